@@ -675,44 +675,46 @@ __global__ __launch_bounds__(256) void blend_count_kernel(BlendArgs a)
 
 // ---- backward (K/cuda_rasterizer_hgs/backward.cu:415-622) ---------------------------------------
 // Each wavefront walks, back to front, the entries the forward filed for its strip, starting at
-// the last one that any of its 64 pixels blended.  The pass is split in two so that no
-// cross-lane reduction is needed per entry:
+// the last one that any of its 64 pixels blended, eight entries at a time.  The pass is split in two so
+// that no cross-lane reduction is needed per entry:
 //  * pixel-parallel part (lane = pixel, as in the forward): the per-pixel recurrences of the
 //    reference loop give, for an entry, two numbers per pixel: u = G dL/dalpha-term and
 //    aT = alpha T.  They are parked in one LDS row per entry.
-//  * entry-parallel part, run whenever 8 rows are full (lane = (entry, strip row, half of the row)):
+//  * entry-parallel part (lane = (entry, strip row, half of the row)):
 //    each lane sweeps 8 pixels and accumulates sum u, sum u dx, sum u dx^2 and
 //    sum aT g_{r,g,b,depth}; dy is constant along a strip row, so the y moments follow from
 //    those; three exchanges inside each group of eight lanes finish the sums, and the group adds its
 //    entry's ten sums into the Gaussian's row of `sums`, eight neighbouring columns in one atomic
-//    instruction and the last two in another.  Eight rows rather than sixteen keep the wavefront's
-//    LDS under 10 KB, which is what lets sixteen of them share a CU.
+//    instruction and the last two in another.
 // All ten sums of the reference (mean2D x/y, conic xx/xy/yy, opacity, colour r/g/b, depth)
 // are linear in u and aT, which is what makes the split possible.
+// (The sums as one product of the eight entries' sixteen rows with a 64 x 10 matrix of pixel moments and upstream
+// gradients, sixteen 16x16x4 matrix instructions in fp32, were built and measured: 0.60 -> 0.66 ms at 1600x1036 with
+// 5.6 M Gaussians.  The fp32 matrix instructions take their time from the vector instructions of the SIMD's other
+// wavefronts, and 512 cycles per eight entries is more than the sweep needs; bf16 ones, which would not, need three
+// terms per factor for the same precision, and splitting them costs what the sweep does.)
 
-constexpr int kRows = 8;      // entries gathered before the entry-parallel part runs
-// Pixel p of the strip sits in column p + (p >> 4) of a row of kRowStride (u, alpha T) pairs, and its four upstream
-// gradients in element p + (p >> 3) of their array: the LDS has 32 banks of 4 bytes, an 8-byte access is served 16
-// lanes at a time and a 16-byte access 8 lanes at a time, and with these numbers neither the per-pixel writes nor
+constexpr int kRows = 8;      // entries per entry-parallel part
+// Pixel p of the strip sits in column p + (p >> 4) of a row of kRowStride (u, alpha T) pairs: the LDS has 32 banks of 4
+// bytes, an 8-byte access is served 16 lanes at a time, and with these numbers neither the per-pixel writes nor
 // the per-(entry, strip row, half row) reads below hit a bank twice within such a group.
 constexpr int kRowStride = 68;
 __device__ __forceinline__ int row_column(int pixel) { return pixel + (pixel >> 4); }
-__device__ __forceinline__ int upstream_column(int pixel) { return pixel + (pixel >> 3); }
 
 struct BackwardPixel {
 	float T;
-	float behind;  // what lies behind the entry being visited, weighted with the upstream gradient: see backward_visit
+	float behind;  // what lies behind the entry being visited, weighted with the upstream gradient: see backward_rows
 	float g_r, g_g, g_b, g_depth, g_alpha;
 };
 
 struct BackwardStage {  // wave-private
-	float4 geom[kChunk + 3];  // + padding up to a multiple of four entries
-	float4 conic[kChunk + 3];  // staged_conic(): -xx / 2, -xy, -yy / 2, opacity
-	float4 cd[kChunk];
-	uint32_t entry[kChunk + 3];  // 0-based position in the tile list
-	uint32_t id[kChunk];
+	float4 geom[kChunk + kRows - 1];   // + padding up to a multiple of eight entries
+	float4 conic[kChunk + kRows - 1];  // staged_conic(): -xx / 2, -xy, -yy / 2, opacity
+	float4 cd[kChunk + kRows - 1];
+	uint32_t entry[kChunk + kRows - 1];  // 0-based position in the tile list
+	uint32_t id[kChunk + kRows - 1];
 	float2 u_at[kRows * kRowStride];  // [row][row_column(pixel)]: (u, alpha T)
-	float4 upstream[72];              // dL/dpixel r, g, b, depth of the strip's 64 pixels, by upstream_column
+	float g_depth[72];                // upstream gradient of the depth image by pixel, eight of nine words
 };
 
 struct StripFrame {
@@ -727,8 +729,13 @@ __device__ __forceinline__ float dpp_exchange_add(float v)
 	return v + __builtin_bit_cast(float, moved);
 }
 
-// Entry-parallel part for the first `rows` rows.  A 16-lane row of the wavefront serves two entries, e in its low
-// eight lanes and e + 4 in its high eight; lane (h = (lane >> 1) & 3, half = lane & 1) of the eight
+// The upstream colour gradients of the eight pixels that a lane sweeps in the entry-parallel part: the same for the whole walk.
+struct SweepUpstream {
+	float r[8], g[8], b[8];   // (those of the depth image, where there are any, stay in LDS: BackwardStage::g_depth)
+};
+
+// Entry-parallel part for the eight entries staged from slot0 on.  A 16-lane row of the wavefront serves two entries, e in
+// its low eight lanes and e + 4 in its high eight; lane (h = (lane >> 1) & 3, half = lane & 1) of the eight
 // sums the entry's row over the 8 pixels of one half of strip row h; the eight lanes of an entry then add up what
 // they hold (three exchanges inside their group of eight) and the entry's ten sums go into the Gaussian's
 // row of `sums` with one atomic instruction: the entry's own lanes add columns 0-7, two lanes of the other eight of
@@ -736,43 +743,35 @@ __device__ __forceinline__ float dpp_exchange_add(float v)
 // (Adding columns 0-7 of all eight entries first and columns 8-9 after them, which needs no exchange between the
 // groups, had every request of the second instruction hit a cache line that one of the first was still at work on:
 // measured, that second instruction cost eight times what the first did, a fifth of the kernel's time.)
-// `row_slots` holds, one byte per row, which staged entry of the current chunk the row belongs to: the entry's centre,
-// conic and Gaussian are read from where the chunk was staged (so the rows are flushed before the next chunk is).
+// The x moments are taken about the lane's first pixel, with constants for factors, and moved to the entry's centre once.
 // kDepth: a gradient arrived for the depth image (without one, the usual case of a loss on the colour image alone, the
 // terms it multiplies are left out: the depth column of `sums` stays zero).
 template <bool kDepth>
-__device__ __forceinline__ void flush_rows(const BackwardStage& st, int rows, uint64_t row_slots, const StripFrame& f,
-                                           const BlendArgs& a, int lane)
+__device__ __forceinline__ void sum_rows(const BackwardStage& st, int slot0, int entries, const SweepUpstream& upstream,
+                                         const StripFrame& f, const BlendArgs& a, int lane)
 {
 #pragma clang fp contract(fast)
 	__builtin_amdgcn_wave_barrier();
 	const int upper = (lane >> 3) & 1;  // which eight of the 16-lane row
 	const int e = (lane >> 4) + 4 * upper, h = (lane >> 1) & 3, half = lane & 1, j = lane & 7;
-	const int slot = (int)((row_slots >> (8 * e)) & 0xFFull);
-	const float4 centre = st.geom[slot];
-	const float2 xy = {centre.x, centre.y};
-	const float dy = xy.y - (f.y0 + (float)h);
-	const float x_first = f.x0 + (float)(8 * half);
-	float s0 = 0.f, sx = 0.f, sxx = 0.f, cr = 0.f, cg = 0.f, cb = 0.f, cdp = 0.f;
-	const int col0 = row_column(h * 16 + 8 * half);
-	const float2* row = st.u_at + e * kRowStride + col0;
-	const float4* upstream = st.upstream + upstream_column(h * 16 + 8 * half);
+	const int slot = slot0 + e;
+	const float2* row = st.u_at + e * kRowStride + row_column(h * 16 + 8 * half);
+	float s0 = 0.f, s1 = 0.f, s2 = 0.f, cr = 0.f, cg = 0.f, cb = 0.f, cdp = 0.f;
 #pragma unroll
 	for (int step = 0; step < 8; step++) {
 		const float2 ua = row[step];
-		const float4 g = upstream[step];
-		const float uu = ua.x, tt = ua.y;
-		const float dx = xy.x - (x_first + (float)step);
-		const float t = uu * dx;
-		s0 += uu;
-		sx += t;
-		sxx += t * dx;
-		cr += tt * g.x;
-		cg += tt * g.y;
-		cb += tt * g.z;
+		s0 += ua.x;
+		s1 += (float)step * ua.x;
+		s2 += (float)(step * step) * ua.x;
+		cr += ua.y * upstream.r[step];
+		cg += ua.y * upstream.g[step];
+		cb += ua.y * upstream.b[step];
 		if (kDepth)
-			cdp += tt * g.w;
+			cdp += ua.y * st.g_depth[9 * (lane & 7) + step];
 	}
+	const float4 centre = st.geom[slot];
+	const float dx = centre.x - (f.x0 + (float)(8 * half)), dy = centre.y - (f.y0 + (float)h);
+	const float sx = dx * s0 - s1, sxx = dx * sx - (dx * s1 - s2);
 	// the two halves of the strip row first (dy is theirs in common), then the four strip rows
 	float w[7] = {s0, sx, sxx, cr, cg, cb, cdp};
 #pragma unroll
@@ -784,22 +783,21 @@ __device__ __forceinline__ void flush_rows(const BackwardStage& st, int rows, ui
 		v[q] = dpp_exchange_add<0x4E>(v[q]);   // quad_perm:[2,3,0,1]
 		v[q] = dpp_exchange_add<0x141>(v[q]);  // row_half_mirror: the other quad of the eight
 	}
-	// (every lane forms all five products and then picks its own: a handful of multiplications more than the one or
-	// two a lane needs, but no branch per column and no wait for the conic inside one)
+	// (every lane forms all five products and then picks its own: a handful of multiplications more than the one or two
+	// a lane needs, but no branch per column and no wait for the conic inside one)
 	const float4 co = st.conic[slot];  // the staged conic: -xx / 2, -xy, -yy / 2, opacity
-	const uint32_t id = e < rows ? st.id[slot] : 0u;
+	const uint32_t id = st.id[slot];
 	const float S0 = v[0], Sx = v[1], Sy = v[2], Sxx = v[3], Sxy = v[4], Syy = v[5];
-	const float m0 = co.w * f.ddelx_dx * (2.f * co.x * Sx + co.y * Sy);
-	const float m1 = co.w * f.ddely_dy * (2.f * co.z * Sy + co.y * Sx);
 	const float half_w = -0.5f * co.w;
+	const float m0 = co.w * f.ddelx_dx * (2.f * co.x * Sx + co.y * Sy), m1 = co.w * f.ddely_dy * (2.f * co.z * Sy + co.y * Sx);
 	const float k0 = half_w * Sxx, k1 = half_w * Sxy, k3 = half_w * Syy;
 	// lane j of the eight holds column j of the row, lanes 0 and 1 also columns 8 and 9: see SumCol
-	float first = j == 0 ? m0 : j == 1 ? m1 : j == 2 ? k0 : j == 3 ? k1 : j == 4 ? k3 : j == 5 ? S0 : j == 6 ? v[6] : v[7];
-	float second = j == 0 ? v[8] : j == 1 ? v[9] : 0.f;
-	if (!(e < rows)) {
-		first = 0.f;
-		second = 0.f;
-	}
+	// (picked bit by bit of j: a chain of comparisons becomes a switch)
+	const bool j0 = (j & 1) != 0, j1 = (j & 2) != 0, j2 = (j & 4) != 0, counts = e < entries;
+	const float c01 = j0 ? m1 : m0, c23 = j0 ? k1 : k0, c45 = j0 ? S0 : k3, c67 = j0 ? v[7] : v[6];
+	const float c03 = j1 ? c23 : c01, c47 = j1 ? c67 : c45;
+	const float c89 = j0 ? (kDepth ? v[9] : 0.f) : v[8];
+	const float first = counts ? (j2 ? c47 : c03) : 0.f, second = counts && !j1 && !j2 ? c89 : 0.f;
 	// columns 8 and 9 and the Gaussian's index go to the same lanes of the other eight of the 16-lane row (row_ror:8)
 	const float second_there = __builtin_bit_cast(
 		float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, second), 0x128, 0xF, 0xF, true));
@@ -819,62 +817,77 @@ __device__ __forceinline__ void flush_rows(const BackwardStage& st, int rows, ui
 	__builtin_amdgcn_wave_barrier();
 }
 
-// Pixel-parallel part for one entry; `rows` (wave-uniform) counts the LDS rows in use.
-template <bool kDepth>
-__device__ __forceinline__ void backward_visit(BackwardPixel& p, uint64_t candidates, float power, const float4 g,
-                                               const float4 co, BackwardStage& st, int slot, int& rows, uint64_t& row_slots,
-                                               const StripFrame& f, const PixelRay& ray, const BlendArgs& a, int lane)
+// Pixel-parallel part for the four entries staged from slot k on; their rows are those from `row` on.  Returns whether
+// any pixel blended any of them.
+template <bool kDepth, bool kBoxed>
+__device__ __forceinline__ bool backward_rows(BackwardPixel& p, uint32_t last_contributor, BackwardStage& st, int k, int row,
+                                              const float2 pixf, const PixelRay& ray, const BoxFrame& box, int lane)
 {
-	if (candidates == 0ull)
-		return;
-	// Every lane evaluates alpha (an instruction costs the wavefront the same whatever its lanes); the decisions are
-	// lane masks, and one masked region holds what only a blended sample computes.
-	const float4 cd = st.cd[slot];  // asked for ahead of its use in the masked region: the wait falls behind the exp
-	const float G = exp_of_exponent(power);
-	const float alpha = fminf(0.99f, co.w * G);
-	uint64_t blended = candidates & lanes_where(!(alpha < 1.0f / 255.0f));
-	// the box and the inverse projection are read where they are needed (few strips straddle a face of their
-	// box): kept in scalar registers for the whole walk they crowd out the candidate masks of a step
-	const float clip_w = g.w;  // the same for every lane; NaN: the whole strip is inside the box
-	if (lanes_where(clip_w == clip_w) != 0ull)
-		blended &= lanes_where(!clipped_by_box(ray, clip_w, load_box_frame(a)));
-	if (blended == 0ull)
-		return;
-	float u = 0.f, aT = 0.f;
-	if (__builtin_amdgcn_inverse_ballot_w64(blended)) {
-		// From here on nothing feeds a decision: gradients are compared by tolerance, so the
-		// compiler may contract multiply-adds and the divisions use the hardware reciprocal.
-#pragma clang fp contract(fast)
-		const float inv_one_minus_alpha = __builtin_amdgcn_rcpf(1.f - alpha);
-		p.T = p.T * inv_one_minus_alpha;
-		aT = alpha * p.T;
-		// The pixel's outputs are sums over its blended entries j of w_j (colour_j, depth_j, 1) with w_j = alpha_j T_j,
-		// T_j the product of (1 - alpha_k) over the entries in front, plus T_final times the background.  Their
-		// derivative with respect to alpha_i is T_i (colour_i, depth_i, 1) minus (the sum over the entries behind i +
-		// T_final background) / (1 - alpha_i).  The reference carries that sum per channel and per unit of transmittance
-		// (K/cuda_rasterizer_hgs/backward.cu:568-599: accum_rec = last_alpha * last_color + (1 - last_alpha) * accum_rec,
-		// and the background term apart); only its product with the upstream gradient is needed, so one number per
-		// pixel does for all channels: `behind` = sum over the entries behind of w_j <g, (colour_j, depth_j, 1)> +
-		// T_final <g, background>, started with the latter.  Same quantity, a third of the arithmetic.
-		float weighted = __builtin_fmaf(cd.x, p.g_r, __builtin_fmaf(cd.y, p.g_g, __builtin_fmaf(cd.z, p.g_b, p.g_alpha)));
+	float power[4], clip_w[4], opacity[4];
+	uint64_t mask[4];
+#pragma unroll
+	for (int i = 0; i < 4; i++) {
+		const float4 g = st.geom[k + i];
+		const float4 co = st.conic[k + i];
+		power[i] = exponent_of_staged(g, co, pixf);
+		clip_w[i] = g.w;
+		opacity[i] = co.w;
+		// (each mask from single comparisons: a comparison's result is the mask; nearly every walked entry is blended
+		// by some pixel, so the exponent's floor, which would spare an exponential now and then, is not looked at)
+		mask[i] = lanes_where(st.entry[k + i] < last_contributor) & lanes_where(!(power[i] > 0.0f));
+	}
+	// the entries' colours are asked for ahead of the exponentials
+	float4 cd[4];
+#pragma unroll
+	for (int i = 0; i < 4; i++)
+		cd[i] = st.cd[k + i];
+	__builtin_amdgcn_sched_barrier(0);
+	float alpha[4], G[4], inv[4], weighted[4], u[4], aT[4];
+#pragma unroll
+	for (int i = 0; i < 4; i++) {
+		G[i] = exp_of_exponent(power[i]);
+		alpha[i] = fminf(0.99f, opacity[i] * G[i]);
+		mask[i] &= lanes_where(!(alpha[i] < 1.0f / 255.0f));
+		// (an entry that has the whole strip inside the box carries a NaN: never clipped)
+		if (kBoxed && (mask[i] & lanes_where(clip_w[i] == clip_w[i])) != 0ull)
+			mask[i] &= ~lanes_where(clipped_by_box(ray, clip_w[i], box));
+		// From here on nothing feeds a decision: gradients are compared by tolerance, so the divisions use the hardware
+		// reciprocal.
+		inv[i] = __builtin_amdgcn_rcpf(1.f - alpha[i]);
+		weighted[i] = __builtin_fmaf(cd[i].x, p.g_r, __builtin_fmaf(cd[i].y, p.g_g, __builtin_fmaf(cd[i].z, p.g_b, p.g_alpha)));
 		if (kDepth)
-			weighted = __builtin_fmaf(cd.w, p.g_depth, weighted);
-		const float dL_dopa = weighted * p.T - p.behind * inv_one_minus_alpha;
-		p.behind = __builtin_fmaf(aT, weighted, p.behind);
-		u = G * dL_dopa;
+			weighted[i] = __builtin_fmaf(cd[i].w, p.g_depth, weighted[i]);
+		u[i] = aT[i] = 0.f;
 	}
-	st.u_at[rows * kRowStride + row_column(lane)] = float2{u, aT};
-	row_slots |= (uint64_t)slot << (8 * rows);
-	rows++;
-	if (rows == kRows) {
-		flush_rows<kDepth>(st, kRows, row_slots, f, a, lane);
-		rows = 0;
-		row_slots = 0ull;
+	// The pixel's outputs are sums over its blended entries j of w_j (colour_j, depth_j, 1) with w_j = alpha_j T_j,
+	// T_j the product of (1 - alpha_k) over the entries in front, plus T_final times the background.  Their
+	// derivative with respect to alpha_i is T_i (colour_i, depth_i, 1) minus (the sum over the entries behind i +
+	// T_final background) / (1 - alpha_i).  The reference carries that sum per channel and per unit of transmittance
+	// (K/cuda_rasterizer_hgs/backward.cu:568-599: accum_rec = last_alpha * last_color + (1 - last_alpha) * accum_rec,
+	// and the background term apart); only its product with the upstream gradient is needed, so one number per
+	// pixel does for all channels: `behind` = sum over the entries behind of w_j <g, (colour_j, depth_j, 1)> +
+	// T_final <g, background>, started with the latter.
+	// Under the mask of the pixels that blend the entry, written out: the compiler would put a branch around each of the
+	// four (all 64 lanes are active around it; the mask's move is also the instruction that has to lie between a
+	// reciprocal and the first use of it).
+#pragma unroll
+	for (int i = 0; i < 4; i++) {
+		float dL_dopa;
+		asm("s_mov_b64 exec, %[lanes]\n\t"
+		    "v_mul_f32 %[T], %[T], %[inv]\n\t"
+		    "v_mul_f32 %[d], %[behind], %[inv]\n\t"
+		    "v_mul_f32 %[aT], %[alpha], %[T]\n\t"
+		    "v_fma_f32 %[d], %[weighted], %[T], -%[d]\n\t"
+		    "v_fmac_f32 %[behind], %[aT], %[weighted]\n\t"
+		    "v_mul_f32 %[u], %[G], %[d]\n\t"
+		    "s_mov_b64 exec, -1"
+		    : [T] "+v"(p.T), [behind] "+v"(p.behind), [aT] "+v"(aT[i]), [u] "+v"(u[i]), [d] "=&v"(dL_dopa)
+		    : [lanes] "s"(mask[i]), [inv] "v"(inv[i]), [alpha] "v"(alpha[i]), [weighted] "v"(weighted[i]), [G] "v"(G[i]));
+		st.u_at[(row + i) * kRowStride + row_column(lane)] = float2{u[i], aT[i]};
 	}
+	return (mask[0] | mask[1] | mask[2] | mask[3]) != 0ull;
 }
 
-// 128 registers and under 10 KB of LDS: four wavefronts per SIMD (three, as the compiler chooses by itself, were
-// measured 19 % slower; five spill)
 template <bool kDepth>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void blend_backward_kernel(BlendBatch batch)
 {
@@ -923,9 +936,23 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 		p.g_alpha = a.dL_dalpha ? a.dL_dalpha[pix_id] : 0.f;
 	}
 	p.behind = T_final * ((0.f + a.bg[0] * p.g_r + a.bg[1] * p.g_g) + a.bg[2] * p.g_b);
-	st.upstream[upstream_column(lane)] = float4{p.g_r, p.g_g, p.g_b, p.g_depth};
-	int rows = 0;
-	uint64_t row_slots = 0ull;
+
+	SweepUpstream upstream;
+	{
+		float4* by_pixel = st.geom;  // (not in use yet)
+		by_pixel[lane] = float4{p.g_r, p.g_g, p.g_b, 0.f};
+		if (kDepth)
+			st.g_depth[lane + (lane >> 3)] = p.g_depth;
+		__builtin_amdgcn_wave_barrier();
+#pragma unroll
+		for (int s = 0; s < 8; s++) {
+			const float4 g = by_pixel[8 * (lane & 7) + s];  // pixels of strip row (lane >> 1) & 3, half lane & 1
+			upstream.r[s] = g.x;
+			upstream.g[s] = g.y;
+			upstream.b[s] = g.z;
+		}
+		__builtin_amdgcn_wave_barrier();
+	}
 
 	// Lane l of the chunk that starts `first` entries from the back takes filed entry
 	// filed-1-first-l: its list position (and box flag), through that the Gaussian's index,
@@ -952,11 +979,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 			st.entry[lane] = pos_cur & kPosition;
 			st.id[lane] = cur.id;
 		}
-		if (lane < 3) {  // pad to a multiple of four with entries that never pass the floor test
-			st.geom[count + lane] = float4{0.f, 0.f, INFINITY, 0.f};
+		if (lane < kRows - 1) {  // pad to a multiple of eight with entries behind every pixel's last one
+			st.geom[count + lane] = float4{0.f, 0.f, 0.f, 0.f};
 			st.conic[count + lane] = float4{0.f, 0.f, 0.f, 0.f};
+			st.cd[count + lane] = float4{0.f, 0.f, 0.f, 0.f};
 			st.entry[count + lane] = 0xFFFFFFFFu;
+			st.id[count + lane] = 0u;
 		}
+		const bool boxed = lanes_where(lane < count && (pos_cur & 0x80000000u) == 0u) != 0ull;
 		__builtin_amdgcn_wave_barrier();
 		// the chunk is in LDS now: its registers take the next chunk's records, loaded during the walk
 		cur = load_record(a, id_next, pos_next != kNone);
@@ -966,29 +996,22 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 		const uint32_t e3 = first + 192 + (uint32_t)lane;
 		pos_after = e3 < filed ? filed_list[filed - 1 - e3] : kNone;
 
-		for (int k = 0; k < count; k += 4) {
-			const float4 g0 = st.geom[k], g1 = st.geom[k + 1], g2 = st.geom[k + 2], g3 = st.geom[k + 3];
-			const float4 c0 = st.conic[k], c1 = st.conic[k + 1], c2 = st.conic[k + 2], c3 = st.conic[k + 3];
-			const uint32_t p0 = st.entry[k], p1 = st.entry[k + 1], p2 = st.entry[k + 2], p3 = st.entry[k + 3];
-			const float w0 = exponent_of_staged(g0, c0, pixf), w1 = exponent_of_staged(g1, c1, pixf),
-			            w2 = exponent_of_staged(g2, c2, pixf), w3 = exponent_of_staged(g3, c3, pixf);
-			// Each entry's candidates are formed right where its visit looks at them: nearly every walked entry has
-			// some, so a test for the four together would save little.  Each mask comes from single comparisons (a
-			// comparison's result is the mask; that of a combined flag is formed through a register).
-			backward_visit<kDepth>(p, lanes_where(p0 < last_contributor) & lanes_where(!(w0 > 0.0f)) & lanes_where(!(w0 < g0.z)), w0,
-			                       g0, c0, st, k, rows, row_slots, frame, ray, a, lane);
-			backward_visit<kDepth>(p, lanes_where(p1 < last_contributor) & lanes_where(!(w1 > 0.0f)) & lanes_where(!(w1 < g1.z)), w1,
-			                       g1, c1, st, k + 1, rows, row_slots, frame, ray, a, lane);
-			backward_visit<kDepth>(p, lanes_where(p2 < last_contributor) & lanes_where(!(w2 > 0.0f)) & lanes_where(!(w2 < g2.z)), w2,
-			                       g2, c2, st, k + 2, rows, row_slots, frame, ray, a, lane);
-			backward_visit<kDepth>(p, lanes_where(p3 < last_contributor) & lanes_where(!(w3 > 0.0f)) & lanes_where(!(w3 < g3.z)), w3,
-			                       g3, c3, st, k + 3, rows, row_slots, frame, ray, a, lane);
-		}
-		// the rows point into this chunk's staged entries: they go before the next chunk takes their place
-		if (rows > 0) {
-			flush_rows<kDepth>(st, rows, row_slots, frame, a, lane);
-			rows = 0;
-			row_slots = 0ull;
+		// (few strips straddle a face of their box: their chunks run a copy of the loop that has the test)
+		if (boxed) {
+			const BoxFrame box = load_box_frame(a);
+			for (int k = 0; k < count; k += kRows) {
+				const bool front = backward_rows<kDepth, true>(p, last_contributor, st, k, 0, pixf, ray, box, lane);
+				const bool back = backward_rows<kDepth, true>(p, last_contributor, st, k + 4, 4, pixf, ray, box, lane);
+				if (front || back)
+					sum_rows<kDepth>(st, k, count - k, upstream, frame, a, lane);
+			}
+		} else {
+			for (int k = 0; k < count; k += kRows) {
+				const bool front = backward_rows<kDepth, false>(p, last_contributor, st, k, 0, pixf, ray, BoxFrame{}, lane);
+				const bool back = backward_rows<kDepth, false>(p, last_contributor, st, k + 4, 4, pixf, ray, BoxFrame{}, lane);
+				if (front || back)
+					sum_rows<kDepth>(st, k, count - k, upstream, frame, a, lane);
+			}
 		}
 		__builtin_amdgcn_wave_barrier();
 	}
