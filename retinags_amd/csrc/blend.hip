@@ -23,9 +23,9 @@
 // 8-pixel-wide half of the strip, the entries whose ellipse reaches that half, and the lanes of
 // each half walk their own packed entries side by side (as many steps as the longer of the two).
 //
-// Inside the walk, alpha >= 1/255 needs power >= -ln(255 * opacity); that floor (minus a margin) is
-// stored with the Gaussian, and a group of four entries is skipped with one ballot when no live
-// lane reaches it, before exp() is evaluated.
+// (Inside the walk the floor power >= -ln(255 * opacity), which alpha >= 1/255 needs and the packing uses, is not looked at
+// again: skipping a group of four entries that no live lane reaches, before exp() is evaluated, was measured to cost more
+// than it saves once the walk had no other branches: 0.313 -> 0.289 ms without it at 1600x1036 with 5.6 M Gaussians.)
 #include "rgs_kernels.h"
 #include "strip_filing.h"
 #include "tile_order.h"
@@ -35,6 +35,22 @@ namespace rgs {
 struct PixelRay {
 	float ndc_x, ndc_y;  // pixel centre in NDC
 };
+
+// NDC of a strip's pixel columns and rows, in LDS: only chunks that straddle a face of the box use them, and in registers
+// they would cost the walks of all others two.
+struct StripRays {
+	float x[16], y[4];
+};
+__device__ __forceinline__ void stage_rays(StripRays& r, const float2 pixf, const BlendArgs& a, int lane)
+{
+	r.x[lane & 15] = pix_to_ndc(pixf.x, a.W);  // (four lanes write the same value)
+	r.y[lane >> 4] = pix_to_ndc(pixf.y, a.H);
+}
+__device__ __forceinline__ PixelRay ray_of(const StripRays& r)
+{
+	const int lane = threadIdx.x & 63;
+	return PixelRay{r.x[lane & 15], r.y[lane >> 4]};
+}
 
 __device__ __forceinline__ BoxFrame load_box_frame(const BlendArgs& a)
 {
@@ -50,6 +66,52 @@ __device__ __forceinline__ bool clipped_by_box(const PixelRay& ray, float w, con
 	const float wy = b.m[0][1] * ph.x + b.m[1][1] * ph.y + b.m[2][1] * ph.z + b.m[3][1];
 	const float wz = b.m[0][2] * ph.x + b.m[1][2] * ph.y + b.m[2][2] * ph.z + b.m[3][2];
 	return (wx <= b.lo.x) || (wx > b.hi.x) || (wy <= b.lo.y) || (wy > b.hi.y) || (wz <= b.lo.z) || (wz > b.hi.z);
+}
+
+// The clip w, all positive, between which clipped_by_box() lets a sample of a pixel's ray pass: at none outside of
+// [from, to], at all inside of (from_sure, to_sure).  The ray sample's world coordinates are affine in clip w, slope w +
+// offset, so each face of the box bounds w on one side; slope and offset get room for the rounding of the exact test (about
+// seven roundings of half a unit each, relative to the terms and not to their possibly cancelling sum) and of this one.
+// Four comparisons with it replace the exact test, which is as long as all the rest of a visit, for nearly every sample.
+struct BoxSpan {
+	float from, to, from_sure, to_sure;
+};
+
+__device__ __forceinline__ BoxSpan w_inside_box(const PixelRay& ray, const BoxFrame& b)
+{
+	const float rx = ray.ndc_x * b.tanx, ry = ray.ndc_y * b.tany;
+	const float lo[3] = {b.lo.x, b.lo.y, b.lo.z}, hi[3] = {b.hi.x, b.hi.y, b.hi.z};
+	BoxSpan s = {0.f, INFINITY, 0.f, INFINITY};
+#pragma unroll
+	for (int k = 0; k < 3; k++) {
+		const float t0 = b.m[0][k] * rx, t1 = b.m[1][k] * ry, t2 = b.m[2][k], offset = b.m[3][k];
+		const float slope = t0 + t1 + t2, room = 2e-6f * (fabsf(t0) + fabsf(t1) + fabsf(t2));
+		const float room_offset = 2e-6f * fabsf(offset);
+		// slope w > lo - offset and, mirrored, -slope w > -(hi - offset)
+#pragma unroll
+		for (int side = 0; side < 2; side++) {
+			const float rise = side ? -slope : slope, need = side ? offset - hi[k] : lo[k] - offset;
+			const float rise_p = rise + room, rise_s = rise - room;
+			const float at_p = (need - room_offset) * __builtin_amdgcn_rcpf(rise_p);
+			const float at_s = (need + room_offset) * __builtin_amdgcn_rcpf(rise_s);
+			s.from = fmaxf(s.from, rise_p > 0.f ? at_p : 0.f);
+			s.to = fminf(s.to, rise_p < 0.f ? at_p : INFINITY);
+			s.from_sure = fmaxf(s.from_sure, rise_s > 0.f ? at_s : rise_s < 0.f ? 0.f : INFINITY);
+			s.to_sure = fminf(s.to_sure, rise_s < 0.f ? at_s : INFINITY);
+		}
+	}
+	return BoxSpan{s.from * 0.9999f, s.to * 1.0001f, s.from_sure * 1.0001f, s.to_sure * 0.9999f};
+}
+
+// The lanes among `lanes` whose sample at clip w the box does not clip (a NaN, which marks an entry that has the whole
+// strip inside the box: all of them).
+__device__ __forceinline__ uint64_t lanes_inside_box(uint64_t lanes, float w, const BoxSpan& s, const StripRays& rays, const BlendArgs& a)
+{
+	lanes &= ~(lanes_where(w < s.from) | lanes_where(w > s.to));
+	const uint64_t unsure = lanes & (lanes_where(w <= s.from_sure) | lanes_where(w >= s.to_sure));
+	if (unsure != 0ull)
+		lanes &= ~lanes_where(clipped_by_box(ray_of(rays), w, load_box_frame(a)));
+	return lanes;
 }
 
 // exp(x) for the exponents of the blend (-6 < x <= 0 where the result is used): 2^(x log2 e) on the hardware exp2 unit.
@@ -279,8 +341,11 @@ struct ForwardSlot {
 struct ForwardStage {  // one per workgroup (a single wavefront)
 	// The chunk's entries once per 8-pixel-wide half of the strip they can reach, each half's packed to the front, so
 	// that a step's reads are at addresses known when the step begins (and from one base):
-	ForwardSlot slot[2][kChunk + 3];
-	uint8_t entry[2][kChunk + 4]; // which entry of the chunk a packed slot holds
+	ForwardSlot slots[2 * kChunk + 1];  // of half h from h (kChunk + 1) on: one apart, or both halves' reads would meet in the same banks
+	__device__ __forceinline__ ForwardSlot* slot(int half) { return slots + half * (kChunk + 1); }
+	__device__ __forceinline__ const ForwardSlot* slot(int half) const { return slots + half * (kChunk + 1); }
+	uint8_t entry[2][kChunk];     // which entry of the chunk a packed slot holds
+	StripRays rays;
 };
 
 // Adds a sample to the pixels of `lanes`: one product alpha T (`weight`) and a fused multiply-add per channel instead
@@ -308,43 +373,59 @@ __device__ __forceinline__ void blend_sample(ForwardPixel& p, uint64_t lanes, fl
 // Instructions that only some entries need are few (most visited entries blend somewhere), while a branch per entry
 // had the wavefront wait for its scalar masks four times a group: a walk alone on its SIMD advanced at 280 cycles per
 // entry, two and a half times what issuing its instructions takes.
-template <bool kBoxed>
-__device__ __forceinline__ void forward_group(ForwardPixel& p, uint64_t& live, const ForwardStage& st, int half, int k,
-                                              const float2 pixf, const PixelRay& ray, const BoxFrame& box)
-{
-	const ForwardSlot* slot = st.slot[half] + k;
-	float power[4], clip_w[4], opacity[4];
+struct FourEntries {
+	float power[4], clip_w[4], opacity[4], alpha[4];
 	uint64_t mask[4];
+};
+
+// What four slots hold, read ahead of its use: left to itself the compiler puts each read in front of the entry that
+// needs it, and a wavefront that is alone on its SIMD then waits for LDS four times.
+struct FourSlots {
+	float4 geom[4], conic[4];
+};
+__device__ __forceinline__ FourSlots read_four(const ForwardSlot* slot)
+{
+	FourSlots r;
 #pragma unroll
 	for (int i = 0; i < 4; i++) {
-		const float4 g = slot[i].geom;
-		const float4 co = slot[i].conic;
-		power[i] = exponent_of_staged(g, co, pixf);
-		clip_w[i] = g.w;
-		opacity[i] = co.w;
-		// written with negations so that a NaN exponent is kept, as in the exact loop; each mask from single
-		// comparisons (a comparison's result is the mask; that of a combined flag is formed through a register)
-		mask[i] = lanes_where(!(power[i] > 0.0f)) & lanes_where(!(power[i] < g.z));
+		r.geom[i] = slot[i].geom;
+		r.conic[i] = slot[i].conic;
 	}
-	if (((mask[0] | mask[1] | mask[2] | mask[3]) & live) == 0ull)
-		return;
-	// the entries' colours are asked for ahead of the exponentials and used behind the transmittances
-	float4 cd[4];
+	return r;
+}
+
+// The exponent of entry i, and as a mask the lanes that it leaves candidates.
+__device__ __forceinline__ void forward_candidate(FourEntries& e, int i, const float4 geom, const float4 conic, const float2 pixf)
+{
+	e.power[i] = exponent_of_staged(geom, conic, pixf);
+	e.clip_w[i] = geom.w;
+	e.opacity[i] = conic.w;
+	// written with a negation so that a NaN exponent is kept, as in the exact loop; each mask from single
+	// comparisons (a comparison's result is the mask; that of a combined flag is formed through a register)
+	e.mask[i] = lanes_where(!(e.power[i] > 0.0f));
+}
+
+// Alphas, zero where the pixel does not take the entry, and the masks of those that do (as far as alpha and box decide).
+// boxed: some entries of the chunk straddle a face of the box in the strip.
+__device__ __forceinline__ void forward_alphas(FourEntries& e, uint64_t live, bool boxed, const StripRays& rays, const BoxSpan& span,
+                                               const BlendArgs& a)
+{
+#pragma unroll
+	for (int i = 0; i < 4; i++) {
+		e.alpha[i] = fminf(0.99f, e.opacity[i] * exp_of_exponent(e.power[i]));
+		e.mask[i] &= lanes_where(!(e.alpha[i] < 1.0f / 255.0f));
+	}
+	if (boxed)
+#pragma unroll
+		for (int i = 0; i < 4; i++)
+			e.mask[i] = lanes_inside_box(e.mask[i] & live, e.clip_w[i], span, rays, a);
 #pragma unroll
 	for (int i = 0; i < 4; i++)
-		cd[i] = slot[i].cd;
-	__builtin_amdgcn_sched_barrier(0);
-	float alpha[4];
-#pragma unroll
-	for (int i = 0; i < 4; i++) {
-		alpha[i] = fminf(0.99f, opacity[i] * exp_of_exponent(power[i]));
-		mask[i] &= lanes_where(!(alpha[i] < 1.0f / 255.0f));
-		// (an entry that has the whole strip inside the box carries a NaN; few entries of a chunk that straddles a
-		// face of the box are candidates of a live pixel, and the test is as long as all the rest: a branch pays)
-		if (kBoxed && (mask[i] & live & lanes_where(clip_w[i] == clip_w[i])) != 0ull)
-			mask[i] &= ~lanes_where(clipped_by_box(ray, clip_w[i], box));
-		alpha[i] = __builtin_amdgcn_inverse_ballot_w64(mask[i]) ? alpha[i] : 0.f;
-	}
+		e.alpha[i] = __builtin_amdgcn_inverse_ballot_w64(e.mask[i]) ? e.alpha[i] : 0.f;
+}
+
+__device__ __forceinline__ void forward_blend(ForwardPixel& p, const float* alpha, uint64_t* mask, const float4* cd, int slot)
+{
 	float weight[4];
 #pragma unroll
 	for (int i = 0; i < 4; i++) {
@@ -356,7 +437,27 @@ __device__ __forceinline__ void forward_group(ForwardPixel& p, uint64_t& live, c
 	}
 #pragma unroll
 	for (int i = 0; i < 4; i++)
-		blend_sample(p, mask[i], weight[i], cd[i], k + i);
+		blend_sample(p, mask[i], weight[i], cd[i], slot + i);
+}
+
+__device__ __forceinline__ void forward_group(ForwardPixel& p, uint64_t& live, const ForwardStage& st, int half, int k,
+                                              const float2 pixf, bool boxed, const BoxSpan& span, const BlendArgs& a)
+{
+	const ForwardSlot* slot = st.slot(half) + k;
+	FourEntries e;
+	const FourSlots r = read_four(slot);
+	__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+	for (int i = 0; i < 4; i++)
+		forward_candidate(e, i, r.geom[i], r.conic[i], pixf);
+	// the entries' colours are asked for ahead of the exponentials and used behind the transmittances
+	float4 cd[4];
+#pragma unroll
+	for (int i = 0; i < 4; i++)
+		cd[i] = slot[i].cd;
+	__builtin_amdgcn_sched_barrier(0);
+	forward_alphas(e, live, boxed, st.rays, span, a);
+	forward_blend(p, e.alpha, e.mask, cd, k);
 	live = lanes_where(p.T > 0.f);
 }
 
@@ -379,34 +480,6 @@ __device__ __forceinline__ float4 live_box(uint64_t live, int column)
 	              (float)(__builtin_ctzll(mine) >> 4), (float)((63 - __builtin_clzll(mine)) >> 4)};
 }
 
-// Bounds of the clip w at which clipped_by_box() can let a sample of the pixel's ray pass (x > y: at none).  The ray
-// sample's world coordinates are affine in clip w, slope w + from, so each face of the box bounds w on one side; slope and
-// offset get room for the rounding of the exact test (about seven roundings of half a unit each, relative to the terms and
-// not to their possibly cancelling sum) and of this one.  What matters are rays that run along a face, as those of a camera
-// that looks along the plane between two submodels do: they enter, or leave, far from where their neighbours do.
-__device__ __forceinline__ float2 w_inside_box(const PixelRay& ray, const BoxFrame& b)
-{
-	const float rx = ray.ndc_x * b.tanx, ry = ray.ndc_y * b.tany;
-	const float lo[3] = {b.lo.x, b.lo.y, b.lo.z}, hi[3] = {b.hi.x, b.hi.y, b.hi.z};
-	float enter = 0.f, leave = INFINITY;
-#pragma unroll
-	for (int k = 0; k < 3; k++) {
-		const float t0 = b.m[0][k] * rx, t1 = b.m[1][k] * ry, t2 = b.m[2][k], from = b.m[3][k];
-		const float slope = t0 + t1 + t2, room = 2e-6f * (fabsf(t0) + fabsf(t1) + fabsf(t2));
-		const float room_from = 2e-6f * fabsf(from);
-		// (slope + room) w > lo - from - room_from and, mirrored, (-slope + room) w > -(hi - from) - room_from
-#pragma unroll
-		for (int side = 0; side < 2; side++) {
-			const float up = (side ? -slope : slope) + room;
-			const float need = (side ? from - hi[k] : lo[k] - from) - room_from;
-			const float at = need * __builtin_amdgcn_rcpf(up);
-			enter = fmaxf(enter, up > 0.f ? at : 0.f);
-			leave = fminf(leave, up < 0.f ? at : INFINITY);
-		}
-	}
-	return float2{enter * 0.9999f, leave * 1.0001f};
-}
-
 // Per 8-pixel-wide half of the strip (columns: bit 3 of the lane), the largest of its lanes' values, which are not negative
 // (non-negative floats compare like their bits).
 __device__ __forceinline__ uint2 half_max_u32(uint32_t v)
@@ -423,16 +496,118 @@ __device__ __forceinline__ uint2 half_max_u32(uint32_t v)
 	return uint2{(uint32_t)m[0], (uint32_t)m[1]};
 }
 
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 6))) void blend_forward_kernel(BlendBatch batch)
+// Bounds on clip w between which, per half, some pixel that still takes entries can have its sample inside the box.
+struct HalfSpan {
+	float from[2], to[2];
+};
+__device__ __forceinline__ HalfSpan live_w_span(bool takes, const BoxSpan& span)
 {
-	__shared__ ForwardStage st;
+	takes = takes && !(span.from > span.to);
+	// (the smallest entering w through its complement in the order of the bits)
+	const uint2 to = half_max_u32(takes ? __float_as_uint(fmaxf(span.to, 0.f)) : 0u),
+	            from_c = half_max_u32(takes ? 0x7F800000u - __float_as_uint(span.from) : 0u);
+	return HalfSpan{{__uint_as_float(0x7F800000u - from_c.x), __uint_as_float(0x7F800000u - from_c.y)},
+	                {__uint_as_float(to.x), __uint_as_float(to.y)}};
+}
 
-	const int lane = threadIdx.x;
-	// The jobs of a batch (the submodels of a frame) take turns, each handing out its strips longest
-	// list first: a long strip that starts late is what a launch waits for, and with several jobs in one
-	// launch there is other work to run beside the longest strips of each.
-	const BlendArgs& a = batch.job[blockIdx.x % (uint32_t)batch.count];
-	const uint32_t strip_id = a.strip_order_forward[blockIdx.x / (uint32_t)batch.count];
+// Takes the entries that no live pixel can have inside the box out of a chunk whose entries straddle one of its faces in
+// the strip.  False, with nothing done, if one of them lies at a clip w that is not positive: spans do not apply then.
+__device__ __forceinline__ bool prune_by_box(bool straddles, bool takes, float w, const StripRays& rays, const BlendArgs& a,
+                                                bool& left, bool& right)
+{
+	if (lanes_where(straddles && !(w > 0.f)) != 0ull)
+		return false;
+	const HalfSpan h = live_w_span(takes, w_inside_box(ray_of(rays), load_box_frame(a)));
+	if (straddles) {
+		left = left && !(w > h.to[0]) && !(w < h.from[0]);
+		right = right && !(w > h.to[1]) && !(w < h.from[1]);
+	}
+	return true;
+}
+
+// The pixel's span for the visits; one that decides nothing where spans do not apply.
+__device__ __forceinline__ BoxSpan span_for_visits(bool applies, const StripRays& rays, const BlendArgs& a)
+{
+	return applies ? w_inside_box(ray_of(rays), load_box_frame(a)) : BoxSpan{-INFINITY, INFINITY, INFINITY, -INFINITY};
+}
+
+// In which 8-pixel-wide halves of the strip (first pixel x0, ya) an entry's ellipse power >= floor can reach a pixel that
+// still takes entries, by the bounding boxes of the ellipse and of each half's live pixels.  The ellipse's half extents are
+// sqrt(limit c / (a c - b^2)) in x and sqrt(limit a / (a c - b^2)) in y with limit = -2 floor, here with room for the
+// rounding of the exponent the pixels evaluate (relative to its largest terms over the strip) and of the determinant.  An
+// entry outside that box would pass the floor test in none of those pixels, so leaving it out of the half's walk changes no
+// result.  (The rows matter as much as the columns: a ground plane at a grazing angle is made of flat ellipses, and a row
+// of pixels just above the horizon, which nothing fills, kept its strip walking thousands of entries that only its finished
+// rows could see.)
+__device__ __forceinline__ void halves_reached(const LoadedRecord& r, float x0, float ya, const float4 box_l, const float4 box_r,
+                                               bool& left, bool& right)
+{
+	const float ca = r.conic.x, cb = r.conic.y, cc = r.conic.z;
+	const float dxa = r.geom.x - x0, dya = r.geom.y - ya;
+	const float limit = -2.f * r.geom.z;
+	const float far_x = fmaxf(fabsf(dxa), fabsf(dxa - 15.f)), far_y = fmaxf(fabsf(dya), fabsf(dya - 3.f));
+	const float allowed = limit + (1e-3f + 1e-4f * limit + 1e-5f * (ca * far_x * far_x + cc * far_y * far_y));
+	const float det = ca * cc - cb * cb - 1e-6f * ca * cc;
+	float reach_x = INFINITY, reach_y = INFINITY;
+	if ((ca > 0.f) && (cc > 0.f) && (det > 0.f)) {
+		const float scale = allowed * __builtin_amdgcn_rcpf(det);
+		reach_x = __builtin_amdgcn_sqrtf(scale * cc) * 1.001f + 0.01f;
+		reach_y = __builtin_amdgcn_sqrtf(scale * ca) * 1.001f + 0.01f;
+	}
+	// (a NaN, as of a Gaussian whose floor is, excludes nothing)
+	left = !(dxa + reach_x < box_l.x) && !(dxa - reach_x > box_l.y) && !(dya + reach_y < box_l.z) && !(dya - reach_y > box_l.w);
+	right = !(dxa + reach_x < box_r.x) && !(dxa - reach_x > box_r.y) && !(dya + reach_y < box_r.z) && !(dya - reach_y > box_r.w);
+}
+
+constexpr uint32_t kNone = 0xFFFFFFFFu, kPosition = 0x7FFFFFFFu;  // of a filed entry: none, and its list position
+
+// Files an entry in slot `at` of a half.
+__device__ __forceinline__ void stage_slot(ForwardStage& st, int half, uint32_t at, const LoadedRecord& r, uint32_t pos, int entry)
+{
+	float4 g = r.geom;
+	int nan = 0x7FC00000;
+	asm volatile("" : "+v"(nan));  // (made here each time rather than held through the walk)
+	if (pos & 0x80000000u)
+		g.w = __int_as_float(nan);  // the strip lies inside the box: no per-pixel test
+	st.slot(half)[at].geom = g;
+	st.slot(half)[at].conic = staged_conic(r.conic);
+	st.slot(half)[at].cd = r.cd;
+	st.entry[half][at] = (uint8_t)entry;
+}
+
+// A slot that no pixel takes: opacity 0.
+__device__ __forceinline__ void stage_nothing(ForwardStage& st, int half, uint32_t at)
+{
+	float zero = 0.f;
+	asm volatile("" : "+v"(zero));  // (made here each time: four registers held through the walk otherwise)
+	st.slot(half)[at].geom = float4{zero, zero, zero, zero};
+	st.slot(half)[at].conic = float4{zero, zero, zero, zero};
+}
+
+// What a strip's walk leaves: how many of the filed entries the backward has to walk (up to the last one some pixel
+// blended), and the images.  px, py: the lane's pixel.
+__device__ __forceinline__ void forward_finish(const BlendArgs& a, uint32_t strip_id, const ForwardPixel& p, uint32_t filed,
+                                               const uint32_t* filed_list, uint32_t px, uint32_t py, int lane)
+{
+	const uint32_t upto = filed != 0u ? wave_max_u32(p.last_filed) : 0u;  // (zero for a pixel outside the image)
+	if (lane == 0)
+		a.strip_filed[strip_id] = upto;
+	if (px < (uint32_t)a.W && py < (uint32_t)a.H) {
+		const uint32_t pix_id = (uint32_t)a.W * py + px;
+		const size_t plane = (size_t)a.H * a.W;
+		// the reference's n_contrib: the 1-based position in the tile's list of the last entry the pixel blended
+		a.n_contrib[pix_id] = p.last_filed != 0u ? (filed_list[p.last_filed - 1u] & kPosition) + 1u : 0u;
+		a.out_color[pix_id] = p.C0 + fabsf(p.T) * a.bg[0];
+		a.out_color[plane + pix_id] = p.C1 + fabsf(p.T) * a.bg[1];
+		a.out_color[2 * plane + pix_id] = p.C2 + fabsf(p.T) * a.bg[2];
+		a.out_alpha[pix_id] = p.weight;
+		a.out_depth[pix_id] = p.D;
+	}
+}
+
+// One strip by one wavefront.
+__device__ __forceinline__ void forward_strip(const BlendArgs& a, uint32_t strip_id, ForwardStage& st, int lane)
+{
 	const int tile = (int)(strip_id >> 2), wave = (int)(strip_id & 3u);  // wave: which strip of the tile
 	const uint2 range = a.ranges[tile];
 	const uint32_t n = range.y - range.x;
@@ -440,7 +615,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 6))) void
 	const uint32_t px = tx * kTile + (lane & 15), py = ty * kTile + wave * 4 + (lane >> 4);
 	const bool inside = px < (uint32_t)a.W && py < (uint32_t)a.H;
 	const float2 pixf = {(float)px, (float)py};
-	const PixelRay ray = {pix_to_ndc(pixf.x, a.W), pix_to_ndc(pixf.y, a.H)};
 
 	ForwardPixel p = {inside ? 1.0f : -1.0f, 0.f, 0.f, 0.f, 0.f, 0.f, 0u, -1};
 	uint64_t live = lanes_where(inside);
@@ -454,9 +628,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 6))) void
 		__builtin_amdgcn_s_setprio(2);
 
 	if (filed != 0u && live != 0ull) {
+		stage_rays(st.rays, pixf, a, lane);
 		const uint32_t* list = a.point_list + range.x;
 		const uint32_t* filed_list = a.strip_lists + 4 * (size_t)range.x + (size_t)wave * n;
-		constexpr uint32_t kNone = 0xFFFFFFFFu, kPosition = 0x7FFFFFFFu;
 		// Lane l of the chunk that starts at filed entry `first` takes entry first + l: its list
 		// position (and box flag), through that the Gaussian's index, through that its record.
 		// Three chunks are in flight: the records of the next one, the indices of the one after,
@@ -467,136 +641,71 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 6))) void
 		LoadedRecord cur = load_record(a, pos_cur != kNone ? list[pos_cur & kPosition] : 0u, pos_cur != kNone);
 		uint32_t id_next = pos_next != kNone ? list[pos_next & kPosition] : 0u;
 
-		const int half = (lane >> 3) & 1;
-		const float x0 = (float)(tx * kTile), ya = (float)(ty * kTile + wave * 4);
+		const float x0 = wave_uniform((float)(tx * kTile)), ya = wave_uniform((float)(ty * kTile + wave * 4));
 		for (uint32_t first = 0; first < filed && live != 0ull; first += 64) {
 			const int count = (int)min(filed - first, 64u);
-			// In which 8-pixel-wide halves of the strip the entry's ellipse power >= floor can reach a pixel that still
-			// takes entries, by the bounding boxes of the ellipse and of each half's live pixels.  The ellipse's half
-			// extents are sqrt(limit c / (a c - b^2)) in x and sqrt(limit a / (a c - b^2)) in y with limit = -2 floor, here
-			// with room for the rounding of the exponent the pixels evaluate (relative to its largest terms over the
-			// strip) and of the determinant.  An entry outside that box would pass the floor test below in none of those
-			// pixels, so leaving it out of the half's walk changes no result.  (The rows matter as much as the columns: a
-			// ground plane at a grazing angle is made of flat ellipses, and a row of pixels just above the horizon, which
-			// nothing fills, kept its strip walking thousands of entries that only its finished rows could see.)
+			// what follows from the lane's number is worked out per chunk: held through the walk it costs half a dozen registers
+			int l = lane;
+			asm volatile("" : "+v"(l));
+			const int half = (l >> 3) & 1;
 			const float4 box_l = live_box(live, 0), box_r = live_box(live, 8);
 			bool left = false, right = false;
-			if (lane < count) {
-				const float ca = cur.conic.x, cb = cur.conic.y, cc = cur.conic.z;
-				const float dxa = cur.geom.x - x0, dya = cur.geom.y - ya;
-				const float limit = -2.f * cur.geom.z;
-				const float far_x = fmaxf(fabsf(dxa), fabsf(dxa - 15.f)), far_y = fmaxf(fabsf(dya), fabsf(dya - 3.f));
-				const float allowed = limit + (1e-3f + 1e-4f * limit + 1e-5f * (ca * far_x * far_x + cc * far_y * far_y));
-				const float det = ca * cc - cb * cb - 1e-6f * ca * cc;
-				float reach_x = INFINITY, reach_y = INFINITY;
-				if ((ca > 0.f) && (cc > 0.f) && (det > 0.f)) {
-					const float scale = allowed * __builtin_amdgcn_rcpf(det);
-					reach_x = __builtin_amdgcn_sqrtf(scale * cc) * 1.001f + 0.01f;
-					reach_y = __builtin_amdgcn_sqrtf(scale * ca) * 1.001f + 0.01f;
-				}
-				// (a NaN, as of a Gaussian whose floor is, excludes nothing)
-				left = !(dxa + reach_x < box_l.x) && !(dxa - reach_x > box_l.y) && !(dya + reach_y < box_l.z) && !(dya - reach_y > box_l.w);
-				right = !(dxa + reach_x < box_r.x) && !(dxa - reach_x > box_r.y) && !(dya + reach_y < box_r.z) && !(dya - reach_y > box_r.w);
-			}
+			if (l < count)
+				halves_reached(cur, x0, ya, box_l, box_r, left, right);
 			// Entries whose sample the box clips in every pixel of a half that still takes entries are left out too: a
 			// pixel whose ray has left the box, or enters it behind everything, stays unfinished for good, and a strip with
 			// one such pixel walked its list to the end (at 1600x1036 and 5.6 M Gaussians, a camera that looks along a
 			// plane between submodels: one that blends none of its last 2 800 entries walked 3 387; 0.54 ms of launch).
-			const bool straddles = lane < count && (pos_cur & 0x80000000u) == 0u;
+			const bool straddles = l < count && (pos_cur & 0x80000000u) == 0u;
 			const bool boxed = lanes_where(straddles) != 0ull;
-			if (boxed) {
-				const float2 span = w_inside_box(ray, load_box_frame(a));
-				const bool takes = p.T > 0.f && !(span.x > span.y);
-				// first: the smallest entering w, through its complement in the order of the bits
-				const uint2 last = half_max_u32(takes ? __float_as_uint(span.y) : 0u),
-				            first_c = half_max_u32(takes ? 0x7F800000u - __float_as_uint(span.x) : 0u);
-				if (straddles) {
-					left = left && !(cur.geom.w > __uint_as_float(last.x)) && !(cur.geom.w < __uint_as_float(0x7F800000u - first_c.x));
-					right = right && !(cur.geom.w > __uint_as_float(last.y)) && !(cur.geom.w < __uint_as_float(0x7F800000u - first_c.y));
-				}
-			}
+			const bool span_applies = boxed && prune_by_box(straddles, p.T > 0.f, cur.geom.w, st.rays, a, left, right);
 			const uint64_t in_left = lanes_where(left), in_right = lanes_where(right);
 			const int n_left = __popcll(in_left), n_right = __popcll(in_right);
 			const int steps = max(n_left, n_right), padded = (steps + 3) & ~3;
-			if (lane < count) {
-				float4 g = cur.geom;
-				if (pos_cur & 0x80000000u)
-					g.w = __int_as_float(0x7FC00000);  // the strip lies inside the box: no per-pixel test
-				if (left) {
-					const uint32_t r = lanes_below(in_left);
-					st.slot[0][r].geom = g;
-					st.slot[0][r].conic = staged_conic(cur.conic);
-					st.slot[0][r].cd = cur.cd;
-					st.entry[0][r] = (uint8_t)lane;
-				}
-				if (right) {
-					const uint32_t r = lanes_below(in_right);
-					st.slot[1][r].geom = g;
-					st.slot[1][r].conic = staged_conic(cur.conic);
-					st.slot[1][r].cd = cur.cd;
-					st.entry[1][r] = (uint8_t)lane;
-				}
-			}
-			// both halves are walked for `padded` slots: the rest get entries that never pass the floor test (an
-			// infinite floor; their conic may be any finite one, and the lane's own record is at hand: a real one or zeros)
-			if (lane >= n_left && lane < padded) {
-				st.slot[0][lane].geom = float4{0.f, 0.f, INFINITY, 0.f};
-				st.slot[0][lane].conic = cur.conic;
-			}
-			if (lane >= n_right && lane < padded) {
-				st.slot[1][lane].geom = float4{0.f, 0.f, INFINITY, 0.f};
-				st.slot[1][lane].conic = cur.conic;
-			}
+			if (left)
+				stage_slot(st, 0, lanes_below(in_left), cur, pos_cur, l);
+			if (right)
+				stage_slot(st, 1, lanes_below(in_right), cur, pos_cur, l);
+			// both halves are walked for `padded` slots: the rest get entries that nothing takes
+			if (l >= n_left && l < padded)
+				stage_nothing(st, 0, (uint32_t)l);
+			if (l >= n_right && l < padded)
+				stage_nothing(st, 1, (uint32_t)l);
 			__builtin_amdgcn_wave_barrier();
 			// the chunk is in LDS now: its registers take the next chunk's records, loaded during the walk
 			cur = load_record(a, id_next, pos_next != kNone);
 			pos_cur = pos_next;
 			pos_next = pos_after;
 			id_next = pos_next != kNone ? list[pos_next & kPosition] : 0u;
-			const uint32_t e3 = first + 192 + (uint32_t)lane;
+			const uint32_t e3 = first + 192 + (uint32_t)l;
 			pos_after = e3 < filed ? filed_list[e3] : kNone;
 
-			if (boxed) {
-				const BoxFrame box = load_box_frame(a);
-				for (int k = 0; k < steps && live != 0ull; k += 4)
-					forward_group<true>(p, live, st, half, k, pixf, ray, box);
-			} else {
-				for (int k = 0; k < steps && live != 0ull; k += 4)
-					forward_group<false>(p, live, st, half, k, pixf, ray, BoxFrame{});
-			}
+			BoxSpan span = {0.f, 0.f, 0.f, 0.f};
+			if (boxed)
+				span = span_for_visits(span_applies, st.rays, a);
+			for (int k = 0; k < steps && live != 0ull; k += 4)
+				forward_group(p, live, st, half, k, pixf, boxed, span, a);
 			if (p.last_slot >= 0)
 				p.last_filed = first + st.entry[half][p.last_slot] + 1u;
 			p.last_slot = -1;
 			__builtin_amdgcn_wave_barrier();
 		}
 	}
-
-	{
-		// how many of the filed entries the backward has to walk: up to the last one some pixel blended
-		const uint32_t upto = filed != 0u ? wave_max_u32(p.last_filed) : 0u;  // (zero for a pixel outside the image)
-		if (lane == 0)
-			a.strip_filed[strip_id] = upto;
-	}
 	// (the pixel's place is worked out again, from the lane's number as the hardware counts it: kept from the start it would
 	// hold a register through the whole walk, one more than the kernel's wavefronts per SIMD leave it)
 	const int lane_again = (int)lanes_below(~0ull);
-	const uint32_t out_x = tx * kTile + (lane_again & 15), out_y = ty * kTile + wave * 4 + (lane_again >> 4);
-	if (out_x < (uint32_t)a.W && out_y < (uint32_t)a.H) {
-		const uint32_t pix_id = (uint32_t)a.W * out_y + out_x;
-		const size_t plane = (size_t)a.H * a.W;
-		// the reference's n_contrib: the 1-based position in the tile's list of the last entry the pixel blended
-		uint32_t last_contributor = 0u;
-		if (p.last_filed != 0u) {
-			const uint32_t* filed_list = a.strip_lists + 4 * (size_t)range.x + (size_t)wave * n;
-			last_contributor = (filed_list[p.last_filed - 1u] & 0x7FFFFFFFu) + 1u;
-		}
-		a.n_contrib[pix_id] = last_contributor;
-		a.out_color[pix_id] = p.C0 + fabsf(p.T) * a.bg[0];
-		a.out_color[plane + pix_id] = p.C1 + fabsf(p.T) * a.bg[1];
-		a.out_color[2 * plane + pix_id] = p.C2 + fabsf(p.T) * a.bg[2];
-		a.out_alpha[pix_id] = p.weight;
-		a.out_depth[pix_id] = p.D;
-	}
+	forward_finish(a, strip_id, p, filed, a.strip_lists + 4 * (size_t)range.x + (size_t)wave * n, tx * kTile + (lane_again & 15),
+	               ty * kTile + wave * 4 + (lane_again >> 4), lane_again);
+}
+
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 6))) void blend_forward_kernel(BlendBatch batch)
+{
+	__shared__ ForwardStage st;
+	// The jobs of a batch (the submodels of a frame) take turns, each handing out its strips longest
+	// list first: a long strip that starts late is what a launch waits for, and with several jobs in one
+	// launch there is other work to run beside the longest strips of each.
+	const BlendArgs& a = batch.job[blockIdx.x % (uint32_t)batch.count];
+	forward_strip(a, a.strip_order_forward[blockIdx.x / (uint32_t)batch.count], st, threadIdx.x);
 }
 
 // Work accounting: the reference loop taken literally, one list entry at a time with no
@@ -715,6 +824,7 @@ struct BackwardStage {  // wave-private
 	uint32_t id[kChunk + kRows - 1];
 	float2 u_at[kRows * kRowStride];  // [row][row_column(pixel)]: (u, alpha T)
 	float g_depth[72];                // upstream gradient of the depth image by pixel, eight of nine words
+	StripRays rays;
 };
 
 struct StripFrame {
@@ -821,7 +931,7 @@ __device__ __forceinline__ void sum_rows(const BackwardStage& st, int slot0, int
 // any pixel blended any of them.
 template <bool kDepth, bool kBoxed>
 __device__ __forceinline__ bool backward_rows(BackwardPixel& p, uint32_t last_contributor, BackwardStage& st, int k, int row,
-                                              const float2 pixf, const PixelRay& ray, const BoxFrame& box, int lane)
+                                              const float2 pixf, const BoxSpan& span, const BlendArgs& a, int lane)
 {
 	float power[4], clip_w[4], opacity[4];
 	uint64_t mask[4];
@@ -848,9 +958,8 @@ __device__ __forceinline__ bool backward_rows(BackwardPixel& p, uint32_t last_co
 		G[i] = exp_of_exponent(power[i]);
 		alpha[i] = fminf(0.99f, opacity[i] * G[i]);
 		mask[i] &= lanes_where(!(alpha[i] < 1.0f / 255.0f));
-		// (an entry that has the whole strip inside the box carries a NaN: never clipped)
-		if (kBoxed && (mask[i] & lanes_where(clip_w[i] == clip_w[i])) != 0ull)
-			mask[i] &= ~lanes_where(clipped_by_box(ray, clip_w[i], box));
+		if (kBoxed)
+			mask[i] = lanes_inside_box(mask[i], clip_w[i], span, st.rays, a);
 		// From here on nothing feeds a decision: gradients are compared by tolerance, so the divisions use the hardware
 		// reciprocal.
 		inv[i] = __builtin_amdgcn_rcpf(1.f - alpha[i]);
@@ -910,7 +1019,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 	const bool inside = px < (uint32_t)a.W && py < (uint32_t)a.H;
 	const uint32_t pix_id = (uint32_t)a.W * py + px;
 	const float2 pixf = {(float)px, (float)py};
-	const PixelRay ray = {pix_to_ndc(pixf.x, a.W), pix_to_ndc(pixf.y, a.H)};
 	const size_t plane = (size_t)a.H * a.W;
 	const float strip_x0 = (float)(tx * kTile), strip_y0 = (float)(ty * kTile + wave * 4);
 	const StripFrame frame = {strip_x0, strip_y0, (float)(0.5 * a.W), (float)(0.5 * a.H)};
@@ -937,6 +1045,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 	}
 	p.behind = T_final * ((0.f + a.bg[0] * p.g_r + a.bg[1] * p.g_g) + a.bg[2] * p.g_b);
 
+	stage_rays(st.rays, pixf, a, lane);
 	SweepUpstream upstream;
 	{
 		float4* by_pixel = st.geom;  // (not in use yet)
@@ -960,7 +1069,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 	// indices of the one after, the positions of the one after that.
 	const uint32_t* list = a.point_list + range.x;
 	const uint32_t* filed_list = a.strip_lists + 4 * (size_t)range.x + (size_t)wave * n;
-	constexpr uint32_t kNone = 0xFFFFFFFFu, kPosition = 0x7FFFFFFFu;
 	uint32_t pos_cur = (uint32_t)lane < filed ? filed_list[filed - 1 - lane] : kNone;
 	uint32_t pos_next = (uint32_t)(64 + lane) < filed ? filed_list[filed - 1 - (64 + lane)] : kNone;
 	uint32_t pos_after = (uint32_t)(128 + lane) < filed ? filed_list[filed - 1 - (128 + lane)] : kNone;
@@ -986,7 +1094,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 			st.entry[count + lane] = 0xFFFFFFFFu;
 			st.id[count + lane] = 0u;
 		}
-		const bool boxed = lanes_where(lane < count && (pos_cur & 0x80000000u) == 0u) != 0ull;
+		const bool straddles = lane < count && (pos_cur & 0x80000000u) == 0u;
+		const bool boxed = lanes_where(straddles) != 0ull, all_in_front = lanes_where(straddles && !(cur.geom.w > 0.f)) == 0ull;
 		__builtin_amdgcn_wave_barrier();
 		// the chunk is in LDS now: its registers take the next chunk's records, loaded during the walk
 		cur = load_record(a, id_next, pos_next != kNone);
@@ -998,17 +1107,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 
 		// (few strips straddle a face of their box: their chunks run a copy of the loop that has the test)
 		if (boxed) {
-			const BoxFrame box = load_box_frame(a);
+			const BoxSpan span = span_for_visits(all_in_front, st.rays, a);
 			for (int k = 0; k < count; k += kRows) {
-				const bool front = backward_rows<kDepth, true>(p, last_contributor, st, k, 0, pixf, ray, box, lane);
-				const bool back = backward_rows<kDepth, true>(p, last_contributor, st, k + 4, 4, pixf, ray, box, lane);
+				const bool front = backward_rows<kDepth, true>(p, last_contributor, st, k, 0, pixf, span, a, lane);
+				const bool back = backward_rows<kDepth, true>(p, last_contributor, st, k + 4, 4, pixf, span, a, lane);
 				if (front || back)
 					sum_rows<kDepth>(st, k, count - k, upstream, frame, a, lane);
 			}
 		} else {
 			for (int k = 0; k < count; k += kRows) {
-				const bool front = backward_rows<kDepth, false>(p, last_contributor, st, k, 0, pixf, ray, BoxFrame{}, lane);
-				const bool back = backward_rows<kDepth, false>(p, last_contributor, st, k + 4, 4, pixf, ray, BoxFrame{}, lane);
+				const bool front = backward_rows<kDepth, false>(p, last_contributor, st, k, 0, pixf, BoxSpan{}, a, lane);
+				const bool back = backward_rows<kDepth, false>(p, last_contributor, st, k + 4, 4, pixf, BoxSpan{}, a, lane);
 				if (front || back)
 					sum_rows<kDepth>(st, k, count - k, upstream, frame, a, lane);
 			}
