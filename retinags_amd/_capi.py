@@ -71,9 +71,10 @@ class RgsError(RuntimeError):
 def _load():
     if not os.path.exists(LIB_PATH):
         raise ImportError(
-            f"{LIB_PATH} is missing: build it with `python -m retinags_amd.build` "
+            f"{LIB_PATH} is missing: build it with `python retinags_amd/build.py` "
             "(hipcc, gfx950). There is no fallback implementation.")
-    lib = C.CDLL(LIB_PATH)
+    # its symbols are global: the native host path (csrc/host.cpp) resolves the entry points from them
+    lib = C.CDLL(LIB_PATH, mode=C.RTLD_GLOBAL)
     vp, f, i, sz = C.c_void_p, C.c_float, C.c_int, C.c_size_t
     lib.rgs_version.restype = i
     lib.rgs_last_error.restype = C.c_char_p
@@ -192,10 +193,3 @@ def ptr(t) -> C.c_void_p:
     if t is None or t.numel() == 0:
         return C.c_void_p(0)
     return C.c_void_p(t.data_ptr())
-
-
-def ptr_table(tensors):
-    arr = (C.c_void_p * len(tensors))()
-    for k, t in enumerate(tensors):
-        arr[k] = t.data_ptr()
-    return arr

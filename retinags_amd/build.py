@@ -1,18 +1,22 @@
-"""Builds librgs_gfx950.so from the HIP sources in csrc/ with hipcc, in-tree.
+"""Builds librgs_gfx950.so from the HIP sources in csrc/ with hipcc, and _host.so (the host path between PyTorch and the
+library, csrc/host.cpp) with the host compiler, in-tree.
 
-Usage: ``python -m retinags_amd.build`` (add ``--force`` to rebuild everything).
+Usage: ``python retinags_amd/build.py`` (add ``--force`` to rebuild everything).
 There is no GPU requirement: hipcc cross-compiles for gfx950.
 """
 from __future__ import annotations
 
+import importlib.util
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "librgs_gfx950.so")
+HOST = os.path.join(HERE, "_host.so")
 
 COMMON = [
     "--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function",
@@ -34,6 +38,7 @@ SOURCES = {
     "training.hip": [],
 }
 
+HOST_SOURCES = ["host.cpp"]
 HEADERS = ["rgs_device.h", "rgs_kernels.h", "strip_filing.h", "tile_order.h", os.path.join("..", "..", "include", "rgs.h")]
 
 
@@ -51,6 +56,28 @@ def _stale(target: str, deps) -> bool:
     return any(os.path.getmtime(d) > t for d in deps)
 
 
+def _host_commands():
+    """(source, compile command, object) of every part of the host path, and the link command.  The library's entry points stay
+    undefined in _host.so: they come from the librgs_gfx950.so that is loaded first."""
+    torch_dir = os.path.dirname(importlib.util.find_spec("torch").origin)
+    include = os.path.join(torch_dir, "include")
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    cxx = os.environ.get("CXX", "g++")
+    flags = ["-O2", "-fPIC", "-std=c++17", "-fvisibility=hidden", "-Wall", "-Wno-unknown-pragmas", "-D__HIP_PLATFORM_AMD__=1",
+             "-DUSE_ROCM=1"]
+    for d in (include, os.path.join(include, "torch", "csrc", "api", "include"), os.path.join(rocm, "include"),
+              sysconfig.get_paths()["include"]):
+        flags += ["-isystem", d]
+    parts = []
+    for name in HOST_SOURCES:
+        source = os.path.join(CSRC, name)
+        parts.append((source, [cxx] + flags + ["-c", source, "-o", source.replace(".cpp", ".o")], source.replace(".cpp", ".o")))
+    link = [cxx, "-shared", "-fPIC", "-o", HOST] + [o for _, _, o in parts] + [
+        "-L" + os.path.join(torch_dir, "lib"), "-L" + os.path.join(rocm, "lib"), "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu",
+        "-ltorch_python", "-lamdhip64"]
+    return parts, link
+
+
 def build(force: bool = False, verbose: bool = True) -> str:
     hipcc = _hipcc()
     hdrs = [os.path.join(CSRC, h) for h in HEADERS]
@@ -61,6 +88,11 @@ def build(force: bool = False, verbose: bool = True) -> str:
         objs.append(o)
         if force or _stale(o, [s] + hdrs):
             jobs.append([hipcc] + COMMON + extra + ["-c", s, "-o", o])
+    link = force or bool(jobs) or _stale(LIB, objs)
+    host_parts, host_link = _host_commands()
+    for source, command, o in host_parts:
+        if force or _stale(o, [source, os.path.join(CSRC, "host.h"), hdrs[-1]]):
+            jobs.insert(0, command)
 
     def run(cmd):
         if verbose:
@@ -69,14 +101,16 @@ def build(force: bool = False, verbose: bool = True) -> str:
         # the host pass of hipcc reports that it does not know the packed-fp32 feature; harmless
         err = "\n".join(l for l in r.stderr.splitlines() if "packed-fp32-ops" not in l)
         if r.returncode != 0:
-            raise RuntimeError(f"hipcc failed:\n{' '.join(cmd)}\n{err}")
+            raise RuntimeError(f"the compiler failed:\n{' '.join(cmd)}\n{err}")
         if verbose and err.strip():
             print(err, file=sys.stderr)
 
     with ThreadPoolExecutor(max_workers=min(4, max(1, len(jobs)))) as ex:
         list(ex.map(run, jobs))
-    if force or jobs or _stale(LIB, objs):
+    if link or _stale(LIB, objs):
         run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", LIB] + objs)
+    if force or _stale(HOST, [o for _, _, o in host_parts]):
+        run(host_link)
     return LIB
 
 

@@ -13,7 +13,7 @@ from typing import Dict, List, Optional
 import numpy as np
 import torch
 
-from ..rasterizer import GaussianRasterizationSettings, GaussianRasterizer, rasterize_frame
+from ..rasterizer import GaussianRasterizationSettings, GaussianRasterizer, _rasterize_layers
 from ..compositor import blender_render_result
 from .partition import Partition, partition_scene, relation_vector
 from .scenes import Camera
@@ -346,21 +346,20 @@ def render_frame(cam: Camera, subs: List[Submodel], relation: np.ndarray, backgr
     if together:
         if instance_bounds is not None or host_threads:
             raise ValueError("together=True takes neither instance_bounds nor host_threads")
-        main = torch.cuda.current_stream(device)
-        lanes = streams if streams else [main]
-        rasterizers, inputs = [], []
+        lanes = streams
+        settings, inputs = [], []
         for m in related:
             sub = subs[m]
             means2D = sub.means2D
             if means2D is None:
                 means2D = _screenspace_placeholder(sub)
-            rasterizers.append(GaussianRasterizer(raster_settings=raster_settings(cam, sub, submodel_bg)))
+            settings.append(raster_settings(cam, sub, submodel_bg))
             inputs.append(dict(means3D=sub.means3D, means2D=means2D, shs=sub.shs, opacities=sub.opacity, scales=sub.scales,
                                rotations=sub.rotations))
         taps = [] if keep_workspaces else None
-        outs = rasterize_frame(rasterizers, inputs,
-                               streams=[lanes[k % len(lanes)].cuda_stream for k in range(len(related))] if streams else None,
-                               workspaces=taps)
+        outs = _rasterize_layers(settings, inputs,
+                                 streams=[lanes[k % len(lanes)].cuda_stream for k in range(len(related))] if streams else None,
+                                 workspaces=taps)
         partial = {}
         for k, m in enumerate(related):
             color, radii, depth, alpha = outs[k]
@@ -398,11 +397,12 @@ def render_frame(cam: Camera, subs: List[Submodel], relation: np.ndarray, backgr
                 if torch.is_tensor(t) and t.is_cuda:
                     t.record_stream(main)
     elif not streams:
+        # as below: while the host waits for a submodel's count the next submodels' geometry stages keep the device busy
         partial = {}
+        started = {m: start_submodel(cam, subs[m], submodel_bg) for m in related}
         for m in related:
-            started = start_submodel(cam, subs[m], submodel_bg)
-            stages[m] = started[1]
-            partial[m] = render_submodel(cam, subs[m], submodel_bg, started=started)
+            stages[m] = started[m][1]
+            partial[m] = render_submodel(cam, subs[m], submodel_bg, started=started[m])
     else:
         main = torch.cuda.current_stream(device)
         for side in streams[:len(related)]:
