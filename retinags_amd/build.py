@@ -38,7 +38,7 @@ SOURCES = {
     "training.hip": [],
 }
 
-HOST_SOURCES = ["host.cpp"]
+HOST_SOURCES = ["host.cpp", "host_training.cpp"]
 HEADERS = ["rgs_device.h", "rgs_kernels.h", "strip_filing.h", "tile_order.h", os.path.join("..", "..", "include", "rgs.h")]
 
 

@@ -902,6 +902,7 @@ PYBIND11_MODULE(_host, m)
 	m.def("rasterize_forward", &rasterize_forward);
 	m.def("rasterize_frame", &rasterize_frame);
 	m.def("enqueue_geometry", &enqueue_geometry);
+	define_training(m);
 
 	py::class_<GeometryStage>(m, "GeometryStage",
 	                          "What the first half of a forward call leaves behind: the geometry workspace, the radii and the place "

@@ -197,4 +197,6 @@ inline SlotPool& slot_pool()
 }
 
 
+void define_training(py::module_& m);  // host_training.cpp
+
 }  // namespace rgs_host

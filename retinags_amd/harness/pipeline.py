@@ -13,6 +13,7 @@ from typing import Dict, List, Optional
 import numpy as np
 import torch
 
+from .. import _host
 from ..rasterizer import GaussianRasterizationSettings, GaussianRasterizer, _rasterize_layers
 from ..compositor import blender_render_result
 from .partition import Partition, partition_scene, relation_vector
@@ -89,8 +90,12 @@ def owned_models_from_partition(scene: Dict[str, torch.Tensor], part: Partition,
 
 def submodels_from_shared(merged: List["SharedGSInfo"], part: Partition, device) -> List[Submodel]:
     """Renderer inputs from merged (own + lent) tensors, e.g. those of sharing.merge_shared."""
-    return [Submodel(m.means3D, m.opacity, m.scales, m.rotations, m.shs, torch.from_numpy(part.box_low[k]).to(device),
-                     torch.from_numpy(part.box_up[k]).to(device), means2D=m.means2D) for k, m in enumerate(merged)]
+    # all boxes in one copy, from pinned memory: one per box from pageable memory would each wait for the stream
+    boxes = torch.from_numpy(np.stack([part.box_low, part.box_up], dtype=np.float32))
+    if torch.device(device).type == "cuda":
+        boxes = boxes.pin_memory().to(device, non_blocking=True)
+    return [Submodel(m.means3D, m.opacity, m.scales, m.rotations, m.shs, low, up, means2D=m.means2D)
+            for m, low, up in zip(merged, boxes[0].unbind(), boxes[1].unbind())]
 
 
 def whole_scene_submodel(scene: Dict[str, torch.Tensor], device, margin: float = 1.0) -> Submodel:
@@ -103,24 +108,12 @@ def whole_scene_submodel(scene: Dict[str, torch.Tensor], device, margin: float =
     return Submodel(mv(xyz), mv(scene["opacity"]), mv(scene["scales"]), mv(scene["rotations"]), mv(scene["shs"]), low, up)
 
 
-class GradNormHelper(torch.autograd.Function):
+def gradNormHelpFunction(meta: torch.Tensor, spare_rows: int = 0) -> torch.Tensor:
     """The placeholder through which the reference collects the screen-space gradient norm that
     densification reads (gaussian_renderer/render_half_gs.py:7-19): forward turns an (N,1) meta
-    tensor into the (N,3) zeros passed as means2D; backward hands the meta tensor the length of
-    each row's (x, y) gradient."""
-
-    @staticmethod
-    def forward(ctx, meta: torch.Tensor) -> torch.Tensor:
-        if meta.dim() != 2 or meta.shape[1] != 1:
-            raise RuntimeError("meta must have shape (N, 1)")
-        return torch.zeros((meta.shape[0], 3), dtype=meta.dtype, device=meta.device)
-
-    @staticmethod
-    def backward(ctx, grad_output: torch.Tensor) -> torch.Tensor:
-        return torch.norm(grad_output[:, :2], dim=-1, keepdim=True)
-
-
-gradNormHelpFunction = GradNormHelper.apply
+    tensor into the (N,3) zeros passed as means2D (with room for spare_rows more rows behind them); backward
+    hands the meta tensor the length of each row's (x, y) gradient."""
+    return _host.screen_placeholder(meta, spare_rows)
 
 
 def raster_settings(cam: Camera, sub: Submodel, bg: torch.Tensor, scaling_modifier: float = 1.0,
@@ -500,24 +493,9 @@ class StoredModel:
         """get_xyz, get_opacity, get_scaling, get_rotation, get_features and the means2D placeholder
         (parallel_utils/basic_parallel_trainer/result_aggregator.py:40-52)."""
         from ..activation import activate_gaussians
-        means2D = gradNormHelpFunction(self.means2D_meta)
-        if self.spare_rows:
-            means2D = _RoomBehind.apply(means2D, self.spare_rows)
+        means2D = gradNormHelpFunction(self.means2D_meta, self.spare_rows)
         return activate_gaussians(self.xyz, self.features_dc, self.features_rest, self.scaling, self.rotation,
                                   self.opacity, means2D=means2D, spare_rows=self.spare_rows)
-
-
-class _RoomBehind(torch.autograd.Function):
-    """Identity that moves a tensor to the start of an allocation with spare rows behind it."""
-
-    @staticmethod
-    def forward(ctx, t: torch.Tensor, spare: int) -> torch.Tensor:
-        from ..sharing import with_spare_rows
-        return with_spare_rows(t, spare).detach()
-
-    @staticmethod
-    def backward(ctx, g: torch.Tensor):
-        return g, None
 
 
 def stored_models_from_partition(scene: Dict[str, torch.Tensor], part: Partition, device,
