@@ -363,7 +363,7 @@ int rgs_composite_forward(int K, int height, int width,
                           const float* background, float* out_image, float* out_depth, float* out_alpha,
                           void* stream);
 /* g_depth / g_alpha may be NULL (treated as zero).  d_images[k], d_depths[k], d_alphas[k]
- * receive the gradients and are fully written. */
+ * receive the gradients and are fully written; with g_depth NULL, d_depths may be NULL too. */
 int rgs_composite_backward(int K, int height, int width,
                            const float* const* images, const float* const* depths, const float* const* alphas,
                            const float* background, const float* g_image, const float* g_depth,

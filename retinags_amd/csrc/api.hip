@@ -1296,12 +1296,12 @@ int rgs_composite_backward(int K, int height, int width,
 	rgs::CompositeArgs a;
 	if (int rc = fill_composite(a, K, height, width, images, depths, alphas, background))
 		return rc;
-	RGS_REQUIRE(g_image && d_images && d_depths && d_alphas, "rgs_composite_backward: null pointer");
+	RGS_REQUIRE(g_image && d_images && d_alphas && (d_depths || !g_depth), "rgs_composite_backward: null pointer");
 	a.g_image = g_image; a.g_depth = g_depth; a.g_alpha = g_alpha;
 	for (int k = 0; k < K; k++) {
-		RGS_REQUIRE(d_images[k] && d_depths[k] && d_alphas[k], "rgs_composite_backward: null output plane at k=%d", k);
+		RGS_REQUIRE(d_images[k] && (!d_depths || d_depths[k]) && d_alphas[k], "rgs_composite_backward: null output plane at k=%d", k);
 		a.d_images[k] = d_images[k];
-		a.d_depths[k] = d_depths[k];
+		a.d_depths[k] = d_depths ? d_depths[k] : nullptr;
 		a.d_alphas[k] = d_alphas[k];
 	}
 	rgs::launch_composite_backward(a, s);

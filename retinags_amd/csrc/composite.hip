@@ -42,7 +42,9 @@ __global__ __launch_bounds__(256) void composite_forward_kernel(CompositeArgs a)
 // back-to-front sweep: in registers when the number of layers is at most kLayers (the loops are unrolled over kLayers
 // and guarded by K, so the arrays are indexed by constants), otherwise (kLayers = 0) in an array indexed at run time,
 // which the compiler places in scratch memory: every value then goes out to memory and comes back.
-template <int kLayers>
+// kDepth: there is a gradient of the composited depth.  Without one the layers' depths are not read and their gradients
+// (zero) are written only where the caller has planes for them; the kernel is bound by memory, and both are planes of K.
+template <int kLayers, bool kDepth>
 __global__ __launch_bounds__(256) void composite_backward_kernel(CompositeArgs a)
 {
 	const size_t n = (size_t)a.H * a.W;
@@ -68,7 +70,7 @@ __global__ __launch_bounds__(256) void composite_backward_kernel(CompositeArgs a
 		}
 	}
 	const float gr = a.g_image[p], gg = a.g_image[n + p], gb = a.g_image[2 * n + p];
-	const float gd = a.g_depth ? a.g_depth[p] : 0.f;
+	const float gd = kDepth ? a.g_depth[p] : 0.f;
 	const float ga = a.g_alpha ? a.g_alpha[p] : 0.f;
 	float R = -ga;
 	if (a.bg)
@@ -78,10 +80,12 @@ __global__ __launch_bounds__(256) void composite_backward_kernel(CompositeArgs a
 		di[p] = t * gr;
 		di[n + p] = t * gg;
 		di[2 * n + p] = t * gb;
-		a.d_depths[k][p] = t * gd;
+		if (kDepth || a.d_depths[k])
+			a.d_depths[k][p] = t * gd;
 		a.d_alphas[k][p] = -(t * R);
 		const float* img = a.images[k];
-		R = img[p] * gr + img[n + p] * gg + img[2 * n + p] * gb + a.depths[k][p] * gd + (1.f - alpha_k) * R;
+		const float colour = img[p] * gr + img[n + p] * gg + img[2 * n + p] * gb;
+		R = (kDepth ? colour + a.depths[k][p] * gd : colour) + (1.f - alpha_k) * R;
 	};
 	if (kLayers > 0) {
 #pragma unroll
@@ -101,17 +105,26 @@ void launch_composite_forward(const CompositeArgs& a, hipStream_t s)
 	hipLaunchKernelGGL(composite_forward_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a);
 }
 
-void launch_composite_backward(const CompositeArgs& a, hipStream_t s)
+template <bool kDepth>
+static void launch_composite_backward_as(const CompositeArgs& a, hipStream_t s)
 {
 	const size_t n = (size_t)a.H * a.W;
-	stage_mark("composite_backward", s);
 	const dim3 grid((unsigned)((n + 255) / 256));
 	if (a.K <= 4)
-		hipLaunchKernelGGL(composite_backward_kernel<4>, grid, dim3(256), 0, s, a);
+		hipLaunchKernelGGL((composite_backward_kernel<4, kDepth>), grid, dim3(256), 0, s, a);
 	else if (a.K <= 16)
-		hipLaunchKernelGGL(composite_backward_kernel<16>, grid, dim3(256), 0, s, a);
+		hipLaunchKernelGGL((composite_backward_kernel<16, kDepth>), grid, dim3(256), 0, s, a);
 	else
-		hipLaunchKernelGGL(composite_backward_kernel<0>, grid, dim3(256), 0, s, a);
+		hipLaunchKernelGGL((composite_backward_kernel<0, kDepth>), grid, dim3(256), 0, s, a);
+}
+
+void launch_composite_backward(const CompositeArgs& a, hipStream_t s)
+{
+	stage_mark("composite_backward", s);
+	if (a.g_depth)
+		launch_composite_backward_as<true>(a, s);
+	else
+		launch_composite_backward_as<false>(a, s);
 }
 
 }  // namespace rgs

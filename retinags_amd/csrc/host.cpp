@@ -89,26 +89,27 @@ struct Composite : torch::autograd::Function<Composite> {
 			PlaneTables in;
 			std::array<float*, RGS_MAX_COMPOSITE> d_images, d_depths, d_alphas;
 			// The background is a constant to the loss: no gradient.  Without a gradient of the composited depth the layers'
-			// depths have none either (their planes of the blocks hold the zeros the kernel wrote); told so, the
-			// rasterizer's backward leaves out the terms it would multiply.
+			// depths have none either; told so, the rasterizer's backward leaves out the terms it would multiply.
+			const bool with_depth = g_depth.defined();
+			const int64_t planes = with_depth ? 5 : 4;
 			variable_list out(3 * K + 1);
 			for (int k = 0; k < K; k++) {
 				in.set(k, saved[k], saved[K + k], saved[2 * K + k]);
 				// a layer's three gradients in one (5,H,W) block, the layout of RenderResult.zip_grad
-				// (parallel_utils/basic_parallel_trainer/task_utils.py:187-195)
-				const Tensor block = new_f32({5, H, W}, device);
+				// (parallel_utils/basic_parallel_trainer/task_utils.py:187-195); without the depth's if there is none
+				const Tensor block = new_f32({planes, H, W}, device);
 				d_images[k] = ptr(block);
 				d_depths[k] = d_images[k] + 3 * H * W;
-				d_alphas[k] = d_images[k] + 4 * H * W;
+				d_alphas[k] = d_images[k] + (planes - 1) * H * W;
 				out[k] = block.narrow(0, 0, 3);
-				if (g_depth.defined())
+				if (with_depth)
 					out[K + k] = block.narrow(0, 3, 1);
-				out[2 * K + k] = block.narrow(0, 4, 1);
+				out[2 * K + k] = block.narrow(0, planes - 1, 1);
 			}
 			c10::DeviceGuard guard(device);
 			check(rgs_composite_backward(K, H, W, in.images.data(), in.depths.data(), in.alphas.data(), ptr(saved[3 * K]), ptr(g_image),
-			                             ptr(g_depth), ptr(g_alpha), d_images.data(), d_depths.data(), d_alphas.data(),
-			                             current_stream(device)));
+			                             ptr(g_depth), ptr(g_alpha), d_images.data(), with_depth ? d_depths.data() : nullptr,
+			                             d_alphas.data(), current_stream(device)));
 			return out;
 		});
 	}
