@@ -86,7 +86,7 @@ __device__ __forceinline__ BoxSpan w_inside_box(const PixelRay& ray, const BoxFr
 	for (int k = 0; k < 3; k++) {
 		const float t0 = b.m[0][k] * rx, t1 = b.m[1][k] * ry, t2 = b.m[2][k], offset = b.m[3][k];
 		const float slope = t0 + t1 + t2, room = 2e-6f * (fabsf(t0) + fabsf(t1) + fabsf(t2));
-		const float room_offset = 2e-6f * fabsf(offset);
+		const float room_offset = 2e-6f * fabsf(offset) + 2e-7f * (fabsf(t0) + fabsf(t1));  // (and for the exact test's w + 1e-7)
 		// slope w > lo - offset and, mirrored, -slope w > -(hi - offset)
 #pragma unroll
 		for (int side = 0; side < 2; side++) {

@@ -369,9 +369,15 @@ GradientArrays make_gradients(py::handle module, int64_t P, int64_t M, const at:
 
 py::handle rasterizer_module()
 {
-	static PyObject* module = PyImport_ImportModule("retinags_amd.rasterizer");
-	if (!module)
-		throw py::error_already_set();
+	// (under the interpreter lock, which the import may hand to another thread: a static initialised by the import would have
+	// that thread wait for it while it holds the lock)
+	static PyObject* module = nullptr;
+	if (!module) {
+		PyObject* imported = PyImport_ImportModule("retinags_amd.rasterizer");
+		if (!imported)
+			throw py::error_already_set();
+		module = imported;
+	}
 	return module;
 }
 

@@ -131,6 +131,19 @@ struct CountSlot {
 constexpr int kSlotWords = RGS_MAX_SHARE_BOXES * RGS_MAX_SHARE_BOXES;
 static_assert(kSlotWords >= RGS_MAX_FRAME_LAYERS, "a frame reports one count per layer");
 
+// While a thread captures a graph, queries of events and allocations of pinned memory by any thread would end that capture
+// unless they are told not to matter to it.
+class OutsideCapture {
+public:
+	OutsideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+	~OutsideCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode_); }
+	OutsideCapture(const OutsideCapture&) = delete;
+	OutsideCapture& operator=(const OutsideCapture&) = delete;
+
+private:
+	hipStreamCaptureMode mode_ = hipStreamCaptureModeRelaxed;
+};
+
 // Slots per device, kept for the next call that needs one: at most kKept of them, shared by all threads and streams (a call
 // has its slot to itself).  A slot whose count nobody waited for comes back when its event has passed.
 class SlotPool {
@@ -139,13 +152,21 @@ public:
 	{
 		std::lock_guard<std::mutex> lock(mutex_);
 		PerDevice& d = devices_[device];
+		if (d.in_flight.empty() && !d.free.empty()) {
+			CountSlot s = d.free.back();
+			d.free.pop_back();
+			return s;
+		}
+		OutsideCapture relaxed;
 		for (size_t n = d.in_flight.size(); n > 0; n--) {
 			CountSlot s = d.in_flight.front();
 			d.in_flight.pop_front();
-			if (hipEventQuery(s.event) == hipSuccess)
+			if (hipEventQuery(s.event) == hipSuccess) {
 				keep(d, s);
-			else
+			} else {
+				(void)hipGetLastError();  // not there yet: no error of the caller's
 				d.in_flight.push_back(s);
+			}
 		}
 		if (!d.free.empty()) {
 			CountSlot s = d.free.back();
@@ -183,6 +204,7 @@ private:
 			d.free.push_back(s);
 			return;
 		}
+		OutsideCapture relaxed;
 		(void)hipEventDestroy(s.event);
 		(void)hipHostFree(s.words);
 	}

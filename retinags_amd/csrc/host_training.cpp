@@ -216,7 +216,7 @@ struct MergeShared : torch::autograd::Function<MergeShared> {
 		const at::Device device = flat[0].device();
 		c10::DeviceGuard guard(device);
 		const hipStream_t stream = current_stream(device);
-		m.sh_floats = static_cast<int>(c10::multiply_integers(flat[kFieldSH].sizes().slice(1)));
+		m.sh_floats = flat[kFieldSH].dim() > 1 ? static_cast<int>(c10::multiply_integers(flat[kFieldSH].sizes().slice(1))) : 0;
 		for (const Tensor& t : flat)
 			m.shapes.push_back(t.sizes().vec());
 		variable_list out;
@@ -323,12 +323,14 @@ std::vector<Tensor> merge_shared(const std::vector<int64_t>& own, const py::sequ
 	merge->reuse_gradients = reuse_gradients;
 	merge->append = append;
 	merge->lent.resize(own.size());
-	if (lent.size() != own.size() || flat.size() != kFields * own.size())
+	if (own.empty() || lent.size() != own.size() || flat.size() != kFields * own.size())
 		throw std::runtime_error("merge_shared: six fields and a list of lent rows per submodel");
 	for (size_t d = 0; d < own.size(); d++)
 		for (py::handle h : py::reinterpret_borrow<py::sequence>(lent[d])) {
 			const py::tuple t = py::reinterpret_borrow<py::tuple>(h);
 			merge->lent[d].push_back({py::cast<int>(t[0]), from_python(t[1], "rows"), py::cast<int64_t>(t[2])});
+			if (merge->lent[d].back().source < 0 || merge->lent[d].back().source >= static_cast<int>(own.size()))
+				throw std::runtime_error("merge_shared: rows of a submodel that is not there");
 		}
 	py::gil_scoped_release no_gil;
 	return MergeShared::apply(at::TensorList(flat), &merge);
@@ -378,6 +380,8 @@ py::tuple l1_ssim(const Tensor& image, const Tensor& gt, double lambda_dssim)
 		throw std::runtime_error("image and ground truth differ in shape");
 	if (image.dim() != 3 && image.dim() != 4)
 		throw std::runtime_error("expected (C,H,W) or (B,C,H,W) images");
+	if (image.size(-1) == 0 || image.size(-2) == 0)
+		throw std::runtime_error("the loss of an image without pixels is not defined");
 	if (!image.is_cuda() || !gt.is_cuda())
 		throw std::runtime_error("the loss runs on the GPU only: both images must be device tensors");
 	variable_list out;

@@ -116,6 +116,12 @@ def gradNormHelpFunction(meta: torch.Tensor, spare_rows: int = 0) -> torch.Tenso
     return _host.screen_placeholder(meta, spare_rows)
 
 
+class GradNormHelper:
+    """gradNormHelpFunction under the name of the reference's autograd function."""
+
+    apply = staticmethod(gradNormHelpFunction)
+
+
 def raster_settings(cam: Camera, sub: Submodel, bg: torch.Tensor, scaling_modifier: float = 1.0,
                     debug: bool = False) -> GaussianRasterizationSettings:
     return GaussianRasterizationSettings(

@@ -105,6 +105,30 @@ def test_compositor_forward_and_backward(K, H, W, with_bg):
         assert rel_l2(la[k].grad.cpu().numpy(), wda[k]) <= 1e-4
 
 
+@pytest.mark.parametrize("K", [1, 4, 5, 16, 17])
+def test_compositor_without_a_depth_gradient(K):
+    """With no gradient of the composited depth the layers' depths have none (they are not read, whatever they hold), and the
+    other gradients are those of a depth gradient of zero; a layer count on each side of the register forms' limits."""
+    from retinags_amd import composite_partial_images
+    g = torch.Generator().manual_seed(40 + K)
+    H, W = 19, 33
+    imgs = [torch.rand(3, H, W, generator=g) for _ in range(K)]
+    alps = [torch.rand(1, H, W, generator=g) for _ in range(K)]
+    deps = [torch.rand(1, H, W, generator=g) for _ in range(K)]
+    bg = torch.tensor([0.25, 0.5, 0.75])
+    gi, ga = torch.randn(3, H, W, generator=g), torch.randn(1, H, W, generator=g)
+    wdi, _, wda = orc.composite_backward([np32(t) for t in imgs], [np32(t) for t in deps], [np32(t) for t in alps], np32(bg),
+                                         np32(gi), np.zeros((1, H, W), np.float32), np32(ga))
+    leaf = lambda ts: [t.to(DEV).requires_grad_(True) for t in ts]
+    li, ld, la = leaf(imgs), leaf([torch.full_like(t, float("nan")) for t in deps]), leaf(alps)
+    img, _, alp = composite_partial_images(li, ld, la, bg.to(DEV))
+    torch.autograd.backward([img, alp], [gi.to(DEV), ga.to(DEV)])
+    for k in range(K):
+        assert ld[k].grad is None
+        assert rel_l2(li[k].grad.cpu().numpy(), wdi[k]) <= 1e-4
+        assert rel_l2(la[k].grad.cpu().numpy(), wda[k]) <= 1e-4
+
+
 def test_compositor_colour_only_gradient_and_ordering_rule():
     """blender_render_result composites by ascending relation value and skips negatives."""
     from retinags_amd import blender_render_result

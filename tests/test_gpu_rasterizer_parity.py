@@ -147,6 +147,30 @@ def test_cube_half_box_clips():
     assert st.counters[3] < st.counters[2]  # some samples were clipped by the box
 
 
+_INF = float("inf")
+
+
+@pytest.mark.parametrize("low,up", [
+    ((-0.31, -0.27, 3.6), (0.23, 0.19, 4.3)),          # pixels whose rays miss the box beside pixels that cross it
+    ((-_INF, -_INF, -_INF), (_INF, _INF, 3.9)),        # open sides; the rays leave through one face
+    ((-5.0, 0.05, -1.0), (5.0, 5.0, 9.0)),             # a face that holds the camera's neighbourhood, seen edge on
+    ((0.08, -0.12, 3.0), (0.15, -0.03, 8.0)),          # a shaft along the viewing axis: a few pixels
+    ((-5.0, -5.0, 4.95), (5.0, 5.0, 9.0)),             # behind nearly everything: pixels that stay unfinished
+    ((-5.0, -5.0, -9.0), (5.0, 5.0, 2.0)),             # in front of everything: nothing blends
+])
+@pytest.mark.parametrize("width,height", [(35, 9), (64, 52)])
+def test_box_faces_through_strips_and_halves(low, up, width, height):
+    """The forward blend leaves entries out by the live pixels of each half strip and by the clip w at which their rays are
+    inside the box; both blends decide most box tests by spans of clip w.  Boxes whose faces run through strips, at odd
+    angles to them, against the checker: same last blended entry per pixel, images and gradients within tolerance."""
+    scene = scenes.cube_scene(1200, seed=91)
+    scene["scales"] = scene["scales"] * 8.0
+    cam = scenes.look_at_camera((0.0, 0.0, 0.0), (0.13, -0.07, 4.0), (0.1, -1, 0), width, height, 40.0)
+    sub = _scene_sub(scene, low=torch.tensor(low), up=torch.tensor(up))
+    _check_forward_stages(sub, cam, torch.tensor([0.2, 0.1, 0.05]), max_borderline=2e-3)
+    _check_backward(sub, cam, torch.tensor([0.2, 0.1, 0.05]), seed=17, with_depth_alpha=height > 10)
+
+
 def test_depths_beyond_the_range_of_three_sort_passes():
     """The depth sort looks at 27 bits of the depth's bit pattern in three passes, which tells depths below 8192
     apart; a scene with Gaussians beyond that makes it run its fourth pass over the remaining bits.  Half of the cube
