@@ -816,12 +816,31 @@ struct BackwardPixel {
 	float g_r, g_g, g_b, g_depth, g_alpha;
 };
 
+// An LDS address in a register of its own: left to itself the compiler folds a member's place in the stage into every
+// access, where it exceeds what two-address accesses can encode, and adds it anew for each of them.
+typedef float Pair __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) Pair LdsPair;
+__device__ __forceinline__ LdsPair* lds_base(float2* p)
+{
+	LdsPair* at = (LdsPair*)p;
+	asm volatile("" : "+v"(at));
+	return at;
+}
+
+// Zeros in two neighbouring registers by one instruction (volatile: copies of a shared pair would take two).
+__device__ __forceinline__ Pair zero_pair()
+{
+	Pair z;
+	asm volatile("v_mov_b64 %0, 0" : "=v"(z));
+	return z;
+}
+
 struct BackwardStage {  // wave-private
 	float4 geom[kChunk + kRows - 1];   // + padding up to a multiple of eight entries
 	float4 conic[kChunk + kRows - 1];  // staged_conic(): -xx / 2, -xy, -yy / 2, opacity
 	float4 cd[kChunk + kRows - 1];
 	uint32_t entry[kChunk + kRows - 1];  // 0-based position in the tile list
-	uint32_t id[kChunk + kRows - 1];
+	uint32_t sum_row[kChunk + kRows - 1];  // where the Gaussian's row of `sums` begins, in 16 bytes
 	float2 u_at[kRows * kRowStride];  // [row][row_column(pixel)]: (u, alpha T)
 	float g_depth[72];                // upstream gradient of the depth image by pixel, eight of nine words
 	StripRays rays;
@@ -839,9 +858,12 @@ __device__ __forceinline__ float dpp_exchange_add(float v)
 	return v + __builtin_bit_cast(float, moved);
 }
 
-// The upstream colour gradients of the eight pixels that a lane sweeps in the entry-parallel part: the same for the whole walk.
-struct SweepUpstream {
+// What a lane needs in the entry-parallel part whatever the entries, held for the whole walk: the upstream colour gradients of
+// the eight pixels that it sweeps, their place in its entry's row, and the columns of `sums` that it adds to (of row 0).
+struct Sweep {
 	float r[8], g[8], b[8];   // (those of the depth image, where there are any, stay in LDS: BackwardStage::g_depth)
+	LdsPair* row;
+	float *column_low, *column_high;  // for entries 0-3 and for entries 4-7 of a pass
 };
 
 // Entry-parallel part for the eight entries staged from slot0 on.  A 16-lane row of the wavefront serves two entries, e in
@@ -857,25 +879,31 @@ struct SweepUpstream {
 // kDepth: a gradient arrived for the depth image (without one, the usual case of a loss on the colour image alone, the
 // terms it multiplies are left out: the depth column of `sums` stays zero).
 template <bool kDepth>
-__device__ __forceinline__ void sum_rows(const BackwardStage& st, int slot0, int entries, const SweepUpstream& upstream,
-                                         const StripFrame& f, const BlendArgs& a, int lane)
+__device__ __forceinline__ void sum_rows(const BackwardStage& st, int slot0, int entries, const Sweep& sweep, const StripFrame& f,
+                                         int lane)
 {
 #pragma clang fp contract(fast)
 	__builtin_amdgcn_wave_barrier();
 	const int upper = (lane >> 3) & 1;  // which eight of the 16-lane row
 	const int e = (lane >> 4) + 4 * upper, h = (lane >> 1) & 3, half = lane & 1, j = lane & 7;
 	const int slot = slot0 + e;
-	const float2* row = st.u_at + e * kRowStride + row_column(h * 16 + 8 * half);
-	float s0 = 0.f, s1 = 0.f, s2 = 0.f, cr = 0.f, cg = 0.f, cb = 0.f, cdp = 0.f;
+	// (the first pixel's terms start the sums: added to zeros they would take five instructions)
+	Pair ua = sweep.row[0];
+	float s0 = ua.x, cr = ua.y * sweep.r[0], cg = ua.y * sweep.g[0], cb = ua.y * sweep.b[0];
+	float cdp = kDepth ? ua.y * st.g_depth[9 * (lane & 7)] : 0.f;
+	ua = sweep.row[1];
+	float s1 = ua.x, s2 = ua.x;
 #pragma unroll
-	for (int step = 0; step < 8; step++) {
-		const float2 ua = row[step];
+	for (int step = 1; step < 8; step++) {
+		if (step > 1) {
+			ua = sweep.row[step];
+			s1 += (float)step * ua.x;
+			s2 += (float)(step * step) * ua.x;
+		}
 		s0 += ua.x;
-		s1 += (float)step * ua.x;
-		s2 += (float)(step * step) * ua.x;
-		cr += ua.y * upstream.r[step];
-		cg += ua.y * upstream.g[step];
-		cb += ua.y * upstream.b[step];
+		cr += ua.y * sweep.r[step];
+		cg += ua.y * sweep.g[step];
+		cb += ua.y * sweep.b[step];
 		if (kDepth)
 			cdp += ua.y * st.g_depth[9 * (lane & 7) + step];
 	}
@@ -896,42 +924,40 @@ __device__ __forceinline__ void sum_rows(const BackwardStage& st, int slot0, int
 	// (every lane forms all five products and then picks its own: a handful of multiplications more than the one or two
 	// a lane needs, but no branch per column and no wait for the conic inside one)
 	const float4 co = st.conic[slot];  // the staged conic: -xx / 2, -xy, -yy / 2, opacity
-	const uint32_t id = st.id[slot];
+	const uint32_t sum_row = st.sum_row[slot];
 	const float S0 = v[0], Sx = v[1], Sy = v[2], Sxx = v[3], Sxy = v[4], Syy = v[5];
 	const float half_w = -0.5f * co.w;
 	const float m0 = co.w * f.ddelx_dx * (2.f * co.x * Sx + co.y * Sy), m1 = co.w * f.ddely_dy * (2.f * co.z * Sy + co.y * Sx);
 	const float k0 = half_w * Sxx, k1 = half_w * Sxy, k3 = half_w * Syy;
 	// lane j of the eight holds column j of the row, lanes 0 and 1 also columns 8 and 9: see SumCol
 	// (picked bit by bit of j: a chain of comparisons becomes a switch)
-	const bool j0 = (j & 1) != 0, j1 = (j & 2) != 0, j2 = (j & 4) != 0, counts = e < entries;
+	const bool j0 = (j & 1) != 0, j1 = (j & 2) != 0, j2 = (j & 4) != 0;
 	const float c01 = j0 ? m1 : m0, c23 = j0 ? k1 : k0, c45 = j0 ? S0 : k3, c67 = j0 ? v[7] : v[6];
 	const float c03 = j1 ? c23 : c01, c47 = j1 ? c67 : c45;
 	const float c89 = j0 ? (kDepth ? v[9] : 0.f) : v[8];
-	const float first = counts ? (j2 ? c47 : c03) : 0.f, second = counts && !j1 && !j2 ? c89 : 0.f;
-	// columns 8 and 9 and the Gaussian's index go to the same lanes of the other eight of the 16-lane row (row_ror:8)
+	const float first = j2 ? c47 : c03, second = !j1 && !j2 ? c89 : 0.f;
+	// columns 8 and 9 and the Gaussian's row go to the same lanes of the other eight of the 16-lane row (row_ror:8)
 	const float second_there = __builtin_bit_cast(
 		float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, second), 0x128, 0xF, 0xF, true));
-	const uint32_t id_there = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)id, 0x128, 0xF, 0xF, true);
-	{
-		// entries 0-3: their own (lower) lanes add columns 0-7, the upper lanes columns 8 and 9 for them
-		const float value = upper ? second_there : first;
-		float* at = a.sums + (size_t)kSumCols * (upper ? id_there : id) + (upper ? 8 + j : j);
-		if (value != 0.f) unsafeAtomicAdd(at, value);
-	}
-	{
-		// entries 4-7: the other way round
-		const float value = upper ? first : second_there;
-		float* at = a.sums + (size_t)kSumCols * (upper ? id : id_there) + (upper ? j : 8 + j);
-		if (value != 0.f) unsafeAtomicAdd(at, value);
-	}
+	const uint32_t row_there = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)sum_row, 0x128, 0xF, 0xF, true);
+	// Entries 0-3: their own (lower) lanes add columns 0-7, the upper lanes columns 8 and 9 for them; then entries 4-7 the
+	// other way round.  Which entries there are is asked here alone: with a branch around the choices above, the
+	// compiler moves the last additions of the exchanges into it and their lane moves stay outside as instructions of their own.
+	const float low = upper ? second_there : first, high = upper ? first : second_there;
+	float* at_low = reinterpret_cast<float*>(reinterpret_cast<char*>(sweep.column_low) + ((uint64_t)(upper ? row_there : sum_row) << 4));
+	float* at_high = reinterpret_cast<float*>(reinterpret_cast<char*>(sweep.column_high) + ((uint64_t)(upper ? sum_row : row_there) << 4));
+	if ((lane >> 4) < entries && low != 0.f)
+		unsafeAtomicAdd(at_low, low);
+	if ((lane >> 4) + 4 < entries && high != 0.f)
+		unsafeAtomicAdd(at_high, high);
 	__builtin_amdgcn_wave_barrier();
 }
 
-// Pixel-parallel part for the four entries staged from slot k on; their rows are those from `row` on.  Returns whether
-// any pixel blended any of them.
+// Pixel-parallel part for the four entries staged from slot k on; `rows`: the pixel's place in the first of their rows.
+// Returns whether any pixel blended any of them.
 template <bool kDepth, bool kBoxed>
-__device__ __forceinline__ bool backward_rows(BackwardPixel& p, uint32_t last_contributor, BackwardStage& st, int k, int row,
-                                              const float2 pixf, const BoxSpan& span, const BlendArgs& a, int lane)
+__device__ __forceinline__ bool backward_rows(BackwardPixel& p, uint32_t last_contributor, const BackwardStage& st, int k,
+                                              LdsPair* rows, const float2 pixf, const BoxSpan& span, const BlendArgs& a)
 {
 	float power[4], clip_w[4], opacity[4];
 	uint64_t mask[4];
@@ -952,7 +978,7 @@ __device__ __forceinline__ bool backward_rows(BackwardPixel& p, uint32_t last_co
 	for (int i = 0; i < 4; i++)
 		cd[i] = st.cd[k + i];
 	__builtin_amdgcn_sched_barrier(0);
-	float alpha[4], G[4], inv[4], weighted[4], u[4], aT[4];
+	float alpha[4], G[4], inv[4], weighted[4];
 #pragma unroll
 	for (int i = 0; i < 4; i++) {
 		G[i] = exp_of_exponent(power[i]);
@@ -966,7 +992,6 @@ __device__ __forceinline__ bool backward_rows(BackwardPixel& p, uint32_t last_co
 		weighted[i] = __builtin_fmaf(cd[i].x, p.g_r, __builtin_fmaf(cd[i].y, p.g_g, __builtin_fmaf(cd[i].z, p.g_b, p.g_alpha)));
 		if (kDepth)
 			weighted[i] = __builtin_fmaf(cd[i].w, p.g_depth, weighted[i]);
-		u[i] = aT[i] = 0.f;
 	}
 	// The pixel's outputs are sums over its blended entries j of w_j (colour_j, depth_j, 1) with w_j = alpha_j T_j,
 	// T_j the product of (1 - alpha_k) over the entries in front, plus T_final times the background.  Their
@@ -982,6 +1007,8 @@ __device__ __forceinline__ bool backward_rows(BackwardPixel& p, uint32_t last_co
 #pragma unroll
 	for (int i = 0; i < 4; i++) {
 		float dL_dopa;
+		Pair z = zero_pair();
+		float u = z.x, aT = z.y;
 		asm("s_mov_b64 exec, %[lanes]\n\t"
 		    "v_mul_f32 %[T], %[T], %[inv]\n\t"
 		    "v_mul_f32 %[d], %[behind], %[inv]\n\t"
@@ -990,9 +1017,9 @@ __device__ __forceinline__ bool backward_rows(BackwardPixel& p, uint32_t last_co
 		    "v_fmac_f32 %[behind], %[aT], %[weighted]\n\t"
 		    "v_mul_f32 %[u], %[G], %[d]\n\t"
 		    "s_mov_b64 exec, -1"
-		    : [T] "+v"(p.T), [behind] "+v"(p.behind), [aT] "+v"(aT[i]), [u] "+v"(u[i]), [d] "=&v"(dL_dopa)
+		    : [T] "+v"(p.T), [behind] "+v"(p.behind), [aT] "+v"(aT), [u] "+v"(u), [d] "=&v"(dL_dopa)
 		    : [lanes] "s"(mask[i]), [inv] "v"(inv[i]), [alpha] "v"(alpha[i]), [weighted] "v"(weighted[i]), [G] "v"(G[i]));
-		st.u_at[(row + i) * kRowStride + row_column(lane)] = float2{u[i], aT[i]};
+		rows[i * kRowStride] = Pair{u, aT};
 	}
 	return (mask[0] | mask[1] | mask[2] | mask[3]) != 0ull;
 }
@@ -1046,8 +1073,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 	p.behind = T_final * ((0.f + a.bg[0] * p.g_r + a.bg[1] * p.g_g) + a.bg[2] * p.g_b);
 
 	stage_rays(st.rays, pixf, a, lane);
-	SweepUpstream upstream;
+	Sweep sweep;
 	{
+		const int upper = (lane >> 3) & 1, e = (lane >> 4) + 4 * upper, h = (lane >> 1) & 3, j = lane & 7;
+		sweep.row = lds_base(st.u_at + e * kRowStride + row_column(h * 16 + 8 * (lane & 1)));
+		sweep.column_low = a.sums + (upper ? 8 + j : j);
+		sweep.column_high = a.sums + (upper ? j : 8 + j);
 		float4* by_pixel = st.geom;  // (not in use yet)
 		by_pixel[lane] = float4{p.g_r, p.g_g, p.g_b, 0.f};
 		if (kDepth)
@@ -1056,12 +1087,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 #pragma unroll
 		for (int s = 0; s < 8; s++) {
 			const float4 g = by_pixel[8 * (lane & 7) + s];  // pixels of strip row (lane >> 1) & 3, half lane & 1
-			upstream.r[s] = g.x;
-			upstream.g[s] = g.y;
-			upstream.b[s] = g.z;
+			sweep.r[s] = g.x;
+			sweep.g[s] = g.y;
+			sweep.b[s] = g.z;
 		}
 		__builtin_amdgcn_wave_barrier();
 	}
+
+	LdsPair* const rows[2] = {lds_base(st.u_at + row_column(lane)), lds_base(st.u_at + 4 * kRowStride + row_column(lane))};
 
 	// Lane l of the chunk that starts `first` entries from the back takes filed entry
 	// filed-1-first-l: its list position (and box flag), through that the Gaussian's index,
@@ -1085,14 +1118,14 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 			st.conic[lane] = staged_conic(cur.conic);
 			st.cd[lane] = cur.cd;
 			st.entry[lane] = pos_cur & kPosition;
-			st.id[lane] = cur.id;
+			st.sum_row[lane] = kSumCols / 4 * cur.id;  // (32 bits hold it: a thousand million Gaussians' gradients fit no device)
 		}
 		if (lane < kRows - 1) {  // pad to a multiple of eight with entries behind every pixel's last one
 			st.geom[count + lane] = float4{0.f, 0.f, 0.f, 0.f};
 			st.conic[count + lane] = float4{0.f, 0.f, 0.f, 0.f};
 			st.cd[count + lane] = float4{0.f, 0.f, 0.f, 0.f};
 			st.entry[count + lane] = 0xFFFFFFFFu;
-			st.id[count + lane] = 0u;
+			st.sum_row[count + lane] = 0u;
 		}
 		const bool straddles = lane < count && (pos_cur & 0x80000000u) == 0u;
 		const bool boxed = lanes_where(straddles) != 0ull, all_in_front = lanes_where(straddles && !(cur.geom.w > 0.f)) == 0ull;
@@ -1109,17 +1142,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 		if (boxed) {
 			const BoxSpan span = span_for_visits(all_in_front, st.rays, a);
 			for (int k = 0; k < count; k += kRows) {
-				const bool front = backward_rows<kDepth, true>(p, last_contributor, st, k, 0, pixf, span, a, lane);
-				const bool back = backward_rows<kDepth, true>(p, last_contributor, st, k + 4, 4, pixf, span, a, lane);
+				const bool front = backward_rows<kDepth, true>(p, last_contributor, st, k, rows[0], pixf, span, a);
+				const bool back = backward_rows<kDepth, true>(p, last_contributor, st, k + 4, rows[1], pixf, span, a);
 				if (front || back)
-					sum_rows<kDepth>(st, k, count - k, upstream, frame, a, lane);
+					sum_rows<kDepth>(st, k, count - k, sweep, frame, lane);
 			}
 		} else {
 			for (int k = 0; k < count; k += kRows) {
-				const bool front = backward_rows<kDepth, false>(p, last_contributor, st, k, 0, pixf, BoxSpan{}, a, lane);
-				const bool back = backward_rows<kDepth, false>(p, last_contributor, st, k + 4, 4, pixf, BoxSpan{}, a, lane);
+				const bool front = backward_rows<kDepth, false>(p, last_contributor, st, k, rows[0], pixf, BoxSpan{}, a);
+				const bool back = backward_rows<kDepth, false>(p, last_contributor, st, k + 4, rows[1], pixf, BoxSpan{}, a);
 				if (front || back)
-					sum_rows<kDepth>(st, k, count - k, upstream, frame, a, lane);
+					sum_rows<kDepth>(st, k, count - k, sweep, frame, lane);
 			}
 		}
 		__builtin_amdgcn_wave_barrier();
