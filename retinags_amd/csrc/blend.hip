@@ -1164,7 +1164,29 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 // launch order needs.  Two small kernels: count the strips of every class, then place them; one
 // launch of each serves every job of a batch (blockIdx.y).  Both aggregate in LDS first: most
 // strips fall into one class (nothing to walk), and thousands of global atomics on one word would
-// take longer than the blend itself.
+// take longer than the blend itself.  What bounds them is the additions of all workgroups to the same few counters, so a
+// workgroup takes kOrderStrips strips, four per thread, and the lanes of the last class (little or nothing to walk, often
+// most of a wavefront) add to its LDS counter as one.
+constexpr uint32_t kOrderStrips = 1024;
+
+// The calling lane's place among its workgroup's strips of class c (all lanes come here).
+__device__ __forceinline__ uint32_t count_in_class(uint32_t* s_count, uint32_t c, bool valid)
+{
+	const uint64_t last = lanes_where(valid && c == kStripClasses - 1u);
+	uint32_t rank = 0;
+	if (valid && c != kStripClasses - 1u)
+		rank = atomicAdd(&s_count[c], 1u);
+	if (last != 0ull) {
+		uint32_t base = 0;
+		if (lanes_below(~0ull) == 0u)
+			base = atomicAdd(&s_count[kStripClasses - 1], (uint32_t)__popcll(last));
+		base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+		if (valid && c == kStripClasses - 1u)
+			rank = base + lanes_below(last);
+	}
+	return rank;
+}
+
 struct StripOrderJob {
 	const uint32_t* length;  // per strip
 	uint32_t* classes;       // kStripClasses counters and as many placement cursors, zero beforehand
@@ -1181,9 +1203,15 @@ __global__ __launch_bounds__(256) void strip_count_kernel(StripOrderBatch batch)
 	const StripOrderJob& j = batch.job[blockIdx.y];
 	s_count[threadIdx.x] = 0;
 	__syncthreads();
-	const uint32_t k = blockIdx.x * 256 + threadIdx.x;
-	if (k < batch.strips)
-		atomicAdd(&s_count[strip_class(j.length[k])], 1u);
+	uint32_t length[kOrderStrips / 256];
+#pragma unroll
+	for (uint32_t q = 0; q < kOrderStrips / 256; q++) {
+		const uint32_t k = blockIdx.x * kOrderStrips + 256 * q + threadIdx.x;
+		length[q] = k < batch.strips ? j.length[k] : 0u;
+	}
+#pragma unroll
+	for (uint32_t q = 0; q < kOrderStrips / 256; q++)
+		count_in_class(s_count, strip_class(length[q]), blockIdx.x * kOrderStrips + 256 * q + threadIdx.x < batch.strips);
 	__syncthreads();
 	if (s_count[threadIdx.x] != 0u)
 		atomicAdd(&j.classes[threadIdx.x], s_count[threadIdx.x]);
@@ -1196,21 +1224,29 @@ __global__ __launch_bounds__(256) void strip_place_kernel(StripOrderBatch batch)
 	const StripOrderJob& j = batch.job[blockIdx.y];
 	s_count[threadIdx.x] = 0;
 	__syncthreads();
-	const uint32_t k = blockIdx.x * 256 + threadIdx.x;
-	uint32_t c = 0, rank = 0;
-	if (k < batch.strips) {
-		c = strip_class(j.length[k]);
-		rank = atomicAdd(&s_count[c], 1u);
+	const uint32_t in_class = j.classes[threadIdx.x];
+	uint32_t c[kOrderStrips / 256], rank[kOrderStrips / 256];
+#pragma unroll
+	for (uint32_t q = 0; q < kOrderStrips / 256; q++) {
+		const uint32_t k = blockIdx.x * kOrderStrips + 256 * q + threadIdx.x;
+		c[q] = strip_class(k < batch.strips ? j.length[k] : 0u);
 	}
+#pragma unroll
+	for (uint32_t q = 0; q < kOrderStrips / 256; q++)
+		rank[q] = count_in_class(s_count, c[q], blockIdx.x * kOrderStrips + 256 * q + threadIdx.x < batch.strips);
 	__syncthreads();
 	uint32_t total;
-	const uint32_t start = block256_exclusive_scan_u32(j.classes[threadIdx.x], s_scan, total);
+	const uint32_t start = block256_exclusive_scan_u32(in_class, s_scan, total);
 	const uint32_t mine = s_count[threadIdx.x];
 	__syncthreads();
 	s_count[threadIdx.x] = start + (mine != 0u ? atomicAdd(&j.classes[kStripClasses + threadIdx.x], mine) : 0u);
 	__syncthreads();
-	if (k < batch.strips)
-		j.order[s_count[c] + rank] = k;
+#pragma unroll
+	for (uint32_t q = 0; q < kOrderStrips / 256; q++) {
+		const uint32_t k = blockIdx.x * kOrderStrips + 256 * q + threadIdx.x;
+		if (k < batch.strips)
+			j.order[s_count[c[q]] + rank[q]] = k;
+	}
 }
 
 // which: 0 = the forward's order (by the entries filed), 1 = the backward's (by the entries up to the last one blended)
@@ -1223,7 +1259,7 @@ static void launch_strip_order(const BlendArgs* jobs, int count, int which, hipS
 		b.job[k].classes = jobs[k].strip_classes + (which == 0 ? 2 * kStripClasses : 0);
 		b.job[k].order = which == 0 ? jobs[k].strip_order_forward : jobs[k].strip_order;
 	}
-	const dim3 grid((b.strips + 255) / 256, (unsigned)count);
+	const dim3 grid((b.strips + kOrderStrips - 1) / kOrderStrips, (unsigned)count);
 	hipLaunchKernelGGL(strip_count_kernel, grid, dim3(256), 0, s, b);
 	hipLaunchKernelGGL(strip_place_kernel, grid, dim3(256), 0, s, b);
 }
