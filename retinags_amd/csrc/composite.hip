@@ -15,13 +15,30 @@ __global__ __launch_bounds__(256) void composite_forward_kernel(CompositeArgs a)
 	if (p >= n)
 		return;
 	float T = 1.f, r = 0.f, g = 0.f, b = 0.f, d = 0.f;
-	for (int k = 0; k < a.K; k++) {
-		const float* img = a.images[k];
-		r += T * img[p];
-		g += T * img[n + p];
-		b += T * img[2 * n + p];
-		d += T * a.depths[k][p];
-		T = T * (1.f - a.alphas[k][p]);
+	// kAhead layers' planes are asked for together: one layer at a time, the kernel waited for memory once per layer with five
+	// requests on their way
+	constexpr int kAhead = 4;
+	for (int k0 = 0; k0 < a.K; k0 += kAhead) {
+		float v[kAhead][5];
+#pragma unroll
+		for (int q = 0; q < kAhead; q++)
+			if (k0 + q < a.K) {
+				const float* img = a.images[k0 + q];
+				v[q][0] = img[p];
+				v[q][1] = img[n + p];
+				v[q][2] = img[2 * n + p];
+				v[q][3] = a.depths[k0 + q][p];
+				v[q][4] = a.alphas[k0 + q][p];
+			}
+#pragma unroll
+		for (int q = 0; q < kAhead; q++)
+			if (k0 + q < a.K) {
+				r += T * v[q][0];
+				g += T * v[q][1];
+				b += T * v[q][2];
+				d += T * v[q][3];
+				T = T * (1.f - v[q][4]);
+			}
 	}
 	float bg0 = 0.f, bg1 = 0.f, bg2 = 0.f;
 	if (a.bg) {
