@@ -844,28 +844,28 @@ __global__ __launch_bounds__(256) void sort_onesweep_kernel(Batch<SortJob<KeyT>>
 		val[i] = ok ? vals_in[k] : 0u;
 	}
 
-	const uint64_t lanes_below = (1ull << lane) - 1ull;
 #pragma unroll
 	for (int i = 0; i < kSortItems; i++) {
 		const size_t k = wave_base + (size_t)i * 64 + lane;
 		// Padding elements rank as the last digit value after every real element, so they never disturb one.
 		const uint32_t d = (k < n) ? digit_of(key[i], shift, mask) : (uint32_t)(kBins - 1);
-		uint64_t same = ~0ull;
+		// the lanes with this lane's digit: a vote per bit, taken as it is or inverted by a mask made of the lane's own bit
+		uint32_t same_lo = ~0u, same_hi = ~0u;
 #pragma unroll
 		for (int b = 0; b < kBits; b++) {
-			const bool bit = (d >> b) & 1u;
-			const uint64_t vote = lanes_where(bit);
-			same &= bit ? vote : ~vote;
+			int own = (int)(d << (31 - b)) >> 31;
+			asm("" : "+v"(own));  // (or the compiler forms the bit a second time for the vote)
+			const uint64_t vote = lanes_where(own != 0);
+			// same & ~(vote ^ own), one instruction
+			same_lo = (uint32_t)__builtin_amdgcn_bitop3_b32((int)same_lo, (int)(uint32_t)vote, own, 0x90);
+			same_hi = (uint32_t)__builtin_amdgcn_bitop3_b32((int)same_hi, (int)(uint32_t)(vote >> 32), own, 0x90);
 		}
-		const uint32_t below = (uint32_t)__popcll(same & lanes_below);
-		const uint32_t count = (uint32_t)__popcll(same);
-		const int leader = __ffsll((unsigned long long)same) - 1;
-		uint32_t prior = 0;
-		if (lane == leader) {
-			prior = sc.wave_hist[wave][d];
-			sc.wave_hist[wave][d] = (uint16_t)(prior + count);
-		}
-		prior = __shfl(prior, leader);
+		const uint32_t below = __builtin_amdgcn_mbcnt_hi(same_hi, __builtin_amdgcn_mbcnt_lo(same_lo, 0u));
+		// every lane reads its digit's count (lanes of one digit the same word), then the first of each digit's lanes adds theirs:
+		// a wavefront's LDS accesses are served in order
+		const uint32_t prior = sc.wave_hist[wave][d];
+		if (below == 0u)
+			sc.wave_hist[wave][d] = (uint16_t)(prior + (uint32_t)__popc(same_lo) + (uint32_t)__popc(same_hi));
 		rank[i] = prior + below;
 		__builtin_amdgcn_wave_barrier();
 	}
