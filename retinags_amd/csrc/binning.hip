@@ -766,25 +766,27 @@ enum SortPassKind { kPassPlain = 0, kPassEndsUnless = 1, kPassOnDemand = 2 };
 // Per-wave digit counts fit 16 bits (a wavefront ranks kSortItems * 64 keys), and so does a digit's place inside a tile.
 template <int kBits>
 struct SortCounts {
-	uint16_t wave_hist[4][1 << kBits];  // per-wave digit counts, then exclusive prefix over waves
 	uint16_t digit_base[1 << kBits];    // exclusive prefix over digits within the tile
 	uint32_t global_base[1 << kBits];   // where this tile's run of each digit starts globally
 };
 
+// A workgroup's life is a chain of phases (loads, ranking, look-back, stores) and how many wavefronts stand by to fill the
+// gaps of the others' sets the pace of a pass, not memory: eight wavefronts of eight pairs per lane rank a tile in half the
+// steps that four of sixteen take, and with half the registers 32 instead of 16 of them fit a CU (the counts of the
+// ranking lie where the tile's keys go afterwards, which keeps four workgroups' LDS in a CU).
 template <typename KeyT, int kBits, int kKind>
-__global__ __launch_bounds__(256) void sort_onesweep_kernel(Batch<SortJob<KeyT>> batch, int pass, int shift, uint32_t mask,
-                                                             int spin_limit)
+__global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(sizeof(KeyT) == 4 ? 8 : 4))) void sort_onesweep_kernel(
+	Batch<SortJob<KeyT>> batch, int pass, int shift, uint32_t mask, int spin_limit)
 {
 	constexpr int kBins = 1 << kBits;
-	constexpr int kOwn = kBins / 256;  // digit values a thread owns: kOwn * tid .. kOwn * tid + kOwn - 1
-	static_assert(kOwn == 1 || kOwn == 2, "256 threads own one or two digit values each");
+	constexpr int kWaves = kSortThreads / 64;
+	static_assert(kBins <= kSortThreads, "a thread owns at most one digit value");
 	const SortJob<KeyT>& j = batch.job[blockIdx.y];
 	// the passes ping-pong between the two buffer pairs, starting in -> out
 	const KeyT* __restrict__ keys_in = (pass & 1) ? j.keys_out : j.keys_in;
 	const uint32_t* __restrict__ vals_in = (pass & 1) ? j.vals_out : j.vals_in;
 	KeyT* __restrict__ keys_out = (pass & 1) ? j.keys_in : j.keys_out;
 	uint32_t* __restrict__ vals_out = (pass & 1) ? j.vals_in : j.vals_out;
-	size_t n = j.n;
 	const uint32_t* __restrict__ n_device = j.n_device;
 	const size_t job_tiles = (j.n + kSortBlock - 1) / kSortBlock;
 	if (blockIdx.x >= job_tiles)
@@ -805,40 +807,40 @@ __global__ __launch_bounds__(256) void sort_onesweep_kernel(Batch<SortJob<KeyT>>
 	__shared__ KeyT s_keys[kSortBlock];
 	__shared__ uint32_t s_vals[kSortBlock];
 	__shared__ SortCounts<kBits> sc;
-	__shared__ uint32_t s_scan[8];
+	__shared__ uint32_t s_scan[kWaves];
+	// per-wave digit counts, then their exclusive prefix over waves; the keys take their place when all have been read
+	uint16_t (*const wave_hist)[kBins] = reinterpret_cast<uint16_t (*)[kBins]>(s_keys);
+	static_assert(sizeof(s_keys) >= kWaves * kBins * sizeof(uint16_t), "the counts fit where the keys go");
 	__shared__ uint32_t s_tile;
 
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 	// asked for before anything else: needed only after the look-back, by when it has long arrived
-	uint32_t digit_total[kOwn];
-#pragma unroll
-	for (int o = 0; o < kOwn; o++)
-		digit_total[o] = digit_count[kOwn * tid + o];
+	const bool owns = tid < kBins;
+	const uint32_t digit_total = owns ? digit_count[tid] : 0u;
 	// Tiles are handed out in arrival order, so every tile a block waits for below belongs to
 	// a block that is already running.
 	if (tid == 0)
 		s_tile = atomicAdd(tile_counter, 1u);
 #pragma unroll
-	for (int w = 0; w < 4; w++)
-#pragma unroll
-		for (int o = 0; o < kOwn; o++)
-			sc.wave_hist[w][kOwn * tid + o] = 0;
+	for (int w = 0; w < kWaves * kBins / 2 / kSortThreads; w++)
+		reinterpret_cast<uint32_t*>(s_keys)[w * kSortThreads + tid] = 0u;
 	__syncthreads();
 	const uint32_t tile = s_tile;
-	const size_t block_base = (size_t)tile * kSortBlock;
+	const uint32_t block_base = tile * (uint32_t)kSortBlock;
+	uint32_t n = (uint32_t)j.n;  // (fewer than 2^30: the look-back words hold no more)
 	if (n_device)
-		n = min(n, (size_t)*n_device);
+		n = (uint32_t)min(j.n, (size_t)*n_device);
 	// launched for an upper bound of n: tiles beyond the data leave, and no tile waits for them
 	if (block_base >= n)
 		return;
-	const size_t wave_base = block_base + (size_t)wave * (kSortItems * 64);
+	const uint32_t wave_base = block_base + (uint32_t)wave * (kSortItems * 64);
 
 	KeyT key[kSortItems];
 	uint32_t val[kSortItems];
 	uint32_t rank[kSortItems];
 #pragma unroll
 	for (int i = 0; i < kSortItems; i++) {
-		const size_t k = wave_base + (size_t)i * 64 + lane;
+		const uint32_t k = wave_base + (uint32_t)(i * 64 + lane);
 		const bool ok = k < n;
 		key[i] = ok ? keys_in[k] : (KeyT)~(KeyT)0;
 		val[i] = ok ? vals_in[k] : 0u;
@@ -846,7 +848,7 @@ __global__ __launch_bounds__(256) void sort_onesweep_kernel(Batch<SortJob<KeyT>>
 
 #pragma unroll
 	for (int i = 0; i < kSortItems; i++) {
-		const size_t k = wave_base + (size_t)i * 64 + lane;
+		const uint32_t k = wave_base + (uint32_t)(i * 64 + lane);
 		// Padding elements rank as the last digit value after every real element, so they never disturb one.
 		const uint32_t d = (k < n) ? digit_of(key[i], shift, mask) : (uint32_t)(kBins - 1);
 		// the lanes with this lane's digit: a vote per bit, taken as it is or inverted by a mask made of the lane's own bit
@@ -863,72 +865,56 @@ __global__ __launch_bounds__(256) void sort_onesweep_kernel(Batch<SortJob<KeyT>>
 		const uint32_t below = __builtin_amdgcn_mbcnt_hi(same_hi, __builtin_amdgcn_mbcnt_lo(same_lo, 0u));
 		// every lane reads its digit's count (lanes of one digit the same word), then the first of each digit's lanes adds theirs:
 		// a wavefront's LDS accesses are served in order
-		const uint32_t prior = sc.wave_hist[wave][d];
+		const uint32_t prior = wave_hist[wave][d];
 		if (below == 0u)
-			sc.wave_hist[wave][d] = (uint16_t)(prior + (uint32_t)__popc(same_lo) + (uint32_t)__popc(same_hi));
+			wave_hist[wave][d] = (uint16_t)(prior + (uint32_t)__popc(same_lo) + (uint32_t)__popc(same_hi));
 		rank[i] = prior + below;
 		__builtin_amdgcn_wave_barrier();
 	}
 	__syncthreads();
 
-	// A thread owns kOwn neighbouring digit values: prefix over the 4 waves, publish the tile's counts.
-	const size_t remaining = n - block_base;
-	const uint32_t valid = remaining < (size_t)kSortBlock ? (uint32_t)remaining : (uint32_t)kSortBlock;
-	uint32_t* const my_word = lookback + (size_t)tile * kBins + kOwn * tid;
-	uint32_t count[kOwn], digit_start[kOwn];
+	// A thread owns a digit value: prefix over the waves, publish the tile's count.
+	const uint32_t valid = min(n - block_base, (uint32_t)kSortBlock);
+	uint32_t* const my_word = lookback + (size_t)tile * kBins + tid;
+	uint32_t count = 0, digit_start;
 	{
-		uint32_t mine = 0;
+		if (owns) {
+			uint32_t c[kWaves];
 #pragma unroll
-		for (int o = 0; o < kOwn; o++) {
-			const int d = kOwn * tid + o;
-			const uint32_t c0 = sc.wave_hist[0][d], c1 = sc.wave_hist[1][d], c2 = sc.wave_hist[2][d], c3 = sc.wave_hist[3][d];
-			sc.wave_hist[0][d] = 0;
-			sc.wave_hist[1][d] = (uint16_t)c0;
-			sc.wave_hist[2][d] = (uint16_t)(c0 + c1);
-			sc.wave_hist[3][d] = (uint16_t)(c0 + c1 + c2);
-			count[o] = c0 + c1 + c2 + c3;
-			mine += count[o];
+			for (int w = 0; w < kWaves; w++)
+				c[w] = wave_hist[w][tid];
+#pragma unroll
+			for (int w = 0; w < kWaves; w++) {
+				wave_hist[w][tid] = (uint16_t)count;
+				count += c[w];
+			}
 		}
 		uint32_t total;
-		uint32_t ex = block256_exclusive_scan_u32(mine, s_scan, total);
-#pragma unroll
-		for (int o = 0; o < kOwn; o++) {
-			sc.digit_base[kOwn * tid + o] = (uint16_t)ex;
-			ex += count[o];
-		}
-		if (tid == 255)
-			count[kOwn - 1] -= (uint32_t)kSortBlock - valid;  // padding is not published
-		const uint32_t flag = tile == 0 ? kFlagInclusive : kFlagAggregate;
-		if (kOwn == 1) {
-			__hip_atomic_store(my_word, count[0] | flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-		} else {
-			// both counts in one 8-byte store: a reader sees the pair published or not, never one of the two
-			__hip_atomic_store(reinterpret_cast<uint64_t*>(my_word),
-			                   (uint64_t)(count[0] | flag) | ((uint64_t)(count[kOwn - 1] | flag) << 32), __ATOMIC_RELAXED,
-			                   __HIP_MEMORY_SCOPE_AGENT);
-		}
+		const uint32_t ex = block_exclusive_scan_u32<kWaves>(count, s_scan, total);
+		if (owns)
+			sc.digit_base[tid] = (uint16_t)ex;
+		if (tid == kBins - 1)
+			count -= (uint32_t)kSortBlock - valid;  // padding is not published
+		if (owns)
+			__hip_atomic_store(my_word, count | (tile == 0 ? kFlagInclusive : kFlagAggregate), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 		// where the digit's run starts in the whole array: the exclusive scan of the digit counts
-		uint32_t all, totals = 0;
-#pragma unroll
-		for (int o = 0; o < kOwn; o++)
-			totals += digit_total[o];
-		uint32_t start = block256_exclusive_scan_u32(totals, s_scan, all);
-#pragma unroll
-		for (int o = 0; o < kOwn; o++) {
-			digit_start[o] = start;
-			start += digit_total[o];
-		}
+		uint32_t all;
+		digit_start = block_exclusive_scan_u32<kWaves>(digit_total, s_scan, all);
 	}
 
 	// The tile's pairs in digit order, through LDS.  None of this needs the tiles before this one: by the time
 	// the look-back below starts, more of them have finished theirs and it has fewer words to read.
 #pragma unroll
 	for (int i = 0; i < kSortItems; i++) {
-		const size_t k = wave_base + (size_t)i * 64 + lane;
+		const uint32_t k = wave_base + (uint32_t)(i * 64 + lane);
 		const uint32_t d = (k < n) ? digit_of(key[i], shift, mask) : (uint32_t)(kBins - 1);
-		const uint32_t pos = (uint32_t)sc.digit_base[d] + (uint32_t)sc.wave_hist[wave][d] + rank[i];
-		s_keys[pos] = key[i];
-		s_vals[pos] = val[i];
+		rank[i] += (uint32_t)sc.digit_base[d] + (uint32_t)wave_hist[wave][d];
+	}
+	__syncthreads();  // the counts have been read
+#pragma unroll
+	for (int i = 0; i < kSortItems; i++) {
+		s_keys[rank[i]] = key[i];
+		s_vals[rank[i]] = val[i];
 	}
 	__syncthreads();
 	// every LDS read of the thread is asked for before anything needs one
@@ -936,54 +922,35 @@ __global__ __launch_bounds__(256) void sort_onesweep_kernel(Batch<SortJob<KeyT>>
 	uint32_t out_val[kSortItems];
 #pragma unroll
 	for (int i = 0; i < kSortItems; i++) {
-		const uint32_t p = (uint32_t)i * 256 + tid;
+		const uint32_t p = (uint32_t)i * kSortThreads + tid;
 		const uint32_t q = p < valid ? p : 0u;
 		out_key[i] = s_keys[q];
 		out_val[i] = s_vals[q];
 	}
 
-	// Look back: the pairs of this thread's digit values in all earlier tiles.
-	{
-		uint32_t exclusive[kOwn];
-#pragma unroll
-		for (int o = 0; o < kOwn; o++)
-			exclusive[o] = 0;
+	// Look back: the pairs of this thread's digit value in all earlier tiles.
+	if (owns) {
+		uint32_t exclusive = 0;
 		if (tile != 0) {
 			// Words of the tiles below t are still to be added.  Up to kLookBatch of them are requested
 			// together: walked one load at a time, the chain of tiles and not memory sets the pace of a pass.
 			uint32_t t = tile;
 			bool gave_up = spin_limit < 0, done = false;
 			while (!gave_up && !done) {
-				uint32_t v[kLookBatch][kOwn];
+				uint32_t v[kLookBatch];
 #pragma unroll
-				for (int q = 0; q < kLookBatch; q++) {
-					const uint32_t* word = lookback + (size_t)(t - 1u - (uint32_t)q) * kBins + kOwn * tid;
-					if ((uint32_t)q < t) {
-						if (kOwn == 1) {
-							v[q][0] = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-						} else {
-							const uint64_t both = __hip_atomic_load(reinterpret_cast<const uint64_t*>(word), __ATOMIC_RELAXED,
-							                                        __HIP_MEMORY_SCOPE_AGENT);
-							v[q][0] = (uint32_t)both;
-							v[q][kOwn - 1] = (uint32_t)(both >> 32);
-						}
-					} else {
-#pragma unroll
-						for (int o = 0; o < kOwn; o++)
-							v[q][o] = kFlagInclusive;  // below the first tile there is nothing
-					}
-				}
+				for (int q = 0; q < kLookBatch; q++)
+					v[q] = (uint32_t)q < t ? __hip_atomic_load(lookback + (size_t)(t - 1u - (uint32_t)q) * kBins + tid, __ATOMIC_RELAXED,
+					                                           __HIP_MEMORY_SCOPE_AGENT)
+					                       : kFlagInclusive;  // below the first tile there is nothing
 				uint32_t used = 0;
 #pragma unroll
 				for (int q = 0; q < kLookBatch; q++) {
-					// a word counts once every nearer one has been published and none of them closed the sum (a tile's
-					// words are published together and carry the same flag, so the first tells for all)
-					if (!done && used == (uint32_t)q && (v[q][0] >> 30) != 0u) {
-#pragma unroll
-						for (int o = 0; o < kOwn; o++)
-							exclusive[o] += v[q][o] & kValueMask;
+					// a word counts once every nearer one has been published and none of them closed the sum
+					if (!done && used == (uint32_t)q && (v[q] >> 30) != 0u) {
+						exclusive += v[q] & kValueMask;
 						used = (uint32_t)q + 1u;
-						done = (v[q][0] & kFlagInclusive) != 0u;
+						done = (v[q] & kFlagInclusive) != 0u;
 					}
 				}
 				t -= used < t ? used : t;
@@ -991,7 +958,7 @@ __global__ __launch_bounds__(256) void sort_onesweep_kernel(Batch<SortJob<KeyT>>
 					done = true;
 				if (!done && used < (uint32_t)kLookBatch) {
 					// tile t - 1 has not published yet: wait for its word, then look again from there
-					const uint32_t* word = lookback + (size_t)(t - 1u) * kBins + kOwn * tid;
+					const uint32_t* word = lookback + (size_t)(t - 1u) * kBins + tid;
 					uint32_t w = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 					for (int spins = 0; (w >> 30) == 0u; spins++) {
 						// give up after a bounded wait, or as soon as any other look-back has
@@ -1010,28 +977,18 @@ __global__ __launch_bounds__(256) void sort_onesweep_kernel(Batch<SortJob<KeyT>>
 				atomicOr(status, 1u);
 			// On the (never expected) give-up path `exclusive` is too small, which keeps every
 			// scatter address inside the array; the status word tells the consumer to discard it.
-			if (kOwn == 1) {
-				__hip_atomic_store(my_word, ((exclusive[0] + count[0]) & kValueMask) | kFlagInclusive, __ATOMIC_RELAXED,
-				                   __HIP_MEMORY_SCOPE_AGENT);
-			} else {
-				__hip_atomic_store(reinterpret_cast<uint64_t*>(my_word),
-				                   (uint64_t)(((exclusive[0] + count[0]) & kValueMask) | kFlagInclusive) |
-				                       ((uint64_t)(((exclusive[kOwn - 1] + count[kOwn - 1]) & kValueMask) | kFlagInclusive) << 32),
-				                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-			}
+			__hip_atomic_store(my_word, ((exclusive + count) & kValueMask) | kFlagInclusive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 		}
-#pragma unroll
-		for (int o = 0; o < kOwn; o++)
-			sc.global_base[kOwn * tid + o] = digit_start[o] + exclusive[o];
+		sc.global_base[tid] = digit_start + exclusive;
 	}
 	__syncthreads();
 
-	size_t out_at[kSortItems];
+	uint32_t out_at[kSortItems];  // (fewer than 2^30 pairs)
 #pragma unroll
 	for (int i = 0; i < kSortItems; i++) {
-		const uint32_t p = (uint32_t)i * 256 + tid;
+		const uint32_t p = (uint32_t)i * kSortThreads + tid;
 		const uint32_t d = digit_of(out_key[i], shift, mask);
-		out_at[i] = p < valid ? (size_t)sc.global_base[d] + (p - (uint32_t)sc.digit_base[d]) : n;
+		out_at[i] = p < valid ? sc.global_base[d] + (p - (uint32_t)sc.digit_base[d]) : n;
 	}
 	if (kKind != kPassPlain && ends_here) {
 		// the sort ends here: a value's index and tile count go to arrays of their own (a count stored as all ones did
@@ -1119,7 +1076,7 @@ static void sort_pairs(const SortJob<KeyT>* jobs, int count, int end_bit, bool t
 			const uint32_t mask = (1u << bits) - 1u;
 			if (mark_stages)
 				stage_mark("sort_onesweep", s);
-			hipLaunchKernelGGL((sort_onesweep_kernel<KeyT, kBits, kPassPlain>), dim3(max_tiles, (unsigned)live), dim3(256), 0, s, b, p, shift,
+			hipLaunchKernelGGL((sort_onesweep_kernel<KeyT, kBits, kPassPlain>), dim3(max_tiles, (unsigned)live), dim3(kSortThreads), 0, s, b, p, shift,
 			                   mask, g_lookback_spin_limit.load());
 		}
 	}
@@ -1177,10 +1134,10 @@ void launch_depth_order(const DepthOrderJob* jobs, int count, hipStream_t s)
 		// three passes of nine bits (a -> b -> a -> the order and the tile counts in that order), and the pass on demand
 		const dim3 tiles((unsigned)((max_p + kSortBlock - 1) / kSortBlock), (unsigned)nj);
 		const int spin = g_lookback_spin_limit.load();
-		hipLaunchKernelGGL((sort_onesweep_kernel<uint32_t, 9, kPassPlain>), tiles, dim3(256), 0, s, sorts, 0, 0, 511u, spin);
-		hipLaunchKernelGGL((sort_onesweep_kernel<uint32_t, 9, kPassPlain>), tiles, dim3(256), 0, s, sorts, 1, 9, 511u, spin);
-		hipLaunchKernelGGL((sort_onesweep_kernel<uint32_t, 9, kPassEndsUnless>), tiles, dim3(256), 0, s, sorts, 2, 18, 511u, spin);
-		hipLaunchKernelGGL((sort_onesweep_kernel<uint32_t, 9, kPassOnDemand>), tiles, dim3(256), 0, s, sorts, 3, kDepthKeyBits, 31u, spin);
+		hipLaunchKernelGGL((sort_onesweep_kernel<uint32_t, 9, kPassPlain>), tiles, dim3(kSortThreads), 0, s, sorts, 0, 0, 511u, spin);
+		hipLaunchKernelGGL((sort_onesweep_kernel<uint32_t, 9, kPassPlain>), tiles, dim3(kSortThreads), 0, s, sorts, 1, 9, 511u, spin);
+		hipLaunchKernelGGL((sort_onesweep_kernel<uint32_t, 9, kPassEndsUnless>), tiles, dim3(kSortThreads), 0, s, sorts, 2, 18, 511u, spin);
+		hipLaunchKernelGGL((sort_onesweep_kernel<uint32_t, 9, kPassOnDemand>), tiles, dim3(kSortThreads), 0, s, sorts, 3, kDepthKeyBits, 31u, spin);
 		hipLaunchKernelGGL(order_totals_kernel, grid, dim3(256), 0, s, b);
 		if (!few_groups)
 			hipLaunchKernelGGL(single_block_exclusive_scan_kernel, dim3(1, (unsigned)nj), dim3(1024), 0, s, scan);

@@ -186,25 +186,32 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v)
 	return max(max(r0, r1), max(r2, r3));
 }
 
-// Exclusive prefix sum of one u32 per thread over a 256-thread block.
-// `lds` needs 5 words; returns the block total in `total`.
-__device__ __forceinline__ uint32_t block256_exclusive_scan_u32(uint32_t v, uint32_t* lds, uint32_t& total)
+// Exclusive prefix sum of one u32 per thread over a block of kWaves wavefronts.
+// `lds` needs kWaves words; returns the block total in `total`.
+template <int kWaves>
+__device__ __forceinline__ uint32_t block_exclusive_scan_u32(uint32_t v, uint32_t* lds, uint32_t& total)
 {
 	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 	uint32_t inc = wave_inclusive_scan_u32(v);
 	if (lane == 63)
 		lds[wave] = inc;
 	__syncthreads();
-	uint32_t base = 0;
+	uint32_t base = 0, sum = 0;
 #pragma unroll
-	for (int w = 0; w < 4; w++) {
+	for (int w = 0; w < kWaves; w++) {
 		uint32_t s = lds[w];
 		if (w < wave)
 			base += s;
+		sum += s;
 	}
-	total = lds[0] + lds[1] + lds[2] + lds[3];
+	total = sum;
 	__syncthreads();
 	return base + inc - v;
+}
+
+__device__ __forceinline__ uint32_t block256_exclusive_scan_u32(uint32_t v, uint32_t* lds, uint32_t& total)
+{
+	return block_exclusive_scan_u32<4>(v, lds, total);
 }
 
 }  // namespace rgs

@@ -309,8 +309,9 @@ __host__ __device__ inline int sort_digit_shift(int end_bit, int p, int max_bits
 	const int n = sort_passes(end_bit, max_bits);
 	return p * (end_bit / n) + (p < end_bit % n ? p : end_bit % n);
 }
-constexpr int kSortItems = 16;                    // keys per thread in one sort block
-constexpr int kSortBlock = 256 * kSortItems;      // keys per sort block
+constexpr int kSortThreads = 512;
+constexpr int kSortItems = 8;                           // keys per thread in one sort block
+constexpr int kSortBlock = kSortThreads * kSortItems;   // keys per sort block
 size_t scan_temp_words(size_t n);                 // u32 words of scratch for launch_inclusive_sum
 // `stage` (may be null) names the stage for the timing aid.
 void launch_inclusive_sum(const uint32_t* in, uint32_t* out, size_t n, uint32_t* temp, const char* stage,
