@@ -309,7 +309,7 @@ __host__ __device__ inline int sort_digit_shift(int end_bit, int p, int max_bits
 	const int n = sort_passes(end_bit, max_bits);
 	return p * (end_bit / n) + (p < end_bit % n ? p : end_bit % n);
 }
-constexpr int kSortThreads = 512;
+constexpr int kSortThreads = 1024;
 constexpr int kSortItems = 8;                           // keys per thread in one sort block
 constexpr int kSortBlock = kSortThreads * kSortItems;   // keys per sort block
 size_t scan_temp_words(size_t n);                 // u32 words of scratch for launch_inclusive_sum
