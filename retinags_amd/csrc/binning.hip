@@ -770,16 +770,15 @@ struct SortCounts {
 	uint32_t global_base[1 << kBits];   // where this tile's run of each digit starts globally
 };
 
-// A workgroup's life is a chain of phases (loads, ranking, look-back, stores) and how many wavefronts stand by to fill the
-// gaps of the others' sets the pace of a pass, not memory: eight wavefronts of eight pairs per lane rank a tile in half the
-// steps that four of sixteen take, and with half the registers 32 instead of 16 of them fit a CU (the counts of the
-// ranking lie where the tile's keys go afterwards, which keeps four workgroups' LDS in a CU).
-template <typename KeyT, int kBits, int kKind>
-__global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(sizeof(KeyT) == 4 ? 8 : 4))) void sort_onesweep_kernel(
+// How many wavefronts stand by to fill the gaps of the others' phases (loads, ranking, look-back, stores) and how long the runs are
+// that a tile writes set the pace of a pass: sixteen wavefronts per tile, 32 per CU with up to eight pairs per lane (64
+// registers; the counts of the ranking lie where the tile's keys go afterwards), 16 with sixteen.
+template <typename KeyT, int kBits, int kKind, int kItems>
+__global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(sizeof(KeyT) == 4 && kItems <= 8 ? 8 : 4))) void sort_onesweep_kernel(
 	Batch<SortJob<KeyT>> batch, int pass, int shift, uint32_t mask, int spin_limit)
 {
 	constexpr int kBins = 1 << kBits;
-	constexpr int kWaves = kSortThreads / 64;
+	constexpr int kWaves = kSortThreads / 64, kBlock = kSortThreads * kItems;
 	static_assert(kBins <= kSortThreads, "a thread owns at most one digit value");
 	const SortJob<KeyT>& j = batch.job[blockIdx.y];
 	// the passes ping-pong between the two buffer pairs, starting in -> out
@@ -788,7 +787,7 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 	KeyT* __restrict__ keys_out = (pass & 1) ? j.keys_in : j.keys_out;
 	uint32_t* __restrict__ vals_out = (pass & 1) ? j.vals_in : j.vals_out;
 	const uint32_t* __restrict__ n_device = j.n_device;
-	const size_t job_tiles = (j.n + kSortBlock - 1) / kSortBlock;
+	const size_t job_tiles = (j.n + kBlock - 1) / kBlock;
 	if (blockIdx.x >= job_tiles)
 		return;  // the launch is sized for the job with the most tiles
 	bool ends_here = false;
@@ -804,8 +803,8 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 	uint32_t* __restrict__ lookback = j.temp + kSortHeader + (size_t)pass * kBins * job_tiles;
 	uint32_t* __restrict__ tile_counter = j.temp + kSortCounters + pass;
 	uint32_t* __restrict__ status = j.temp + kSortStatus;
-	__shared__ KeyT s_keys[kSortBlock];
-	__shared__ uint32_t s_vals[kSortBlock];
+	__shared__ KeyT s_keys[kBlock];
+	__shared__ uint32_t s_vals[kBlock];
 	__shared__ SortCounts<kBits> sc;
 	__shared__ uint32_t s_scan[kWaves];
 	// per-wave digit counts, then their exclusive prefix over waves; the keys take their place when all have been read
@@ -826,20 +825,20 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 		reinterpret_cast<uint32_t*>(s_keys)[w * kSortThreads + tid] = 0u;
 	__syncthreads();
 	const uint32_t tile = s_tile;
-	const uint32_t block_base = tile * (uint32_t)kSortBlock;
+	const uint32_t block_base = tile * (uint32_t)kBlock;
 	uint32_t n = (uint32_t)j.n;  // (fewer than 2^30: the look-back words hold no more)
 	if (n_device)
 		n = (uint32_t)min(j.n, (size_t)*n_device);
 	// launched for an upper bound of n: tiles beyond the data leave, and no tile waits for them
 	if (block_base >= n)
 		return;
-	const uint32_t wave_base = block_base + (uint32_t)wave * (kSortItems * 64);
+	const uint32_t wave_base = block_base + (uint32_t)wave * (kItems * 64);
 
-	KeyT key[kSortItems];
-	uint32_t val[kSortItems];
-	uint32_t rank[kSortItems];
+	KeyT key[kItems];
+	uint32_t val[kItems];
+	uint32_t rank[kItems];
 #pragma unroll
-	for (int i = 0; i < kSortItems; i++) {
+	for (int i = 0; i < kItems; i++) {
 		const uint32_t k = wave_base + (uint32_t)(i * 64 + lane);
 		const bool ok = k < n;
 		key[i] = ok ? keys_in[k] : (KeyT)~(KeyT)0;
@@ -847,7 +846,7 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 	}
 
 #pragma unroll
-	for (int i = 0; i < kSortItems; i++) {
+	for (int i = 0; i < kItems; i++) {
 		const uint32_t k = wave_base + (uint32_t)(i * 64 + lane);
 		// Padding elements rank as the last digit value after every real element, so they never disturb one.
 		const uint32_t d = (k < n) ? digit_of(key[i], shift, mask) : (uint32_t)(kBins - 1);
@@ -874,7 +873,7 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 	__syncthreads();
 
 	// A thread owns a digit value: prefix over the waves, publish the tile's count.
-	const uint32_t valid = min(n - block_base, (uint32_t)kSortBlock);
+	const uint32_t valid = min(n - block_base, (uint32_t)kBlock);
 	uint32_t* const my_word = lookback + (size_t)tile * kBins + tid;
 	uint32_t count = 0, digit_start;
 	{
@@ -894,7 +893,7 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 		if (owns)
 			sc.digit_base[tid] = (uint16_t)ex;
 		if (tid == kBins - 1)
-			count -= (uint32_t)kSortBlock - valid;  // padding is not published
+			count -= (uint32_t)kBlock - valid;  // padding is not published
 		if (owns)
 			__hip_atomic_store(my_word, count | (tile == 0 ? kFlagInclusive : kFlagAggregate), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 		// where the digit's run starts in the whole array: the exclusive scan of the digit counts
@@ -905,23 +904,23 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 	// The tile's pairs in digit order, through LDS.  None of this needs the tiles before this one: by the time
 	// the look-back below starts, more of them have finished theirs and it has fewer words to read.
 #pragma unroll
-	for (int i = 0; i < kSortItems; i++) {
+	for (int i = 0; i < kItems; i++) {
 		const uint32_t k = wave_base + (uint32_t)(i * 64 + lane);
 		const uint32_t d = (k < n) ? digit_of(key[i], shift, mask) : (uint32_t)(kBins - 1);
 		rank[i] += (uint32_t)sc.digit_base[d] + (uint32_t)wave_hist[wave][d];
 	}
 	__syncthreads();  // the counts have been read
 #pragma unroll
-	for (int i = 0; i < kSortItems; i++) {
+	for (int i = 0; i < kItems; i++) {
 		s_keys[rank[i]] = key[i];
 		s_vals[rank[i]] = val[i];
 	}
 	__syncthreads();
 	// every LDS read of the thread is asked for before anything needs one
-	KeyT out_key[kSortItems];
-	uint32_t out_val[kSortItems];
+	KeyT out_key[kItems];
+	uint32_t out_val[kItems];
 #pragma unroll
-	for (int i = 0; i < kSortItems; i++) {
+	for (int i = 0; i < kItems; i++) {
 		const uint32_t p = (uint32_t)i * kSortThreads + tid;
 		const uint32_t q = p < valid ? p : 0u;
 		out_key[i] = s_keys[q];
@@ -983,9 +982,9 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 	}
 	__syncthreads();
 
-	uint32_t out_at[kSortItems];  // (fewer than 2^30 pairs)
+	uint32_t out_at[kItems];  // (fewer than 2^30 pairs)
 #pragma unroll
-	for (int i = 0; i < kSortItems; i++) {
+	for (int i = 0; i < kItems; i++) {
 		const uint32_t p = (uint32_t)i * kSortThreads + tid;
 		const uint32_t d = digit_of(out_key[i], shift, mask);
 		out_at[i] = p < valid ? sc.global_base[d] + (p - (uint32_t)sc.digit_base[d]) : n;
@@ -995,7 +994,7 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 		// not fit and is looked up; an index that a sort which gave up left behind may be anything and is clamped)
 		const uint32_t index_bits = j.index_bits, cap = 0xFFFFFFFFu >> index_bits, index_mask = (1u << index_bits) - 1u;
 #pragma unroll
-		for (int i = 0; i < kSortItems; i++) {
+		for (int i = 0; i < kItems; i++) {
 			if (out_at[i] < n) {
 				const uint32_t index = out_val[i] & index_mask;
 				uint32_t c = out_val[i] >> index_bits;
@@ -1008,7 +1007,7 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 		return;
 	}
 #pragma unroll
-	for (int i = 0; i < kSortItems; i++) {
+	for (int i = 0; i < kItems; i++) {
 		if (out_at[i] < n) {
 			keys_out[out_at[i]] = out_key[i];
 			vals_out[out_at[i]] = out_val[i];
@@ -1026,16 +1025,45 @@ const uint32_t* sort_status_word(const uint32_t* temp)
 	return temp + kSortStatus;
 }
 
+static size_t sort_tiles(size_t n, int items)
+{
+	const size_t block = (size_t)kSortThreads * items;
+	return (n + block - 1) / block;
+}
+
+// (a launch takes its tiles by the pairs of all its jobs, n among them: never smaller ones than n alone would have)
 size_t sort_clear_words(size_t n, int end_bit, int max_bits)
 {
-	const size_t tiles = (n + kSortBlock - 1) / kSortBlock;
+	const size_t tiles = sort_tiles(n, sort_items(n));
 	return kSortHeader + (size_t)sort_passes(end_bit, max_bits) * ((size_t)1 << max_bits) * tiles;
 }
 
 size_t depth_sort_clear_words(size_t n)
 {
-	const size_t tiles = (n + kSortBlock - 1) / kSortBlock;
+	const size_t tiles = sort_tiles(n, sort_items(n));
 	return kSortHeader + (size_t)(kDepthPasses + 1) * 512 * tiles;
+}
+
+// One pass over every job of the batch, in tiles of sort_items(pairs) pairs per thread.
+template <typename KeyT, int kBits, int kKind>
+static void launch_sort_pass(const Batch<SortJob<KeyT>>& b, size_t most_pairs, size_t pairs, int jobs, int pass, int shift, uint32_t mask,
+                             hipStream_t s)
+{
+	// (64-bit keys, of the stand-alone entry points alone, take the smallest tiles: larger ones fill the LDS)
+	const int items = sizeof(KeyT) == 4 ? sort_items(pairs) : kSortItemsFew;
+	const dim3 grid((unsigned)sort_tiles(most_pairs, items), (unsigned)jobs);
+	const int spin = g_lookback_spin_limit.load();
+	if constexpr (sizeof(KeyT) == 4) {
+		if (items == kSortItemsMany) {
+			hipLaunchKernelGGL((sort_onesweep_kernel<KeyT, kBits, kKind, kSortItemsMany>), grid, dim3(kSortThreads), 0, s, b, pass, shift, mask, spin);
+			return;
+		}
+		if (items == kSortItems) {
+			hipLaunchKernelGGL((sort_onesweep_kernel<KeyT, kBits, kKind, kSortItems>), grid, dim3(kSortThreads), 0, s, b, pass, shift, mask, spin);
+			return;
+		}
+	}
+	hipLaunchKernelGGL((sort_onesweep_kernel<KeyT, kBits, kKind, kSortItemsFew>), grid, dim3(kSortThreads), 0, s, b, pass, shift, mask, spin);
 }
 
 template <typename KeyT, int kBits>
@@ -1046,17 +1074,17 @@ static void sort_pairs(const SortJob<KeyT>* jobs, int count, int end_bit, bool t
 	for (int at = 0; at < count; at += kMaxBatch) {
 		const int nj = count - at < kMaxBatch ? count - at : kMaxBatch;
 		Batch<SortJob<KeyT>> b = {};
-		uint32_t max_tiles = 0;
+		size_t most = 0, pairs = 0;
 		int live = 0;
 		for (int k = 0; k < nj; k++) {
 			const SortJob<KeyT>& j = jobs[at + k];
 			if (j.n == 0)
 				continue;
 			b.job[live++] = j;
-			const uint32_t tiles = (uint32_t)((j.n + kSortBlock - 1) / kSortBlock);
-			max_tiles = tiles > max_tiles ? tiles : max_tiles;
+			most = j.n > most ? j.n : most;
+			pairs += j.n;
 			if (!temp_cleared)
-				launch_fill_u32(j.temp, 0u, sort_clear_words(j.n, end_bit, kBits), s);
+				launch_fill_u32(j.temp, 0u, kSortHeader + (size_t)passes * (1u << kBits) * sort_tiles(j.n, kSortItemsFew), s);
 		}
 		if (live == 0)
 			continue;
@@ -1065,7 +1093,7 @@ static void sort_pairs(const SortJob<KeyT>* jobs, int count, int end_bit, bool t
 		// every block ends with an atomic add per digit and pass into its job's counts: a few hundred blocks per
 		// job read the keys as fast as thousands would, and queue far fewer adds on the same words
 		const uint32_t most_blocks = live >= 8 ? 256u : 2048u / (uint32_t)live;
-		const uint32_t hist_blocks = max_tiles < most_blocks ? max_tiles : most_blocks;
+		const uint32_t hist_blocks = (uint32_t)min(sort_tiles(most, kSortItemsFew), (size_t)most_blocks);
 		if (!histograms_done) {
 			if constexpr (sizeof(KeyT) == 8)
 				hipLaunchKernelGGL(sort_digit_histogram_kernel<KeyT>, dim3(hist_blocks, (unsigned)live), dim3(256), 0, s, b, passes, end_bit);
@@ -1076,8 +1104,7 @@ static void sort_pairs(const SortJob<KeyT>* jobs, int count, int end_bit, bool t
 			const uint32_t mask = (1u << bits) - 1u;
 			if (mark_stages)
 				stage_mark("sort_onesweep", s);
-			hipLaunchKernelGGL((sort_onesweep_kernel<KeyT, kBits, kPassPlain>), dim3(max_tiles, (unsigned)live), dim3(kSortThreads), 0, s, b, p, shift,
-			                   mask, g_lookback_spin_limit.load());
+			launch_sort_pass<KeyT, kBits, kPassPlain>(b, most, pairs, live, p, shift, mask, s);
 		}
 	}
 }
@@ -1111,8 +1138,11 @@ void launch_depth_order(const DepthOrderJob* jobs, int count, hipStream_t s)
 		Batch<BlockInclusiveJob> inc = {};
 		Batch<SortJob<uint32_t>> sorts = {};
 		int max_p = 0;
-		for (int k = 0; k < nj; k++)
+		size_t pairs = 0;
+		for (int k = 0; k < nj; k++) {
 			max_p = jobs[at + k].P > max_p ? jobs[at + k].P : max_p;
+			pairs += (size_t)jobs[at + k].P;
+		}
 		const bool few_groups = ((size_t)max_p + kScanGroup - 1) / kScanGroup <= 4096;
 		for (int k = 0; k < nj; k++) {
 			const DepthOrderJob& j = jobs[at + k];
@@ -1132,12 +1162,10 @@ void launch_depth_order(const DepthOrderJob* jobs, int count, hipStream_t s)
 		const unsigned most = nj >= 8 ? 256u : 2048u / (unsigned)nj;
 		hipLaunchKernelGGL(depth_pairs_kernel, dim3(grid.x < most ? grid.x : most, (unsigned)nj), dim3(256), 0, s, b);
 		// three passes of nine bits (a -> b -> a -> the order and the tile counts in that order), and the pass on demand
-		const dim3 tiles((unsigned)((max_p + kSortBlock - 1) / kSortBlock), (unsigned)nj);
-		const int spin = g_lookback_spin_limit.load();
-		hipLaunchKernelGGL((sort_onesweep_kernel<uint32_t, 9, kPassPlain>), tiles, dim3(kSortThreads), 0, s, sorts, 0, 0, 511u, spin);
-		hipLaunchKernelGGL((sort_onesweep_kernel<uint32_t, 9, kPassPlain>), tiles, dim3(kSortThreads), 0, s, sorts, 1, 9, 511u, spin);
-		hipLaunchKernelGGL((sort_onesweep_kernel<uint32_t, 9, kPassEndsUnless>), tiles, dim3(kSortThreads), 0, s, sorts, 2, 18, 511u, spin);
-		hipLaunchKernelGGL((sort_onesweep_kernel<uint32_t, 9, kPassOnDemand>), tiles, dim3(kSortThreads), 0, s, sorts, 3, kDepthKeyBits, 31u, spin);
+		launch_sort_pass<uint32_t, 9, kPassPlain>(sorts, (size_t)max_p, pairs, nj, 0, 0, 511u, s);
+		launch_sort_pass<uint32_t, 9, kPassPlain>(sorts, (size_t)max_p, pairs, nj, 1, 9, 511u, s);
+		launch_sort_pass<uint32_t, 9, kPassEndsUnless>(sorts, (size_t)max_p, pairs, nj, 2, 18, 511u, s);
+		launch_sort_pass<uint32_t, 9, kPassOnDemand>(sorts, (size_t)max_p, pairs, nj, 3, kDepthKeyBits, 31u, s);
 		hipLaunchKernelGGL(order_totals_kernel, grid, dim3(256), 0, s, b);
 		if (!few_groups)
 			hipLaunchKernelGGL(single_block_exclusive_scan_kernel, dim3(1, (unsigned)nj), dim3(1024), 0, s, scan);

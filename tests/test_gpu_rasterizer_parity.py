@@ -193,6 +193,39 @@ def test_depths_beyond_the_range_of_three_sort_passes():
         assert (st.radii > 0).sum() > n // 2
 
 
+@pytest.mark.parametrize("n,width,height", [((1 << 20) - 1, 64, 48), (1 << 20, 96, 80), ((1 << 20) + 8193, 4112, 4096), ((1 << 23) + 5, 700, 520)])
+def test_sorts_at_the_sizes_where_their_tiles_change(n, width, height):
+    """Depth order and tile lists against numpy, with as many Gaussians as change the sort's tile size, one more tile's worth and
+    a ragged end; eight- and nine-bit digits (the tile bits of the images)."""
+    from retinags_amd import _capi
+    dev = torch.device("cuda:0")
+    gen = torch.Generator(device=dev).manual_seed(n % 1000)
+    xyz = torch.rand(n, 3, generator=gen, device=dev) * 2.0 - 1.0
+    xyz[:, 2] += 4.0
+    xyz[::7, 2] = xyz[0, 2]      # many Gaussians of one depth: the order among them is that of their indices
+    q = torch.zeros(n, 4, device=dev)
+    q[:, 0] = 1.0
+    sub = dict(xyz=xyz, opacity=torch.full((n, 1), 0.5, device=dev), scales=torch.full((n, 3), 0.003, device=dev), rotations=q,
+               shs=torch.zeros(n, 1, 3, device=dev), low=torch.full((3,), -9.0), up=torch.full((3,), 9.0))
+    cam = scenes.look_at_camera((0.0, 0.0, 0.0), (0.0, 0.0, 1.0), (0, -1, 0), width, height, 60.0)
+    R, _, _, _, radii, geom, binning, _ = _run_gpu_forward(sub, cam, torch.zeros(3), dev, sh_degree=0)
+    torch.cuda.synchronize()
+    g, b = _capi.geom_layout(n), _capi.binning_layout(R, width, height)
+    touched = view_ws(geom, g["tiles_touched"], n, np.uint32)
+    depth_bits = view_ws(geom, g["depths"], n, np.uint32)
+    visible = np.flatnonzero(touched).astype(np.uint32)
+    order = view_ws(geom, g["depth_order"], n, np.uint32)[:len(visible)]
+    assert len(visible) > n // 3 and R == int(touched.sum(dtype=np.int64))
+    assert np.array_equal(order, visible[np.argsort(depth_bits[visible], kind="stable")])
+    tiles = view_ws(binning, b["keys_sorted"], R, np.uint32) & np.uint32(0xFFFFFF)
+    vals = view_ws(binning, b["values_sorted"], R, np.uint32)
+    rank = np.empty(n, np.int64)
+    rank[order] = np.arange(len(order))
+    # sorted by tile, by depth rank inside a tile, every Gaussian as often as it touches tiles
+    assert (np.diff(tiles.astype(np.int64) * n + rank[vals]) > 0).all()
+    assert np.array_equal(np.bincount(vals, minlength=n), touched)
+
+
 def test_garden_odd_resolution():
     """Garden-like scene at a resolution that is not a multiple of the tile size."""
     scene, cam, _ = scenes.make_config("C1", shrink=200, resolution_scale=0.2)
