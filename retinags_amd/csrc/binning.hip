@@ -658,7 +658,7 @@ void launch_duplicate_with_keys(const DuplicateJob* jobs, int count, int grid_x,
 // a stable least-significant-digit sort of (key, u32 value) pairs on key bits [0, end_bit), in the one-sweep form:
 // the digit histogram of every pass is built while the keys are written (or, for the stand-alone entry points, by one
 // kernel that reads them once), then each pass is a single kernel whose blocks take tiles of
-// kSortBlock pairs in arrival order, rank them in LDS, obtain their global digit offsets from
+// kSortThreads * kItems pairs in arrival order, rank them in LDS, obtain their global digit offsets from
 // the blocks before them through a chained look-back over per-tile status words, and scatter.
 // Element order inside a tile is (wave, round, lane); ranking preserves it, and tiles are
 // ordered by their id, so every pass is stable.  A digit has up to kBits bits (template parameter): 9 for 32-bit

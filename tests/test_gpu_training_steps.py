@@ -64,6 +64,14 @@ def test_loss_rejects_host_tensors_and_shape_mismatch():
         L.l1_ssim_loss(torch.zeros(3, 8, 8, device=DEV), torch.zeros(3, 8, 9, device=DEV))
 
 
+def test_loss_of_an_image_without_pixels_is_refused():
+    from retinags_amd.loss import l1_ssim_loss
+    for shape in ((3, 0, 16), (3, 16, 0), (2, 3, 0, 0)):
+        empty = torch.zeros(shape, device="cuda:0")
+        with pytest.raises(RuntimeError, match="without pixels"):
+            l1_ssim_loss(empty, empty)
+
+
 def test_adam_against_torch_on_the_cpu():
     """The reference's parameter groups (scene/gaussian_nn_module.py:433-441) at a small size,
     five steps, against torch.optim.Adam on the CPU; includes the group with learning rate 0."""
