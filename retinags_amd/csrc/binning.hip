@@ -850,7 +850,9 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 		const uint32_t k = wave_base + (uint32_t)(i * 64 + lane);
 		// Padding elements rank as the last digit value after every real element, so they never disturb one.
 		const uint32_t d = (k < n) ? digit_of(key[i], shift, mask) : (uint32_t)(kBins - 1);
-		// the lanes with this lane's digit: a vote per bit, taken as it is or inverted by a mask made of the lane's own bit
+		// The lanes with this lane's digit: a vote per bit, taken as it is or inverted by a mask made of the lane's own bit, four vector
+		// instructions per bit instead of nine (which kept the SIMDs busy for 60 % of a pass: 78 -> 71 us for the instances of
+		// 5.6 M Gaussians at 1600x1036).
 		uint32_t same_lo = ~0u, same_hi = ~0u;
 #pragma unroll
 		for (int b = 0; b < kBits; b++) {

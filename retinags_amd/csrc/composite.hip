@@ -16,7 +16,7 @@ __global__ __launch_bounds__(256) void composite_forward_kernel(CompositeArgs a)
 		return;
 	float T = 1.f, r = 0.f, g = 0.f, b = 0.f, d = 0.f;
 	// kAhead layers' planes are asked for together: one layer at a time, the kernel waited for memory once per layer with five
-	// requests on their way
+	// requests on their way (12 layers at 1920x1080: 140 -> 128 us, 4.2 TB/s; four pixels per thread with 16-byte loads: 132)
 	constexpr int kAhead = 4;
 	for (int k0 = 0; k0 < a.K; k0 += kAhead) {
 		float v[kAhead][5];
@@ -60,7 +60,8 @@ __global__ __launch_bounds__(256) void composite_forward_kernel(CompositeArgs a)
 // and guarded by K, so the arrays are indexed by constants), otherwise (kLayers = 0) in an array indexed at run time,
 // which the compiler places in scratch memory: every value then goes out to memory and comes back.
 // kDepth: there is a gradient of the composited depth.  Without one the layers' depths are not read and their gradients
-// (zero) are written only where the caller has planes for them; the kernel is bound by memory, and both are planes of K.
+// (zero) are written only where the caller has planes for them; the kernel is bound by memory, and both are planes of K
+// (12 layers at 1920x1080: 168 -> 135 us, 6 TB/s).
 template <int kLayers, bool kDepth>
 __global__ __launch_bounds__(256) void composite_backward_kernel(CompositeArgs a)
 {
