@@ -875,10 +875,15 @@ struct Sweep {
 // (Adding columns 0-7 of all eight entries first and columns 8-9 after them, which needs no exchange between the
 // groups, had every request of the second instruction hit a cache line that one of the first was still at work on:
 // measured, that second instruction cost eight times what the first did, a fifth of the kernel's time.)
-// The x moments are taken about the lane's first pixel, with constants for factors, and moved to the entry's centre once.
+// The x moments are summed pixel by pixel about the entry's centre.  About the lane's first pixel, with constants for factors and
+// moved to the centre once, they take 15 vector instructions fewer per pass, and the kernel 4 us less at 1600x1036 with
+// 5.6 M Gaussians (532 for 536) and 39 at 5185x3359 (2855 for 2894), but terms of up to 49 u cancel to one of the Gaussian's
+// own extent squared: for a Gaussian of half a pixel, the usual one of a dense scene, the sum for the conic's xx is then 7.7e-6
+// off (relative L2 against 64 bits) and that for the mean's x 4.9e-7; this way both are 1.3e-7, as the sums in y.
 // No instruction here only moves or repeats: one base address per LDS region, sums that start from the first pixel's terms, exchanges
-// folded into their additions, rows of `sums` addressed by one shifted addition (405 -> 355 vector instructions per pass of
-// eight entries; the kernel 555 -> 520 us at 1600x1036 with 5.6 M Gaussians, 2935 -> 2885 at 5185x3359).
+// folded into their additions, rows of `sums` addressed by one shifted addition (50 vector instructions fewer per pass of eight
+// entries; the kernel 555 -> 520 us at 1600x1036, 2935 -> 2885 at 5185x3359 when that was done, with the moments about the
+// first pixel).
 // kDepth: a gradient arrived for the depth image (without one, the usual case of a loss on the colour image alone, the
 // terms it multiplies are left out: the depth column of `sums` stays zero).
 template <bool kDepth>
@@ -890,29 +895,26 @@ __device__ __forceinline__ void sum_rows(const BackwardStage& st, int slot0, int
 	const int upper = (lane >> 3) & 1;  // which eight of the 16-lane row
 	const int e = (lane >> 4) + 4 * upper, h = (lane >> 1) & 3, half = lane & 1, j = lane & 7;
 	const int slot = slot0 + e;
-	// (the first pixel's terms start the sums: added to zeros they would take five instructions)
+	const float4 centre = st.geom[slot];
+	const float dx_first = centre.x - (f.x0 + (float)(8 * half)), dy = centre.y - (f.y0 + (float)h);
+	// (the first pixel's terms start the sums: added to zeros they would take six instructions)
 	Pair ua = sweep.row[0];
-	float s0 = ua.x, cr = ua.y * sweep.r[0], cg = ua.y * sweep.g[0], cb = ua.y * sweep.b[0];
+	float s0 = ua.x, sx = ua.x * dx_first, sxx = sx * dx_first;
+	float cr = ua.y * sweep.r[0], cg = ua.y * sweep.g[0], cb = ua.y * sweep.b[0];
 	float cdp = kDepth ? ua.y * st.g_depth[9 * (lane & 7)] : 0.f;
-	ua = sweep.row[1];
-	float s1 = ua.x, s2 = ua.x;
 #pragma unroll
 	for (int step = 1; step < 8; step++) {
-		if (step > 1) {
-			ua = sweep.row[step];
-			s1 += (float)step * ua.x;
-			s2 += (float)(step * step) * ua.x;
-		}
+		ua = sweep.row[step];
+		const float dx = dx_first - (float)step, t = ua.x * dx;
 		s0 += ua.x;
+		sx += t;
+		sxx += t * dx;
 		cr += ua.y * sweep.r[step];
 		cg += ua.y * sweep.g[step];
 		cb += ua.y * sweep.b[step];
 		if (kDepth)
 			cdp += ua.y * st.g_depth[9 * (lane & 7) + step];
 	}
-	const float4 centre = st.geom[slot];
-	const float dx = centre.x - (f.x0 + (float)(8 * half)), dy = centre.y - (f.y0 + (float)h);
-	const float sx = dx * s0 - s1, sxx = dx * sx - (dx * s1 - s2);
 	// the two halves of the strip row first (dy is theirs in common), then the four strip rows
 	float w[7] = {s0, sx, sxx, cr, cg, cb, cdp};
 #pragma unroll

@@ -330,3 +330,77 @@ def test_gaussians_that_cover_the_whole_image(width, height):
     tiles = (width // 16) * (height // 16)
     assert (st.tiles_touched[:40] >= tiles // 2).sum() >= 20
     _check_backward(sub, cam, torch.zeros(3), seed=5, with_depth_alpha=True)
+
+
+def _head_on(places, width, height):
+    """Camera at the origin that looks along z, and round Gaussians at `places`: (x, y in pixels, depth, size in pixels)."""
+    cam = scenes.look_at_camera((0.0, 0.0, 0.0), (0.0, 0.0, 1.0), (0, -1, 0), width, height, 60.0)
+    places = torch.as_tensor(places, dtype=torch.float32)
+    z = places[:, 2]
+    xyz = torch.stack([((2 * places[:, 0] + 1) / width - 1) * cam.tanfovx * z, ((2 * places[:, 1] + 1) / height - 1) * cam.tanfovy * z, z], 1)
+    scales = (places[:, 3] * 2 * cam.tanfovx * z / width)[:, None].repeat(1, 3)
+    rotations = torch.zeros(len(places), 4)
+    rotations[:, 0] = 1.0
+    return cam, dict(xyz=xyz, scales=scales, rotations=rotations)
+
+
+def _open_box_settings(cam, dev):
+    from retinags_amd import GaussianRasterizationSettings
+    return GaussianRasterizationSettings(
+        image_height=cam.image_height, image_width=cam.image_width, tanfovx=cam.tanfovx, tanfovy=cam.tanfovy,
+        bg=torch.zeros(3, device=dev), scale_modifier=1.0, viewmatrix=cam.world_view_transform.to(dev),
+        projmatrix=cam.full_proj_transform.to(dev), projmatrix_inv=cam.projection_matrix_inv.to(dev),
+        range_low=torch.full((3,), -99.0, device=dev), range_up=torch.full((3,), 99.0, device=dev), sh_degree=0,
+        campos=cam.camera_center.to(dev), prefiltered=False, debug=False)
+
+
+def test_blend_gradient_sums_of_subpixel_gaussians_against_double_precision(monkeypatch):
+    """The backward blend's sums over the pixels of Gaussians of about half a pixel (the low-pass filter alone), each alone
+    on its pixels, against the same sums in 64 bits from the records that the blend reads.  A pixel's terms carry the
+    exponent's rounding (about three half units of the products, below 5e-7 absolute where the weight is not negligible),
+    exp2's, and three more products: together below 6e-7 of the term, and the sum of some twenty of them six levels of
+    additions, 3.6e-7.  Moments that are taken about another point than the centre and moved there cancel: about the first
+    of a lane's eight pixels, the second moment in x loses two digits (4e-6 to 8e-6)."""
+    from retinags_amd import GaussianRasterizer, _capi, rasterizer
+    dev = torch.device("cuda:0")
+    columns, rows, spacing = 40, 30, 32
+    W, H, n = columns * spacing, rows * spacing, columns * rows
+    gen = torch.Generator().manual_seed(12)
+    gy, gx = torch.meshgrid(torch.arange(rows), torch.arange(columns), indexing="ij")
+    at = torch.stack([gx.reshape(-1), gy.reshape(-1)], 1) * float(spacing) + spacing / 2 + torch.rand(n, 2, generator=gen) * 16.0 - 8.0
+    cam, g = _head_on(torch.cat([at, torch.tensor([[4.0, 0.01]]).repeat(n, 1)], 1), W, H)
+    g["opacity"], g["colors"] = 0.1 + 0.4 * torch.rand(n, 1, generator=gen), torch.rand(n, 3, generator=gen)
+    made = []
+    make = rasterizer._gradient_outputs
+    monkeypatch.setattr(rasterizer, "_gradient_outputs", lambda *a, **k: made.append(make(*a, **k)) or made[-1])
+    leaf = {k: v.to(dev).requires_grad_(True) for k, v in g.items()}
+    workspaces = []
+    color, radii, _, _ = rasterizer.rasterize_frame([GaussianRasterizer(_open_box_settings(cam, dev))], [dict(
+        means3D=leaf["xyz"], means2D=torch.zeros_like(leaf["xyz"], requires_grad=True), opacities=leaf["opacity"],
+        colors_precomp=leaf["colors"], scales=leaf["scales"], rotations=leaf["rotations"])], workspaces=workspaces)[0]
+    upstream = torch.randn(3, H, W, generator=gen) * 1e-2
+    color.backward(upstream.to(dev))
+    torch.cuda.synchronize()
+    assert (radii > 0).all()
+    sums = made[0]["sums"].cpu().numpy().astype(np.float64)
+    rec = view_ws(workspaces[0][1], _capi.geom_layout(n)["blend_record"], 16 * n, np.float32).reshape(n, 16).astype(np.float64)
+    reach = np.arange(-8, 9)
+    px, py = np.broadcast_arrays(np.rint(rec[:, 0])[:, None, None] + reach[None, None, :], np.rint(rec[:, 1])[:, None, None] + reach[None, :, None])
+    within = (px >= 0) & (px < W) & (py >= 0) & (py < H)
+    g_at = upstream.numpy().astype(np.float64)[:, np.clip(py, 0, H - 1).astype(int), np.clip(px, 0, W - 1).astype(int)]
+    dx, dy = rec[:, 0, None, None] - px, rec[:, 1, None, None] - py
+    xx, xy, yy, op = (rec[:, 4 + k, None, None] for k in range(4))
+    G = np.exp(-0.5 * (xx * dx * dx + yy * dy * dy) - xy * dx * dy)
+    alpha = np.where(within & (op * G >= 1.0 / 255.0), op * G, 0.0)
+    assert np.abs(op * G * 255.0 - 1.0).min() > 1e-5          # no pixel sits on the threshold
+    u = np.where(alpha > 0, G, 0.0) * np.einsum("cnij,nc->nij", g_at, rec[:, 8:11])
+    total = lambda a: a.sum(axis=(1, 2))
+    xx, xy, yy, op = xx[:, 0, 0], xy[:, 0, 0], yy[:, 0, 0], op[:, 0, 0]
+    sx, sy = total(u * dx), total(u * dy)
+    want = [-op * 0.5 * W * (xx * sx + xy * sy), -op * 0.5 * H * (yy * sy + xy * sx), -0.5 * op * total(u * dx * dx),
+            -0.5 * op * total(u * dx * dy), -0.5 * op * total(u * dy * dy), total(u)] + [total(alpha * g_at[c]) for c in range(3)]
+    assert 3.0 < np.median(xx) < 3.5                            # half a pixel wide
+    for k, name in enumerate(("mean x", "mean y", "conic xx", "conic xy", "conic yy", "opacity", "red", "green", "blue")):
+        err = rel_l2(sums[:, k], want[k])
+        print(f"{name}: relative L2 {err:.2e}")
+        assert err <= 1e-6, f"sum for {name}: relative L2 {err:.2e}"
