@@ -866,6 +866,11 @@ struct Sweep {
 	float *column_low, *column_high;  // for entries 0-3 and for entries 4-7 of a pass
 };
 
+// Which entries of a pass some pixel blended: entries 0-3 and entries 4-7, 16 lanes each, a row of the wavefront per entry.
+struct Blended {
+	uint64_t low, high;
+};
+
 // Entry-parallel part for the eight entries staged from slot0 on.  A 16-lane row of the wavefront serves two entries, e in
 // its low eight lanes and e + 4 in its high eight; lane (h = (lane >> 1) & 3, half = lane & 1) of the eight
 // sums the entry's row over the 8 pixels of one half of strip row h; the eight lanes of an entry then add up what
@@ -887,8 +892,8 @@ struct Sweep {
 // kDepth: a gradient arrived for the depth image (without one, the usual case of a loss on the colour image alone, the
 // terms it multiplies are left out: the depth column of `sums` stays zero).
 template <bool kDepth>
-__device__ __forceinline__ void sum_rows(const BackwardStage& st, int slot0, int entries, const Sweep& sweep, const StripFrame& f,
-                                         int lane)
+__device__ __forceinline__ void sum_rows(const BackwardStage& st, int slot0, const Blended& blended, const Sweep& sweep,
+                                         const StripFrame& f, int lane)
 {
 #pragma clang fp contract(fast)
 	__builtin_amdgcn_wave_barrier();
@@ -946,22 +951,24 @@ __device__ __forceinline__ void sum_rows(const BackwardStage& st, int slot0, int
 		float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, second), 0x128, 0xF, 0xF, true));
 	const uint32_t row_there = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)sum_row, 0x128, 0xF, 0xF, true);
 	// Entries 0-3: their own (lower) lanes add columns 0-7, the upper lanes columns 8 and 9 for them; then entries 4-7 the
-	// other way round.  Which entries there are is asked here alone: with a branch around the choices above, the
-	// compiler moves the last additions of the exchanges into it and their lane moves stay outside as instructions of their own.
+	// other way round.  Which entries some pixel blended is asked here alone (an entry that none blends, as the slots behind the
+	// last one, has zeros in its row, which an upstream gradient that is not finite would turn into NaN): with a branch around
+	// the choices above, the compiler moves the last additions of the exchanges into it and their lane moves stay outside as
+	// instructions of their own.
 	const float low = upper ? second_there : first, high = upper ? first : second_there;
 	float* at_low = reinterpret_cast<float*>(reinterpret_cast<char*>(sweep.column_low) + ((uint64_t)(upper ? row_there : sum_row) << 4));
 	float* at_high = reinterpret_cast<float*>(reinterpret_cast<char*>(sweep.column_high) + ((uint64_t)(upper ? sum_row : row_there) << 4));
-	if ((lane >> 4) < entries && low != 0.f)
+	if (__builtin_amdgcn_inverse_ballot_w64(blended.low) && low != 0.f)
 		unsafeAtomicAdd(at_low, low);
-	if ((lane >> 4) + 4 < entries && high != 0.f)
+	if (__builtin_amdgcn_inverse_ballot_w64(blended.high) && high != 0.f)
 		unsafeAtomicAdd(at_high, high);
 	__builtin_amdgcn_wave_barrier();
 }
 
 // Pixel-parallel part for the four entries staged from slot k on; `rows`: the pixel's place in the first of their rows.
-// Returns whether any pixel blended any of them.
+// Returns, as sum_rows asks for it (16 lanes per entry), which of them any pixel blended.
 template <bool kDepth, bool kBoxed>
-__device__ __forceinline__ bool backward_rows(BackwardPixel& p, uint32_t last_contributor, const BackwardStage& st, int k,
+__device__ __forceinline__ uint64_t backward_rows(BackwardPixel& p, uint32_t last_contributor, const BackwardStage& st, int k,
                                               LdsPair* rows, const float2 pixf, const BoxSpan& span, const BlendArgs& a)
 {
 	float power[4], clip_w[4], opacity[4];
@@ -1026,7 +1033,11 @@ __device__ __forceinline__ bool backward_rows(BackwardPixel& p, uint32_t last_co
 		    : [lanes] "s"(mask[i]), [inv] "v"(inv[i]), [alpha] "v"(alpha[i]), [weighted] "v"(weighted[i]), [G] "v"(G[i]));
 		rows[i * kRowStride] = Pair{u, aT};
 	}
-	return (mask[0] | mask[1] | mask[2] | mask[3]) != 0ull;
+	uint64_t blended = 0ull;
+#pragma unroll
+	for (int i = 0; i < 4; i++)
+		blended |= mask[i] != 0ull ? 0xFFFFull << (16 * i) : 0ull;
+	return blended;
 }
 
 template <bool kDepth>
@@ -1147,17 +1158,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 		if (boxed) {
 			const BoxSpan span = span_for_visits(all_in_front, st.rays, a);
 			for (int k = 0; k < count; k += kRows) {
-				const bool front = backward_rows<kDepth, true>(p, last_contributor, st, k, rows[0], pixf, span, a);
-				const bool back = backward_rows<kDepth, true>(p, last_contributor, st, k + 4, rows[1], pixf, span, a);
-				if (front || back)
-					sum_rows<kDepth>(st, k, count - k, sweep, frame, lane);
+				const Blended blended = {backward_rows<kDepth, true>(p, last_contributor, st, k, rows[0], pixf, span, a),
+				                         backward_rows<kDepth, true>(p, last_contributor, st, k + 4, rows[1], pixf, span, a)};
+				if ((blended.low | blended.high) != 0ull)
+					sum_rows<kDepth>(st, k, blended, sweep, frame, lane);
 			}
 		} else {
 			for (int k = 0; k < count; k += kRows) {
-				const bool front = backward_rows<kDepth, false>(p, last_contributor, st, k, rows[0], pixf, BoxSpan{}, a);
-				const bool back = backward_rows<kDepth, false>(p, last_contributor, st, k + 4, rows[1], pixf, BoxSpan{}, a);
-				if (front || back)
-					sum_rows<kDepth>(st, k, count - k, sweep, frame, lane);
+				const Blended blended = {backward_rows<kDepth, false>(p, last_contributor, st, k, rows[0], pixf, BoxSpan{}, a),
+				                         backward_rows<kDepth, false>(p, last_contributor, st, k + 4, rows[1], pixf, BoxSpan{}, a)};
+				if ((blended.low | blended.high) != 0ull)
+					sum_rows<kDepth>(st, k, blended, sweep, frame, lane);
 			}
 		}
 		__builtin_amdgcn_wave_barrier();

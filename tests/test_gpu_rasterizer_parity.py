@@ -404,3 +404,32 @@ def test_blend_gradient_sums_of_subpixel_gaussians_against_double_precision(monk
         err = rel_l2(sums[:, k], want[k])
         print(f"{name}: relative L2 {err:.2e}")
         assert err <= 1e-6, f"sum for {name}: relative L2 {err:.2e}"
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_a_gradient_that_is_not_finite_stays_with_the_gaussians_that_are_blended(bad):
+    """The left of a strip is finished by opaque Gaussians in front; one behind them there is filed for the strip and blended
+    by no pixel; a last one is blended in the right half, where a pixel's upstream gradient is not finite.  That reaches the
+    last one; the one that nothing blends has gradients of exactly zero."""
+    from retinags_amd import GaussianRasterizer
+    dev = torch.device("cuda:0")
+    W, H = 32, 16
+    cam, g = _head_on([(2.0, 1.0, 2.0 + 0.05 * k, 3.0) for k in range(16)] + [(2.0, 1.0, 3.0, 0.3), (12.0, 1.0, 3.5, 0.5)], W, H)
+    g["opacity"], g["colors"] = torch.tensor([[0.99]] * 16 + [[0.9], [0.5]]), torch.full((18, 3), 0.5)
+    s = oracle_settings(cam, torch.full((3,), -99.0), torch.full((3,), 99.0), torch.zeros(3), sh_degree=0)
+    st = orc.forward(s, np32(g["xyz"]), np32(g["opacity"]), colors_precomp=np32(g["colors"]), scales=np32(g["scales"]),
+                     rotations=np32(g["rotations"]))
+    want = orc.backward(s, st, np.full((3, H, W), 1e-2, np.float32))
+    assert (st.radii > 0).all() and st.ranges[0].tolist() == [0, 18]
+    assert (want["colors"][16] == 0).all() and (want["colors"][17] != 0).all()
+    leaf = {k: v.to(dev).requires_grad_(True) for k, v in g.items()}
+    color = GaussianRasterizer(_open_box_settings(cam, dev))(
+        means3D=leaf["xyz"], means2D=torch.zeros_like(leaf["xyz"]), opacities=leaf["opacity"], colors_precomp=leaf["colors"],
+        scales=leaf["scales"], rotations=leaf["rotations"])[0]
+    upstream = torch.full((3, H, W), 1e-2)
+    upstream[:, 1, 12] = bad
+    color.backward(upstream.to(dev))
+    for k in ("xyz", "opacity", "colors"):
+        grad = leaf[k].grad.cpu()
+        assert not torch.isfinite(grad[17]).all(), f"{k}: {grad[17]}"   # the last one, under the pixel
+        assert (grad[16] == 0).all(), f"{k}: {grad[16]}"                 # the one that nothing blends
