@@ -352,19 +352,22 @@ struct ForwardStage {  // one per workgroup (a single wavefront)
 // of the reference's two products and an add each (forward.cu:378-385); the sums feed no decision, the images are compared
 // by tolerance.  Under a lane mask, so that a colour that is not finite reaches the pixels that blend it and no others;
 // written out because the compiler puts a branch around every masked region, and four taken branches per group of
-// entries cost a wavefront that is alone on its SIMD more than the additions do.  (All 64 lanes are active around it.)
+// entries cost a wavefront that is alone on its SIMD more than the additions do.  (Lanes that are not active around it stay so.)
 __device__ __forceinline__ void blend_sample(ForwardPixel& p, uint64_t lanes, float weight, const float4 cd, int slot)
 {
-	asm("s_mov_b64 exec, %[lanes]\n\t"
+	uint64_t active;
+	asm("s_and_saveexec_b64 %[active], %[lanes]\n\t"
 	    "v_fmac_f32 %[c0], %[r], %[w]\n\t"
 	    "v_fmac_f32 %[c1], %[g], %[w]\n\t"
 	    "v_fmac_f32 %[c2], %[b], %[w]\n\t"
 	    "v_fmac_f32 %[d], %[z], %[w]\n\t"
 	    "v_add_f32 %[sum], %[sum], %[w]\n\t"
 	    "v_mov_b32 %[last], %[slot]\n\t"
-	    "s_mov_b64 exec, -1"
-	    : [c0] "+v"(p.C0), [c1] "+v"(p.C1), [c2] "+v"(p.C2), [d] "+v"(p.D), [sum] "+v"(p.weight), [last] "+v"(p.last_slot)
-	    : [lanes] "s"(lanes), [w] "v"(weight), [r] "v"(cd.x), [g] "v"(cd.y), [b] "v"(cd.z), [z] "v"(cd.w), [slot] "s"(slot));
+	    "s_mov_b64 exec, %[active]"
+	    : [c0] "+v"(p.C0), [c1] "+v"(p.C1), [c2] "+v"(p.C2), [d] "+v"(p.D), [sum] "+v"(p.weight), [last] "+v"(p.last_slot),
+	      [active] "=&s"(active)
+	    : [lanes] "s"(lanes), [w] "v"(weight), [r] "v"(cd.x), [g] "v"(cd.y), [b] "v"(cd.z), [z] "v"(cd.w), [slot] "s"(slot)
+	    : "scc");
 }
 
 // Four neighbouring slots of the pixel's half.  Alpha of all four first, by every lane, with the decisions kept as lane
@@ -1014,23 +1017,24 @@ __device__ __forceinline__ uint64_t backward_rows(BackwardPixel& p, uint32_t las
 	// pixel does for all channels: `behind` = sum over the entries behind of w_j <g, (colour_j, depth_j, 1)> +
 	// T_final <g, background>, started with the latter.
 	// Under the mask of the pixels that blend the entry, written out: the compiler would put a branch around each of the
-	// four (all 64 lanes are active around it; the mask's move is also the instruction that has to lie between a
-	// reciprocal and the first use of it).
+	// four (the mask's move is also the instruction that has to lie between a reciprocal and the first use of it).
 #pragma unroll
 	for (int i = 0; i < 4; i++) {
 		float dL_dopa;
 		Pair z = zero_pair();
 		float u = z.x, aT = z.y;
-		asm("s_mov_b64 exec, %[lanes]\n\t"
+		uint64_t active;
+		asm("s_and_saveexec_b64 %[active], %[lanes]\n\t"
 		    "v_mul_f32 %[T], %[T], %[inv]\n\t"
 		    "v_mul_f32 %[d], %[behind], %[inv]\n\t"
 		    "v_mul_f32 %[aT], %[alpha], %[T]\n\t"
 		    "v_fma_f32 %[d], %[weighted], %[T], -%[d]\n\t"
 		    "v_fmac_f32 %[behind], %[aT], %[weighted]\n\t"
 		    "v_mul_f32 %[u], %[G], %[d]\n\t"
-		    "s_mov_b64 exec, -1"
-		    : [T] "+v"(p.T), [behind] "+v"(p.behind), [aT] "+v"(aT), [u] "+v"(u), [d] "=&v"(dL_dopa)
-		    : [lanes] "s"(mask[i]), [inv] "v"(inv[i]), [alpha] "v"(alpha[i]), [weighted] "v"(weighted[i]), [G] "v"(G[i]));
+		    "s_mov_b64 exec, %[active]"
+		    : [T] "+v"(p.T), [behind] "+v"(p.behind), [aT] "+v"(aT), [u] "+v"(u), [d] "=&v"(dL_dopa), [active] "=&s"(active)
+		    : [lanes] "s"(mask[i]), [inv] "v"(inv[i]), [alpha] "v"(alpha[i]), [weighted] "v"(weighted[i]), [G] "v"(G[i])
+		    : "scc");
 		rows[i * kRowStride] = Pair{u, aT};
 	}
 	uint64_t blended = 0ull;

@@ -300,3 +300,17 @@ def test_exponent_of_a_conic_staged_pre_scaled_has_the_bits_of_the_reference_exp
     staged = (sxx * dx * dx + syy * dy * dy) + sxy * dx * dy
     assert reference.dtype == np.float32 and staged.dtype == np.float32
     assert np.array_equal(reference.view(np.uint32), staged.view(np.uint32))
+
+
+def test_inline_assembly_gives_back_the_lanes_that_were_active():
+    """Assembly that masks lanes off must bring back those that were active around it and no others: setting the execution
+    mask to a constant afterwards is right only while the code around it happens to run with every lane on."""
+    writes = 0
+    for name in os.listdir(os.path.join(ROOT, "retinags_amd", "csrc")):
+        if name.endswith((".hip", ".h")):
+            text = open(os.path.join(ROOT, "retinags_amd", "csrc", name)).read()
+            for source in re.findall(r"s_mov_b(?:32|64)\s+exec\w*,\s*([^\\\"\s]+)", text):
+                assert re.fullmatch(r"%\[\w+\]", source), f"{name}: exec set to {source}"
+                writes += 1
+            assert len(re.findall(r"s_mov_b64\s+exec", text)) == len(re.findall(r"s_and_saveexec_b64", text)), name
+    assert writes > 0
