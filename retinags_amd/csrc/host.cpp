@@ -892,14 +892,18 @@ using namespace rgs_host;
 PYBIND11_MODULE(_host, m)
 {
 	library_error_type = py::object(py::module_::import("retinags_amd._capi").attr("RgsError")).release().ptr();
-	py::register_exception_translator([](std::exception_ptr p) {
+	// For the functions of this module alone: the library's errors by their own type, those of tensor code (out of memory among
+	// them, which callers catch to make room and try again) and of Python code that it ran by the types that PyTorch gives them.
+	py::register_local_exception_translator([](std::exception_ptr p) {
 		try {
 			if (p)
 				std::rethrow_exception(p);
 		} catch (const LibraryError& e) {
 			PyErr_SetString(library_error_type, e.what());
-		} catch (const c10::Error& e) {
-			PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
+		} catch (const c10::Error&) {
+			torch::translate_exception_to_python(p);
+		} catch (const python_error&) {
+			torch::translate_exception_to_python(p);
 		}
 	});
 

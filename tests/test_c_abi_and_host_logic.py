@@ -314,3 +314,12 @@ def test_inline_assembly_gives_back_the_lanes_that_were_active():
                 writes += 1
             assert len(re.findall(r"s_mov_b64\s+exec", text)) == len(re.findall(r"s_and_saveexec_b64", text)), name
     assert writes > 0
+
+
+def test_errors_of_tensor_code_keep_their_types_through_the_host_path():
+    """What tensor code throws in the native host path arrives as the type that PyTorch gives it, not as a plain RuntimeError."""
+    from retinags_amd import _host, rasterizer
+    with pytest.raises(NotImplementedError):
+        rasterizer._gradient_outputs(4, 1, torch.device("xla"))      # a backend this build of PyTorch does not have
+    with pytest.raises(RuntimeError, match="between one layer"):
+        _host.composite(None, [])

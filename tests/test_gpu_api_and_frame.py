@@ -664,3 +664,45 @@ def test_rasterize_frame_with_an_empty_layer_and_without_stages():
     once = full["means3D"].grad.clone()
     (c0.sum() + c1.sum()).backward()
     assert rel_l2(full["means3D"].grad.cpu().numpy(), 2.0 * once.cpu().numpy()) <= 1e-5
+
+
+def test_out_of_memory_and_hooks_keep_their_types_and_the_call_can_be_repeated():
+    """A forward that finds no memory raises torch.OutOfMemoryError, as the allocator does, and the same call goes through
+    once there is room; what a saved-tensor hook raises arrives as it is."""
+    from retinags_amd import GaussianRasterizer
+    from retinags_amd.compositor import composite_partial_images
+    scene, cam, low, up = _small_inputs(n=5000, seed=4)
+    r = GaussianRasterizer(_settings(oracle_settings(cam, low, up, torch.tensor([0.3, 0.2, 0.1]))))
+    kw = dict(means3D=scene["xyz"].to(DEV), means2D=torch.zeros_like(scene["xyz"]).to(DEV), opacities=scene["opacity"].to(DEV),
+              shs=scene["shs"].to(DEV), scales=scene["scales"].to(DEV), rotations=scene["rotations"].to(DEV))
+    want = [t.clone() for t in r(**kw)]
+    plane = torch.rand(1, cam.image_height, cam.image_width, device=DEV)
+    layers = [plane.expand(3, -1, -1).contiguous()], [plane], [plane.clone()]
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 1024) / total)
+        filler = []
+        with pytest.raises(torch.OutOfMemoryError):
+            while True:                      # what is free inside the segments already reserved
+                filler.append(torch.empty(4096, dtype=torch.uint8, device=DEV))
+        with pytest.raises(torch.OutOfMemoryError):
+            r(**kw)
+        with pytest.raises(torch.OutOfMemoryError):
+            composite_partial_images(*layers)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+        del filler
+    for a, b in zip(r(**kw), want):
+        assert torch.equal(a, b)
+
+    class Refused(Exception):
+        pass
+
+    def refuse(t):
+        raise Refused("not this one")
+
+    leaf = layers[0][0].requires_grad_(True)
+    with torch.autograd.graph.saved_tensors_hooks(refuse, lambda t: t), pytest.raises(Refused):
+        composite_partial_images([leaf], layers[1], layers[2])
