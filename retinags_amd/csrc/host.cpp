@@ -156,15 +156,15 @@ Settings settings_from_python(py::handle s)
 	r.W = py::cast<int64_t>(py::int_(s.attr("image_width")));
 	r.tanfovx = py::cast<double>(py::float_(s.attr("tanfovx")));
 	r.tanfovy = py::cast<double>(py::float_(s.attr("tanfovy")));
-	r.bg = from_python(s.attr("bg"), "bg");
+	r.bg = tensor_from_python(s.attr("bg"), "bg");
 	r.scale_modifier = py::cast<double>(py::float_(s.attr("scale_modifier")));
-	r.view = from_python(s.attr("viewmatrix"), "viewmatrix");
-	r.proj = from_python(s.attr("projmatrix"), "projmatrix");
-	r.proj_inv = from_python(s.attr("projmatrix_inv"), "projmatrix_inv");
-	r.low = from_python(s.attr("range_low"), "range_low");
-	r.up = from_python(s.attr("range_up"), "range_up");
+	r.view = tensor_from_python(s.attr("viewmatrix"), "viewmatrix");
+	r.proj = tensor_from_python(s.attr("projmatrix"), "projmatrix");
+	r.proj_inv = tensor_from_python(s.attr("projmatrix_inv"), "projmatrix_inv");
+	r.low = tensor_from_python(s.attr("range_low"), "range_low");
+	r.up = tensor_from_python(s.attr("range_up"), "range_up");
 	r.sh_degree = static_cast<int>(py::cast<int64_t>(py::int_(s.attr("sh_degree"))));
-	r.campos = from_python(s.attr("campos"), "campos");
+	r.campos = tensor_from_python(s.attr("campos"), "campos");
 	r.prefiltered = truth(s.attr("prefiltered"));
 	r.debug = truth(s.attr("debug"));
 	return r;
@@ -507,13 +507,17 @@ struct RasterizeCall : torch::autograd::Function<RasterizeCall> {
 	}
 };
 
+// An absent input comes as an empty tensor; only the placeholder for the screen-space gradient, whose values nobody reads, may be None.
 std::array<Tensor, kInputs> inputs_from_python(const py::handle* given)
 {
 	std::array<Tensor, kInputs> in;
 	for (int k = 0; k < kInputs; k++) {
-		in[k] = from_python(given[k], kInputNames[k]);
-		if (!in[k].defined())
-			in[k] = at::empty({0});  // stands for an absent input
+		if (k != kMeans2D)
+			in[k] = tensor_from_python(given[k], kInputNames[k]);
+		else if (THPVariable_Check(given[k].ptr()))
+			in[k] = THPVariable_Unpack(given[k].ptr());
+		else
+			in[k] = at::empty({0});
 	}
 	return in;
 }
@@ -822,7 +826,7 @@ struct RasterizeFrame : torch::autograd::Function<RasterizeFrame> {
 	}
 };
 
-// `inputs`: per layer the kInputs tensors, None for those that are absent.  `streams`: None, or a stream handle per layer.
+// `inputs`: per layer the kInputs tensors, empty ones for those that are absent.  `streams`: None, or a stream handle per layer.
 // `workspaces`: None, or a list that receives (instances, geometry, binning and image workspace) per layer.
 py::list rasterize_frame(const py::sequence& settings, const py::sequence& inputs, py::handle streams, py::handle workspaces)
 {
@@ -834,20 +838,18 @@ py::list rasterize_frame(const py::sequence& settings, const py::sequence& input
 	auto frame = c10::make_intrusive<Frame>();
 	frame->layers.resize(K);
 	frame->keep_workspaces = !workspaces.is_none();
-	variable_list flat(K * kInputs);
-	Tensor absent;
+	variable_list flat;
+	flat.reserve(K * kInputs);
 	for (size_t k = 0; k < K; k++) {
 		frame->layers[k].s = settings_from_python(settings[k]);
 		if (!streams.is_none())
 			frame->layers[k].side = reinterpret_cast<hipStream_t>(py::cast<uintptr_t>(py::reinterpret_borrow<py::sequence>(streams)[k]));
-		for (int i = 0; i < kInputs; i++) {
-			flat[k * kInputs + i] = from_python(inputs[k * kInputs + i], kInputNames[i]);
-			if (!flat[k * kInputs + i].defined()) {
-				if (!absent.defined())
-					absent = at::empty({0});
-				flat[k * kInputs + i] = absent;
-			}
-		}
+		std::array<py::object, kInputs> held;
+		std::array<py::handle, kInputs> given;
+		for (int i = 0; i < kInputs; i++)
+			given[i] = held[i] = inputs[k * kInputs + i];
+		const std::array<Tensor, kInputs> in = inputs_from_python(given.data());
+		flat.insert(flat.end(), in.begin(), in.end());
 	}
 	variable_list out;
 	{

@@ -84,6 +84,14 @@ inline Tensor from_python(py::handle h, const char* name)
 	return THPVariable_Unpack(h.ptr());
 }
 
+// The same where a tensor has to be given.
+inline Tensor tensor_from_python(py::handle h, const char* name)
+{
+	if (!THPVariable_Check(h.ptr()))
+		throw py::type_error(std::string(name) + " must be a tensor");
+	return THPVariable_Unpack(h.ptr());
+}
+
 inline py::object to_python(const Tensor& t) { return t.defined() ? py::cast(t) : py::none(); }
 
 inline bool present(const Tensor& t) { return t.defined() && t.numel() != 0; }

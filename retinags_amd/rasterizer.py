@@ -57,6 +57,9 @@ def _dev_f32(t: torch.Tensor, device, name: str) -> torch.Tensor:
     return t.contiguous()
 
 
+_EMPTY = torch.Tensor([])  # stands for an absent input, as in the reference (it becomes a null pointer)
+
+
 def _stream_ptr(device) -> C.c_void_p:
     return C.c_void_p(torch.cuda.current_stream(device).cuda_stream)
 
@@ -164,20 +167,23 @@ def _rasterize_layers(settings, inputs, streams=None, workspaces=None):
     """rasterize_frame from the layers' settings."""
     flat = []
     for kw in inputs:
-        shs, colors_precomp, scales, rotations, cov3D = (kw.get("shs"), kw.get("colors_precomp"), kw.get("scales"),
-                                                         kw.get("rotations"), kw.get("cov3D_precomp"))
-        _check_inputs(shs, colors_precomp, scales, rotations, cov3D)
+        shs, colors_precomp, scales, rotations, cov3D = _checked_inputs(kw.get("shs"), kw.get("colors_precomp"), kw.get("scales"),
+                                                                        kw.get("rotations"), kw.get("cov3D_precomp"))
         flat += (kw["means3D"], kw["means2D"], shs, colors_precomp, kw["opacities"], scales, rotations, cov3D)
     return _host.rasterize_frame(settings, flat, streams, workspaces)
 
 
-def _check_inputs(shs, colors_precomp, scales, rotations, cov3D_precomp):
+def _checked_inputs(shs, colors_precomp, scales, rotations, cov3D_precomp):
+    """The five inputs of which a call takes some, empty tensors for those that are absent."""
     if (shs is None and colors_precomp is None) or (shs is not None and colors_precomp is not None):
         raise Exception('Please provide excatly one of either SHs or precomputed colors!')
 
     if ((scales is None or rotations is None) and cov3D_precomp is None) or \
             ((scales is not None or rotations is not None) and cov3D_precomp is not None):
         raise Exception('Please provide exactly one of either scale/rotation pair or precomputed 3D covariance!')
+    return (_EMPTY if shs is None else shs, _EMPTY if colors_precomp is None else colors_precomp,
+            _EMPTY if scales is None else scales, _EMPTY if rotations is None else rotations,
+            _EMPTY if cov3D_precomp is None else cov3D_precomp)
 
 
 class GaussianRasterizer(nn.Module):
@@ -198,7 +204,8 @@ class GaussianRasterizer(nn.Module):
                 cov3D_precomp=None, geometry=None):
         """As the reference's forward.  `geometry`, if given, is what enqueue_geometry returned for
         these same inputs: the call then only waits for that stage and goes on from there."""
-        _check_inputs(shs, colors_precomp, scales, rotations, cov3D_precomp)
+        shs, colors_precomp, scales, rotations, cov3D_precomp = _checked_inputs(shs, colors_precomp, scales, rotations,
+                                                                                cov3D_precomp)
         return rasterize_gaussians(means3D, means2D, shs, colors_precomp, opacities, scales, rotations, cov3D_precomp,
                                    self.raster_settings, geometry)
 
@@ -216,7 +223,8 @@ class GaussianRasterizer(nn.Module):
         K/rasterize_points.cu:27-33).  The caller must then ask stage.within_bound() after the
         forward has been issued (at the end of the iteration is early enough) and, if it is
         false, repeat the forward with a bound of at least stage.instances()."""
-        _check_inputs(shs, colors_precomp, scales, rotations, cov3D_precomp)
+        shs, colors_precomp, scales, rotations, cov3D_precomp = _checked_inputs(shs, colors_precomp, scales, rotations,
+                                                                                cov3D_precomp)
         if instance_bound is not None:
             instance_bound = int(instance_bound)
             if instance_bound < 0:

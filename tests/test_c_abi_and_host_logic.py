@@ -323,3 +323,35 @@ def test_errors_of_tensor_code_keep_their_types_through_the_host_path():
         rasterizer._gradient_outputs(4, 1, torch.device("xla"))      # a backend this build of PyTorch does not have
     with pytest.raises(RuntimeError, match="between one layer"):
         _host.composite(None, [])
+
+
+def _none_refusals():
+    """(name, call) of every tensor argument for which None is no tensor."""
+    from retinags_amd import GaussianRasterizationSettings, rasterizer
+    z = torch.zeros
+    settings = GaussianRasterizationSettings(
+        image_height=32, image_width=32, tanfovx=0.5, tanfovy=0.5, bg=z(3), scale_modifier=1.0, viewmatrix=torch.eye(4),
+        projmatrix=torch.eye(4), projmatrix_inv=torch.eye(4), range_low=-torch.ones(3), range_up=torch.ones(3),
+        sh_degree=3, campos=z(3), prefiltered=False, debug=False)
+    inputs = dict(means3D=z(5, 3), means2D=z(5, 3), sh=z(5, 16, 3), colors_precomp=torch.Tensor([]), opacities=z(5, 1), scales=z(5, 3),
+                  rotations=z(5, 4), cov3Ds_precomp=torch.Tensor([]))
+    for name in ("bg", "viewmatrix", "projmatrix", "projmatrix_inv", "range_low", "range_up", "campos"):
+        changed = settings._replace(**{name: None})
+        yield name, lambda s=changed: rasterizer.rasterize_gaussians(**inputs, raster_settings=s)
+        yield name, lambda s=changed: rasterizer._rasterize_layers([s], [dict(
+            means3D=z(5, 3), means2D=z(5, 3), shs=z(5, 16, 3), opacities=z(5, 1), scales=z(5, 3), rotations=z(5, 4))])
+        yield name, lambda s=changed: rasterizer.GaussianRasterizer(s).enqueue_geometry(z(5, 3), z(5, 1), z(5, 16, 3), None, z(5, 3), z(5, 4))
+    for name in inputs:
+        if name not in ("means3D", "means2D"):
+            yield name, lambda n=name: rasterizer.rasterize_gaussians(**dict(inputs, **{n: None}), raster_settings=settings)
+    yield "opacities", lambda: rasterizer._rasterize_layers([settings], [dict(
+        means3D=z(5, 3), means2D=z(5, 3), shs=z(5, 16, 3), opacities=None, scales=z(5, 3), rotations=z(5, 4))])
+    yield "opacities", lambda: rasterizer.GaussianRasterizer(settings).enqueue_geometry(z(5, 3), None, z(5, 16, 3), None, z(5, 3), z(5, 4))
+
+
+def test_none_in_the_place_of_a_tensor_is_a_type_error_that_names_it():
+    """The settings' tensors and a call's inputs have to be tensors (an absent input is an empty one; GaussianRasterizer makes
+    it of None); only the screen-space placeholder, whose values nobody reads, may be missing."""
+    for name, call in _none_refusals():
+        with pytest.raises(TypeError, match=name):
+            call()
