@@ -417,9 +417,9 @@ struct Call : torch::CustomClassHolder {
 	Rendered rendered;
 };
 
-variable_list call_backward(const Call& call, const variable_list& saved, const variable_list& grads)
+// `grads`: of the colour, of nothing, of the depth and of the alpha image; those that are not defined or empty are null pointers.
+GradientArrays gradients_of_call(const Settings& s, int64_t instances, const variable_list& saved, const variable_list& grads)
 {
-	const Settings& s = call.s;
 	const Tensor& means3D = saved[kSavedMeans3D];
 	const at::Device device = means3D.device();
 	const int64_t P = means3D.size(0), H = s.H, W = s.W;
@@ -439,7 +439,7 @@ variable_list call_backward(const Call& call, const variable_list& saved, const 
 		             proj_inv = device_f32(s.proj_inv, device), low = device_f32(s.low, device), up = device_f32(s.up, device),
 		             campos = device_f32(s.campos, device);
 		auto g = [&](int k) { return ptr(out.g[k]); };
-		check(rgs_backward(P, s.sh_degree, M, call.rendered.instances, W, H, ptr(bg), ptr(means3D), ptr(saved[kSavedSH]),
+		check(rgs_backward(P, s.sh_degree, M, instances, W, H, ptr(bg), ptr(means3D), ptr(saved[kSavedSH]),
 		                   ptr(saved[kSavedColors]), ptr(saved[kSavedAlpha]), ptr(saved[kSavedScales]), s.scale_modifier,
 		                   ptr(saved[kSavedRotations]), ptr(saved[kSavedCov3D]), ptr(view), ptr(proj), ptr(proj_inv), ptr(low), ptr(up),
 		                   ptr(campos), s.tanfovx, s.tanfovy, ptr<int>(saved[kSavedRadii]), ptr<void>(saved[kSavedGeom]),
@@ -447,6 +447,12 @@ variable_list call_backward(const Call& call, const variable_list& saved, const 
 		                   ptr(out.sums), g(kGradMeans2D), g(kGradOpacity), g(kGradColors), g(kGradMeans3D), g(kGradCov3D), g(kGradSH),
 		                   g(kGradScales), g(kGradRotations), 0, current_stream(device), s.debug));
 	}
+	return out;
+}
+
+variable_list call_backward(const Call& call, const variable_list& saved, const variable_list& grads)
+{
+	const GradientArrays out = gradients_of_call(call.s, call.rendered.instances, saved, grads);
 	variable_list result(kInputs + 1);
 	gradients_of_inputs(result, 0, out, present(saved[kSavedSH]), present(saved[kSavedColors]), present(saved[kSavedScales]),
 	                    present(saved[kSavedRotations]), present(saved[kSavedCov3D]));
@@ -522,6 +528,12 @@ std::array<Tensor, kInputs> inputs_from_python(const py::handle* given)
 	return in;
 }
 
+void check_stage(const GeometryStage& g, const Tensor& means3D, py::handle settings)
+{
+	if (g.source != means3D.data_ptr() || g.P != means3D.size(0) || g.settings.ptr() != settings.ptr() || g.used)
+		throw std::runtime_error("the geometry stage was enqueued for other inputs or settings, or already used");
+}
+
 py::tuple rasterize(py::handle means3D, py::handle means2D, py::handle sh, py::handle colors, py::handle opacities, py::handle scales,
                     py::handle rotations, py::handle cov3D, py::handle settings, py::handle geometry)
 {
@@ -531,9 +543,7 @@ py::tuple rasterize(py::handle means3D, py::handle means2D, py::handle sh, py::h
 	call->s = settings_from_python(settings);
 	if (!geometry.is_none()) {
 		call->stage = &py::cast<GeometryStage&>(geometry);
-		const GeometryStage& g = *call->stage;
-		if (g.source != in[kMeans3D].data_ptr() || g.P != in[kMeans3D].size(0) || g.settings.ptr() != settings.ptr() || g.used)
-			throw std::runtime_error("the geometry stage was enqueued for other inputs or settings, or already used");
+		check_stage(*call->stage, in[kMeans3D], settings);
 	}
 	variable_list out;
 	{
@@ -583,6 +593,44 @@ py::tuple rasterize_forward(Tensor bg, py::handle means3D, py::handle colors, py
 		r = run_raster(stage);
 	}
 	return py::make_tuple(r.instances, r.color, r.depth, r.alpha, stage.radii, stage.geom, r.binning, r.image);
+}
+
+// The same 8-tuple from a stage that is already on its way.
+py::tuple rasterize_forward_from_stage(GeometryStage& stage, const Tensor& means3D, py::handle settings)
+{
+	check_stage(stage, means3D, settings);
+	Rendered r;
+	{
+		py::gil_scoped_release no_gil;
+		at::NoGradGuard no_grad;
+		r = run_raster(stage);
+	}
+	return py::make_tuple(r.instances, r.color, r.depth, r.alpha, stage.radii, stage.geom, r.binning, r.image);
+}
+
+// RasterizeGaussiansBackwardCUDA_hgs (K/rasterize_points.cu:127-220): its arguments in its order, its 8 tensors.
+py::tuple rasterize_backward(Tensor bg, Tensor means3D, Tensor radii, Tensor colors, Tensor scales, Tensor rotations, double scale_modifier,
+                             Tensor cov3D, Tensor view, Tensor proj, Tensor proj_inv, Tensor low, Tensor up, double tanfovx, double tanfovy,
+                             Tensor grad_color, Tensor grad_depth, Tensor grad_alpha, Tensor sh, int sh_degree, Tensor campos, Tensor geom,
+                             int64_t instances, Tensor binning, Tensor image, Tensor alpha, bool debug)
+{
+	check_means(means3D);
+	if (grad_color.dim() != 3 || grad_color.size(0) != 3)
+		throw std::runtime_error("grad_color must have dimensions (3, height, width)");
+	const at::Device device = means3D.device();
+	const Settings s = {grad_color.size(1), grad_color.size(2), tanfovx, tanfovy,   bg,     scale_modifier, view, proj, proj_inv,
+	                    low,                up,                 sh_degree, campos, false, debug};
+	GradientArrays out;
+	{
+		py::gil_scoped_release no_gil;
+		at::NoGradGuard no_grad;
+		auto f = [&](const Tensor& t) { return device_f32(t, device); };
+		out = gradients_of_call(s, instances, {f(colors), f(means3D), f(scales), f(rotations), f(cov3D), radii, f(sh), geom, binning, image, f(alpha)},
+		                        {grad_color, Tensor(), grad_depth, grad_alpha});
+	}
+	const auto& g = out.g;
+	return py::make_tuple(g[kGradMeans2D], g[kGradColors], g[kGradOpacity], g[kGradMeans3D], g[kGradCov3D], g[kGradSH], g[kGradScales],
+	                      g[kGradRotations]);
 }
 
 // ---- the layers of a frame together ------------------------------------------------------------------------------
@@ -913,6 +961,8 @@ PYBIND11_MODULE(_host, m)
 	m.def("gradient_outputs", &gradient_outputs);
 	m.def("rasterize", &rasterize);
 	m.def("rasterize_forward", &rasterize_forward);
+	m.def("rasterize_forward_from_stage", &rasterize_forward_from_stage);
+	m.def("rasterize_backward", &rasterize_backward);
 	m.def("rasterize_frame", &rasterize_frame);
 	m.def("enqueue_geometry", &enqueue_geometry);
 	define_training(m);

@@ -116,10 +116,23 @@ def gradNormHelpFunction(meta: torch.Tensor, spare_rows: int = 0) -> torch.Tenso
     return _host.screen_placeholder(meta, spare_rows)
 
 
-class GradNormHelper:
-    """gradNormHelpFunction under the name of the reference's autograd function."""
+class GradNormHelper(torch.autograd.Function):
+    """gradNormHelpFunction under the name of the reference's autograd function.  apply() is the native one; forward and
+    backward are for those who call them or derive from them, and a derived class's apply() runs them."""
 
-    apply = staticmethod(gradNormHelpFunction)
+    @classmethod
+    def apply(cls, meta, *spare_rows):
+        return gradNormHelpFunction(meta, *spare_rows) if cls is GradNormHelper else super().apply(meta, *spare_rows)
+
+    @staticmethod
+    def forward(ctx, meta: torch.Tensor) -> torch.Tensor:
+        if meta.dim() != 2 or meta.shape[1] != 1:
+            raise RuntimeError("meta must have shape (N, 1)")
+        return torch.zeros((meta.shape[0], 3), dtype=meta.dtype, device=meta.device)
+
+    @staticmethod
+    def backward(ctx, grad_output: torch.Tensor) -> torch.Tensor:
+        return torch.norm(grad_output[:, :2], dim=-1, keepdim=True)
 
 
 def raster_settings(cam: Camera, sub: Submodel, bg: torch.Tensor, scaling_modifier: float = 1.0,

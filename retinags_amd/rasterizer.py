@@ -89,6 +89,18 @@ def _gradient_outputs(P, M, device, scratch=()):
     return _host.gradient_outputs(P, M, device, scratch)
 
 
+def _rasterize_backward(bg, means3D, radii, colors_precomp, scales, rotations, scale_modifier, cov3Ds_precomp,
+                        viewmatrix, projmatrix, projmatrix_inv, range_low, range_up, tanfovx, tanfovy, grad_color,
+                        grad_depth, grad_alpha, sh, sh_degree, campos, geomBuffer, num_rendered, binningBuffer,
+                        imgBuffer, alpha, debug):
+    """Counterpart of RasterizeGaussiansBackwardCUDA_hgs (K/rasterize_points.cu:127-220);
+    returns the same 8 tensors in the same order."""
+    return _host.rasterize_backward(bg, means3D, radii, colors_precomp, scales, rotations, float(scale_modifier),
+                                    cov3Ds_precomp, viewmatrix, projmatrix, projmatrix_inv, range_low, range_up,
+                                    float(tanfovx), float(tanfovy), grad_color, grad_depth, grad_alpha, sh, int(sh_degree),
+                                    campos, geomBuffer, int(num_rendered), binningBuffer, imgBuffer, alpha, bool(debug))
+
+
 def _mark_visible(means3D, viewmatrix, projmatrix):
     """Counterpart of markVisible_hgs (K/rasterize_points.cu:222-241)."""
     device = means3D.device
@@ -112,42 +124,92 @@ def rasterize_gaussians(means3D, means2D, sh, colors_precomp, opacities, scales,
                                      cov3Ds_precomp, raster_settings, geometry)
 
 
-class _RasterizeGaussians:
-    """K/diff_gaussian_rasterization_half_gaussian/__init__.py:44-164: forward and backward of one call as an autograd
-    function (RasterizeCall of csrc/host.cpp)."""
-
-    @staticmethod
-    def apply(means3D, means2D, sh, colors_precomp, opacities, scales, rotations, cov3Ds_precomp, raster_settings,
-              geometry=None):
-        run = lambda: _host.rasterize(means3D, means2D, sh, colors_precomp, opacities, scales, rotations, cov3Ds_precomp,
-                                      raster_settings, geometry)
-        if not raster_settings.debug or geometry is not None:
-            return run()
-        args = (
-            raster_settings.bg, means3D, colors_precomp, opacities, scales, rotations, raster_settings.scale_modifier,
-            cov3Ds_precomp, raster_settings.viewmatrix, raster_settings.projmatrix, raster_settings.projmatrix_inv,
-            raster_settings.range_low, raster_settings.range_up, raster_settings.tanfovx, raster_settings.tanfovy,
-            raster_settings.image_height, raster_settings.image_width, sh, raster_settings.sh_degree,
-            raster_settings.campos, raster_settings.prefiltered, raster_settings.debug,
-        )
-        cpu_args = cpu_deep_copy_tuple(args)  # copy them before they can be corrupted
-        try:
-            return run()
-        except Exception as ex:
-            torch.save(cpu_args, "snapshot_fw.dump")
-            print("\nAn error occured in forward. Please forward snapshot_fw.dump for debugging.")
-            raise ex
+def _forward_in_debug(args, run):
+    """A forward in debug mode: its arguments are kept aside and written to a file if it fails."""
+    cpu_args = cpu_deep_copy_tuple(args)  # copy them before they can be corrupted
+    try:
+        return run()
+    except Exception as ex:
+        torch.save(cpu_args, "snapshot_fw.dump")
+        print("\nAn error occured in forward. Please forward snapshot_fw.dump for debugging.")
+        raise ex
 
 
 def _backward_in_debug(args, run):
     """The backward of a call in debug mode: its arguments are kept aside and written to a file if it fails."""
     cpu_args = cpu_deep_copy_tuple(args)
     try:
-        run()
+        return run()
     except Exception as ex:
         torch.save(cpu_args, "snapshot_bw.dump")
         print("\nAn error occured in backward. Writing snapshot_bw.dump for debugging.\n")
         raise ex
+
+
+class _RasterizeGaussians(torch.autograd.Function):
+    """K/diff_gaussian_rasterization_half_gaussian/__init__.py:44-164: forward and backward of one call as an autograd
+    function.  apply() goes through the native one (RasterizeCall of csrc/host.cpp), which does the same without coming back
+    to Python; forward and backward are for those who call them or derive from them, and a derived class's apply() runs them."""
+
+    @classmethod
+    def apply(cls, means3D, means2D, sh, colors_precomp, opacities, scales, rotations, cov3Ds_precomp, raster_settings,
+              geometry=None):
+        if cls is not _RasterizeGaussians:
+            return super().apply(means3D, means2D, sh, colors_precomp, opacities, scales, rotations, cov3Ds_precomp,
+                                 raster_settings, geometry)
+        run = lambda: _host.rasterize(means3D, means2D, sh, colors_precomp, opacities, scales, rotations, cov3Ds_precomp,
+                                      raster_settings, geometry)
+        if not raster_settings.debug or geometry is not None:
+            return run()
+        return _forward_in_debug(_forward_arguments(means3D, sh, colors_precomp, opacities, scales, rotations, cov3Ds_precomp,
+                                                    raster_settings), run)
+
+    @staticmethod
+    def forward(ctx, means3D, means2D, sh, colors_precomp, opacities, scales, rotations, cov3Ds_precomp,
+                raster_settings, geometry=None):
+        if geometry is not None:
+            outs = _host.rasterize_forward_from_stage(geometry, means3D, raster_settings)
+        else:
+            args = _forward_arguments(means3D, sh, colors_precomp, opacities, scales, rotations, cov3Ds_precomp, raster_settings)
+            run = lambda: _rasterize_forward(*args)
+            outs = _forward_in_debug(args, run) if raster_settings.debug else run()
+        num_rendered, color, depth, alpha, radii, geomBuffer, binningBuffer, imgBuffer = outs
+
+        ctx.set_materialize_grads(False)  # an output that took no part in the loss comes back as None, not as a tensor of zeros
+        ctx.raster_settings = raster_settings
+        ctx.num_rendered = num_rendered
+        ctx.save_for_backward(colors_precomp, means3D, scales, rotations, cov3Ds_precomp, radii, sh, geomBuffer,
+                              binningBuffer, imgBuffer, alpha)
+        ctx.mark_non_differentiable(radii)
+        return color, radii, depth, alpha
+
+    @staticmethod
+    def backward(ctx, grad_color, grad_radii, grad_depth, grad_alpha):
+        rs = ctx.raster_settings
+        (colors_precomp, means3D, scales, rotations, cov3Ds_precomp, radii, sh, geomBuffer, binningBuffer, imgBuffer,
+         alpha) = ctx.saved_tensors
+        # The reference's C++ side always receives dense tensors; here an absent depth / alpha gradient goes down as a null
+        # pointer, which the library takes as zero.
+        if grad_color is None:
+            grad_color = torch.zeros((3,) + tuple(alpha.shape[1:]), dtype=alpha.dtype, device=alpha.device)
+        args = (rs.bg, means3D, radii, colors_precomp, scales, rotations, rs.scale_modifier, cov3Ds_precomp, rs.viewmatrix,
+                rs.projmatrix, rs.projmatrix_inv, rs.range_low, rs.range_up, rs.tanfovx, rs.tanfovy, grad_color,
+                _EMPTY if grad_depth is None else grad_depth, _EMPTY if grad_alpha is None else grad_alpha, sh, rs.sh_degree,
+                rs.campos, geomBuffer, ctx.num_rendered, binningBuffer, imgBuffer, alpha, rs.debug)
+        run = lambda: _rasterize_backward(*args)
+        (grad_means2D, grad_colors_precomp, grad_opacities, grad_means3D, grad_cov3Ds_precomp, grad_sh, grad_scales,
+         grad_rotations) = _backward_in_debug(args, run) if rs.debug else run()
+        return (grad_means3D, grad_means2D, grad_sh if sh.numel() else None,
+                grad_colors_precomp if colors_precomp.numel() else None, grad_opacities,
+                grad_scales if scales.numel() else None, grad_rotations if rotations.numel() else None,
+                grad_cov3Ds_precomp if cov3Ds_precomp.numel() else None, None, None)
+
+
+def _forward_arguments(means3D, sh, colors_precomp, opacities, scales, rotations, cov3Ds_precomp, rs):
+    """The arguments of the reference's C++ forward in its order (K/rasterize_points.cu:35-58)."""
+    return (rs.bg, means3D, colors_precomp, opacities, scales, rotations, rs.scale_modifier, cov3Ds_precomp, rs.viewmatrix,
+            rs.projmatrix, rs.projmatrix_inv, rs.range_low, rs.range_up, rs.tanfovx, rs.tanfovy, rs.image_height, rs.image_width,
+            sh, rs.sh_degree, rs.campos, rs.prefiltered, rs.debug)
 
 
 def rasterize_frame(rasterizers, inputs, streams=None, workspaces=None):

@@ -355,3 +355,26 @@ def test_none_in_the_place_of_a_tensor_is_a_type_error_that_names_it():
     for name, call in _none_refusals():
         with pytest.raises(TypeError, match=name):
             call()
+
+
+def test_the_names_of_the_reference_are_autograd_functions():
+    """_RasterizeGaussians and GradNormHelper can be derived from and their forward and backward called, whatever their own
+    apply() goes through."""
+    from retinags_amd import _RasterizeGaussians
+    from retinags_amd.harness.pipeline import GradNormHelper
+    assert issubclass(_RasterizeGaussians, torch.autograd.Function) and issubclass(GradNormHelper, torch.autograd.Function)
+    assert callable(_RasterizeGaussians.forward) and callable(_RasterizeGaussians.backward)
+
+    class Doubled(GradNormHelper):
+        @staticmethod
+        def backward(ctx, grad_output):
+            return 2.0 * GradNormHelper.backward(ctx, grad_output)
+
+    got = []
+    for function in (GradNormHelper, Doubled):
+        meta = torch.zeros(5, 1, requires_grad=True)
+        placeholder = function.apply(meta)
+        assert placeholder.shape == (5, 3) and (placeholder == 0).all()
+        (placeholder * torch.arange(15.0).reshape(5, 3)).sum().backward()
+        got.append(meta.grad)
+    assert torch.equal(got[0][:, 0], torch.arange(15.0).reshape(5, 3)[:, :2].norm(dim=1)) and torch.equal(got[1], 2.0 * got[0])

@@ -706,3 +706,36 @@ def test_out_of_memory_and_hooks_keep_their_types_and_the_call_can_be_repeated()
     leaf = layers[0][0].requires_grad_(True)
     with torch.autograd.graph.saved_tensors_hooks(refuse, lambda t: t), pytest.raises(Refused):
         composite_partial_images([leaf], layers[1], layers[2])
+
+
+@pytest.mark.parametrize("staged", [False, True])
+def test_the_autograd_function_of_a_derived_class_does_what_the_native_one_does(staged):
+    """apply() of a class derived from _RasterizeGaussians runs forward and backward as Python calls them (8-tuples), with and
+    without a geometry stage; results of the native function, gradients up to the order of the float atomics."""
+    from retinags_amd import GaussianRasterizer, rasterizer
+
+    class Derived(rasterizer._RasterizeGaussians):
+        pass
+
+    scene, cam, low, up = _small_inputs(n=5000, seed=6)
+    settings = _settings(oracle_settings(cam, low, up, torch.tensor([0.3, 0.2, 0.1])))
+    empty = torch.Tensor([])
+
+    def run(function):
+        leaves = {k: scene[k].to(DEV).requires_grad_(True) for k in ("xyz", "opacity", "shs", "scales", "rotations")}
+        m2d = torch.zeros_like(leaves["xyz"], requires_grad=True)
+        stage = GaussianRasterizer(settings).enqueue_geometry(leaves["xyz"], leaves["opacity"], shs=leaves["shs"], scales=leaves["scales"],
+                                                              rotations=leaves["rotations"]) if staged else None
+        out = function.apply(leaves["xyz"], m2d, leaves["shs"], empty, leaves["opacity"], leaves["scales"], leaves["rotations"], empty,
+                             settings, stage)
+        color, radii, depth, alpha = out
+        gen = torch.Generator().manual_seed(9)
+        g = [torch.randn(t.shape, generator=gen).to(DEV) * 1e-2 for t in (color, alpha)]
+        return out, torch.autograd.grad([color, alpha], [m2d] + list(leaves.values()), g, retain_graph=True)
+
+    native, derived = run(rasterizer._RasterizeGaussians), run(Derived)
+    assert len(derived[0][0].grad_fn.saved_tensors) == 11
+    for a, b in zip(native[0], derived[0]):
+        assert torch.equal(a, b)
+    for a, b in zip(native[1], derived[1]):
+        assert rel_l2(b.cpu().numpy(), a.cpu().numpy()) <= 1e-4
