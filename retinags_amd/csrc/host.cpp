@@ -334,37 +334,32 @@ struct GradientArrays {
 	Tensor sums;
 };
 
+// The gradient arrays of a layer but for those that are left out, each an allocation of its own: a gradient that the caller keeps
+// holds no other.
+GradientArrays new_gradients(int64_t P, int64_t M, const at::Device& device, const std::array<bool, kGradients>& left_out)
+{
+	const std::array<std::vector<int64_t>, kGradients> shapes = {{{P, 3}, {P, 1}, {P, 3}, {P, 3}, {P, 6}, {P, M, 3}, {P, 3}, {P, 4}}};
+	GradientArrays r;
+	for (int k = 0; k < kGradients; k++)
+		if (!left_out[k])
+			r.g[k] = new_f32(shapes[k], device);
+	r.sums = new_f32({P, kSumFloats}, device);
+	return r;
+}
+
 py::dict gradient_outputs(int64_t P, int64_t M, py::handle device_object, py::handle scratch)
 {
 	const at::Device device = THPDevice_Check(device_object.ptr()) ? reinterpret_cast<THPDevice*>(device_object.ptr())->device
 	                                                               : at::Device(py::cast<std::string>(device_object));
-	const std::array<std::vector<int64_t>, kGradients> shapes = {{{P, 3}, {P, 1}, {P, 3}, {P, 3}, {P, 6}, {P, M, 3}, {P, 3}, {P, 4}}};
-	std::array<int64_t, kGradients> at_element;
-	int64_t total = 0;
-	for (int k = 0; k < kGradients; k++) {
-		const bool made = !scratch.contains(kGradientNames[k]);
-		at_element[k] = made ? total : -1;
-		if (made)
-			total += (c10::multiply_integers(shapes[k]) + 63) / 64 * 64;  // 256-byte aligned parts
-	}
-	const Tensor block = new_f32({total}, device);
+	std::array<bool, kGradients> left_out;
+	for (int k = 0; k < kGradients; k++)
+		left_out[k] = scratch.contains(kGradientNames[k]);
+	const GradientArrays made = new_gradients(P, M, device, left_out);
 	py::dict out;
 	for (int k = 0; k < kGradients; k++)
-		out[kGradientNames[k]] = at_element[k] < 0 ? py::none() : py::cast(carved(block, at_element[k], shapes[k]));
-	out["sums"] = new_f32({P, kSumFloats}, device);
+		out[kGradientNames[k]] = to_python(made.g[k]);
+	out["sums"] = made.sums;
 	return out;
-}
-
-// The gradient arrays of a layer, by way of the Python function of that name, which is where they are made.
-GradientArrays make_gradients(py::handle module, int64_t P, int64_t M, const at::Device& device, const py::tuple& scratch)
-{
-	py::object made = module.attr("_gradient_outputs")(P, M, py::reinterpret_steal<py::object>(THPDevice_New(device)),
-	                                                   py::arg("scratch") = scratch);
-	GradientArrays r;
-	for (int k = 0; k < kGradients; k++)
-		r.g[k] = from_python(made[kGradientNames[k]], kGradientNames[k]);
-	r.sums = from_python(made["sums"], "sums");
-	return r;
 }
 
 py::handle rasterizer_module()
@@ -379,6 +374,32 @@ py::handle rasterizer_module()
 		module = imported;
 	}
 	return module;
+}
+
+// _gradient_outputs of that module as it was when the module was imported.
+PyObject* original_gradient_outputs = nullptr;
+void set_original_gradient_outputs(py::object f) { original_gradient_outputs = f.release().ptr(); }
+
+// The gradient arrays of a layer: made here, or by the module's function of that name where another has been put in its place.
+GradientArrays make_gradients(int64_t P, int64_t M, const at::Device& device, const std::array<bool, kGradients>& left_out)
+{
+	{
+		py::gil_scoped_acquire gil;
+		const py::object f = rasterizer_module().attr("_gradient_outputs");
+		if (f.ptr() != original_gradient_outputs) {
+			py::list scratch;
+			for (int k = 0; k < kGradients; k++)
+				if (left_out[k])
+					scratch.append(kGradientNames[k]);
+			const py::object made = f(P, M, py::reinterpret_steal<py::object>(THPDevice_New(device)), py::arg("scratch") = py::tuple(scratch));
+			GradientArrays r;
+			for (int k = 0; k < kGradients; k++)
+				r.g[k] = from_python(made[kGradientNames[k]], kGradientNames[k]);
+			r.sums = tensor_from_python(made["sums"], "sums");
+			return r;
+		}
+	}
+	return new_gradients(P, M, device, left_out);
 }
 
 // The gradients of a layer without Gaussians.
@@ -428,10 +449,7 @@ GradientArrays gradients_of_call(const Settings& s, int64_t instances, const var
 	if (P == 0) {
 		out = empty_gradients(M, device);
 	} else {
-		{
-			py::gil_scoped_acquire gil;
-			out = make_gradients(rasterizer_module(), P, M, device, py::tuple());
-		}
+		out = make_gradients(P, M, device, {});
 		c10::DeviceGuard guard(device);
 		const Tensor g_color = grads[0].defined() ? device_f32(grads[0], device) : new_f32({3, H, W}, device).zero_();
 		const Tensor g_depth = device_f32(grads[2], device), g_alpha = device_f32(grads[3], device);
@@ -796,21 +814,15 @@ struct RasterizeFrame : torch::autograd::Function<RasterizeFrame> {
 			const hipStream_t main = current_stream(device);
 			auto sv = [&](int k, int i) -> const Tensor& { return saved[k * kSavedPerLayer + i]; };
 			std::vector<GradientArrays> made(K);
-			{
-				py::gil_scoped_acquire gil;
-				const py::handle module = rasterizer_module();
-				for (int k = 0; k < K; k++) {
-					if (frame.layers[k].P == 0)
-						continue;
-					// arrays nobody gets to see are not made: the colour gradient when the colours come from SH, the covariance
-					// gradient when it comes from scale and rotation
-					py::list scratch;
-					if (!present(sv(k, kSavedColors)))
-						scratch.append(kGradientNames[kGradColors]);
-					if (!present(sv(k, kSavedCov3D)))
-						scratch.append(kGradientNames[kGradCov3D]);
-					made[k] = make_gradients(module, frame.layers[k].P, frame.layers[k].M, device, py::tuple(scratch));
-				}
+			for (int k = 0; k < K; k++) {
+				if (frame.layers[k].P == 0)
+					continue;
+				// arrays nobody gets to see are not made: the colour gradient when the colours come from SH, the covariance
+				// gradient when it comes from scale and rotation
+				std::array<bool, kGradients> left_out{};
+				left_out[kGradColors] = !present(sv(k, kSavedColors));
+				left_out[kGradCov3D] = !present(sv(k, kSavedCov3D));
+				made[k] = make_gradients(frame.layers[k].P, frame.layers[k].M, device, left_out);
 			}
 			const std::array<Tensor, 4> vt = view_tensors(s0, device);
 			const rgs_frame_view view = view_of(s0, vt);
@@ -959,6 +971,7 @@ PYBIND11_MODULE(_host, m)
 
 	m.def("composite", &composite);
 	m.def("gradient_outputs", &gradient_outputs);
+	m.def("set_original_gradient_outputs", &set_original_gradient_outputs);
 	m.def("rasterize", &rasterize);
 	m.def("rasterize_forward", &rasterize_forward);
 	m.def("rasterize_forward_from_stage", &rasterize_forward_from_stage);

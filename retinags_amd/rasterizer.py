@@ -76,17 +76,19 @@ def _rasterize_forward(bg, means3D, colors_precomp, opacities, scales, rotations
 
 
 def _gradient_outputs(P, M, device, scratch=()):
-    """The eight dense gradient tensors of K/rasterize_points.cu:165-174, carved out of one
-    uninitialised allocation (the library writes every row of them: those of Gaussians that were
-    not rendered as zeros), and the backward's scratch for the per-Gaussian sums in an
-    allocation of its own (the library clears it), so that a
-    gradient the caller keeps (the means2D gradient, say, for densification statistics) does not
-    hold on to the scratch.  The eight do share one block: keeping any of them keeps all (about
-    280 bytes per Gaussian with SH degree 3).  `scratch` names those of the eight that the caller
+    """The eight dense gradient tensors of K/rasterize_points.cu:165-174, uninitialised (the library
+    writes every row of them: those of Gaussians that were not rendered as zeros), and the
+    backward's scratch for the per-Gaussian sums (the library clears it).  Each is an allocation of
+    its own: what a caller keeps, a leaf's .grad or the means2D gradient for densification
+    statistics, holds nothing else.  `scratch` names those of the eight that the caller
     hands to nobody (the colour gradient when the colours come from SH, the covariance gradient
     when it comes from scale and rotation): they are not made at all (None), and the library
-    does not write them.  The backward nodes ask for their arrays here."""
+    does not write them.  The backward nodes make the same arrays without coming here, unless
+    another function has been put in the place of this one: that one is asked."""
     return _host.gradient_outputs(P, M, device, scratch)
+
+
+_host.set_original_gradient_outputs(_gradient_outputs)
 
 
 def _rasterize_backward(bg, means3D, radii, colors_precomp, scales, rotations, scale_modifier, cov3Ds_precomp,

@@ -739,3 +739,20 @@ def test_the_autograd_function_of_a_derived_class_does_what_the_native_one_does(
         assert torch.equal(a, b)
     for a, b in zip(native[1], derived[1]):
         assert rel_l2(b.cpu().numpy(), a.cpu().numpy()) <= 1e-4
+
+
+@pytest.mark.parametrize("through_frame", [False, True])
+def test_a_gradient_that_is_kept_holds_no_other(through_frame):
+    """What a caller keeps of a backward, a leaf's .grad or a gradient by itself, is an allocation of its own: it keeps no other
+    gradient's memory alive."""
+    from retinags_amd import GaussianRasterizer, rasterizer
+    scene, cam, low, up = _small_inputs(n=5003, seed=4)
+    r = GaussianRasterizer(_settings(oracle_settings(cam, low, up, torch.zeros(3))))
+    leaves = {k: scene[k].to(DEV).requires_grad_(True) for k in ("xyz", "opacity", "shs", "scales", "rotations")}
+    m2d = torch.zeros_like(leaves["xyz"], requires_grad=True)
+    kw = dict(means3D=leaves["xyz"], means2D=m2d, opacities=leaves["opacity"], shs=leaves["shs"], scales=leaves["scales"],
+              rotations=leaves["rotations"])
+    color = (rasterizer.rasterize_frame([r], [kw])[0] if through_frame else r(**kw))[0]
+    color.sum().backward()
+    for name, t in dict(leaves, means2D=m2d).items():
+        assert t.grad.untyped_storage().nbytes() == 4 * t.numel(), name
