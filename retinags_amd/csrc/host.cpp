@@ -195,11 +195,12 @@ struct GeometryStage {
 	std::array<Tensor, kInputs> in;
 	Tensor radii, geom;
 	const void* source = nullptr;
-	bool used = false;
+	std::atomic<bool> used{false};
 	std::optional<int64_t> bound, count;
 	bool in_flight = false;
 	CountSlot slot;
-	py::object settings;  // of a stage that Python holds
+	std::mutex count_mutex;  // several threads may ask for the count, without the interpreter lock
+	py::object settings;     // of a stage that Python holds
 
 	GeometryStage() = default;
 	GeometryStage(const GeometryStage&) = delete;
@@ -213,6 +214,7 @@ struct GeometryStage {
 	// The number of (Gaussian, tile) instances; waits for it if it is still on its way.
 	int64_t instances()
 	{
+		std::lock_guard<std::mutex> lock(count_mutex);
 		if (!count) {
 			if (!in_flight)
 				throw std::runtime_error("this stage has no instance count");
@@ -294,9 +296,8 @@ void make_package(Rendered& r, int64_t H, int64_t W, const at::Device& device)
 // Second half: waits for the instance count if it is still on its way, sizes the binning workspace with it, sorts and blends.
 Rendered run_raster(GeometryStage& g)
 {
-	if (g.used)
+	if (g.used.exchange(true))
 		throw std::runtime_error("this geometry stage has already been consumed");
-	g.used = true;
 	if (current_stream(g.device) != g.stream)
 		throw std::runtime_error("the geometry stage was enqueued on another stream than the one current now");
 	Rendered r;
@@ -987,7 +988,7 @@ PYBIND11_MODULE(_host, m)
 	    .def_readonly("P", &GeometryStage::P)
 	    .def_readonly("H", &GeometryStage::H)
 	    .def_readonly("W", &GeometryStage::W)
-	    .def_readonly("used", &GeometryStage::used)
+	    .def_property_readonly("used", [](const GeometryStage& g) { return g.used.load(); })
 	    .def_property_readonly("settings", [](const GeometryStage& g) { return g.settings; })
 	    .def_readonly("radii", &GeometryStage::radii)
 	    .def_readonly("geomBuffer", &GeometryStage::geom)

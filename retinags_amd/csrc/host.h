@@ -11,6 +11,7 @@
 #include <c10/hip/HIPStream.h>
 
 #include <array>
+#include <atomic>
 #include <deque>
 #include <map>
 #include <mutex>

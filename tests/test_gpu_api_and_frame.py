@@ -756,3 +756,42 @@ def test_a_gradient_that_is_kept_holds_no_other(through_frame):
     color.sum().backward()
     for name, t in dict(leaves, means2D=m2d).items():
         assert t.grad.untyped_storage().nbytes() == 4 * t.numel(), name
+
+
+def test_threads_that_ask_one_stage_for_its_count_and_forward():
+    """Threads that ask the same stage for its count at once all get it, and its landing place goes back once: stages that are
+    under way together afterwards have their own.  Of threads that forward one stage together exactly one may."""
+    import threading
+    from retinags_amd import GaussianRasterizer
+    inputs = []
+    for n in (3000, 5000):
+        scene, cam, low, up = _small_inputs(n=n, seed=n)
+        r = GaussianRasterizer(_settings(oracle_settings(cam, low, up, torch.zeros(3))))
+        d = {k: scene[k].to(DEV) for k in ("xyz", "opacity", "shs", "scales", "rotations")}
+        inputs.append((r, d, lambda r=r, d=d: r.enqueue_geometry(d["xyz"], d["opacity"], shs=d["shs"], scales=d["scales"], rotations=d["rotations"])))
+    counts = [enqueue().instances() for _, _, enqueue in inputs]
+    assert counts[0] != counts[1]
+
+    def together(work, threads=8):
+        got, gate = [], threading.Barrier(threads)
+
+        def run():
+            gate.wait()
+            try:
+                got.append(work())
+            except RuntimeError as e:
+                got.append(e)
+        ts = [threading.Thread(target=run) for _ in range(threads)]
+        [t.start() for t in ts]
+        [t.join() for t in ts]
+        return got
+
+    for _ in range(10):
+        assert together(inputs[0][2]().instances) == [counts[0]] * 8
+        under_way = [inputs[k % 2][2]() for k in range(6)]
+        assert [s.instances() for s in under_way] == counts * 3
+    r, d, enqueue = inputs[0]
+    stage = enqueue()
+    got = together(lambda: r(means3D=d["xyz"], means2D=torch.zeros_like(d["xyz"]), opacities=d["opacity"], shs=d["shs"], scales=d["scales"],
+                             rotations=d["rotations"], geometry=stage))
+    assert sum(isinstance(g, tuple) for g in got) == 1 and stage.used
