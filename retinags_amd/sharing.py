@@ -69,6 +69,8 @@ def select_straddlers(models: Sequence[SharedGSInfo], box_low, box_up, capacity:
     K = len(models)
     if K > _capi.MAX_SHARE_BOXES:
         raise RuntimeError(f"{K} submodels: at most {_capi.MAX_SHARE_BOXES} per call")
+    if capacity is not None and int(capacity) < 0:
+        raise RuntimeError(f"a capacity of {capacity} rows: it must not be negative")
     low = np.ascontiguousarray(np.asarray(box_low, dtype=np.float32).reshape(K, 3))
     up = np.ascontiguousarray(np.asarray(box_up, dtype=np.float32).reshape(K, 3))
     own = [len(m) for m in models]

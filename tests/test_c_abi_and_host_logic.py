@@ -378,3 +378,10 @@ def test_the_names_of_the_reference_are_autograd_functions():
         (placeholder * torch.arange(15.0).reshape(5, 3)).sum().backward()
         got.append(meta.grad)
     assert torch.equal(got[0][:, 0], torch.arange(15.0).reshape(5, 3)[:, :2].norm(dim=1)) and torch.equal(got[1], 2.0 * got[0])
+
+
+def test_a_negative_capacity_of_straddlers_is_refused():
+    """(In the native host path a negative one stands for a capacity that depends on the submodel's size.)"""
+    from retinags_amd.sharing import select_straddlers
+    with pytest.raises(RuntimeError, match="negative"):
+        select_straddlers([], torch.zeros(0, 3), torch.zeros(0, 3), capacity=-5)
