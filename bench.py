@@ -325,7 +325,10 @@ def measure(args, config, forward_only, asides, cpu, apart_too=False, morton_too
     N = W * H
     tile_bits = int(_capi.lib.rgs_get_higher_msb(T))
     passes = min((tile_bits + 8) // 9, (tile_bits + 7) // 8)   # of the instance sort, on the tile key: digits of up to 9 bits
-    # The backward revisits, per pixel, the entries up to the last blended one: nAl of the nA visits.
+    # The backward revisits, per pixel, the entries up to the last blended one: nAl of the nA visits.  These are the visits of
+    # the reference's loop, which looks at every entry of a tile's list in every pixel; the kernels here leave out most of those
+    # that blend nothing.  So achieved_TFLOPs of the blends is the rate at which that loop's work gets done, and not that of the
+    # instructions executed, which may be fewer: for those see valu_issue.
     flops_fwd = 12 * nA + 3 * nB + 27 * nC + 3 * nD + 14 * nE
     flops_bwd = 12 * nAl + 3 * nBl + 27 * nCl + 80 * nE
     # Algorithmic bytes per frame of every HBM-bound stage (one launch per submodel; the sort
@@ -397,10 +400,10 @@ def measure(args, config, forward_only, asides, cpu, apart_too=False, morton_too
             roofline = {"kernel": dominant, "bound": "valu", "achieved": d["achieved_TFLOPs"],
                         "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": d["frac"], "traffic": None,
                         "bound_note": "fp32 vector-ALU issue (per-pixel compare / exp / blend arithmetic, no dense "
-                                      "contraction, so no MFMA); peak is the published 157.3 TFLOP/s fp32 figure, which "
-                                      "counts packed two-wide fp32 instructions; the library is built with those switched "
-                                      "off, so full-rate issue of fused multiply-adds is 78.6 TFLOP/s",
-                        "frac_of_unpacked_fp32_issue_peak": round(d["achieved_TFLOPs"] / (FP32_PEAK_TFLOPS / 2), 4)}
+                                      "contraction, so no MFMA); achieved is the rate of the reference loop's flops, of "
+                                      "which the kernel leaves out visits that blend nothing (executed instructions: "
+                                      "valu_issue); peak is the published 157.3 TFLOP/s fp32 figure, which counts packed "
+                                      "two-wide fp32 instructions, and the library is built with those switched off"}
         if roofline is not None:
             full_c1 = config == "C1" and args.shrink == 1.0 and args.resolution_scale == 1.0
             traffic, commit = load_traffic_table()

@@ -1033,7 +1033,7 @@ static size_t sort_tiles(size_t n, int items)
 	return (n + block - 1) / block;
 }
 
-// (a launch takes its tiles by the pairs of all its jobs, n among them: never smaller ones than n alone would have)
+// (a launch takes its tiles by the room of all its jobs, n among them: never smaller ones than n alone would have)
 size_t sort_clear_words(size_t n, int end_bit, int max_bits)
 {
 	const size_t tiles = sort_tiles(n, sort_items(n));

@@ -24,8 +24,10 @@
 // each half walk their own packed entries side by side (as many steps as the longer of the two).
 //
 // (Inside the walk the floor power >= -ln(255 * opacity), which alpha >= 1/255 needs and the packing uses, is not looked at
-// again: skipping a group of four entries that no live lane reaches, before exp() is evaluated, was measured to cost more
-// than it saves once the walk had no other branches: 0.313 -> 0.289 ms without it at 1600x1036 with 5.6 M Gaussians.)
+// again: skipping a group of four entries that no live lane reaches, before exp() is evaluated, costs more than it saves where
+// most visited entries blend somewhere.  Without the test and with it (in a build for five wavefronts per SIMD, since it needs
+// registers that six do not leave), us: 287 and 300 at 1600x1036 with 5.6 M Gaussians, 1847 and 1919 at 5185x3359, 158 and 168
+// for the view of a city; but 924 and 896 for the scene of 62.9 M Gaussians, where one visit in twenty blends.)
 #include "rgs_kernels.h"
 #include "strip_filing.h"
 #include "tile_order.h"

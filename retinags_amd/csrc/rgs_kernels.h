@@ -312,9 +312,12 @@ __host__ __device__ inline int sort_digit_shift(int end_bit, int p, int max_bits
 constexpr int kSortThreads = 1024;
 // Pairs per thread in one tile of the sort: what a pass writes of a tile are runs of one digit value, and the longer they are the
 // fewer cache lines two workgroups (on two XCDs) share; but fewer, larger tiles leave part of the chip idle when the pairs
-// are few.  By the pairs of all jobs of a launch.  Per pass, us, with 4 / 8 / 16: 62.9 M Gaussians' instances 219 / 195 / 198
-// and depths 163 / 137 / 122, the instances of a 5185x3359 frame 482 / 436 / 350 (both passes / 2), of 1600x1036 69 / 64 / 64;
-// a call of 100 000 Gaussians takes 272 us as a whole with 4 and 288 with 16.
+// are few.  By what a launch has room for: the instances of all its jobs, which the host knows, and for the depth sort all their
+// Gaussians, of which the host does not know how many are visible.  Per pass, us, with 4 / 8 / 16:
+//   instances: 62.9 M Gaussians 256 / 196 / 197, 1600x1036 with 5.6 M 78 / 64 / 64, a call of 333 333 Gaussians 22 / 20 / 21;
+//   depths: 62.9 M Gaussians, a third visible 184 / 138 / 121; 27 M, a twentieth visible 40 / 31 / 25 (few of its tiles hold
+//   pairs, but a workgroup without any costs its start); 5.6 M, a third visible 24 / 26 / 24; 333 333, all visible 13 / 18 / 19.
+// A call of 100 000 Gaussians takes 260 / 275 / 287 us as a whole.
 constexpr int kSortItemsFew = 4, kSortItems = 8, kSortItemsMany = 16;
 constexpr size_t kSortSome = (size_t)1 << 20, kSortMany = (size_t)1 << 23;  // pairs from which 8, and 16, are taken
 constexpr int kSortBlock = kSortThreads * kSortItemsFew;  // pairs of the smallest tile
