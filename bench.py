@@ -355,7 +355,9 @@ def measure(args, config, forward_only, asides, cpu, apart_too=False, morton_too
         # ones that were not rendered)
         "preprocess_backward": 285.0 * P_vis + (4.0 + 248.0) * P_tot,
         "composite_forward": (20.0 * K + 20.0) * N,
-        "composite_backward": (40.0 * K + 20.0) * N,
+        # colour and alpha planes of every layer in and their gradients out, the gradient of the image in (the loss looks at
+        # neither depth nor alpha of the composite, so the depths take no part)
+        "composite_backward": (32.0 * K + 12.0) * N,
     }
     alg_flops = {"blend_forward": flops_fwd, "blend_backward": flops_bwd}
     # Where this design's bytes differ from those of the reference's design, both are carried.  The reference's backward
