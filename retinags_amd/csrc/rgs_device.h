@@ -125,6 +125,21 @@ __device__ __forceinline__ float2 alpha_ellipse_half_extent(const float4 conic, 
 	return float2{sqrtf(c * conic.z / det) * 1.0001f + 1e-2f, sqrtf(c * conic.x / det) * 1.0001f + 1e-2f};
 }
 
+// ---- streaming accesses -----------------------------------------------------------------------
+
+// 16 bytes that nothing reads again soon (or wrote a moment ago): the access does not push what other kernels left in the
+// caches out to memory.
+typedef float StreamVec __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ float4 load_streaming(const float4* p)
+{
+	const StreamVec v = __builtin_nontemporal_load(reinterpret_cast<const StreamVec*>(p));
+	return float4{v.x, v.y, v.z, v.w};
+}
+__device__ __forceinline__ void store_streaming(float4* p, const float4 v)
+{
+	__builtin_nontemporal_store(StreamVec{v.x, v.y, v.z, v.w}, reinterpret_cast<StreamVec*>(p));
+}
+
 // ---- wave64 cross-lane primitives (DPP) -----------------------------------------------
 
 template <int Ctrl, int RowMask, int BankMask>

@@ -272,7 +272,9 @@ __global__ __launch_bounds__(256) void ssim_backward_kernel(LossArgs a)
 //   m = b1 m + (1 - b1) g;  v = b2 v + (1 - b2) g g;
 //   p = p - (lr / (1 - b1^t)) * m / (sqrt(v) / sqrt(1 - b2^t) + eps)
 // One launch updates every tensor of a parameter-group list; a workgroup takes kAdamBlock
-// consecutive elements of one tensor.
+// consecutive elements of one tensor.  Bound by memory, 28 bytes per element, none of which another kernel reads soon:
+// streaming accesses leave the caches to the others and run at 5.7 instead of 4.9 TB/s (168 M floats: 965 us with plain accesses,
+// 844 with the loads streaming, 828 with the stores as well; from 3.6 M floats on, the smallest tried, no slower).
 constexpr int kAdamBlock = 4096;
 
 __device__ __forceinline__ void adam_one(float& p, float g, float& m, float& v, const AdamTensor& t, const AdamArgs& a)
@@ -296,17 +298,17 @@ __global__ __launch_bounds__(256) void adam_step_kernel(AdamArgs a)
 		if (i >= t.n)
 			break;
 		if (i + 4 <= t.n && t.by_16_bytes) {
-			float4 p = *reinterpret_cast<float4*>(t.param + i);
-			const float4 g = *reinterpret_cast<const float4*>(t.grad + i);
-			float4 m = *reinterpret_cast<float4*>(t.exp_avg + i);
-			float4 v = *reinterpret_cast<float4*>(t.exp_avg_sq + i);
+			float4 p = load_streaming(reinterpret_cast<const float4*>(t.param + i));
+			const float4 g = load_streaming(reinterpret_cast<const float4*>(t.grad + i));
+			float4 m = load_streaming(reinterpret_cast<const float4*>(t.exp_avg + i));
+			float4 v = load_streaming(reinterpret_cast<const float4*>(t.exp_avg_sq + i));
 			adam_one(p.x, g.x, m.x, v.x, t, a);
 			adam_one(p.y, g.y, m.y, v.y, t, a);
 			adam_one(p.z, g.z, m.z, v.z, t, a);
 			adam_one(p.w, g.w, m.w, v.w, t, a);
-			*reinterpret_cast<float4*>(t.param + i) = p;
-			*reinterpret_cast<float4*>(t.exp_avg + i) = m;
-			*reinterpret_cast<float4*>(t.exp_avg_sq + i) = v;
+			store_streaming(reinterpret_cast<float4*>(t.param + i), p);
+			store_streaming(reinterpret_cast<float4*>(t.exp_avg + i), m);
+			store_streaming(reinterpret_cast<float4*>(t.exp_avg_sq + i), v);
 		} else {
 			for (size_t j = i; j < t.n && j < i + 4; j++) {
 				float p = t.param[j], m = t.exp_avg[j], v = t.exp_avg_sq[j];
