@@ -1549,6 +1549,7 @@ int rgs_activate_forward(int n, int rest, const float* features_dc, const float*
 	a.features_dc = features_dc; a.features_rest = features_rest; a.scaling = scaling; a.rotation = rotation;
 	a.opacity = opacity;
 	a.shs = shs; a.scales = scales; a.rotations = rotations; a.opacities = opacities;
+	a.features_by_16_bytes = aligned16(features_dc) && aligned16(features_rest);
 	rgs::launch_activate_forward(a, s);
 	RGS_STAGE("activate_forward");
 	return 0;
@@ -1579,6 +1580,7 @@ int rgs_activate_backward(int n, int rest, const float* rotation, const float* s
 	a.g_shs = g_shs; a.g_scales = g_scales; a.g_rotations = g_rotations; a.g_opacities = g_opacities;
 	a.d_features_dc = d_features_dc; a.d_features_rest = d_features_rest; a.d_scaling = d_scaling;
 	a.d_rotation = d_rotation; a.d_opacity = d_opacity;
+	a.features_by_16_bytes = aligned16(d_features_dc) && aligned16(d_features_rest);
 	rgs::launch_activate_backward(a, s);
 	RGS_STAGE("activate_backward");
 	return 0;

@@ -221,6 +221,7 @@ struct ActivateArgs {
 	float* scales;
 	float* rotations;
 	float* opacities;
+	bool features_by_16_bytes;   // both feature tensors start at a multiple of 16 bytes (the others have to)
 };
 struct ActivateBackwardArgs {
 	int n, rest;
@@ -236,6 +237,7 @@ struct ActivateBackwardArgs {
 	float* d_scaling;
 	float* d_rotation;
 	float* d_opacity;
+	bool features_by_16_bytes;   // as above, for their gradients
 };
 constexpr int kMaxAdamTensors = 16;
 struct AdamTensor {

@@ -321,48 +321,193 @@ __global__ __launch_bounds__(256) void adam_step_kernel(AdamArgs a)
 	}
 }
 
-// Both activation kernels are flat passes over four arrays; a workgroup works on one of them
-// (its part is the same for all its threads), 1024 sixteen-byte units per workgroup, so every
-// store is a full 16 bytes to consecutive addresses.  The SH rows are the one place where that
-// takes care: a row of the joined tensor is 3 floats of one source followed by 3 * rest of the
-// other, so the 16-byte units of the output (or of its gradient) straddle the two sources and
-// are put together from 4-byte accesses on the source side.
+// Both activation kernels are flat passes over four arrays; a workgroup works on one of them (its part is the same for all
+// its threads) and reads and writes 16 bytes per lane.  The SH rows are the one place where that takes care: a row of the joined
+// tensor is 3 floats of one source followed by 3 * rest of the other.  A workgroup takes kActRows whole rows, whose floats are
+// consecutive in all three tensors, and joins (or splits) them in LDS, where the shift by a row's 3 floats is 4-byte accesses.
+// Bound by memory, 4 bytes read and 4 written per float.  With 4-byte accesses on the side of the two tensors, the form that is
+// left for more coefficients than kActMaxRest and for arrays that do not start at a multiple of 16 bytes, 2.8 M Gaussians of 16
+// coefficients took 268 us forward and 348 backward; now 220 and 240.
 constexpr int kActUnits = 1024;   // 16-byte units per workgroup: 4 per thread
+constexpr int kActRows = 128;     // SH rows per workgroup: six workgroups' rows fit a CU's LDS
+constexpr int kActMaxRest = 15;
+static_assert(kActRows % 4 == 0, "a workgroup's rows begin at a multiple of 16 bytes in each of the tensors");
 
 struct ActParts {
 	uint32_t sh_blocks, rot_blocks, scale_blocks, opacity_blocks;
+	uint32_t rest_reciprocal;  // 0: the SH rows go by 4-byte accesses, kActUnits per workgroup; otherwise kActRows rows per workgroup
 };
 
-__host__ __device__ inline ActParts act_parts(int n, int rest)
+// f / (3 rest) is (f * reciprocal) >> 20 for every float f of a workgroup's rows: the excess of the reciprocal over 2^20 / d,
+// less than 1, adds f / 2^20 < 1 / d to the quotient.
+static_assert((size_t)kActRows * 3 * kActMaxRest * 3 * kActMaxRest < (1u << 20), "exact division");
+
+inline ActParts act_parts(int n, int rest, bool sh_by_16_bytes)
 {
 	const size_t sh_floats = 3 * (size_t)(1 + rest);
-	auto blocks = [](size_t units) { return (uint32_t)((units + kActUnits - 1) / kActUnits); };
+	auto blocks = [](size_t units, size_t per_block) { return (uint32_t)((units + per_block - 1) / per_block); };
 	ActParts p;
-	p.sh_blocks = blocks(((size_t)n * sh_floats + 3) / 4);
-	p.rot_blocks = blocks((size_t)n);
-	p.scale_blocks = blocks(((size_t)n * 3 + 3) / 4);
-	p.opacity_blocks = blocks(((size_t)n + 3) / 4);
+	const bool by_rows = sh_by_16_bytes && rest >= 1 && rest <= kActMaxRest;
+	p.rest_reciprocal = by_rows ? ((1u << 20) + 3 * (uint32_t)rest - 1) / (3 * (uint32_t)rest) : 0u;
+	p.sh_blocks = by_rows ? blocks((size_t)n, kActRows) : blocks(((size_t)n * sh_floats + 3) / 4, kActUnits);
+	p.rot_blocks = blocks((size_t)n, kActUnits);
+	p.scale_blocks = blocks(((size_t)n * 3 + 3) / 4, kActUnits);
+	p.opacity_blocks = blocks(((size_t)n + 3) / 4, kActUnits);
 	return p;
 }
 
-// floats [4u, 4u+4) of a flat array of `total` floats, element by element where the array ends
-template <typename F>
-__device__ __forceinline__ void flat_unit(size_t u, size_t total, const float* __restrict__ in, float* __restrict__ out, F f)
+// Unit u (floats [4u, 4u+4)) of `total` floats that start at a multiple of 16 bytes.
+__device__ __forceinline__ float4 read_unit(const float* __restrict__ in, uint32_t u, uint32_t total)
+{
+	if (4 * u + 4 <= total)
+		return load_streaming(reinterpret_cast<const float4*>(in) + u);
+	float4 v = {0.f, 0.f, 0.f, 0.f};
+	if (4 * u < total)
+		v.x = in[4 * u];
+	if (4 * u + 1 < total)
+		v.y = in[4 * u + 1];
+	if (4 * u + 2 < total)
+		v.z = in[4 * u + 2];
+	return v;
+}
+__device__ __forceinline__ void write_unit(float* __restrict__ out, uint32_t u, uint32_t total, const float4 v)
 {
 	if (4 * u + 4 <= total) {
-		const float4 v = reinterpret_cast<const float4*>(in)[u];
-		reinterpret_cast<float4*>(out)[u] = float4{f(v.x, 4 * u), f(v.y, 4 * u + 1), f(v.z, 4 * u + 2), f(v.w, 4 * u + 3)};
-	} else {
-		for (size_t k = 4 * u; k < total; k++)
-			out[k] = f(in[k], k);
+		store_streaming(reinterpret_cast<float4*>(out) + u, v);
+		return;
+	}
+	if (4 * u < total)
+		out[4 * u] = v.x;
+	if (4 * u + 1 < total)
+		out[4 * u + 1] = v.y;
+	if (4 * u + 2 < total)
+		out[4 * u + 2] = v.z;
+}
+
+// Where float f of a workgroup's dc or rest floats (floats_per_row of a row) lies among its joined rows.
+struct JoinedPlace {
+	uint32_t at, left;  // left: floats of the row from this one on
+};
+__device__ __forceinline__ JoinedPlace joined_place(uint32_t f, uint32_t floats_per_row, uint32_t reciprocal, uint32_t sh_floats, uint32_t shift)
+{
+	const uint32_t row = (f * reciprocal) >> 20, col = f - row * floats_per_row;
+	return JoinedPlace{row * sh_floats + shift + col, floats_per_row - col};
+}
+
+constexpr uint32_t kThirds = ((1u << 20) + 2) / 3;  // the reciprocal of a row of dc
+
+constexpr int kActRestTurns = (kActRows * 3 * kActMaxRest / 4 + 255) / 256, kActRowTurns = (kActRows * 3 * (1 + kActMaxRest) / 4 + 255) / 256;
+
+// Rows [first, first + rows) of dc and rest joined into shs.
+__device__ __forceinline__ void join_rows(const ActivateArgs& a, uint32_t reciprocal, size_t first, uint32_t rows, float* joined)
+{
+	const uint32_t tid = threadIdx.x, rest_floats = 3u * (uint32_t)a.rest, sh_floats = rest_floats + 3u;
+	const uint32_t rest_total = rows * rest_floats, dc_total = 3u * rows, total = rows * sh_floats;
+	const float* rest = a.features_rest + first * rest_floats;
+	float4 v[kActRestTurns], d = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+	for (int t = 0; t < kActRestTurns; t++)
+		if (4 * (256 * t + tid) < rest_total)
+			v[t] = read_unit(rest, 256 * t + tid, rest_total);
+	if (4 * tid < dc_total)
+		d = read_unit(a.features_dc + first * 3, tid, dc_total);
+	auto place = [&](uint32_t f, uint32_t end, uint32_t floats_per_row, uint32_t recip, uint32_t shift, const float4 q) {
+		const JoinedPlace p = joined_place(f, floats_per_row, recip, sh_floats, shift);
+		const uint32_t gap = sh_floats - floats_per_row;  // between a row's last float and the next row's first
+		const float x[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+		for (uint32_t k = 0; k < 4; k++)
+			if (f + k < end)
+				joined[p.at + k + (k >= p.left ? gap : 0u) + (k >= p.left + floats_per_row ? gap : 0u)] = x[k];
+	};
+#pragma unroll
+	for (int t = 0; t < kActRestTurns; t++)
+		place(4 * (256 * t + tid), rest_total, rest_floats, reciprocal, 3u, v[t]);
+	place(4 * tid, dc_total, 3u, kThirds, 0u, d);
+	__syncthreads();
+	float* out = a.shs + first * sh_floats;
+#pragma unroll
+	for (int t = 0; t < kActRowTurns; t++) {
+		const uint32_t u = 256 * t + tid;
+		if (4 * u < total)
+			write_unit(out, u, total, reinterpret_cast<const float4*>(joined)[u]);
+	}
+}
+
+// ... and the gradient of those rows split.
+__device__ __forceinline__ void split_rows(const ActivateBackwardArgs& a, uint32_t reciprocal, size_t first, uint32_t rows, float* joined)
+{
+	const uint32_t tid = threadIdx.x, rest_floats = 3u * (uint32_t)a.rest, sh_floats = rest_floats + 3u;
+	const uint32_t rest_total = rows * rest_floats, dc_total = 3u * rows, total = rows * sh_floats;
+	const float* in = a.g_shs + first * sh_floats;
+	float4 v[kActRowTurns];
+#pragma unroll
+	for (int t = 0; t < kActRowTurns; t++)
+		if (4 * (256 * t + tid) < total)
+			v[t] = read_unit(in, 256 * t + tid, total);
+#pragma unroll
+	for (int t = 0; t < kActRowTurns; t++)
+		if (4 * (256 * t + tid) < total)
+			reinterpret_cast<float4*>(joined)[256 * t + tid] = v[t];
+	__syncthreads();
+	auto pick = [&](uint32_t f, uint32_t end, uint32_t floats_per_row, uint32_t recip, uint32_t shift) {
+		const JoinedPlace p = joined_place(f, floats_per_row, recip, sh_floats, shift);
+		const uint32_t gap = sh_floats - floats_per_row;
+		float x[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+		for (uint32_t k = 0; k < 4; k++)
+			if (f + k < end)
+				x[k] = joined[p.at + k + (k >= p.left ? gap : 0u) + (k >= p.left + floats_per_row ? gap : 0u)];
+		return float4{x[0], x[1], x[2], x[3]};
+	};
+#pragma unroll
+	for (int t = 0; t < kActRestTurns; t++) {
+		const uint32_t u = 256 * t + tid;
+		if (4 * u < rest_total)
+			write_unit(a.d_features_rest + first * rest_floats, u, rest_total, pick(4 * u, rest_total, rest_floats, reciprocal, 3u));
+	}
+	if (4 * tid < dc_total)
+		write_unit(a.d_features_dc + first * 3, tid, dc_total, pick(4 * tid, dc_total, 3u, kThirds, 0u));
+}
+
+// Four 16-byte units of a flat array of `total` floats per thread, element by element where the array ends; f(value, other): `other`
+// is the element of a second array (null: 0).
+template <typename F>
+__device__ __forceinline__ void flat_units(uint32_t block, size_t total, const float* __restrict__ in, const float* __restrict__ other,
+                                           float* __restrict__ out, F f)
+{
+	constexpr int kTurns = kActUnits / 256;
+	float4 v[kTurns], o[kTurns];
+	const size_t u0 = (size_t)block * kActUnits + threadIdx.x;
+#pragma unroll
+	for (int t = 0; t < kTurns; t++)
+		if (4 * (u0 + 256 * t) + 4 <= total) {
+			v[t] = load_streaming(reinterpret_cast<const float4*>(in) + u0 + 256 * t);
+			o[t] = other ? load_streaming(reinterpret_cast<const float4*>(other) + u0 + 256 * t) : float4{0.f, 0.f, 0.f, 0.f};
+		}
+#pragma unroll
+	for (int t = 0; t < kTurns; t++) {
+		const size_t u = u0 + 256 * t;
+		if (4 * u + 4 <= total)
+			store_streaming(reinterpret_cast<float4*>(out) + u,
+			                float4{f(v[t].x, o[t].x), f(v[t].y, o[t].y), f(v[t].z, o[t].z), f(v[t].w, o[t].w)});
+		else
+			for (size_t k = 4 * u; k < total; k++)
+				out[k] = f(in[k], other ? other[k] : 0.f);
 	}
 }
 
 __global__ __launch_bounds__(256) void activate_forward_kernel(ActivateArgs a, ActParts parts)
 {
+	__shared__ __attribute__((aligned(16))) float joined[kActRows * 3 * (1 + kActMaxRest)];
 	uint32_t block = blockIdx.x;
 	const size_t n = (size_t)a.n;
 	if (block < parts.sh_blocks) {
+		if (parts.rest_reciprocal != 0u) {
+			const size_t first = (size_t)block * kActRows;
+			join_rows(a, parts.rest_reciprocal, first, (uint32_t)min((size_t)kActRows, n - first), joined);
+			return;
+		}
 		const size_t sh_floats = 3 * (size_t)(1 + a.rest), rest_floats = 3 * (size_t)a.rest, total = n * sh_floats;
 		for (int it = 0; it < kActUnits / 256; it++) {
 			const size_t u = (size_t)block * kActUnits + it * 256 + threadIdx.x;
@@ -389,36 +534,44 @@ __global__ __launch_bounds__(256) void activate_forward_kernel(ActivateArgs a, A
 	}
 	block -= parts.sh_blocks;
 	if (block < parts.rot_blocks) {
-		for (int it = 0; it < kActUnits / 256; it++) {
-			const size_t i = (size_t)block * kActUnits + it * 256 + threadIdx.x;
-			if (i >= n)
-				break;
-			const float4 q = reinterpret_cast<const float4*>(a.rotation)[i];
-			const float len = fmaxf(sqrtf(q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w), 1e-12f);  // torch.nn.functional.normalize
-			reinterpret_cast<float4*>(a.rotations)[i] = float4{q.x / len, q.y / len, q.z / len, q.w / len};
-		}
+		constexpr int kTurns = kActUnits / 256;
+		const size_t i0 = (size_t)block * kActUnits + threadIdx.x;
+		float4 v[kTurns];
+#pragma unroll
+		for (int t = 0; t < kTurns; t++)
+			if (i0 + 256 * t < n)
+				v[t] = load_streaming(reinterpret_cast<const float4*>(a.rotation) + i0 + 256 * t);
+#pragma unroll
+		for (int t = 0; t < kTurns; t++)
+			if (i0 + 256 * t < n) {
+				const float4 q = v[t];
+				const float len = fmaxf(sqrtf(q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w), 1e-12f);  // torch.nn.functional.normalize
+				store_streaming(reinterpret_cast<float4*>(a.rotations) + i0 + 256 * t, float4{q.x / len, q.y / len, q.z / len, q.w / len});
+			}
 		return;
 	}
 	block -= parts.rot_blocks;
 	if (block < parts.scale_blocks) {
-		for (int it = 0; it < kActUnits / 256; it++)
-			flat_unit((size_t)block * kActUnits + it * 256 + threadIdx.x, 3 * n, a.scaling, a.scales,
-			          [](float v, size_t) { return expf(v); });
+		flat_units(block, 3 * n, a.scaling, nullptr, a.scales, [](float v, float) { return expf(v); });
 		return;
 	}
 	block -= parts.scale_blocks;
-	for (int it = 0; it < kActUnits / 256; it++)
-		flat_unit((size_t)block * kActUnits + it * 256 + threadIdx.x, n, a.opacity, a.opacities,
-		          [](float v, size_t) { return 1.0f / (1.0f + expf(-v)); });
+	flat_units(block, n, a.opacity, nullptr, a.opacities, [](float v, float) { return 1.0f / (1.0f + expf(-v)); });
 }
 
 __global__ __launch_bounds__(256) void activate_backward_kernel(ActivateBackwardArgs a, ActParts parts)
 {
+	__shared__ __attribute__((aligned(16))) float joined[kActRows * 3 * (1 + kActMaxRest)];
 	uint32_t block = blockIdx.x;
 	const size_t n = (size_t)a.n;
 	if (block < parts.sh_blocks) {
 		if (!a.g_shs)
 			return;
+		if (parts.rest_reciprocal != 0u) {
+			const size_t first = (size_t)block * kActRows;
+			split_rows(a, parts.rest_reciprocal, first, (uint32_t)min((size_t)kActRows, n - first), joined);
+			return;
+		}
 		const size_t sh_floats = 3 * (size_t)(1 + a.rest), rest_floats = 3 * (size_t)a.rest, total = n * sh_floats;
 		for (int it = 0; it < kActUnits / 256; it++) {
 			const size_t u = (size_t)block * kActUnits + it * 256 + threadIdx.x;
@@ -450,40 +603,38 @@ __global__ __launch_bounds__(256) void activate_backward_kernel(ActivateBackward
 	if (block < parts.rot_blocks) {
 		if (!a.g_rotations)
 			return;
-		for (int it = 0; it < kActUnits / 256; it++) {
-			const size_t i = (size_t)block * kActUnits + it * 256 + threadIdx.x;
-			if (i >= n)
-				break;
-			// d/dq of q / |q|: (g - u (u . g)) / |q| with u = q / |q|
-			const float4 q = reinterpret_cast<const float4*>(a.rotation)[i];
-			const float4 g = reinterpret_cast<const float4*>(a.g_rotations)[i];
-			const float len = fmaxf(sqrtf(q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w), 1e-12f);
-			const float u0 = q.x / len, u1 = q.y / len, u2 = q.z / len, u3 = q.w / len;
-			const float along = u0 * g.x + u1 * g.y + u2 * g.z + u3 * g.w;
-			reinterpret_cast<float4*>(a.d_rotation)[i] =
-			    float4{(g.x - u0 * along) / len, (g.y - u1 * along) / len, (g.z - u2 * along) / len, (g.w - u3 * along) / len};
-		}
+		constexpr int kTurns = kActUnits / 256;
+		const size_t i0 = (size_t)block * kActUnits + threadIdx.x;
+		float4 v[kTurns], w[kTurns];
+#pragma unroll
+		for (int t = 0; t < kTurns; t++)
+			if (i0 + 256 * t < n) {
+				v[t] = load_streaming(reinterpret_cast<const float4*>(a.rotation) + i0 + 256 * t);
+				w[t] = load_streaming(reinterpret_cast<const float4*>(a.g_rotations) + i0 + 256 * t);
+			}
+#pragma unroll
+		for (int t = 0; t < kTurns; t++)
+			if (i0 + 256 * t < n) {
+				// d/dq of q / |q|: (g - u (u . g)) / |q| with u = q / |q|
+				const float4 q = v[t], g = w[t];
+				const float len = fmaxf(sqrtf(q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w), 1e-12f);
+				const float u0 = q.x / len, u1 = q.y / len, u2 = q.z / len, u3 = q.w / len;
+				const float along = u0 * g.x + u1 * g.y + u2 * g.z + u3 * g.w;
+				store_streaming(reinterpret_cast<float4*>(a.d_rotation) + i0 + 256 * t,
+				                float4{(g.x - u0 * along) / len, (g.y - u1 * along) / len, (g.z - u2 * along) / len,
+				                       (g.w - u3 * along) / len});
+			}
 		return;
 	}
 	block -= parts.rot_blocks;
 	if (block < parts.scale_blocks) {
-		if (!a.g_scales)
-			return;
-		const float* scales = a.scales;
-		for (int it = 0; it < kActUnits / 256; it++)
-			flat_unit((size_t)block * kActUnits + it * 256 + threadIdx.x, 3 * n, a.g_scales, a.d_scaling,
-			          [scales](float g, size_t k) { return g * scales[k]; });
+		if (a.g_scales)
+			flat_units(block, 3 * n, a.g_scales, a.scales, a.d_scaling, [](float g, float s) { return g * s; });
 		return;
 	}
 	block -= parts.scale_blocks;
-	if (!a.g_opacities)
-		return;
-	const float* opacities = a.opacities;
-	for (int it = 0; it < kActUnits / 256; it++)
-		flat_unit((size_t)block * kActUnits + it * 256 + threadIdx.x, n, a.g_opacities, a.d_opacity, [opacities](float g, size_t k) {
-			const float o = opacities[k];
-			return g * (o * (1.0f - o));
-		});
+	if (a.g_opacities)
+		flat_units(block, n, a.g_opacities, a.opacities, a.d_opacity, [](float g, float o) { return g * (o * (1.0f - o)); });
 }
 
 }  // namespace
@@ -493,7 +644,7 @@ void launch_activate_forward(const ActivateArgs& a, hipStream_t s)
 	stage_mark("activate_forward", s);
 	if (a.n <= 0)
 		return;
-	const ActParts p = act_parts(a.n, a.rest);
+	const ActParts p = act_parts(a.n, a.rest, a.features_by_16_bytes);
 	hipLaunchKernelGGL(activate_forward_kernel, dim3(p.sh_blocks + p.rot_blocks + p.scale_blocks + p.opacity_blocks), dim3(256),
 	                   0, s, a, p);
 }
@@ -503,7 +654,7 @@ void launch_activate_backward(const ActivateBackwardArgs& a, hipStream_t s)
 	stage_mark("activate_backward", s);
 	if (a.n <= 0)
 		return;
-	const ActParts p = act_parts(a.n, a.rest);
+	const ActParts p = act_parts(a.n, a.rest, a.features_by_16_bytes);
 	hipLaunchKernelGGL(activate_backward_kernel, dim3(p.sh_blocks + p.rot_blocks + p.scale_blocks + p.opacity_blocks), dim3(256),
 	                   0, s, a, p);
 }
