@@ -856,6 +856,9 @@ void fill_backward_geometry(rgs::PreprocessBackwardArgs& p, int P, int D, int M,
 	p.dL_dmean2D = dL_dmean2D; p.dL_dopacity = dL_dopacity; p.dL_dcolor = dL_dcolor;
 	p.dL_dmeans = dL_dmean3D; p.dL_dcov3D = dL_dcov3D; p.dL_dsh = dL_dsh; p.dL_dscale = dL_dscale; p.dL_drot = dL_drot;
 	p.sh_rows_by_16_bytes = sh_rows_by_16_bytes(shs, M, D) && (reinterpret_cast<uintptr_t>(dL_dsh) & 15) == 0;
+	p.rows_by_16_bytes = true;
+	for (const float* out : {dL_dmean2D, dL_dcolor, dL_dmean3D, dL_dcov3D, dL_dscale})
+		p.rows_by_16_bytes = p.rows_by_16_bytes && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
 }
 
 // Events for ordering a frame's stream against its layers' own streams: a few per host thread and device, reused.

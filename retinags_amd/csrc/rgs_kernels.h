@@ -61,6 +61,7 @@ struct PreprocessBackwardArgs {
 	float focal_x, focal_y, tanfovx, tanfovy;
 	const float* sums;  // (P, kSumCols): what the backward blend accumulated, see SumCol
 	bool sh_rows_by_16_bytes;       // SH rows are 16-byte aligned, a multiple of 16 bytes long and at most 48 floats
+	bool rows_by_16_bytes;          // every output that is made starts at a multiple of 16 bytes
 	// outputs: every row is written, zeros where radii[i] <= 0
 	float* dL_dmean2D;  // (P,3), third column 0
 	float* dL_dopacity; // (P)

@@ -51,3 +51,50 @@ def test_activated_values_at_the_edges_of_a_workgroup(n):
     for got, ref in zip(grads, want_grads):
         # (the quaternion's gradient is a difference of terms as large as the upstream gradient)
         assert float((got.double() - ref).norm() / ref.norm()) < 2e-6
+
+
+@pytest.mark.parametrize("n", (1, 63, 64, 65, 127, 128, 129, 777))
+def test_gradient_rows_leave_alike_on_and_off_a_16_byte_boundary(n, monkeypatch):
+    """Rows of whole wavefronts go out 16 bytes per lane, those of the last and of arrays off a 16-byte boundary one float at a
+    time; every row is written either way.  Two runs differ by the order of the atomic additions alone (1e-4, as between
+    repeats)."""
+    from helpers import rel_l2
+    from retinags_amd import GaussianRasterizationSettings, GaussianRasterizer, rasterizer
+    from retinags_amd.harness import scenes
+    gen = torch.Generator().manual_seed(n)
+    cam = scenes.look_at_camera((0, 0, 0), (0, 0, 1), (0, -1, 0), 96, 64, 60.0).to(DEV)
+    given = dict(means3D=torch.cat((torch.rand(n, 2, generator=gen) * 4 - 2, torch.rand(n, 1, generator=gen) * 6 - 1), 1),
+                 opacities=torch.rand(n, 1, generator=gen), shs=torch.randn(n, 16, 3, generator=gen) * 0.2,
+                 scales=torch.rand(n, 3, generator=gen) * 0.2, rotations=torch.nn.functional.normalize(torch.randn(n, 4, generator=gen)))
+    given = {k: v.to(DEV).requires_grad_(True) for k, v in given.items()}
+    given["means2D"] = torch.zeros(n, 3, device=DEV, requires_grad=True)
+    settings = GaussianRasterizationSettings(
+        image_height=64, image_width=96, tanfovx=cam.tanfovx, tanfovy=cam.tanfovy, bg=torch.zeros(3, device=DEV), scale_modifier=1.0,
+        viewmatrix=cam.world_view_transform, projmatrix=cam.full_proj_transform, projmatrix_inv=cam.projection_matrix_inv,
+        range_low=torch.full((3,), -99.0, device=DEV), range_up=torch.full((3,), 99.0, device=DEV), sh_degree=3,
+        campos=cam.camera_center, prefiltered=False, debug=False)
+    upstream = torch.randn(3, 64, 96, generator=gen).to(DEV)
+    make, made = rasterizer._gradient_outputs, []
+
+    def run(offset):
+        def arrays(*args, **kwargs):
+            out = make(*args, **kwargs)
+            for name, t in out.items():
+                if t is not None and name != "sums":
+                    if offset and t.dim() == 2 and t.shape[1] in (3, 6):
+                        out[name] = torch.empty(t.numel() + offset, device=DEV)[offset:].view(t.shape)
+                    out[name].fill_(float("nan"))
+            made.append(out)
+            return out
+        monkeypatch.setattr(rasterizer, "_gradient_outputs", arrays)
+        color, radii = GaussianRasterizer(settings)(**given)[:2]
+        torch.autograd.grad([color], list(given.values()), [upstream])
+        return radii, {k: v for k, v in made[-1].items() if v is not None and k != "sums"}
+
+    radii, even = run(0)
+    for offset in (1, 2):
+        odd = run(offset)[1]
+        for name, t in even.items():
+            assert not torch.isnan(t).any() and not torch.isnan(odd[name]).any(), name
+            assert rel_l2(odd[name].cpu().numpy(), t.cpu().numpy()) <= 1e-4, name
+            assert (t[radii <= 0] == 0).all() and (odd[name][radii <= 0] == 0).all(), name
