@@ -115,6 +115,13 @@ __device__ __forceinline__ uint64_t lanes_inside_box(uint64_t lanes, float w, co
 		lanes &= ~lanes_where(clipped_by_box(ray_of(rays), w, load_box_frame(a)));
 	return lanes;
 }
+// The same by the exact test alone, where some entry of the chunk lies at a clip w that is not positive.
+__device__ __forceinline__ uint64_t lanes_inside_box(uint64_t lanes, float w, const StripRays& rays, const BlendArgs& a)
+{
+	return lanes & ~lanes_where(clipped_by_box(ray_of(rays), w, load_box_frame(a)));
+}
+// How a chunk's samples are tested against the box: not at all (it has the strip inside for every entry), by spans, exactly.
+enum BoxTest { kBoxNone, kBoxSpans, kBoxExact };
 
 // exp(x) for the exponents of the blend (-6 < x <= 0 where the result is used): 2^(x log2 e) on the hardware exp2 unit.
 // The product's rounding (half a unit in the last place of a number below 8) and the unit's own leave the result within
@@ -411,8 +418,7 @@ __device__ __forceinline__ void forward_candidate(FourEntries& e, int i, const f
 }
 
 // Alphas, zero where the pixel does not take the entry, and the masks of those that do (as far as alpha and box decide).
-// boxed: some entries of the chunk straddle a face of the box in the strip.
-__device__ __forceinline__ void forward_alphas(FourEntries& e, uint64_t live, bool boxed, const StripRays& rays, const BoxSpan& span,
+__device__ __forceinline__ void forward_alphas(FourEntries& e, uint64_t live, BoxTest box, const StripRays& rays, const BoxSpan& span,
                                                const BlendArgs& a)
 {
 #pragma unroll
@@ -420,10 +426,14 @@ __device__ __forceinline__ void forward_alphas(FourEntries& e, uint64_t live, bo
 		e.alpha[i] = fminf(0.99f, e.opacity[i] * exp_of_exponent(e.power[i]));
 		e.mask[i] &= lanes_where(!(e.alpha[i] < 1.0f / 255.0f));
 	}
-	if (boxed)
+	if (box == kBoxSpans)
 #pragma unroll
 		for (int i = 0; i < 4; i++)
 			e.mask[i] = lanes_inside_box(e.mask[i] & live, e.clip_w[i], span, rays, a);
+	else if (box == kBoxExact)
+#pragma unroll
+		for (int i = 0; i < 4; i++)
+			e.mask[i] = lanes_inside_box(e.mask[i] & live, e.clip_w[i], rays, a);
 #pragma unroll
 	for (int i = 0; i < 4; i++)
 		e.alpha[i] = __builtin_amdgcn_inverse_ballot_w64(e.mask[i]) ? e.alpha[i] : 0.f;
@@ -446,7 +456,7 @@ __device__ __forceinline__ void forward_blend(ForwardPixel& p, const float* alph
 }
 
 __device__ __forceinline__ void forward_group(ForwardPixel& p, uint64_t& live, const ForwardStage& st, int half, int k,
-                                              const float2 pixf, bool boxed, const BoxSpan& span, const BlendArgs& a)
+                                              const float2 pixf, BoxTest box, const BoxSpan& span, const BlendArgs& a)
 {
 	const ForwardSlot* slot = st.slot(half) + k;
 	FourEntries e;
@@ -461,7 +471,7 @@ __device__ __forceinline__ void forward_group(ForwardPixel& p, uint64_t& live, c
 	for (int i = 0; i < 4; i++)
 		cd[i] = slot[i].cd;
 	__builtin_amdgcn_sched_barrier(0);
-	forward_alphas(e, live, boxed, st.rays, span, a);
+	forward_alphas(e, live, box, st.rays, span, a);
 	forward_blend(p, e.alpha, e.mask, cd, k);
 	live = lanes_where(p.T > 0.f);
 }
@@ -516,24 +526,14 @@ __device__ __forceinline__ HalfSpan live_w_span(bool takes, const BoxSpan& span)
 }
 
 // Takes the entries that no live pixel can have inside the box out of a chunk whose entries straddle one of its faces in
-// the strip.  False, with nothing done, if one of them lies at a clip w that is not positive: spans do not apply then.
-__device__ __forceinline__ bool prune_by_box(bool straddles, bool takes, float w, const StripRays& rays, const BlendArgs& a,
-                                                bool& left, bool& right)
+// the strip, all of them at a positive clip w.
+__device__ __forceinline__ void prune_by_box(bool straddles, bool takes, float w, const BoxSpan& span, bool& left, bool& right)
 {
-	if (lanes_where(straddles && !(w > 0.f)) != 0ull)
-		return false;
-	const HalfSpan h = live_w_span(takes, w_inside_box(ray_of(rays), load_box_frame(a)));
+	const HalfSpan h = live_w_span(takes, span);
 	if (straddles) {
 		left = left && !(w > h.to[0]) && !(w < h.from[0]);
 		right = right && !(w > h.to[1]) && !(w < h.from[1]);
 	}
-	return true;
-}
-
-// The pixel's span for the visits; one that decides nothing where spans do not apply.
-__device__ __forceinline__ BoxSpan span_for_visits(bool applies, const StripRays& rays, const BlendArgs& a)
-{
-	return applies ? w_inside_box(ray_of(rays), load_box_frame(a)) : BoxSpan{-INFINITY, INFINITY, INFINITY, -INFINITY};
 }
 
 // In which 8-pixel-wide halves of the strip (first pixel x0, ya) an entry's ellipse power >= floor can reach a pixel that
@@ -647,6 +647,11 @@ __device__ __forceinline__ void forward_strip(const BlendArgs& a, uint32_t strip
 		uint32_t id_next = pos_next != kNone ? list[pos_next & kPosition] : 0u;
 
 		const float x0 = wave_uniform((float)(tx * kTile)), ya = wave_uniform((float)(ty * kTile + wave * 4));
+		// Where an entry straddles a face of the box, the pixel's span is worked out once, at the first such chunk: a strip
+		// with a pixel that stays unfinished walks hundreds of chunks that hold nothing for it, and with the span (150 instructions
+		// and the box from memory) formed twice in each, as once, such a walk took 3.9 us a chunk (62.9 M Gaussians: 232 chunks).
+		BoxSpan span = {0.f, 0.f, 0.f, 0.f};
+		bool have_span = false;
 		for (uint32_t first = 0; first < filed && live != 0ull; first += 64) {
 			const int count = (int)min(filed - first, 64u);
 			// what follows from the lane's number is worked out per chunk: held through the walk it costs half a dozen registers
@@ -662,8 +667,14 @@ __device__ __forceinline__ void forward_strip(const BlendArgs& a, uint32_t strip
 			// one such pixel walked its list to the end (at 1600x1036 and 5.6 M Gaussians, a camera that looks along a
 			// plane between submodels: one that blends none of its last 2 800 entries walked 3 387; 0.54 ms of launch).
 			const bool straddles = l < count && (pos_cur & 0x80000000u) == 0u;
-			const bool boxed = lanes_where(straddles) != 0ull;
-			const bool span_applies = boxed && prune_by_box(straddles, p.T > 0.f, cur.geom.w, st.rays, a, left, right);
+			const BoxTest box = lanes_where(straddles) == 0ull ? kBoxNone : lanes_where(straddles && !(cur.geom.w > 0.f)) == 0ull ? kBoxSpans : kBoxExact;
+			if (box == kBoxSpans) {
+				if (!have_span) {
+					span = w_inside_box(ray_of(st.rays), load_box_frame(a));
+					have_span = true;
+				}
+				prune_by_box(straddles, p.T > 0.f, cur.geom.w, span, left, right);
+			}
 			const uint64_t in_left = lanes_where(left), in_right = lanes_where(right);
 			const int n_left = __popcll(in_left), n_right = __popcll(in_right);
 			const int steps = max(n_left, n_right), padded = (steps + 3) & ~3;
@@ -685,11 +696,8 @@ __device__ __forceinline__ void forward_strip(const BlendArgs& a, uint32_t strip
 			const uint32_t e3 = first + 192 + (uint32_t)l;
 			pos_after = e3 < filed ? filed_list[e3] : kNone;
 
-			BoxSpan span = {0.f, 0.f, 0.f, 0.f};
-			if (boxed)
-				span = span_for_visits(span_applies, st.rays, a);
 			for (int k = 0; k < steps && live != 0ull; k += 4)
-				forward_group(p, live, st, half, k, pixf, boxed, span, a);
+				forward_group(p, live, st, half, k, pixf, box, span, a);
 			if (p.last_slot >= 0)
 				p.last_filed = first + st.entry[half][p.last_slot] + 1u;
 			p.last_slot = -1;
@@ -972,7 +980,7 @@ __device__ __forceinline__ void sum_rows(const BackwardStage& st, int slot0, con
 
 // Pixel-parallel part for the four entries staged from slot k on; `rows`: the pixel's place in the first of their rows.
 // Returns, as sum_rows asks for it (16 lanes per entry), which of them any pixel blended.
-template <bool kDepth, bool kBoxed>
+template <bool kDepth, BoxTest kBox>
 __device__ __forceinline__ uint64_t backward_rows(BackwardPixel& p, uint32_t last_contributor, const BackwardStage& st, int k,
                                               LdsPair* rows, const float2 pixf, const BoxSpan& span, const BlendArgs& a)
 {
@@ -1001,8 +1009,10 @@ __device__ __forceinline__ uint64_t backward_rows(BackwardPixel& p, uint32_t las
 		G[i] = exp_of_exponent(power[i]);
 		alpha[i] = fminf(0.99f, opacity[i] * G[i]);
 		mask[i] &= lanes_where(!(alpha[i] < 1.0f / 255.0f));
-		if (kBoxed)
+		if (kBox == kBoxSpans)
 			mask[i] = lanes_inside_box(mask[i], clip_w[i], span, st.rays, a);
+		if (kBox == kBoxExact)
+			mask[i] = lanes_inside_box(mask[i], clip_w[i], st.rays, a);
 		// From here on nothing feeds a decision: gradients are compared by tolerance, so the divisions use the hardware
 		// reciprocal.
 		inv[i] = __builtin_amdgcn_rcpf(1.f - alpha[i]);
@@ -1044,6 +1054,20 @@ __device__ __forceinline__ uint64_t backward_rows(BackwardPixel& p, uint32_t las
 	for (int i = 0; i < 4; i++)
 		blended |= mask[i] != 0ull ? 0xFFFFull << (16 * i) : 0ull;
 	return blended;
+}
+
+// The entries of a chunk, eight at a time.
+template <bool kDepth, BoxTest kBox>
+__device__ __forceinline__ void backward_chunk(BackwardPixel& p, uint32_t last_contributor, const BackwardStage& st, int count,
+                                               LdsPair* const (&rows)[2], const float2 pixf, const BoxSpan& span, const Sweep& sweep,
+                                               const StripFrame& frame, int lane, const BlendArgs& a)
+{
+	for (int k = 0; k < count; k += kRows) {
+		const Blended blended = {backward_rows<kDepth, kBox>(p, last_contributor, st, k, rows[0], pixf, span, a),
+		                         backward_rows<kDepth, kBox>(p, last_contributor, st, k + 4, rows[1], pixf, span, a)};
+		if ((blended.low | blended.high) != 0ull)
+			sum_rows<kDepth>(st, k, blended, sweep, frame, lane);
+	}
 }
 
 template <bool kDepth>
@@ -1130,6 +1154,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 	LoadedRecord cur = load_record(a, pos_cur != kNone ? list[min(pos_cur & kPosition, n - 1u)] : 0u, pos_cur != kNone);
 	uint32_t id_next = pos_next != kNone ? list[min(pos_next & kPosition, n - 1u)] : 0u;
 
+	BoxSpan span = {0.f, 0.f, 0.f, 0.f};  // of the pixel, from the first chunk that straddles a face of the box on
+	bool have_span = false;
 	for (uint32_t first = 0; first < filed; first += 64) {
 		const int count = (int)min(filed - first, 64u);
 		if (lane < count) {
@@ -1160,22 +1186,17 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 		const uint32_t e3 = first + 192 + (uint32_t)lane;
 		pos_after = e3 < filed ? filed_list[filed - 1 - e3] : kNone;
 
-		// (few strips straddle a face of their box: their chunks run a copy of the loop that has the test)
-		if (boxed) {
-			const BoxSpan span = span_for_visits(all_in_front, st.rays, a);
-			for (int k = 0; k < count; k += kRows) {
-				const Blended blended = {backward_rows<kDepth, true>(p, last_contributor, st, k, rows[0], pixf, span, a),
-				                         backward_rows<kDepth, true>(p, last_contributor, st, k + 4, rows[1], pixf, span, a)};
-				if ((blended.low | blended.high) != 0ull)
-					sum_rows<kDepth>(st, k, blended, sweep, frame, lane);
+		// (few strips straddle a face of their box: their chunks run copies of the loop that have the test)
+		if (boxed && all_in_front) {
+			if (!have_span) {
+				span = w_inside_box(ray_of(st.rays), load_box_frame(a));
+				have_span = true;
 			}
+			backward_chunk<kDepth, kBoxSpans>(p, last_contributor, st, count, rows, pixf, span, sweep, frame, lane, a);
+		} else if (boxed) {
+			backward_chunk<kDepth, kBoxExact>(p, last_contributor, st, count, rows, pixf, span, sweep, frame, lane, a);
 		} else {
-			for (int k = 0; k < count; k += kRows) {
-				const Blended blended = {backward_rows<kDepth, false>(p, last_contributor, st, k, rows[0], pixf, BoxSpan{}, a),
-				                         backward_rows<kDepth, false>(p, last_contributor, st, k + 4, rows[1], pixf, BoxSpan{}, a)};
-				if ((blended.low | blended.high) != 0ull)
-					sum_rows<kDepth>(st, k, blended, sweep, frame, lane);
-			}
+			backward_chunk<kDepth, kBoxNone>(p, last_contributor, st, count, rows, pixf, span, sweep, frame, lane, a);
 		}
 		__builtin_amdgcn_wave_barrier();
 	}

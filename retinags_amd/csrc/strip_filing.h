@@ -32,17 +32,21 @@ struct BoxFrame {
 	float tanx, tany;
 };
 
-__device__ __forceinline__ BoxFrame load_box_frame(const float* __restrict__ projinv, const float* __restrict__ range_low,
-                                                   const float* __restrict__ range_up, float tanx, float tany)
+// A pointer to what no kernel writes while it is read: such loads go through the scalar unit, straight into scalar registers.
+typedef const __attribute__((address_space(4))) float* ConstantFloats;
+__device__ __forceinline__ ConstantFloats constant_floats(const float* p) { return (ConstantFloats)(uintptr_t)p; }
+
+__device__ __forceinline__ BoxFrame load_box_frame(const float* projinv, const float* range_low, const float* range_up, float tanx, float tany)
 {
 	BoxFrame b;
+	const ConstantFloats m = constant_floats(projinv), lo = constant_floats(range_low), hi = constant_floats(range_up);
 #pragma unroll
 	for (int c = 0; c < 4; c++)
 #pragma unroll
 		for (int r = 0; r < 3; r++)
-			b.m[c][r] = wave_uniform(projinv[4 * c + r]);
-	b.lo = float3{wave_uniform(range_low[0]), wave_uniform(range_low[1]), wave_uniform(range_low[2])};
-	b.hi = float3{wave_uniform(range_up[0]), wave_uniform(range_up[1]), wave_uniform(range_up[2])};
+			b.m[c][r] = m[4 * c + r];
+	b.lo = float3{lo[0], lo[1], lo[2]};
+	b.hi = float3{hi[0], hi[1], hi[2]};
 	b.tanx = tanx;
 	b.tany = tany;
 	return b;
