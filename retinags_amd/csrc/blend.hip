@@ -135,9 +135,13 @@ __device__ __forceinline__ float exp_of_exponent(float x)
 
 // Launch-order classes of the backward's strips, by the number of entries they have to walk.
 constexpr int kStripClasses = 256;
-__device__ __forceinline__ uint32_t strip_class(uint32_t filed) { return 255u - min(filed >> 3, 255u); }
+constexpr uint32_t kEmptyClass = kStripClasses;  // of the strips without entries: the last ones of an order
+__device__ __forceinline__ uint32_t strip_class(uint32_t filed) { return filed == 0u ? kEmptyClass : 255u - min(filed >> 3, 255u); }
+// Words of strip_classes behind the counters and cursors of the two orders (1: the forward's, 0: the backward's).
+constexpr int kStripTail = 4 * kStripClasses;
+constexpr int strip_empty_word(int forward) { return kStripTail + 2 * forward; }  // how many strips are empty; behind it the placement cursor
+static_assert(strip_empty_word(1) + 1 < kRangeTailWords, "the words lie behind the ranges");
 
-constexpr uint32_t kLongList = 2048;    // filed entries from which a strip's wavefront takes the highest issue priority
 constexpr int kPerLane = 1;             // list entries per lane and step (2 was measured slower)
 constexpr int kChunk = 64 * kPerLane;   // list entries a wavefront takes per step
 
@@ -625,13 +629,6 @@ __device__ __forceinline__ void forward_strip(const BlendArgs& a, uint32_t strip
 	uint64_t live = lanes_where(inside);
 	// the entries filed for this strip, in list order: list position, bit 31 = strip inside the box
 	const uint32_t filed = a.strip_total[strip_id];
-	// A long list is a long chain of dependent steps: its wavefront goes first where it shares a SIMD with
-	// wavefronts of short lists, which lose little by waiting and would otherwise stretch the launch's longest walk.
-	if (filed > kLongList)
-		__builtin_amdgcn_s_setprio(3);
-	else if (filed > kLongList / 4)
-		__builtin_amdgcn_s_setprio(2);
-
 	if (filed != 0u && live != 0ull) {
 		stage_rays(st.rays, pixf, a, lane);
 		const uint32_t* list = a.point_list + range.x;
@@ -711,14 +708,58 @@ __device__ __forceinline__ void forward_strip(const BlendArgs& a, uint32_t strip
 	               ty * kTile + wave * 4 + (lane_again >> 4), lane_again);
 }
 
+// The place in the order of a workgroup's first, second ... strip.
+__device__ __forceinline__ uint32_t turn_of_workgroup(uint32_t number, uint32_t turn, uint32_t workgroups)
+{
+	return turn * workgroups + ((turn & 1u) != 0u ? workgroups - 1u - number : number);
+}
+
+// Strips without entries, at most 64 of them: background, and nothing for the backward to walk.
+__device__ __forceinline__ void forward_empty(const BlendArgs& a, const uint32_t* order, uint32_t count, int lane)
+{
+	const uint32_t mine = (uint32_t)lane < count ? order[lane] : 0u;
+	const size_t plane = (size_t)a.H * a.W;
+	const float r = a.bg[0], g = a.bg[1], b = a.bg[2];
+	for (uint32_t k = 0; k < count; k++) {
+		const uint32_t strip_id = (uint32_t)__builtin_amdgcn_readlane((int)mine, (int)k), tile = strip_id >> 2;
+		const uint32_t px = (tile % (uint32_t)a.grid_x) * kTile + (lane & 15), py = (tile / (uint32_t)a.grid_x) * kTile + 4u * (strip_id & 3u) + (lane >> 4);
+		if (lane == 0)
+			a.strip_filed[strip_id] = 0u;
+		if (px < (uint32_t)a.W && py < (uint32_t)a.H) {
+			const uint32_t pix_id = (uint32_t)a.W * py + px;
+			a.n_contrib[pix_id] = 0u;
+			a.out_color[pix_id] = r;
+			a.out_color[plane + pix_id] = g;
+			a.out_color[2 * plane + pix_id] = b;
+			a.out_alpha[pix_id] = 0.f;
+			a.out_depth[pix_id] = 0.f;
+		}
+	}
+}
+
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 6))) void blend_forward_kernel(BlendBatch batch)
 {
 	__shared__ ForwardStage st;
 	// The jobs of a batch (the submodels of a frame) take turns, each handing out its strips longest
 	// list first: a long strip that starts late is what a launch waits for, and with several jobs in one
-	// launch there is other work to run beside the longest strips of each.
+	// launch there is other work to run beside the longest strips of each.  Most strips of a large image are empty
+	// in most jobs, and workgroups are launched at about one per nanosecond, so a job has batch.workgroups of them, a
+	// share of its strips: strips with entries beyond that number are second turns, the last of them that of the workgroup
+	// with the longest first one.  The empty ones are dealt out evenly and come first: their stores leave while the walk goes on.
 	const BlendArgs& a = batch.job[blockIdx.x % (uint32_t)batch.count];
-	forward_strip(a, a.strip_order_forward[blockIdx.x / (uint32_t)batch.count], st, threadIdx.x);
+	const int lane = threadIdx.x;
+	const uint32_t number = blockIdx.x / (uint32_t)batch.count, workgroups = batch.workgroups;
+	uint32_t strip_id = a.strip_order_forward[number];  // (asked for beside the number of empty ones; workgroups <= strips)
+	const uint32_t none = min(a.strip_classes[strip_empty_word(1)], batch.strips), filled = batch.strips - none;
+	const uint32_t share = (none + workgroups - 1u) / workgroups;
+	for (uint32_t first = number * share, end = min(first + share, none); first < end; first += 64u)
+		forward_empty(a, a.strip_order_forward + filled + first, min(64u, end - first), lane);
+	for (uint32_t at = number, turn = 0; at < filled;) {
+		forward_strip(a, strip_id, st, lane);
+		at = turn_of_workgroup(number, ++turn, workgroups);
+		if (at < filled)
+			strip_id = a.strip_order_forward[at];
+	}
 }
 
 // Work accounting: the reference loop taken literally, one list entry at a time with no
@@ -1071,18 +1112,8 @@ __device__ __forceinline__ void backward_chunk(BackwardPixel& p, uint32_t last_c
 }
 
 template <bool kDepth>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void blend_backward_kernel(BlendBatch batch)
+__device__ __forceinline__ void backward_strip(const BlendArgs& a, uint32_t strip_id, BackwardStage& st, int lane)
 {
-	__shared__ BackwardStage s_stage;
-
-	const int lane = threadIdx.x;
-	// the jobs of the batch take turns; each hands out its strips with the most entries first: a long
-	// strip that starts late is what the whole launch waits for
-	const BlendArgs& a = batch.job[blockIdx.x % (uint32_t)batch.count];
-	// What the forward left in the workspaces (the strips' order, the tiles' ranges, the lists, the walk lengths) comes
-	// back through the caller's hands: every index taken from it is held inside the arrays' bounds, so that a
-	// workspace that is not the forward's (stale, or another frame's) gives wrong gradients and no stray access.
-	const uint32_t strip_id = min(a.strip_order[blockIdx.x / (uint32_t)batch.count], 4u * (uint32_t)(a.grid_x * a.grid_y) - 1u);
 	const int tile = (int)(strip_id >> 2), wave = (int)(strip_id & 3u);  // wave: which strip of the tile
 	uint2 range = a.ranges[tile];
 	range.y = min(range.y, a.capacity);
@@ -1095,7 +1126,6 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 	const size_t plane = (size_t)a.H * a.W;
 	const float strip_x0 = (float)(tx * kTile), strip_y0 = (float)(ty * kTile + wave * 4);
 	const StripFrame frame = {strip_x0, strip_y0, (float)(0.5 * a.W), (float)(0.5 * a.H)};
-	BackwardStage& st = s_stage;
 
 	// The forward blend has written down which entries of the tile's list matter to this strip
 	// (its conservative filters, not repeated here), up to the last one that any pixel blended.
@@ -1154,7 +1184,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 	LoadedRecord cur = load_record(a, pos_cur != kNone ? list[min(pos_cur & kPosition, n - 1u)] : 0u, pos_cur != kNone);
 	uint32_t id_next = pos_next != kNone ? list[min(pos_next & kPosition, n - 1u)] : 0u;
 
-	BoxSpan span = {0.f, 0.f, 0.f, 0.f};  // of the pixel, from the first chunk that straddles a face of the box on
+	BoxSpan span;  // of the pixel, from the first chunk that straddles a face of the box on
 	bool have_span = false;
 	for (uint32_t first = 0; first < filed; first += 64) {
 		const int count = (int)min(filed - first, 64u);
@@ -1188,7 +1218,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 
 		// (few strips straddle a face of their box: their chunks run copies of the loop that have the test)
 		if (boxed && all_in_front) {
-			if (!have_span) {
+			if (kDepth || !have_span) {  // (with the depth terms no registers are left to hold it)
 				span = w_inside_box(ray_of(st.rays), load_box_frame(a));
 				have_span = true;
 			}
@@ -1202,30 +1232,54 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 	}
 }
 
+template <bool kDepth>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void blend_backward_kernel(BlendBatch batch)
+{
+	__shared__ BackwardStage st;
+	// the jobs of the batch take turns; each hands out its strips with the most entries first: a long
+	// strip that starts late is what the whole launch waits for (workgroups and their turns as in blend_forward_kernel; a strip
+	// without entries to walk needs nothing)
+	const BlendArgs& a = batch.job[blockIdx.x % (uint32_t)batch.count];
+	const uint32_t number = blockIdx.x / (uint32_t)batch.count;
+	uint32_t strip_id = a.strip_order[number];
+	const uint32_t filled = batch.strips - min(a.strip_classes[strip_empty_word(0)], batch.strips);
+	for (uint32_t at = number, turn = 0; at < filled;) {
+		// What the forward left in the workspaces (the strips' order, the tiles' ranges, the lists, the walk lengths) comes
+		// back through the caller's hands: every index taken from it is held inside the arrays' bounds, so that a
+		// workspace that is not the forward's (stale, or another frame's) gives wrong gradients and no stray access.
+		int lane = threadIdx.x;
+		asm volatile("" : "+v"(lane));  // (what follows from it is worked out per turn: held from the first on, it costs registers)
+		backward_strip<kDepth>(a, min(strip_id, batch.strips - 1u), st, lane);
+		at = turn_of_workgroup(number, ++turn, batch.workgroups);
+		if (at < filled)
+			strip_id = a.strip_order[at];
+	}
+}
+
 // Strips by decreasing number of entries to walk, in kStripClasses classes of 8 (longer ones share
 // the first class); the order inside a class is whatever the atomics give, which is all a
-// launch order needs.  Two small kernels: count the strips of every class, then place them; one
+// launch order needs; the strips without any come last.  Two small kernels: count the strips of every class, then place them; one
 // launch of each serves every job of a batch (blockIdx.y).  Both aggregate in LDS first: most
 // strips fall into one class (nothing to walk), and thousands of global atomics on one word would
 // take longer than the blend itself.  What bounds them is the additions of all workgroups to the same few counters, so a
-// workgroup takes kOrderStrips strips, four per thread, and the lanes of the last class (little or nothing to walk, often
-// most of a wavefront) add to its LDS counter as one
+// workgroup takes kOrderStrips strips, four per thread, and the lanes with empty strips (often most of a wavefront) add to their
+// LDS counter as one
 // (5185x3359, both kernels and both orders: 92 us with a strip per thread, 31 now; 1600x1036: 19 and 20).
 constexpr uint32_t kOrderStrips = 1024;
 
 // The calling lane's place among its workgroup's strips of class c (all lanes come here).
 __device__ __forceinline__ uint32_t count_in_class(uint32_t* s_count, uint32_t c, bool valid)
 {
-	const uint64_t last = lanes_where(valid && c == kStripClasses - 1u);
+	const uint64_t last = lanes_where(valid && c == kEmptyClass);
 	uint32_t rank = 0;
-	if (valid && c != kStripClasses - 1u)
+	if (valid && c != kEmptyClass)
 		rank = atomicAdd(&s_count[c], 1u);
 	if (last != 0ull) {
 		uint32_t base = 0;
 		if (lanes_below(~0ull) == 0u)
-			base = atomicAdd(&s_count[kStripClasses - 1], (uint32_t)__popcll(last));
+			base = atomicAdd(&s_count[kEmptyClass], (uint32_t)__popcll(last));
 		base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
-		if (valid && c == kStripClasses - 1u)
+		if (valid && c == kEmptyClass)
 			rank = base + lanes_below(last);
 	}
 	return rank;
@@ -1234,6 +1288,7 @@ __device__ __forceinline__ uint32_t count_in_class(uint32_t* s_count, uint32_t c
 struct StripOrderJob {
 	const uint32_t* length;  // per strip
 	uint32_t* classes;       // kStripClasses counters and as many placement cursors, zero beforehand
+	uint32_t* empty;         // how many strips are empty, and their placement cursor, zero beforehand
 	uint32_t* order;
 };
 struct StripOrderBatch {
@@ -1243,9 +1298,11 @@ struct StripOrderBatch {
 
 __global__ __launch_bounds__(256) void strip_count_kernel(StripOrderBatch batch)
 {
-	__shared__ uint32_t s_count[kStripClasses];
+	__shared__ uint32_t s_count[kStripClasses + 1];
 	const StripOrderJob& j = batch.job[blockIdx.y];
 	s_count[threadIdx.x] = 0;
+	if (threadIdx.x == 0)
+		s_count[kEmptyClass] = 0;
 	__syncthreads();
 	uint32_t length[kOrderStrips / 256];
 #pragma unroll
@@ -1259,14 +1316,18 @@ __global__ __launch_bounds__(256) void strip_count_kernel(StripOrderBatch batch)
 	__syncthreads();
 	if (s_count[threadIdx.x] != 0u)
 		atomicAdd(&j.classes[threadIdx.x], s_count[threadIdx.x]);
+	if (threadIdx.x == 0 && s_count[kEmptyClass] != 0u)
+		atomicAdd(&j.empty[0], s_count[kEmptyClass]);
 }
 
 __global__ __launch_bounds__(256) void strip_place_kernel(StripOrderBatch batch)
 {
-	__shared__ uint32_t s_count[kStripClasses];  // strips of this block per class, then where they go
+	__shared__ uint32_t s_count[kStripClasses + 1];  // strips of this block per class, then where they go
 	__shared__ uint32_t s_scan[8];
 	const StripOrderJob& j = batch.job[blockIdx.y];
 	s_count[threadIdx.x] = 0;
+	if (threadIdx.x == 0)
+		s_count[kEmptyClass] = 0;
 	__syncthreads();
 	const uint32_t in_class = j.classes[threadIdx.x];
 	uint32_t c[kOrderStrips / 256], rank[kOrderStrips / 256];
@@ -1284,6 +1345,8 @@ __global__ __launch_bounds__(256) void strip_place_kernel(StripOrderBatch batch)
 	const uint32_t mine = s_count[threadIdx.x];
 	__syncthreads();
 	s_count[threadIdx.x] = start + (mine != 0u ? atomicAdd(&j.classes[kStripClasses + threadIdx.x], mine) : 0u);
+	if (threadIdx.x == 0)
+		s_count[kEmptyClass] = total + (s_count[kEmptyClass] != 0u ? atomicAdd(&j.empty[1], s_count[kEmptyClass]) : 0u);
 	__syncthreads();
 #pragma unroll
 	for (uint32_t q = 0; q < kOrderStrips / 256; q++) {
@@ -1301,6 +1364,7 @@ static void launch_strip_order(const BlendArgs* jobs, int count, int which, hipS
 	for (int k = 0; k < count; k++) {
 		b.job[k].length = which == 0 ? jobs[k].strip_total : jobs[k].strip_filed;
 		b.job[k].classes = jobs[k].strip_classes + (which == 0 ? 2 * kStripClasses : 0);
+		b.job[k].empty = jobs[k].strip_classes + strip_empty_word(which == 0 ? 1 : 0);
 		b.job[k].order = which == 0 ? jobs[k].strip_order_forward : jobs[k].strip_order;
 	}
 	const dim3 grid((b.strips + kOrderStrips - 1) / kOrderStrips, (unsigned)count);
@@ -1332,6 +1396,17 @@ void launch_strip_filing(const BlendArgs* jobs, int count, hipStream_t s)
 	}
 }
 
+// Workgroups of a job in a blend launch (see blend_forward_kernel): one per strip up to kStripWorkgroups of all jobs together,
+// beyond that half as many as strips.  Forward and backward in us with one per strip, half and a quarter as many, all with the
+// empty strips dealt out: 104 000 strips of which 28 700 have entries (1600x1036, 4 jobs) 281 + 542, 278 + 539, 286 + 554;
+// 1 094 000 strips (5185x3359) 1 735 + 2 889, 1 612 + 2 773, 1 600 + 2 770; 130 560 of which 36 800 (view of a city) 157, 145, 151.
+// Where all strips nearly fit the chip at once, second turns only lengthen the launch (12 288 strips at 1013x761: 59 -> 64).
+constexpr unsigned kStripWorkgroups = 32768;
+static unsigned blend_workgroups(unsigned strips, int jobs)
+{
+	return (size_t)strips * (size_t)jobs <= kStripWorkgroups ? strips : (strips + 1) / 2;
+}
+
 // All jobs share the image size (they are the submodels of one frame, or a single call).
 void launch_blend_forward(const BlendArgs* jobs, int count, hipStream_t s)
 {
@@ -1344,7 +1419,9 @@ void launch_blend_forward(const BlendArgs* jobs, int count, hipStream_t s)
 		stage_mark("strip_order", s);
 		launch_strip_order(jobs + at, batch.count, 0, s);
 		stage_mark("blend_forward", s);
-		hipLaunchKernelGGL(blend_forward_kernel, dim3(strips * (unsigned)batch.count), dim3(64), 0, s, batch);
+		batch.strips = strips;
+		batch.workgroups = blend_workgroups(strips, batch.count);
+		hipLaunchKernelGGL(blend_forward_kernel, dim3(batch.workgroups * (unsigned)batch.count), dim3(64), 0, s, batch);
 		// the order in which the backward will take the strips
 		stage_mark("strip_order", s);
 		launch_strip_order(jobs + at, batch.count, 1, s);
@@ -1360,13 +1437,16 @@ void launch_blend_backward(const BlendArgs* jobs, int count, hipStream_t s)
 		batch.count = count - at < kMaxBlendBatch ? count - at : kMaxBlendBatch;
 		for (int k = 0; k < batch.count; k++)
 			batch.job[k] = jobs[at + k];
+		batch.strips = strips;
+		batch.workgroups = blend_workgroups(strips, batch.count);
+		const dim3 grid(batch.workgroups * (unsigned)batch.count);
 		bool depth = false;  // does any job of the batch bring a gradient of the depth image?
 		for (int k = 0; k < batch.count; k++)
 			depth = depth || batch.job[k].dL_dpix_depth != nullptr;
 		if (depth)
-			hipLaunchKernelGGL(blend_backward_kernel<true>, dim3(strips * (unsigned)batch.count), dim3(64), 0, s, batch);
+			hipLaunchKernelGGL(blend_backward_kernel<true>, grid, dim3(64), 0, s, batch);
 		else
-			hipLaunchKernelGGL(blend_backward_kernel<false>, dim3(strips * (unsigned)batch.count), dim3(64), 0, s, batch);
+			hipLaunchKernelGGL(blend_backward_kernel<false>, grid, dim3(64), 0, s, batch);
 	}
 }
 

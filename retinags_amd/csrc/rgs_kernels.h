@@ -101,8 +101,8 @@ struct BlendArgs {
 	const uint32_t* order_status;
 	uint32_t* strip_order;  // strips by decreasing strip_filed, written behind the forward blend
 	uint32_t* strip_order_forward;  // strips by decreasing strip_total, written ahead of the forward blend
-	uint32_t* strip_classes;  // 4 x 256 words, zero before the forward blend: strips per class and placement cursors,
-	                          // for strip_order and then for strip_order_forward
+	uint32_t* strip_classes;  // kRangeTailWords words, zero before the forward blend: 256 strips per class and 256 placement cursors,
+	                          // for strip_order and then for strip_order_forward; then the numbers of empty strips and cursors
 	uint64_t* counters;  // non-null selects the work-accounting twin of the forward blend (7 sums)
 	// backward
 	const float* dL_dpix;
@@ -457,7 +457,7 @@ void launch_report_sort_status(const uint32_t* temp, uint32_t* fault, uint32_t* 
 // and sets *fault (host memory the device can write, may be null).  The caller has cleared `ranges`.  With a non-null
 // n_device the number of keys is min(n, *n_device) and the launch is sized for n.  file_tail (may be null)
 // receives, per kFileGroup keys, how many entries of the tile of the last of them have each strip bit set.
-constexpr int kRangeTailWords = 1024;   // words behind the ranges: the strip class counters of the blend
+constexpr int kRangeTailWords = 1028;   // words behind the ranges: the strip class counters of the blend
 struct TileRangesJob {
 	const uint32_t* keys;
 	size_t n;
@@ -476,6 +476,7 @@ constexpr int kMaxBlendBatch = 16;   // jobs one launch of a blend kernel can ta
 struct BlendBatch {
 	BlendArgs job[kMaxBlendBatch];
 	int count;
+	uint32_t strips, workgroups;  // of each job (set by the launchers)
 };
 void launch_strip_filing(const BlendArgs* jobs, int count, hipStream_t s);   // the per-strip lists, from the sorted keys' strip bits
 // `jobs` (host array) share one image size; more than kMaxBlendBatch take several launches.
