@@ -54,6 +54,8 @@ __device__ __forceinline__ PixelRay ray_of(const StripRays& r)
 	return PixelRay{r.x[lane & 15], r.y[lane >> 4]};
 }
 
+__device__ __forceinline__ PixelRay ray_of(const PixelRay& r) { return r; }
+
 __device__ __forceinline__ BoxFrame load_box_frame(const BlendArgs& a)
 {
 	return load_box_frame(a.projinv, a.range_low, a.range_up, a.tanfovx, a.tanfovy);
@@ -107,7 +109,8 @@ __device__ __forceinline__ BoxSpan w_inside_box(const PixelRay& ray, const BoxFr
 
 // The lanes among `lanes` whose sample at clip w the box does not clip (a NaN, which marks an entry that has the whole
 // strip inside the box: all of them).
-__device__ __forceinline__ uint64_t lanes_inside_box(uint64_t lanes, float w, const BoxSpan& s, const StripRays& rays, const BlendArgs& a)
+template <typename Rays>
+__device__ __forceinline__ uint64_t lanes_inside_box(uint64_t lanes, float w, const BoxSpan& s, const Rays& rays, const BlendArgs& a)
 {
 	lanes &= ~(lanes_where(w < s.from) | lanes_where(w > s.to));
 	const uint64_t unsure = lanes & (lanes_where(w <= s.from_sure) | lanes_where(w >= s.to_sure));
@@ -116,7 +119,8 @@ __device__ __forceinline__ uint64_t lanes_inside_box(uint64_t lanes, float w, co
 	return lanes;
 }
 // The same by the exact test alone, where some entry of the chunk lies at a clip w that is not positive.
-__device__ __forceinline__ uint64_t lanes_inside_box(uint64_t lanes, float w, const StripRays& rays, const BlendArgs& a)
+template <typename Rays>
+__device__ __forceinline__ uint64_t lanes_inside_box(uint64_t lanes, float w, const Rays& rays, const BlendArgs& a)
 {
 	return lanes & ~lanes_where(clipped_by_box(ray_of(rays), w, load_box_frame(a)));
 }
@@ -574,8 +578,10 @@ __device__ __forceinline__ void prune_by_box(bool straddles, bool takes, float w
 // result.  (The rows matter as much as the columns: a ground plane at a grazing angle is made of flat ellipses, and a row
 // of pixels just above the horizon, which nothing fills, kept its strip walking thousands of entries that only its finished
 // rows could see.)
-__device__ __forceinline__ void halves_reached(const LoadedRecord& r, float x0, float ya, const float4 box_l, const float4 box_r,
-                                               bool& left, bool& right)
+struct EllipseBox {
+	float dx, dy, reach_x, reach_y;  // centre relative to the strip's first pixel, half extents
+};
+__device__ __forceinline__ EllipseBox ellipse_box(const LoadedRecord& r, float x0, float ya)
 {
 	const float ca = r.conic.x, cb = r.conic.y, cc = r.conic.z;
 	const float dxa = r.geom.x - x0, dya = r.geom.y - ya;
@@ -583,15 +589,19 @@ __device__ __forceinline__ void halves_reached(const LoadedRecord& r, float x0, 
 	const float far_x = fmaxf(fabsf(dxa), fabsf(dxa - 15.f)), far_y = fmaxf(fabsf(dya), fabsf(dya - 3.f));
 	const float allowed = limit + (1e-3f + 1e-4f * limit + 1e-5f * (ca * far_x * far_x + cc * far_y * far_y));
 	const float det = ca * cc - cb * cb - 1e-6f * ca * cc;
-	float reach_x = INFINITY, reach_y = INFINITY;
+	EllipseBox b = {dxa, dya, INFINITY, INFINITY};
 	if ((ca > 0.f) && (cc > 0.f) && (det > 0.f)) {
 		const float scale = allowed * __builtin_amdgcn_rcpf(det);
-		reach_x = __builtin_amdgcn_sqrtf(scale * cc) * 1.001f + 0.01f;
-		reach_y = __builtin_amdgcn_sqrtf(scale * ca) * 1.001f + 0.01f;
+		b.reach_x = __builtin_amdgcn_sqrtf(scale * cc) * 1.001f + 0.01f;
+		b.reach_y = __builtin_amdgcn_sqrtf(scale * ca) * 1.001f + 0.01f;
 	}
-	// (a NaN, as of a Gaussian whose floor is, excludes nothing)
-	left = !(dxa + reach_x < box_l.x) && !(dxa - reach_x > box_l.y) && !(dya + reach_y < box_l.z) && !(dya - reach_y > box_l.w);
-	right = !(dxa + reach_x < box_r.x) && !(dxa - reach_x > box_r.y) && !(dya + reach_y < box_r.z) && !(dya - reach_y > box_r.w);
+	return b;
+}
+// box: first and last column, first and last row, relative to the strip's first pixel.  (A NaN, as of a Gaussian whose floor is,
+// excludes nothing.)
+__device__ __forceinline__ bool reaches(const EllipseBox& e, const float4 box)
+{
+	return !(e.dx + e.reach_x < box.x) && !(e.dx - e.reach_x > box.y) && !(e.dy + e.reach_y < box.z) && !(e.dy - e.reach_y > box.w);
 }
 
 constexpr uint32_t kNone = 0xFFFFFFFFu, kPosition = 0x7FFFFFFFu;  // of a filed entry: none, and its list position
@@ -685,8 +695,11 @@ __device__ __forceinline__ void forward_strip(const BlendArgs& a, uint32_t strip
 			const int half = (l >> 3) & 1;
 			const float4 box_l = live_box(live, 0), box_r = live_box(live, 8);
 			bool left = false, right = false;
-			if (l < count)
-				halves_reached(cur, x0, ya, box_l, box_r, left, right);
+			if (l < count) {
+				const EllipseBox e = ellipse_box(cur, x0, ya);
+				left = reaches(e, box_l);
+				right = reaches(e, box_r);
+			}
 			// Entries whose sample the box clips in every pixel of a half that still takes entries are left out too: a
 			// pixel whose ray has left the box, or enters it behind everything, stays unfinished for good, and a strip with
 			// one such pixel walked its list to the end (at 1600x1036 and 5.6 M Gaussians, a camera that looks along a
@@ -743,6 +756,195 @@ __device__ __forceinline__ void forward_strip(const BlendArgs& a, uint32_t strip
 	               ty * kTile + wave * 4 + (lane_again >> 4), lane_again);
 }
 
+// ---- a walk shared by four wavefronts ------------------------------------------------------------
+// A wavefront alone on its SIMD advances four entries in 1 200 cycles, of which it issues in 430: the rest is the latency of
+// one chain of LDS reads, dependent instructions and masks.  A launch with fewer strips than fill that time lasts as long as
+// its longest walk.  There (see blend_shared) a strip is walked by four wavefronts, one per quarter of 8x2 pixels, and each takes
+// four entries at a time: lane 4 p + e is pixel p's view of entry e, so that one exponential, one comparison serves
+// four entries.  What depends on order is kept bit for bit: the transmittances in front of the four entries are the same products
+// in the same order, taken by three multiplications inside each quad of lanes, and lane c of a quad adds channel c of
+// the four samples one after the other.  In all it is twice the work.  (The backward shared in the same way adds to each Gaussian's row
+// four times as often, and additions to one address take 12 ns each: 5 000 Gaussians at 512x512 took 303 us a pass for 200.)
+constexpr uint32_t kSharedList = 64;  // entries from which a strip is worth four wavefronts (24 to 128 measure the same, 192 up to 3 us more)
+
+template <int Ctrl>
+__device__ __forceinline__ float quad_move(float v)
+{
+	return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), Ctrl, 0xF, 0xF, true));
+}
+// Lane e of a quad: start times (plus) the f of lanes 0 to e - 1, in that order.
+__device__ __forceinline__ float product_in_front(float start, float f, int e)
+{
+	const float shifted = quad_move<0x90>(f);                      // quad_perm:[0,0,1,2]
+	const float in_front = e == 0 ? 1.f : shifted;
+	return start * quad_move<0x54>(in_front) * quad_move<0xA0>(in_front) * quad_move<0xC0>(in_front);  // [0,1,1,1], [0,0,2,2], [0,0,0,3]
+}
+
+struct QuarterPlace {
+	int tile, strip, column, row;  // the quarter's first pixel relative to the strip's
+	uint32_t px, py;               // the lane's pixel
+	bool inside;
+};
+__device__ __forceinline__ QuarterPlace quarter_place(const BlendArgs& a, uint32_t strip_id, int quarter, int lane)
+{
+	QuarterPlace q;
+	q.tile = (int)(strip_id >> 2);
+	q.strip = (int)(strip_id & 3u);
+	q.column = 8 * (quarter & 1);
+	q.row = 2 * (quarter >> 1);
+	q.px = (uint32_t)(q.tile % a.grid_x * kTile + q.column + ((lane >> 2) & 7));
+	q.py = (uint32_t)(q.tile / a.grid_x * kTile + 4 * q.strip + q.row + (lane >> 5));
+	q.inside = q.px < (uint32_t)a.W && q.py < (uint32_t)a.H;
+	return q;
+}
+
+struct QuarterPixel {
+	float T;        // transmittance in front of the next entry (of a finished pixel: in front of the entry that finished it)
+	float C;        // lane c: channel c (r, g, b, depth)
+	float weight;
+	int last_slot;  // the last of the lane's entries that the pixel blended, as a packed slot of the chunk (-1: none)
+};
+
+// The four entries of slots k to k + 3.  odd_colours: some colour of the chunk is not finite, so that one which is not blended
+// must not be multiplied by its weight, zero.
+__device__ __forceinline__ void quarter_group(QuarterPixel& p, uint64_t& live, const ForwardSlot* slots, int k, int lane,
+                                              const float2 pixf, BoxTest box, const BoxSpan& span, const PixelRay& ray, bool odd_colours,
+                                              const BlendArgs& a)
+{
+	const int e = lane & 3;
+	const float4 centre_conic = slots[k + e].centre_conic, rest = slots[k + e].rest;
+	float colour[4];
+#pragma unroll
+	for (int i = 0; i < 4; i++)
+		colour[i] = reinterpret_cast<const float*>(&slots[k + i].cd)[e];
+	__builtin_amdgcn_sched_barrier(0);
+	const float power = exponent_of_staged(centre_conic, rest.x, pixf);
+	float alpha = fminf(0.99f, rest.y * exp_of_exponent(power));
+	uint64_t mask = live & lanes_where(!(power > 0.0f)) & lanes_where(!(alpha < 1.0f / 255.0f));
+	if (box == kBoxSpans)
+		mask = lanes_inside_box(mask, rest.z, span, ray, a);
+	else if (box == kBoxExact)
+		mask = lanes_inside_box(mask, rest.z, ray, a);
+	alpha = __builtin_amdgcn_inverse_ballot_w64(mask) ? alpha : 0.f;
+	const float beyond = 1 - alpha;
+	const float T = product_in_front(p.T, beyond, e), test_T = T * beyond;
+	const bool ok = !(test_T < 0.0001f);            // (false for every entry behind one for which it is)
+	const uint64_t passed = lanes_where(ok);
+	const float weight = ok ? alpha * T : 0.f;
+	p.last_slot = __builtin_amdgcn_inverse_ballot_w64(mask & passed) ? k + e : p.last_slot;
+	// in front of the next group: behind the last entry that passed
+	float t = ok ? test_T : p.T;
+	t = fminf(t, quad_move<0xB1>(t));     // quad_perm:[1,0,3,2]
+	p.T = fminf(t, quad_move<0x4E>(t));   // quad_perm:[2,3,0,1]
+	const uint64_t through = (passed >> 3) & 0x1111111111111111ull;  // pixels that entry 3 has passed
+	live &= (through << 4) - through;
+	const float w[4] = {quad_move<0x00>(weight), quad_move<0x55>(weight), quad_move<0xAA>(weight), quad_move<0xFF>(weight)};
+#pragma unroll
+	for (int i = 0; i < 4; i++)
+		p.weight += w[i];
+	if (!odd_colours) {
+#pragma unroll
+		for (int i = 0; i < 4; i++)
+			p.C = __builtin_fmaf(w[i], colour[i], p.C);
+	} else {
+#pragma unroll
+		for (int i = 0; i < 4; i++)
+			p.C = w[i] != 0.f ? __builtin_fmaf(w[i], colour[i], p.C) : p.C;  // (the weight of a blended sample is not zero)
+	}
+}
+
+// Bounding box of a quarter's live pixels, relative to the strip's first pixel.
+__device__ __forceinline__ float4 quarter_box(uint64_t live, const QuarterPlace& q)
+{
+	const uint32_t upper = (uint32_t)live & 0x11111111u, lower = (uint32_t)(live >> 32) & 0x11111111u, columns = upper | lower;
+	return float4{(float)(q.column + (__builtin_ctz(columns) >> 2)), (float)(q.column + ((31 - __builtin_clz(columns)) >> 2)),
+	              (float)(q.row + (upper == 0u ? 1 : 0)), (float)(q.row + (lower == 0u ? 0 : 1))};
+}
+
+__device__ __forceinline__ void forward_quarter(const BlendArgs& a, uint32_t strip_id, uint32_t filed, int quarter, ForwardStage& st, int lane)
+{
+	const QuarterPlace q = quarter_place(a, strip_id, quarter, lane);
+	const uint2 range = a.ranges[q.tile];
+	const uint32_t n = range.y - range.x;
+	const int e = lane & 3;
+	const float2 pixf = {(float)q.px, (float)q.py};
+	uint64_t live = lanes_where(q.inside);
+	if (live == 0ull)
+		return;
+	const PixelRay ray = {pix_to_ndc(pixf.x, a.W), pix_to_ndc(pixf.y, a.H)};
+	const float x0 = wave_uniform((float)(q.tile % a.grid_x * kTile)), ya = wave_uniform((float)(q.tile / a.grid_x * kTile + 4 * q.strip));
+	const uint32_t* list = a.point_list + range.x;
+	const uint32_t* filed_list = a.strip_lists + 4 * (size_t)range.x + (size_t)q.strip * n;
+	QuarterPixel p = {1.f, 0.f, 0.f, -1};
+	uint32_t last_filed = 0u;
+	BoxSpan span = {0.f, 0.f, 0.f, 0.f};
+	bool have_span = false;
+	// (chunks as in forward_strip)
+	uint32_t pos_cur = (uint32_t)lane < filed ? filed_list[lane] : kNone;
+	uint32_t pos_next = (uint32_t)(64 + lane) < filed ? filed_list[64 + lane] : kNone;
+	uint32_t pos_after = (uint32_t)(128 + lane) < filed ? filed_list[128 + lane] : kNone;
+	LoadedRecord cur = load_record(a, pos_cur != kNone ? list[pos_cur & kPosition] : 0u, pos_cur != kNone);
+	uint32_t id_next = pos_next != kNone ? list[pos_next & kPosition] : 0u;
+	for (uint32_t first = 0; first < filed && live != 0ull; first += 64) {
+		const int count = (int)min(filed - first, 64u);
+		bool reached = lane < count && reaches(ellipse_box(cur, x0, ya), quarter_box(live, q));
+		const bool straddles = lane < count && (pos_cur & 0x80000000u) == 0u;
+		const BoxTest box = lanes_where(straddles) == 0ull ? kBoxNone : lanes_where(straddles && !(cur.geom.w > 0.f)) == 0ull ? kBoxSpans : kBoxExact;
+		if (box == kBoxSpans) {
+			if (!have_span) {
+				span = w_inside_box(ray, load_box_frame(a));
+				have_span = true;
+			}
+			// entries that the box clips in every live pixel (as prune_by_box, over the quarter)
+			const bool takes = __builtin_amdgcn_inverse_ballot_w64(live) && !(span.from > span.to);
+			const float to = __uint_as_float(wave_max_u32(takes ? __float_as_uint(fmaxf(span.to, 0.f)) : 0u));
+			const float from = __uint_as_float(0x7F800000u - wave_max_u32(takes ? 0x7F800000u - __float_as_uint(span.from) : 0u));
+			if (straddles)
+				reached = reached && !(cur.geom.w > to) && !(cur.geom.w < from);
+		}
+		const uint64_t in = lanes_where(reached);
+		const int steps = __popcll(in);
+		// (a sum that is not finite names a colour that is not; one of finite colours may overflow, which only costs time)
+		const bool odd_colours = lanes_where(reached && !(fabsf(cur.cd.x + cur.cd.y + cur.cd.z + cur.cd.w) < INFINITY)) != 0ull;
+		if (reached)
+			stage_slot(st, 0, lanes_below(in), cur, pos_cur, lane);
+		if (lane < 3) {  // up to a multiple of four
+			stage_nothing(st, 0, (uint32_t)(steps + lane));
+			st.slots[steps + lane].cd = float4{0.f, 0.f, 0.f, 0.f};
+		}
+		__builtin_amdgcn_wave_barrier();
+		cur = load_record(a, id_next, pos_next != kNone);
+		pos_cur = pos_next;
+		pos_next = pos_after;
+		id_next = pos_next != kNone ? list[pos_next & kPosition] : 0u;
+		const uint32_t e3 = first + 192 + (uint32_t)lane;
+		pos_after = e3 < filed ? filed_list[e3] : kNone;
+		for (int k = 0; k < steps && live != 0ull; k += 4)
+			quarter_group(p, live, st.slots, k, lane, pixf, box, span, ray, odd_colours, a);
+		if (p.last_slot >= 0)
+			last_filed = first + st.entry[0][p.last_slot] + 1u;
+		p.last_slot = -1;
+		__builtin_amdgcn_wave_barrier();
+	}
+	const uint32_t upto = wave_max_u32(last_filed);
+	if (lane == 0 && upto != 0u)
+		atomicMax(&a.strip_filed[strip_id], upto);  // (zero before the launch)
+	last_filed = max(last_filed, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)last_filed, 0xB1, 0xF, 0xF, true));
+	last_filed = max(last_filed, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)last_filed, 0x4E, 0xF, 0xF, true));
+	if (q.inside) {
+		const uint32_t pix_id = (uint32_t)a.W * q.py + q.px;
+		const size_t plane = (size_t)a.H * a.W;
+		if (e < 3)
+			a.out_color[e * plane + pix_id] = p.C + p.T * a.bg[e];
+		else
+			a.out_depth[pix_id] = p.C;
+		if (e == 0)
+			a.out_alpha[pix_id] = p.weight;
+		if (e == 1)
+			a.n_contrib[pix_id] = last_filed != 0u ? (filed_list[last_filed - 1u] & kPosition) + 1u : 0u;
+	}
+}
+
 // The place in the order of a workgroup's first, second ... strip.
 __device__ __forceinline__ uint32_t turn_of_workgroup(uint32_t number, uint32_t turn, uint32_t workgroups)
 {
@@ -772,6 +974,7 @@ __device__ __forceinline__ void forward_empty(const BlendArgs& a, const uint32_t
 	}
 }
 
+template <bool kShared>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 6))) void blend_forward_kernel(BlendBatch batch)
 {
 	__shared__ ForwardStage st;
@@ -784,11 +987,23 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(6, 6))) void
 	const BlendArgs& a = batch.job[blockIdx.x % (uint32_t)batch.count];
 	const int lane = threadIdx.x;
 	const uint32_t number = blockIdx.x / (uint32_t)batch.count, workgroups = batch.workgroups;
-	uint32_t strip_id = a.strip_order_forward[number];  // (asked for beside the number of empty ones; workgroups <= strips)
+	uint32_t strip_id = a.strip_order_forward[min(number, batch.strips - 1u)];  // (asked for beside the number of empty ones)
 	const uint32_t none = min(a.strip_classes[strip_empty_word(1)], batch.strips), filled = batch.strips - none;
 	const uint32_t share = (none + workgroups - 1u) / workgroups;
 	for (uint32_t first = number * share, end = min(first + share, none); first < end; first += 64u)
 		forward_empty(a, a.strip_order_forward + filled + first, min(64u, end - first), lane);
+	if (kShared) {
+		// four neighbouring workgroups per strip
+		if (number / 4u >= filled)
+			return;
+		strip_id = a.strip_order_forward[number / 4u];
+		const uint32_t entries = a.strip_total[strip_id];
+		if (entries >= kSharedList)
+			forward_quarter(a, strip_id, entries, (int)(number & 3u), st, lane);
+		else if ((number & 3u) == ((number >> 3) & 3u))  // (not always the same of the four: they lie on different XCDs)
+			forward_strip(a, strip_id, st, lane);
+		return;
+	}
 	for (uint32_t at = number, turn = 0; at < filled;) {
 		forward_strip(a, strip_id, st, lane);
 		at = turn_of_workgroup(number, ++turn, workgroups);
@@ -1336,6 +1551,7 @@ struct StripOrderJob {
 	uint32_t* classes;       // kStripClasses counters and as many placement cursors, zero beforehand
 	uint32_t* empty;         // how many strips are empty, and their placement cursor, zero beforehand
 	uint32_t* order;
+	uint32_t* clear;         // per strip, set to zero (may be null)
 };
 struct StripOrderBatch {
 	StripOrderJob job[kMaxBlendBatch];
@@ -1397,8 +1613,11 @@ __global__ __launch_bounds__(256) void strip_place_kernel(StripOrderBatch batch)
 #pragma unroll
 	for (uint32_t q = 0; q < kOrderStrips / 256; q++) {
 		const uint32_t k = blockIdx.x * kOrderStrips + 256 * q + threadIdx.x;
-		if (k < batch.strips)
+		if (k < batch.strips) {
 			j.order[s_count[c[q]] + rank[q]] = k;
+			if (j.clear)
+				j.clear[k] = 0u;
+		}
 	}
 }
 
@@ -1410,6 +1629,7 @@ static void launch_strip_order(const BlendArgs* jobs, int count, int which, hipS
 	for (int k = 0; k < count; k++) {
 		b.job[k].length = which == 0 ? jobs[k].strip_total : jobs[k].strip_filed;
 		b.job[k].classes = jobs[k].strip_classes + (which == 0 ? 2 * kStripClasses : 0);
+		b.job[k].clear = which == 0 ? jobs[k].strip_filed : nullptr;  // (the wavefronts that share a strip take the largest of theirs)
 		b.job[k].empty = jobs[k].strip_classes + strip_empty_word(which == 0 ? 1 : 0);
 		b.job[k].order = which == 0 ? jobs[k].strip_order_forward : jobs[k].strip_order;
 	}
@@ -1453,6 +1673,13 @@ static unsigned blend_workgroups(unsigned strips, int jobs)
 	return (size_t)strips * (size_t)jobs <= kStripWorkgroups ? strips : (strips + 1) / 2;
 }
 
+// Whether a launch's strips are shared by four wavefronts each: up to 4 strips per SIMD of the chip, of all jobs together.  Forward blend
+// in us, one and four wavefronts per strip: 320 strips 28.9 and 22.8 (4 000 Gaussians), 52 and 36 (60 000); 1 900 strips 28.7 and 26.2,
+// 51.7 and 39.7; 3 200 strips of two submodels, with walks that the box leaves unfinished, 123 and 62; 4 096 strips 27.8 and 27.8 (5 000
+// Gaussians), 39.7 and 36.7, 53.3 and 49.9; a call with 4 400 to 10 000 strips is 7 to 30 us slower, a frame with 17 700 by 37.
+constexpr unsigned kSharedStrips = 4096;
+static bool blend_shared(unsigned strips, int jobs) { return (size_t)strips * (size_t)jobs <= kSharedStrips; }
+
 // All jobs share the image size (they are the submodels of one frame, or a single call).
 void launch_blend_forward(const BlendArgs* jobs, int count, hipStream_t s)
 {
@@ -1466,8 +1693,13 @@ void launch_blend_forward(const BlendArgs* jobs, int count, hipStream_t s)
 		launch_strip_order(jobs + at, batch.count, 0, s);
 		stage_mark("blend_forward", s);
 		batch.strips = strips;
-		batch.workgroups = blend_workgroups(strips, batch.count);
-		hipLaunchKernelGGL(blend_forward_kernel, dim3(batch.workgroups * (unsigned)batch.count), dim3(64), 0, s, batch);
+		const bool shared = blend_shared(strips, batch.count);
+		batch.workgroups = shared ? 4 * strips : blend_workgroups(strips, batch.count);
+		const dim3 grid(batch.workgroups * (unsigned)batch.count);
+		if (shared)
+			hipLaunchKernelGGL(blend_forward_kernel<true>, grid, dim3(64), 0, s, batch);
+		else
+			hipLaunchKernelGGL(blend_forward_kernel<false>, grid, dim3(64), 0, s, batch);
 		// the order in which the backward will take the strips
 		stage_mark("strip_order", s);
 		launch_strip_order(jobs + at, batch.count, 1, s);

@@ -25,6 +25,49 @@ def test_more_strips_than_workgroups(width, height, n, grow):
     _check_backward(sub, cam, torch.tensor([0.2, 0.1, 0.05]), seed=3, with_depth_alpha=False)
 
 
+# (up to 4 096 strips, as in most tests of small images, a forward walk is shared by four wavefronts)
+@pytest.mark.parametrize("low,up", [((-0.31, -0.27, 3.6), (0.23, 0.19, 4.3)), ((-5.0, 0.05, -1.0), (5.0, 5.0, 9.0)),
+                                    ((-5.0, -5.0, 4.95), (5.0, 5.0, 9.0))])
+@pytest.mark.parametrize("width,height", [(515, 497), (511, 505)])   # 4 224 and 4 096 strips
+def test_box_faces_with_and_without_shared_walks(low, up, width, height):
+    scene = scenes.cube_scene(2500, seed=92)
+    scene["scales"] = scene["scales"] * 5.0
+    cam = scenes.look_at_camera((0.0, 0.0, 0.0), (0.13, -0.07, 4.0), (0.1, -1, 0), width, height, 40.0)
+    sub = _scene_sub(scene, low=torch.tensor(low), up=torch.tensor(up))
+    _check_forward_stages(sub, cam, torch.tensor([0.2, 0.1, 0.05]), max_borderline=2e-3)
+    _check_backward(sub, cam, torch.tensor([0.2, 0.1, 0.05]), seed=17, with_depth_alpha=width == 511)
+
+
+def test_shared_and_whole_walks_give_the_same_bits():
+    """The same view as one job of a launch (4 096 strips: shared walks) and as two (whole ones): transmittances are the
+    same products in the same order and the sums add in the same order, so images and last blended entries are equal.
+    Some colours are infinite: they reach the pixels that blend them and no others."""
+    from retinags_amd import GaussianRasterizationSettings, GaussianRasterizer, rasterizer
+    dev = "cuda:0"
+    scene = scenes.cube_scene(20_000, seed=93)
+    cam = scenes.look_at_camera((0.0, 0.0, 0.0), (0.13, -0.07, 4.0), (0.1, -1, 0), 509, 501, 40.0).to(dev)
+    inf = float("inf")
+    rasterizers, inputs = [], []
+    for low, up in (((-0.4, -9.0, -9.0), (9.0, 9.0, 9.0)), ((-inf,) * 3, (inf,) * 3)):
+        rasterizers.append(GaussianRasterizer(GaussianRasterizationSettings(
+            image_height=501, image_width=509, tanfovx=cam.tanfovx, tanfovy=cam.tanfovy, bg=torch.zeros(3, device=dev), scale_modifier=1.0,
+            viewmatrix=cam.world_view_transform, projmatrix=cam.full_proj_transform, projmatrix_inv=cam.projection_matrix_inv,
+            range_low=torch.tensor(low, device=dev), range_up=torch.tensor(up, device=dev), sh_degree=0, campos=cam.camera_center,
+            prefiltered=False, debug=False)))
+        colours = torch.rand(20_000, 3, generator=torch.Generator().manual_seed(1))
+        colours[::200, 1] = inf
+        inputs.append(dict(means3D=scene["xyz"].to(dev), means2D=torch.zeros(20_000, 3, device=dev), colors_precomp=colours.to(dev),
+                           opacities=scene["opacity"].to(dev), scales=scene["scales"].to(dev) * 2, rotations=scene["rotations"].to(dev)))
+    with torch.no_grad():
+        together = rasterizer.rasterize_frame(rasterizers, inputs)
+        for k, (r, given) in enumerate(zip(rasterizers, inputs)):
+            for name, one, both in zip(("colour", "radii", "depth", "alpha"), r(**given), together[k]):
+                assert torch.equal(one, both), name
+            infinite = torch.isinf(together[k][0][1])
+            assert not torch.isnan(together[k][0]).any() and infinite.any() and infinite.float().mean() < 0.9
+            assert torch.isfinite(together[k][0][0]).all() and torch.isfinite(together[k][0][2]).all()
+
+
 @pytest.mark.parametrize("case", ("opaque", "needles", "some of each", "opacity is NaN"))
 def test_entries_that_need_every_comparison_of_a_visit(case):
     """Alphas that the 0.99 bound cuts, conics whose exponent may round to above zero at the centre, and both among entries
