@@ -155,6 +155,8 @@ __device__ __forceinline__ void wave_lds_fence()
 
 constexpr int kShRowStride = 13;  // float4 per parked row: 52 words, so 8 lanes' 16-byte reads meet no bank twice
 
+// kStream: records and per-Gaussian arrays are stored as streaming data (see launch_preprocess_forward).
+template <bool kStream>
 __global__ __launch_bounds__(256) void preprocess_forward_kernel(Batch<PreprocessArgs> batch)
 {
 	__shared__ uint32_t s_scan[8];
@@ -304,9 +306,9 @@ __global__ __launch_bounds__(256) void preprocess_forward_kernel(Batch<Preproces
 			if (!a.colors_precomp)
 				a.clamped[idx] = (uint8_t)clamp_bits;
 		}
-		a.radii[idx] = (int)my_radius;
-		a.tiles_touched[idx] = touched;
-		a.depths[idx] = view_z;  // 0 for a Gaussian that touches no tile: the depth order lists the others by this alone
+		store<kStream>(a.radii + idx, (int)my_radius);
+		store<kStream>(a.tiles_touched + idx, touched);
+		store<kStream>(a.depths + idx, view_z);  // 0 for a Gaussian that touches no tile: the depth order lists the others by this alone
 	}
 	{
 		// Everything later stages read of a rendered Gaussian goes into one 64-byte record: a
@@ -331,7 +333,7 @@ __global__ __launch_bounds__(256) void preprocess_forward_kernel(Batch<Preproces
 		for (int base = 0; base < n_seen; base += 16) {
 			const int slot = base + (lane >> 2);
 			if (slot < n_seen)
-				records[4 * (size_t)listed[slot] + (lane & 3)] = parked[slot * kRecordStride + (lane & 3)];
+				store<kStream>(records + 4 * (size_t)listed[slot] + (lane & 3), parked[slot * kRecordStride + (lane & 3)]);
 		}
 	}
 
@@ -793,6 +795,13 @@ void launch_mark_visible(int P, const float* means, const float* view, uint8_t* 
 	hipLaunchKernelGGL(mark_visible_kernel, dim3((P + 255) / 256), dim3(256), 0, s, P, means, view, present);
 }
 
+// From this many Gaussians on, all jobs together, the kernel's stores are streaming ones: the next kernels read the records and the three
+// arrays from end to end, later than the caches would keep them, and the rows that this kernel reads keep their place (1 598 ->
+// 1 463 us at 62.9 M Gaussians, 182 -> 177 at 5.6 M; with loads of the rows or of scale and rotation streaming as well it is slower
+// again, 1 620 to 1 700).  The 21 MB of records of 333 000 Gaussians are still there: streaming, the key duplication takes 44.5
+// instead of 42.2 us.
+constexpr size_t kStreamedGaussians = (size_t)1 << 20;
+
 void launch_preprocess_forward(const PreprocessArgs* jobs, int count, hipStream_t s)
 {
 	stage_mark("preprocess_forward", s);
@@ -800,11 +809,17 @@ void launch_preprocess_forward(const PreprocessArgs* jobs, int count, hipStream_
 		const int nj = count - at < kMaxBatch ? count - at : kMaxBatch;
 		Batch<PreprocessArgs> b = {};
 		int max_p = 0;
+		size_t all = 0;
 		for (int k = 0; k < nj; k++) {
 			b.job[k] = jobs[at + k];
 			max_p = b.job[k].P > max_p ? b.job[k].P : max_p;
+			all += (size_t)b.job[k].P;
 		}
-		hipLaunchKernelGGL(preprocess_forward_kernel, dim3((unsigned)((max_p + 255) / 256), (unsigned)nj), dim3(256), 0, s, b);
+		const dim3 grid((unsigned)((max_p + 255) / 256), (unsigned)nj);
+		if (all >= kStreamedGaussians)
+			hipLaunchKernelGGL(preprocess_forward_kernel<true>, grid, dim3(256), 0, s, b);
+		else
+			hipLaunchKernelGGL(preprocess_forward_kernel<false>, grid, dim3(256), 0, s, b);
 	}
 }
 

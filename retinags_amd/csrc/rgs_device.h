@@ -139,6 +139,22 @@ __device__ __forceinline__ void store_streaming(float4* p, const float4 v)
 {
 	__builtin_nontemporal_store(StreamVec{v.x, v.y, v.z, v.w}, reinterpret_cast<StreamVec*>(p));
 }
+template <bool kStream>
+__device__ __forceinline__ void store(float4* p, const float4 v)
+{
+	if (kStream)
+		store_streaming(p, v);
+	else
+		*p = v;
+}
+template <bool kStream, typename T>
+__device__ __forceinline__ void store(T* p, const T v)
+{
+	if (kStream)
+		__builtin_nontemporal_store(v, p);
+	else
+		*p = v;
+}
 
 // ---- wave64 cross-lane primitives (DPP) -----------------------------------------------
 

@@ -98,3 +98,27 @@ def test_gradient_rows_leave_alike_on_and_off_a_16_byte_boundary(n, monkeypatch)
             assert not torch.isnan(t).any() and not torch.isnan(odd[name]).any(), name
             assert rel_l2(odd[name].cpu().numpy(), t.cpu().numpy()) <= 1e-4, name
             assert (t[radii <= 0] == 0).all() and (odd[name][radii <= 0] == 0).all(), name
+
+
+@pytest.mark.parametrize("n", (2**20 - 1, 2**20, 2**20 + 1))
+def test_geometry_is_the_same_with_and_without_streaming_stores(n):
+    """Up to 2^20 - 1 Gaussians the forward's geometry is stored one way and beyond the other; radii and images of a scene whose
+    further Gaussians lie behind the camera do not depend on how many those are."""
+    from retinags_amd import GaussianRasterizationSettings, GaussianRasterizer
+    from retinags_amd.harness import scenes
+    cam = scenes.look_at_camera((0, 0, 0), (0, 0, 1), (0, -1, 0), 160, 120, 60.0).to(DEV)
+    settings = GaussianRasterizationSettings(
+        image_height=120, image_width=160, tanfovx=cam.tanfovx, tanfovy=cam.tanfovy, bg=torch.zeros(3, device=DEV), scale_modifier=1.0,
+        viewmatrix=cam.world_view_transform, projmatrix=cam.full_proj_transform, projmatrix_inv=cam.projection_matrix_inv,
+        range_low=torch.full((3,), -99.0, device=DEV), range_up=torch.full((3,), 99.0, device=DEV), sh_degree=3,
+        campos=cam.camera_center, prefiltered=False, debug=False)
+    scene = scenes.cube_scene(3000, seed=8)
+    few = dict(means3D=scene["xyz"], opacities=scene["opacity"], shs=scene["shs"], scales=scene["scales"] * 3, rotations=scene["rotations"])
+    few = {k: v.to(DEV) for k, v in few.items()}
+    many = {k: torch.cat((torch.ones(n - 3000, *v.shape[1:], device=DEV), v)) for k, v in few.items()}
+    many["means3D"][:n - 3000, 2] = -5.0
+    with torch.no_grad():
+        color, radii, depth, alpha = GaussianRasterizer(settings)(means2D=torch.zeros_like(few["means3D"]), **few)
+        color_m, radii_m, depth_m, alpha_m = GaussianRasterizer(settings)(means2D=torch.zeros_like(many["means3D"]), **many)
+    assert (radii > 0).sum() > 2000 and torch.equal(radii, radii_m[n - 3000:]) and (radii_m[:n - 3000] == 0).all()
+    assert torch.equal(color, color_m) and torch.equal(depth, depth_m) and torch.equal(alpha, alpha_m)
