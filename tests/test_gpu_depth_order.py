@@ -1,0 +1,52 @@
+"""The depth order's small kernels at the sizes where they change their way."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import orc, scenes
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("totals", (8191, 8192, 8193, 32767, 32768, 32769))   # of 256 each: from memory, through LDS, from memory again
+def test_scan_of_block_totals(totals):
+    from retinags_amd import _capi
+    n = 256 * totals - 3
+    x = np.random.default_rng(totals).integers(0, 50, size=n, dtype=np.uint32)
+    xi = torch.from_numpy(x.view(np.int32).copy()).to(DEV)
+    out = torch.empty_like(xi)
+    temp = torch.empty(_capi.lib.rgs_scan_temp_bytes(n), dtype=torch.uint8, device=DEV)
+    _capi.check(_capi.lib.rgs_inclusive_sum(_capi.ptr(xi), _capi.ptr(out), n, _capi.ptr(temp),
+                                            torch.cuda.current_stream(torch.device(DEV)).cuda_stream))
+    assert np.array_equal(out.cpu().numpy().view(np.uint32), orc.inclusive_sum(x))
+
+
+@pytest.mark.parametrize("n", (8 * 2**20, 8 * 2**20 + 1025))   # 8 192 groups of 1 024 Gaussians: the most of which all are looked at; more
+@pytest.mark.parametrize("spread", (1, 700, 2500))             # neighbours in memory, a few per group, one in some groups
+def test_groups_without_listed_gaussians(n, spread):
+    """3 000 Gaussians of a view among millions behind the camera, `spread` places apart, the last one at the very end: the same
+    images, bit for bit, as those 3 000 alone (ties in depth keep their order)."""
+    from retinags_amd import GaussianRasterizationSettings, GaussianRasterizer
+    cam = scenes.look_at_camera((0, 0, 0), (0, 0, 1), (0, -1, 0), 160, 120, 60.0).to(DEV)
+    settings = GaussianRasterizationSettings(
+        image_height=120, image_width=160, tanfovx=cam.tanfovx, tanfovy=cam.tanfovy, bg=torch.zeros(3, device=DEV), scale_modifier=1.0,
+        viewmatrix=cam.world_view_transform, projmatrix=cam.full_proj_transform, projmatrix_inv=cam.projection_matrix_inv,
+        range_low=torch.full((3,), -99.0, device=DEV), range_up=torch.full((3,), 99.0, device=DEV), sh_degree=0,
+        campos=cam.camera_center, prefiltered=False, debug=False)
+    scene = scenes.cube_scene(3000, seed=8)
+    scene["xyz"][1500:] = scene["xyz"][:1500]
+    few = dict(means3D=scene["xyz"], opacities=scene["opacity"], colors_precomp=torch.rand(3000, 3, generator=torch.Generator().manual_seed(2)),
+               scales=scene["scales"] * 3, rotations=scene["rotations"])
+    few = {k: v.to(DEV) for k, v in few.items()}
+    at = n - 1 - spread * torch.arange(2999, -1, -1, device=DEV)
+    many = {k: torch.ones(n, *v.shape[1:], device=DEV) for k, v in few.items()}
+    many["means3D"][:, 2] = -5.0
+    for k, v in few.items():
+        many[k][at] = v
+    with torch.no_grad():
+        want = GaussianRasterizer(settings)(means2D=torch.zeros_like(few["means3D"]), **few)
+        got = GaussianRasterizer(settings)(means2D=torch.zeros_like(many["means3D"]), **many)
+    assert (want[1] > 0).sum() > 2000 and torch.equal(want[1], got[1][at]) and int((got[1] > 0).sum()) == int((want[1] > 0).sum())
+    for k in (0, 2, 3):
+        assert torch.equal(want[k], got[k])
