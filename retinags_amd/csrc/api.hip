@@ -224,7 +224,7 @@ struct Carver {
 
 // Scratch of the depth sort of the Gaussians, inside the geometry workspace.
 struct OrderScratch {
-	size_t keys_a, keys_b, vals_a, vals_b, tiles_in_order, sort_temp, scan_temp, dup_first, tile_digits, total;
+	size_t keys_a, keys_b, vals_a, vals_b, tiles_in_order, digits, sort_temp, scan_temp, dup_first, total;
 };
 
 OrderScratch order_scratch(size_t P)
@@ -236,10 +236,10 @@ OrderScratch order_scratch(size_t P)
 	o.vals_a = c.take(4 * P);
 	o.vals_b = c.take(4 * P);
 	o.tiles_in_order = c.take(4 * P);
-	o.sort_temp = c.take(4 * rgs::sort_temp_words(P));
+	o.digits = c.take(4 * rgs::kDigitCopies * rgs::kDigitWords);
+	o.sort_temp = c.take(4 * rgs::sort_temp_words(P));  // right behind the counts: both are cleared in one go
 	o.scan_temp = c.take(4 * rgs::scan_temp_words(P));
 	o.dup_first = c.take(4 * rgs::dup_first_words(P));
-	o.tile_digits = c.take(4 * rgs::kTileDigitWords);
 	o.total = c.cursor;
 	return o;
 }
@@ -565,8 +565,8 @@ static int forward_geom(bool wait_for_count, void* count_ready_event, const char
 		a.sh_rows_by_16_bytes = sh_rows_by_16_bytes(c.shs, c.M, c.D);
 		const OrderScratch o = order_scratch((size_t)c.P);
 		char* scratch = at<char>(ws, off[RGS_GEOM_ORDER_SCRATCH]);
-		a.clear = at<uint32_t>(scratch, o.sort_temp);
-		a.clear_words = rgs::depth_sort_clear_words((size_t)c.P);
+		a.clear = at<uint32_t>(scratch, o.digits);
+		a.clear_words = (o.sort_temp - o.digits) / 4 + rgs::depth_sort_clear_words((size_t)c.P);
 
 		totals[(size_t)k] = rgs::TotalsJob{a.block_sums, a.block_visible, c.P, at<uint32_t>(ws, off[RGS_GEOM_TOTAL]),
 		                                   frame_counts + k, at<uint32_t>(ws, off[RGS_GEOM_VISIBLE_COUNT])};
@@ -581,7 +581,7 @@ static int forward_geom(bool wait_for_count, void* count_ready_event, const char
 		d.offsets_in_order = at<uint32_t>(ws, off[RGS_GEOM_POINT_OFFSETS]);
 		d.sort_temp = at<uint32_t>(scratch, o.sort_temp); d.scan_temp = at<uint32_t>(scratch, o.scan_temp);
 		d.dup_first = at<uint32_t>(scratch, o.dup_first);
-		d.tile_digits = at<uint32_t>(scratch, o.tile_digits);
+		d.digits = at<uint32_t>(scratch, o.digits);
 	}
 	rgs::launch_preprocess_forward(pre.data(), K, s);
 	RGS_STAGE("preprocess");
@@ -769,16 +769,17 @@ int forward_binning(const char* who, bool count_on_device, int K, const RasterCa
 		d.clear = temp; d.clear_words = rgs::sort_clear_words((size_t)R, end_bit, rgs::sort_max_digit_bits_u32(end_bit));
 		// it also clears the tile ranges (and the counters and totals behind them) and counts the digits of the tiles
 		// it writes, so the sort starts with its passes
-		uint32_t* tile_digits = at<uint32_t>(at<char>(c.geom_ws, goff[RGS_GEOM_ORDER_SCRATCH]), order_scratch((size_t)P).tile_digits);
-		d.tile_digits = tile_digits; d.end_bit = end_bit;
+		uint32_t* tile_digits = at<uint32_t>(at<char>(c.geom_ws, goff[RGS_GEOM_ORDER_SCRATCH]), order_scratch((size_t)P).digits);
+		const uint32_t digit_copies = rgs::digit_copies(((size_t)R + rgs::kDupPositions - 1) / rgs::kDupPositions);
+		d.tile_digits = tile_digits; d.digit_copies = digit_copies; d.end_bit = end_bit;
 		d.also_clear = reinterpret_cast<uint32_t*>(ranges); d.also_clear_words = clear_words;
 		dups.push_back(d);
 		rgs::SortJob<uint32_t> sj = {};
 		sj.keys_in = keys_a; sj.keys_out = keys_b; sj.vals_in = vals_a; sj.vals_out = vals_b;
-		sj.n = (size_t)R; sj.n_device = count; sj.temp = temp; sj.digit_counts = tile_digits;
+		sj.n = (size_t)R; sj.n_device = count; sj.temp = temp; sj.digit_counts = tile_digits; sj.digit_copies = digit_copies;
 		sorts.push_back(sj);
 		ranges_jobs.push_back(rgs::TileRangesJob{a.tile_keys, (size_t)R, count, ranges, a.sort_status, a.order_status, fault,
-		                                         at<uint4>(c.binning_ws, b.file_tail), tile_digits});
+		                                         at<uint4>(c.binning_ws, b.file_tail), tile_digits, digit_copies * (uint32_t)rgs::kDigitWords});
 		with_instances.push_back(k);
 	}
 	if (with_instances.empty())

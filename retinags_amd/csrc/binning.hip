@@ -284,8 +284,8 @@ __host__ __device__ inline uint32_t depth_index_bits(uint32_t P)
 // (depth key, index and tile count) pairs of the Gaussians that touch a tile, compacted in index order: the
 // group of Gaussians [kScanGroup b, kScanGroup (b + 1)), four neighbouring ones per thread, is written
 // from visible_base[4 b] on (the bases are per 256 Gaussians).  A workgroup takes every gridDim.x-th group and
-// counts the digits of the keys it writes on the way: at the end it adds its counts to the digit histograms
-// the sort of these pairs starts from (cleared beforehand), which saves that sort its own pass over the keys.
+// counts the digits of the keys it writes on the way: at the end it adds its counts to a copy of the digit counts
+// the sort of these pairs starts from (see kDigitCopies; cleared beforehand), which saves that sort its own pass over the keys.
 __global__ __launch_bounds__(256) void depth_pairs_kernel(Batch<DepthOrderJob> batch)
 {
 	__shared__ uint32_t lds[8];
@@ -311,7 +311,7 @@ __global__ __launch_bounds__(256) void depth_pairs_kernel(Batch<DepthOrderJob> b
 	__syncthreads();
 	uint32_t written = 0;
 	// How many of a group's Gaussians are listed is known ahead of it.  Where neighbours in memory are neighbours in the scene most
-	// groups have none (a city stored along a space-filling curve, 5 % in view: 39.5 -> 29 us; 62.9 M Gaussians in random order 124 -> 101), so a workgroup with many groups
+	// groups have none (a city stored along a space-filling curve, 5 % in view: 39.5 -> 29 us; 62.9 M Gaussians in random order 124 -> 101; both before the digit counts had copies), so a workgroup with many groups
 	// looks for those that have some, 64 at a time; one with few would only wait for the answer.
 	const size_t blocks = (P + 255) / 256, groups = (P + kScanGroup - 1) / kScanGroup;
 	const bool many = groups > 4 * (size_t)gridDim.x;
@@ -369,13 +369,14 @@ __global__ __launch_bounds__(256) void depth_pairs_kernel(Batch<DepthOrderJob> b
 	}
 	}
 	__syncthreads();
+	uint32_t* digits = j.digits + (blockIdx.x & (j.digit_copies - 1u)) * kDigitWords;
 #pragma unroll
 	for (int p = 0; p < kDepthPasses; p++)
 #pragma unroll
 		for (int h = 0; h < 2; h++) {
 			const uint32_t c = s_hist[p][256 * h + threadIdx.x];
 			if (c)
-				atomicAdd(&j.sort_temp[512 * p + 256 * h + threadIdx.x], c);
+				atomicAdd(&digits[512 * p + 256 * h + threadIdx.x], c);
 		}
 	// the digit of the pass on demand: value 0 takes every key that was not counted under another value
 	uint32_t all_written;
@@ -391,7 +392,7 @@ __global__ __launch_bounds__(256) void depth_pairs_kernel(Batch<DepthOrderJob> b
 				atomicOr(&j.sort_temp[kSortExtraPass], 1u);
 		}
 		if (c)
-			atomicAdd(&j.sort_temp[512 * kDepthPasses + threadIdx.x], c);
+			atomicAdd(&digits[512 * kDepthPasses + threadIdx.x], c);
 	}
 }
 
@@ -401,9 +402,9 @@ __global__ __launch_bounds__(256) void order_totals_kernel(Batch<DepthOrderJob> 
 {
 	__shared__ uint32_t lds[8];
 	const DepthOrderJob& j = batch.job[blockIdx.y];
-	if (blockIdx.x == 0)  // what the key duplication will count the digits of its tiles into
-		for (int w = threadIdx.x; w < kTileDigitWords; w += 256)
-			j.tile_digits[w] = 0u;
+	// what the key duplication will count the digits of its tiles into
+	for (int w = (int)(blockIdx.x * 256 + threadIdx.x); w < (int)j.digit_copies * kDigitWords / 4; w += (int)gridDim.x * 256)
+		reinterpret_cast<uint4*>(j.digits)[w] = uint4{0u, 0u, 0u, 0u};
 	const size_t n = min((size_t)*j.visible_count, (size_t)j.P);
 	if ((size_t)blockIdx.x * kScanGroup >= n)
 		return;
@@ -457,6 +458,7 @@ __global__ __launch_bounds__(256) void duplicate_with_keys_kernel(Batch<Duplicat
 {
 	__shared__ DuplicateStage st;
 	__shared__ uint32_t s_first;
+	constexpr int kTileDigitWords = 3 * 512;  // tiles have at most 24 bits: three passes at most
 	__shared__ uint32_t s_digits[kTileDigitWords];  // digit counts of the tiles this workgroup writes
 	extern __shared__ __align__(16) float s_ndc[];  // NDC of every tile column's first and last pixel, then of every strip's first and last row
 	const DuplicateJob& job = batch.job[blockIdx.y];
@@ -662,7 +664,7 @@ __global__ __launch_bounds__(256) void duplicate_with_keys_kernel(Batch<Duplicat
 	for (int w = tid; w < 512 * passes; w += 256) {
 		const uint32_t c = s_digits[w];
 		if (c)
-			atomicAdd(&job.tile_digits[w], c);
+			atomicAdd(&job.tile_digits[(blockIdx.x & (job.digit_copies - 1u)) * kDigitWords + w], c);
 	}
 }
 
@@ -683,8 +685,9 @@ void launch_duplicate_with_keys(const DuplicateJob* jobs, int count, int grid_x,
 			blocks = need > blocks ? need : blocks;
 		}
 		// every workgroup ends with an atomic add per digit into its job's counts: enough of them to fill the GPU several
-		// times over, each over many runs of positions, rather than one per run
-		const size_t most = nj >= 8 ? 512 : nj >= 4 ? 4096 / (size_t)nj : 1024;  // twice and four times as many were measured slower
+		// times over, each over many runs of positions, rather than one per run.  (Half and twice as many: 16.6 and 14.9 us for 12.4 at
+		// 100 000 Gaussians, 44 and 50 for 45 in the city, 691 and 595 for 610 in the scene of 62.9 M.)
+		const size_t most = nj >= 8 ? 512 : nj >= 4 ? 4096 / (size_t)nj : 1024;
 		blocks = blocks < most ? blocks : most;
 		hipLaunchKernelGGL(duplicate_with_keys_kernel, dim3((unsigned)blocks, (unsigned)nj), dim3(256),
 		                   ndc_in_lds ? table * sizeof(float) : 0, s, b, grid_x, grid_y, ndc_in_lds);
@@ -704,7 +707,7 @@ void launch_duplicate_with_keys(const DuplicateJob* jobs, int count, int grid_x,
 // pairs fill the LDS.
 //
 // Scratch layout (u32 words), B = 2^kBits:
-//   [0, 2048)      digit histograms, B words per pass (every block of a pass scans its counts itself)
+//   [0, 2048)      digit histograms, B words per pass, where the job names no digit_counts (every block of a pass scans its counts itself)
 //   [2048, 2056)   tile counter of each pass
 //   [2056]         status: non-zero if a look-back ever gave up waiting (never expected)
 //   [2057]         depth sort only: non-zero if its pass on demand is needed (kSortExtraPass)
@@ -853,7 +856,11 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 	// asked for before anything else: needed only after the look-back, by when it has long arrived
 	const bool owns = tid < kBins;
-	const uint32_t digit_total = owns ? digit_count[tid] : 0u;
+	uint32_t digit_total = owns ? digit_count[tid] : 0u;
+	if (owns && j.digit_copies > 1u)
+#pragma unroll
+		for (int c = 1; c < kDigitCopies; c++)
+			digit_total += digit_count[c * kDigitWords + tid];
 	// Tiles are handed out in arrival order, so every tile a block waits for below belongs to
 	// a block that is already running.
 	if (tid == 0)
@@ -1184,12 +1191,18 @@ void launch_depth_order(const DepthOrderJob* jobs, int count, hipStream_t s)
 			pairs += (size_t)jobs[at + k].P;
 		}
 		const bool few_groups = ((size_t)max_p + kScanGroup - 1) / kScanGroup <= 4096;
+		const dim3 grid((unsigned)((max_p + kScanGroup - 1) / kScanGroup), (unsigned)nj);
+		// few workgroups per job, each over many groups: every one ends with an atomic add per digit into its job's counts (half and twice
+		// as many: 17 and 27 us for 20 at two submodels of 2.8 M, 105 and 94 for 99 at four of 15.7 M)
+		const unsigned most = nj >= 8 ? 256u : 2048u / (unsigned)nj;
+		const dim3 pairs_grid(grid.x < most ? grid.x : most, (unsigned)nj);
 		for (int k = 0; k < nj; k++) {
-			const DepthOrderJob& j = jobs[at + k];
-			b.job[k] = j;
+			DepthOrderJob& j = b.job[k];
+			j = jobs[at + k];
+			j.digit_copies = digit_copies(pairs_grid.x);
 			SortJob<uint32_t>& sj = sorts.job[k];
 			sj.keys_in = j.keys_a; sj.keys_out = j.keys_b; sj.vals_in = j.vals_a; sj.vals_out = j.vals_b;
-			sj.n = (size_t)j.P; sj.n_device = j.visible_count; sj.temp = j.sort_temp;
+			sj.n = (size_t)j.P; sj.n_device = j.visible_count; sj.temp = j.sort_temp; sj.digit_counts = j.digits; sj.digit_copies = j.digit_copies;
 			sj.final_index = j.order; sj.final_count = j.tiles_in_order; sj.count_of = j.tiles_touched;
 			sj.index_bits = depth_index_bits((uint32_t)j.P); sj.in_size = (uint32_t)j.P;
 			scan.job[k] = BlockScanJob{j.scan_temp, ((size_t)j.P + kScanGroup - 1) / kScanGroup, j.visible_count, (uint32_t)kScanGroup, nullptr, nullptr,
@@ -1197,10 +1210,7 @@ void launch_depth_order(const DepthOrderJob* jobs, int count, hipStream_t s)
 			inc.job[k] = BlockInclusiveJob{j.tiles_in_order, j.scan_temp, (size_t)j.P, j.visible_count, j.offsets_in_order, j.dup_first,
 			                               (uint32_t)dup_first_words((size_t)j.P), few_groups ? 1u : 0u};
 		}
-		const dim3 grid((unsigned)((max_p + kScanGroup - 1) / kScanGroup), (unsigned)nj);
-		// few workgroups per job, each over many groups: every one ends with an atomic add per digit into its job's counts
-		const unsigned most = nj >= 8 ? 256u : 2048u / (unsigned)nj;
-		hipLaunchKernelGGL(depth_pairs_kernel, dim3(grid.x < most ? grid.x : most, (unsigned)nj), dim3(256), 0, s, b);
+		hipLaunchKernelGGL(depth_pairs_kernel, pairs_grid, dim3(256), 0, s, b);
 		// three passes of nine bits (a -> b -> a -> the order and the tile counts in that order), and the pass on demand
 		launch_sort_pass<uint32_t, 9, kPassPlain>(sorts, (size_t)max_p, pairs, nj, 0, 0, 511u, s);
 		launch_sort_pass<uint32_t, 9, kPassPlain>(sorts, (size_t)max_p, pairs, nj, 1, 9, 511u, s);
@@ -1298,9 +1308,12 @@ __global__ __launch_bounds__(kFileBlock) void tile_ranges_kernel(Batch<TileRange
 	const size_t first = (size_t)blockIdx.x * kFileGroup;
 	if (first >= j.n)
 		return;  // the launch is sized for the job with the most keys
-	if (blockIdx.x == 0 && j.rezero)  // the sort has read its digit counts: zero again for the next to count into them
-		for (int w = threadIdx.x; w < kTileDigitWords; w += kFileBlock)
+	// the sort has read its digit counts: zero again for the next to count into them
+	if (j.rezero) {
+		const size_t threads = (j.n + kFileGroup - 1) / kFileGroup * kFileBlock;
+		for (size_t w = (size_t)blockIdx.x * kFileBlock + threadIdx.x; w < (size_t)j.rezero_words; w += threads)
 			j.rezero[w] = 0u;
+	}
 	if ((sort_status && *sort_status != 0u) || (order_status && *order_status != 0u)) {
 		if (blockIdx.x == 0 && threadIdx.x == 0 && fault)
 			__hip_atomic_store(fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);

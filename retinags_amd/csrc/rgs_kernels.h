@@ -341,11 +341,20 @@ struct TotalsJob {
 };
 void launch_totals_from_block_sums(const TotalsJob* jobs, int count, hipStream_t s);
 // Depth order of the Gaussians that touch a tile.  block_visible holds the exclusive scan of
-// their count per 256 Gaussians and *visible_count the total; sort_temp has been cleared
-// (sort_clear_words(P, 32) words).  On return order[0..count)
+// their count per 256 Gaussians and *visible_count the total; sort_temp (sort_clear_words(P, 32) words) and
+// digits have been cleared.  On return order[0..count)
 // lists them by increasing depth, ties by index, and offsets_in_order is the inclusive scan of
 // their tile counts in that order.  The count stays on the device: every kernel is launched
 // for P elements and reads it.
+// The counts that a 32-bit sort starts from are made by the kernel that writes its keys: word 512 p + d of kDigitWords counts the keys whose
+// digit p is d.  Additions to one word take about 12 ns each whoever makes them, and every workgroup of that kernel ends with one to almost
+// every word: a thousand workgroups that end together wait 12 us.  So the counts lie in memory kDigitCopies times, a workgroup adds to the
+// copy of its number, and the sort adds the copies up (0.2 us per launch).  With 1, 4, 8 and 16 copies the key duplication takes 27.0, 14.2,
+// 12.8 and 12.4 us at 100 000 Gaussians and 77, 45, 45 and 45 for three submodels of a city; with 1 and 8 the listing of pairs 39 and 15 us
+// there, 36 and 20 for two submodels of 2.8 M each.  Up to 128 workgroups (4 000 Gaussians: 4) one copy is the faster.
+constexpr int kDigitWords = 4 * 512;  // keys have at most four digits
+constexpr int kDigitCopies = 8;
+constexpr uint32_t digit_copies(size_t workgroups) { return workgroups > 128 ? kDigitCopies : 1; }
 struct DepthOrderJob {
 	int P;
 	const float* depths;
@@ -362,7 +371,8 @@ struct DepthOrderJob {
 	uint32_t* sort_temp;
 	uint32_t* scan_temp;
 	uint32_t* dup_first;       // dup_first_words(P) words: see launch_duplicate_with_keys
-	uint32_t* tile_digits;     // kTileDigitWords words, left zero: see DuplicateJob
+	uint32_t* digits;          // kDigitCopies x kDigitWords words, zero beforehand and left zero: see also DuplicateJob
+	uint32_t digit_copies;     // how many of the copies the launch uses: it sets this itself
 };
 void launch_depth_order(const DepthOrderJob* jobs, int count, hipStream_t s);
 // Also sets clear[0..clear_words) to zero (the scratch of the sort that follows).  Instances whose
@@ -377,9 +387,8 @@ constexpr int kDupPositions = 256;
 constexpr size_t dup_first_words(size_t P) { return P / 16 + 2; }
 // The key duplication also counts the digits of the tiles it writes, which is what the sort of its keys starts
 // from: counts[512 p + d] = keys whose digit p of the tile bits (sort_digit_shift / sort_digit_bits with
-// sort_max_digit_bits_u32(end_bit)) is d, in kTileDigitWords words that are zero when it starts (the depth order leaves them so, and so does the
+// sort_max_digit_bits_u32(end_bit)) is d, in kDigitWords words that are zero when it starts (the depth order leaves them so, and so does the
 // tile-range kernel, the last to run after they were read).
-constexpr int kTileDigitWords = 3 * 512;  // tiles have at most 24 bits: three passes at most
 struct DuplicateJob {
 	int P;
 	const uint32_t* visible_count;
@@ -387,7 +396,8 @@ struct DuplicateJob {
 	const uint32_t* offsets;   // inclusive, in depth order
 	const uint32_t* total;     // the last of them
 	const uint32_t* first_of_block;  // dup_first_words(P) words
-	uint32_t* tile_digits;     // kTileDigitWords words, zero beforehand
+	uint32_t* tile_digits;     // kDigitCopies x kDigitWords words, zero beforehand
+	uint32_t digit_copies;     // how many of the copies are used: digit_copies(its workgroups)
 	int end_bit;               // bits of the tile the sort will look at
 	uint32_t* also_clear;      // a second array to clear (the tile ranges and what lies behind them)
 	size_t also_clear_words;
@@ -430,7 +440,8 @@ struct SortJob {
 	uint32_t* temp;
 	uint32_t* also_clear;
 	size_t also_clear_words;
-	const uint32_t* digit_counts;  // null: the counts are at the start of temp
+	const uint32_t* digit_counts;  // digit_copies x kDigitWords words; null: the counts are at the start of temp, once
+	uint32_t digit_copies;
 	// Only for the passes that end the depth sort (launch_depth_order): the values are a Gaussian's index in the low
 	// index_bits bits and above them its tile count (all ones: too large to fit, look it up in count_of); the last pass
 	// writes index and count apart, to final_index and final_count, instead of keys and values.
@@ -467,7 +478,8 @@ struct TileRangesJob {
 	const uint32_t* order_status;
 	uint32_t* fault;
 	uint4* file_tail;
-	uint32_t* rezero;  // may be null: kTileDigitWords words set to zero (the digit counts the sort has read)
+	uint32_t* rezero;  // may be null: rezero_words words set to zero (the digit counts the sort has read)
+	uint32_t rezero_words;
 };
 void launch_tile_ranges(const TileRangesJob* jobs, int count, hipStream_t s);
 

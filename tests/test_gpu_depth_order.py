@@ -22,18 +22,51 @@ def test_scan_of_block_totals(totals):
     assert np.array_equal(out.cpu().numpy().view(np.uint32), orc.inclusive_sum(x))
 
 
+def _view(width, height):
+    from retinags_amd import GaussianRasterizationSettings, GaussianRasterizer
+    cam = scenes.look_at_camera((0, 0, 0), (0, 0, 1), (0, -1, 0), width, height, 60.0).to(DEV)
+    return GaussianRasterizer(GaussianRasterizationSettings(
+        image_height=height, image_width=width, tanfovx=cam.tanfovx, tanfovy=cam.tanfovy, bg=torch.zeros(3, device=DEV), scale_modifier=1.0,
+        viewmatrix=cam.world_view_transform, projmatrix=cam.full_proj_transform, projmatrix_inv=cam.projection_matrix_inv,
+        range_low=torch.full((3,), -99.0, device=DEV), range_up=torch.full((3,), 99.0, device=DEV), sh_degree=0,
+        campos=cam.camera_center, prefiltered=False, debug=False))
+
+
+def test_copies_of_the_digit_counts():
+    """The counts a sort starts from lie in memory once for up to 128 workgroups of the kernel that makes them and several times
+    for more: Gaussians behind the camera take the depth order from one to the other (131 072 and 131 073 of them), bounds for
+    the instances the key duplication (32 768 and 32 769 positions).  The images stay the same, bit for bit."""
+    rasterizer = _view(320, 200)
+    scene = scenes.cube_scene(6000, seed=4)
+    scene["xyz"][3000:] = scene["xyz"][:3000]
+    colors = torch.rand(6000, 3, generator=torch.Generator().manual_seed(2))
+    kw = {k: v.to(DEV) for k, v in dict(means3D=scene["xyz"], opacities=scene["opacity"], colors_precomp=colors,
+                                        scales=scene["scales"], rotations=scene["rotations"]).items()}
+
+    def run(n, bound):
+        padded = {k: torch.cat((v, torch.ones(n - 6000, *v.shape[1:], device=DEV))) for k, v in kw.items()}
+        padded["means3D"][6000:, 2] = -5.0
+        with torch.no_grad():
+            stage = rasterizer.enqueue_geometry(**padded, **({} if bound is None else {"instance_bound": bound}))
+            out = rasterizer(means2D=torch.zeros_like(padded["means3D"]), geometry=stage, **padded)
+            again = rasterizer(means2D=torch.zeros_like(padded["means3D"]), **padded)
+        assert all(torch.equal(a, b) for a, b in zip(out, again))
+        return stage.instances(), out
+
+    instances, want = run(6000, None)
+    assert 5000 < instances <= 32767 and want[0].max() > 0
+    for n, bound in ((131072, None), (131073, None), (6000, 32768), (6000, 32769), (131073, 32767), (131072, 100000), (400001, 3000001)):
+        count, got = run(n, bound)
+        assert count == instances and torch.equal(got[1][:6000], want[1])
+        assert all(torch.equal(got[k], want[k]) for k in (0, 2, 3)), (n, bound)
+
+
 @pytest.mark.parametrize("n", (8 * 2**20, 8 * 2**20 + 1025))   # 8 192 groups of 1 024 Gaussians: the most of which all are looked at; more
 @pytest.mark.parametrize("spread", (1, 700, 2500))             # neighbours in memory, a few per group, one in some groups
 def test_groups_without_listed_gaussians(n, spread):
     """3 000 Gaussians of a view among millions behind the camera, `spread` places apart, the last one at the very end: the same
     images, bit for bit, as those 3 000 alone (ties in depth keep their order)."""
-    from retinags_amd import GaussianRasterizationSettings, GaussianRasterizer
-    cam = scenes.look_at_camera((0, 0, 0), (0, 0, 1), (0, -1, 0), 160, 120, 60.0).to(DEV)
-    settings = GaussianRasterizationSettings(
-        image_height=120, image_width=160, tanfovx=cam.tanfovx, tanfovy=cam.tanfovy, bg=torch.zeros(3, device=DEV), scale_modifier=1.0,
-        viewmatrix=cam.world_view_transform, projmatrix=cam.full_proj_transform, projmatrix_inv=cam.projection_matrix_inv,
-        range_low=torch.full((3,), -99.0, device=DEV), range_up=torch.full((3,), 99.0, device=DEV), sh_degree=0,
-        campos=cam.camera_center, prefiltered=False, debug=False)
+    rasterizer = _view(160, 120)
     scene = scenes.cube_scene(3000, seed=8)
     scene["xyz"][1500:] = scene["xyz"][:1500]
     few = dict(means3D=scene["xyz"], opacities=scene["opacity"], colors_precomp=torch.rand(3000, 3, generator=torch.Generator().manual_seed(2)),
@@ -45,8 +78,8 @@ def test_groups_without_listed_gaussians(n, spread):
     for k, v in few.items():
         many[k][at] = v
     with torch.no_grad():
-        want = GaussianRasterizer(settings)(means2D=torch.zeros_like(few["means3D"]), **few)
-        got = GaussianRasterizer(settings)(means2D=torch.zeros_like(many["means3D"]), **many)
+        want = rasterizer(means2D=torch.zeros_like(few["means3D"]), **few)
+        got = rasterizer(means2D=torch.zeros_like(many["means3D"]), **many)
     assert (want[1] > 0).sum() > 2000 and torch.equal(want[1], got[1][at]) and int((got[1] > 0).sum()) == int((want[1] > 0).sum())
     for k in (0, 2, 3):
         assert torch.equal(want[k], got[k])
