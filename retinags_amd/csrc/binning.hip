@@ -813,7 +813,10 @@ struct SortCounts {
 
 // How many wavefronts stand by to fill the gaps of the others' phases (loads, ranking, look-back, stores) and how long the runs are
 // that a tile writes set the pace of a pass: sixteen wavefronts per tile, 32 per CU with up to eight pairs per lane (64
-// registers; the counts of the ranking lie where the tile's keys go afterwards), 16 with sixteen.
+// registers; the counts of the ranking lie where the tile's keys go afterwards), 16 with sixteen.  A lane keeps three registers per pair
+// from phase to phase (key, value, rank): with the parts of the ranks and the digits' addresses kept too, eight pairs per lane spilled
+// to memory, ahead of the ranking, and sixteen took 119 registers instead of 89 (per pass, us: instances of two submodels of 2.8 M
+// 64 -> 58, of two at 5185x3359 378 -> 328, of one of 2.8 M in training 45 -> 42, its depths 20 -> 17).
 template <typename KeyT, int kBits, int kKind, int kItems>
 __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(sizeof(KeyT) == 4 && kItems <= 8 ? 8 : 4))) void sort_onesweep_kernel(
 	Batch<SortJob<KeyT>> batch, int pass, int shift, uint32_t mask, int spin_limit)
@@ -829,8 +832,14 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 	uint32_t* __restrict__ vals_out = (pass & 1) ? j.vals_in : j.vals_out;
 	const uint32_t* __restrict__ n_device = j.n_device;
 	const size_t job_tiles = (j.n + kBlock - 1) / kBlock;
-	if (blockIdx.x >= job_tiles)
-		return;  // the launch is sized for the job with the most tiles
+	uint32_t n = (uint32_t)j.n;  // (fewer than 2^30: the look-back words hold no more)
+	if (n_device)  // (no kernel writes it meanwhile: read by the scalar unit)
+		n = (uint32_t)min(j.n, (size_t)*(const __attribute__((address_space(4))) uint32_t*)(uintptr_t)n_device);
+	// The launch is sized for the job with the most tiles, and for an upper bound of n: as many workgroups take a tile as there are
+	// tiles, the others leave at once.  (Most of a depth sort's, which is launched for all Gaussians: 25 -> 22 us per pass for three
+	// submodels of a city, a twentieth of 27 M in view, when they no longer took a ticket first.)
+	if (blockIdx.x >= (n + (uint32_t)kBlock - 1u) / (uint32_t)kBlock)
+		return;
 	bool ends_here = false;
 	if (kKind != kPassPlain) {
 		const bool extra = j.temp[kSortExtraPass] != 0u;
@@ -854,13 +863,7 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 	__shared__ uint32_t s_tile;
 
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-	// asked for before anything else: needed only after the look-back, by when it has long arrived
 	const bool owns = tid < kBins;
-	uint32_t digit_total = owns ? digit_count[tid] : 0u;
-	if (owns && j.digit_copies > 1u)
-#pragma unroll
-		for (int c = 1; c < kDigitCopies; c++)
-			digit_total += digit_count[c * kDigitWords + tid];
 	// Tiles are handed out in arrival order, so every tile a block waits for below belongs to
 	// a block that is already running.
 	if (tid == 0)
@@ -871,30 +874,33 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 	__syncthreads();
 	const uint32_t tile = s_tile;
 	const uint32_t block_base = tile * (uint32_t)kBlock;
-	uint32_t n = (uint32_t)j.n;  // (fewer than 2^30: the look-back words hold no more)
-	if (n_device)
-		n = (uint32_t)min(j.n, (size_t)*n_device);
-	// launched for an upper bound of n: tiles beyond the data leave, and no tile waits for them
-	if (block_base >= n)
-		return;
 	const uint32_t wave_base = block_base + (uint32_t)wave * (kItems * 64);
 
 	KeyT key[kItems];
 	uint32_t val[kItems];
 	uint32_t rank[kItems];
+	// Behind the data a tile is filled up with keys of ones: the last digit value, and after every pair in the tile that has it.
+	if (block_base + (uint32_t)kBlock <= n) {
+		const KeyT* const keys_at = keys_in + wave_base;
+		const uint32_t* const vals_at = vals_in + wave_base;
 #pragma unroll
-	for (int i = 0; i < kItems; i++) {
-		const uint32_t k = wave_base + (uint32_t)(i * 64 + lane);
-		const bool ok = k < n;
-		key[i] = ok ? keys_in[k] : (KeyT)~(KeyT)0;
-		val[i] = ok ? vals_in[k] : 0u;
+		for (int i = 0; i < kItems; i++) {
+			key[i] = keys_at[i * 64 + lane];
+			val[i] = vals_at[i * 64 + lane];
+		}
+	} else {
+#pragma unroll
+		for (int i = 0; i < kItems; i++) {
+			const uint32_t k = wave_base + (uint32_t)(i * 64 + lane);
+			const bool ok = k < n;
+			key[i] = ok ? keys_in[k] : (KeyT)~(KeyT)0;
+			val[i] = ok ? vals_in[k] : 0u;
+		}
 	}
 
 #pragma unroll
 	for (int i = 0; i < kItems; i++) {
-		const uint32_t k = wave_base + (uint32_t)(i * 64 + lane);
-		// Padding elements rank as the last digit value after every real element, so they never disturb one.
-		const uint32_t d = (k < n) ? digit_of(key[i], shift, mask) : (uint32_t)(kBins - 1);
+		const uint32_t d = digit_of(key[i], shift, mask);
 		// The lanes with this lane's digit: a vote per bit, taken as it is or inverted by a mask made of the lane's own bit, four vector
 		// instructions per bit instead of nine (which kept the SIMDs busy for 60 % of a pass: 78 -> 71 us for the instances of
 		// 5.6 M Gaussians at 1600x1036).
@@ -915,13 +921,24 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 		if (below == 0u)
 			wave_hist[wave][d] = (uint16_t)(prior + (uint32_t)__popc(same_lo) + (uint32_t)__popc(same_hi));
 		rank[i] = prior + below;
+		asm volatile("" : "+v"(rank[i]), "+v"(key[i]));  // (the sum is made here, and the digit taken from the key again later)
 		__builtin_amdgcn_wave_barrier();
+	}
+	// the counts of the thread's digit value in all tiles, needed once this tile's are published
+	uint32_t totals[kDigitCopies] = {};
+	if (owns) {
+		totals[0] = digit_count[tid];
+		if (j.digit_copies > 1u)
+#pragma unroll
+			for (int c = 1; c < kDigitCopies; c++)
+				totals[c] = digit_count[c * kDigitWords + tid];
 	}
 	__syncthreads();
 
 	// A thread owns a digit value: prefix over the waves, publish the tile's count.
 	const uint32_t valid = min(n - block_base, (uint32_t)kBlock);
-	uint32_t* const my_word = lookback + (size_t)tile * kBins + tid;
+	// (by its distance in bytes, below 2^32: an address of 64 bits takes its registers through the whole kernel)
+	auto word_of = [&](uint32_t t) { return reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(lookback) + (t * (uint32_t)kBins + (uint32_t)tid) * 4u); };
 	uint32_t count = 0, digit_start;
 	{
 		if (owns) {
@@ -939,12 +956,15 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 		const uint32_t ex = block_exclusive_scan_u32<kWaves>(count, s_scan, total);
 		if (owns)
 			sc.digit_base[tid] = (uint16_t)ex;
-		if (tid == kBins - 1)
-			count -= (uint32_t)kBlock - valid;  // padding is not published
+		if ((uint32_t)tid == mask)
+			count -= (uint32_t)kBlock - valid;  // what fills the tile up is not published
 		if (owns)
-			__hip_atomic_store(my_word, count | (tile == 0 ? kFlagInclusive : kFlagAggregate), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+			__hip_atomic_store(word_of(tile), count | (tile == 0 ? kFlagInclusive : kFlagAggregate), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 		// where the digit's run starts in the whole array: the exclusive scan of the digit counts
-		uint32_t all;
+		uint32_t all, digit_total = 0;
+#pragma unroll
+		for (int c = 0; c < kDigitCopies; c++)
+			digit_total += totals[c];
 		digit_start = block_exclusive_scan_u32<kWaves>(digit_total, s_scan, all);
 	}
 
@@ -952,8 +972,7 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 	// the look-back below starts, more of them have finished theirs and it has fewer words to read.
 #pragma unroll
 	for (int i = 0; i < kItems; i++) {
-		const uint32_t k = wave_base + (uint32_t)(i * 64 + lane);
-		const uint32_t d = (k < n) ? digit_of(key[i], shift, mask) : (uint32_t)(kBins - 1);
+		const uint32_t d = digit_of(key[i], shift, mask);
 		rank[i] += (uint32_t)sc.digit_base[d] + (uint32_t)wave_hist[wave][d];
 	}
 	__syncthreads();  // the counts have been read
@@ -986,7 +1005,7 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 				uint32_t v[kLookBatch];
 #pragma unroll
 				for (int q = 0; q < kLookBatch; q++)
-					v[q] = (uint32_t)q < t ? __hip_atomic_load(lookback + (size_t)(t - 1u - (uint32_t)q) * kBins + tid, __ATOMIC_RELAXED,
+					v[q] = (uint32_t)q < t ? __hip_atomic_load(word_of(t - 1u - (uint32_t)q), __ATOMIC_RELAXED,
 					                                           __HIP_MEMORY_SCOPE_AGENT)
 					                       : kFlagInclusive;  // below the first tile there is nothing
 				uint32_t used = 0;
@@ -1004,7 +1023,7 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 					done = true;
 				if (!done && used < (uint32_t)kLookBatch) {
 					// tile t - 1 has not published yet: wait for its word, then look again from there
-					const uint32_t* word = lookback + (size_t)(t - 1u) * kBins + tid;
+					const uint32_t* word = word_of(t - 1u);
 					uint32_t w = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 					for (int spins = 0; (w >> 30) == 0u; spins++) {
 						// give up after a bounded wait, or as soon as any other look-back has
@@ -1023,7 +1042,7 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 				atomicOr(status, 1u);
 			// On the (never expected) give-up path `exclusive` is too small, which keeps every
 			// scatter address inside the array; the status word tells the consumer to discard it.
-			__hip_atomic_store(my_word, ((exclusive + count) & kValueMask) | kFlagInclusive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+			__hip_atomic_store(word_of(tile), ((exclusive + count) & kValueMask) | kFlagInclusive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 		}
 		sc.global_base[tid] = digit_start + exclusive;
 	}
@@ -1081,29 +1100,38 @@ static size_t sort_tiles(size_t n, int items)
 // (a launch takes its tiles by the room of all its jobs, n among them: never smaller ones than n alone would have)
 size_t sort_clear_words(size_t n, int end_bit, int max_bits)
 {
-	const size_t tiles = sort_tiles(n, sort_items(n));
+	const size_t tiles = sort_tiles(n, sort_items(n, max_bits));
 	return kSortHeader + (size_t)sort_passes(end_bit, max_bits) * ((size_t)1 << max_bits) * tiles;
+}
+
+// (a view lists between a twentieth and a third of the Gaussians of a large scene)
+static int depth_sort_items(size_t n)
+{
+	const int items = sort_items(n, 9);
+	return items == kSortItemsMany ? sort_items(n / 2, 9) : items;
 }
 
 size_t depth_sort_clear_words(size_t n)
 {
-	const size_t tiles = sort_tiles(n, sort_items(n));
+	const size_t tiles = sort_tiles(n, depth_sort_items(n));
 	return kSortHeader + (size_t)(kDepthPasses + 1) * 512 * tiles;
 }
 
-// One pass over every job of the batch, in tiles of sort_items(pairs) pairs per thread.
-template <typename KeyT, int kBits, int kKind>
+// One pass over every job of the batch, in tiles by the room for pairs of all its jobs.
+template <typename KeyT, int kBits, int kKind, bool kDepth>
 static void launch_sort_pass(const Batch<SortJob<KeyT>>& b, size_t most_pairs, size_t pairs, int jobs, int pass, int shift, uint32_t mask,
                              hipStream_t s)
 {
 	// (64-bit keys, of the stand-alone entry points alone, take the smallest tiles: larger ones fill the LDS)
-	const int items = sizeof(KeyT) == 4 ? sort_items(pairs) : kSortItemsFew;
+	const int items = sizeof(KeyT) != 4 ? kSortItemsFew : kDepth ? depth_sort_items(pairs) : sort_items(pairs, kBits);
 	const dim3 grid((unsigned)sort_tiles(most_pairs, items), (unsigned)jobs);
 	const int spin = g_lookback_spin_limit.load();
 	if constexpr (sizeof(KeyT) == 4) {
-		if (items == kSortItemsMany) {
-			hipLaunchKernelGGL((sort_onesweep_kernel<KeyT, kBits, kKind, kSortItemsMany>), grid, dim3(kSortThreads), 0, s, b, pass, shift, mask, spin);
-			return;
+		if constexpr (kBits == 9) {
+			if (items == kSortItemsMany) {
+				hipLaunchKernelGGL((sort_onesweep_kernel<KeyT, kBits, kKind, kSortItemsMany>), grid, dim3(kSortThreads), 0, s, b, pass, shift, mask, spin);
+				return;
+			}
 		}
 		if (items == kSortItems) {
 			hipLaunchKernelGGL((sort_onesweep_kernel<KeyT, kBits, kKind, kSortItems>), grid, dim3(kSortThreads), 0, s, b, pass, shift, mask, spin);
@@ -1151,7 +1179,7 @@ static void sort_pairs(const SortJob<KeyT>* jobs, int count, int end_bit, bool t
 			const uint32_t mask = (1u << bits) - 1u;
 			if (mark_stages)
 				stage_mark("sort_onesweep", s);
-			launch_sort_pass<KeyT, kBits, kPassPlain>(b, most, pairs, live, p, shift, mask, s);
+			launch_sort_pass<KeyT, kBits, kPassPlain, false>(b, most, pairs, live, p, shift, mask, s);
 		}
 	}
 }
@@ -1212,10 +1240,10 @@ void launch_depth_order(const DepthOrderJob* jobs, int count, hipStream_t s)
 		}
 		hipLaunchKernelGGL(depth_pairs_kernel, pairs_grid, dim3(256), 0, s, b);
 		// three passes of nine bits (a -> b -> a -> the order and the tile counts in that order), and the pass on demand
-		launch_sort_pass<uint32_t, 9, kPassPlain>(sorts, (size_t)max_p, pairs, nj, 0, 0, 511u, s);
-		launch_sort_pass<uint32_t, 9, kPassPlain>(sorts, (size_t)max_p, pairs, nj, 1, 9, 511u, s);
-		launch_sort_pass<uint32_t, 9, kPassEndsUnless>(sorts, (size_t)max_p, pairs, nj, 2, 18, 511u, s);
-		launch_sort_pass<uint32_t, 9, kPassOnDemand>(sorts, (size_t)max_p, pairs, nj, 3, kDepthKeyBits, 31u, s);
+		launch_sort_pass<uint32_t, 9, kPassPlain, true>(sorts, (size_t)max_p, pairs, nj, 0, 0, 511u, s);
+		launch_sort_pass<uint32_t, 9, kPassPlain, true>(sorts, (size_t)max_p, pairs, nj, 1, 9, 511u, s);
+		launch_sort_pass<uint32_t, 9, kPassEndsUnless, true>(sorts, (size_t)max_p, pairs, nj, 2, 18, 511u, s);
+		launch_sort_pass<uint32_t, 9, kPassOnDemand, true>(sorts, (size_t)max_p, pairs, nj, 3, kDepthKeyBits, 31u, s);
 		hipLaunchKernelGGL(order_totals_kernel, grid, dim3(256), 0, s, b);
 		if (!few_groups)
 			hipLaunchKernelGGL(single_block_exclusive_scan_kernel, dim3(1, (unsigned)nj), dim3(1024), 0, s, scan);

@@ -316,15 +316,18 @@ constexpr int kSortThreads = 1024;
 // Pairs per thread in one tile of the sort: what a pass writes of a tile are runs of one digit value, and the longer they are the
 // fewer cache lines two workgroups (on two XCDs) share; but fewer, larger tiles leave part of the chip idle when the pairs
 // are few.  By what a launch has room for: the instances of all its jobs, which the host knows, and for the depth sort all their
-// Gaussians, of which the host does not know how many are visible.  Per pass, us, with 4 / 8 / 16:
-//   instances: 62.9 M Gaussians 256 / 196 / 197, 1600x1036 with 5.6 M 78 / 64 / 64, a call of 333 333 Gaussians 22 / 20 / 21;
-//   depths: 62.9 M Gaussians, a third visible 184 / 138 / 121; 27 M, a twentieth visible 40 / 31 / 25 (few of its tiles hold
-//   pairs, but a workgroup without any costs its start); 5.6 M, a third visible 24 / 26 / 24; 333 333, all visible 13 / 18 / 19.
-// A call of 100 000 Gaussians takes 260 / 275 / 287 us as a whole.
+// Gaussians, of which the host does not know how many are visible (16 from twice as many on).  Per pass, us, with 4 / 8 / 16:
+//   instances: 5185x3359 with 5.6 M Gaussians (nine-bit digits; those that follow have eight bits) 501 / 350 / 328, 62.9 M at 1600x1036 259 / 174 / 186, 5.6 M there
+//   78 / 58 / 60, 2.8 M in training 51 / 42 / 42, a call of 333 333 Gaussians 22 / 18 / 21, of 100 000 12 / 13 / 17;
+//   depths: 62.9 M, a third visible 153 / 100 / 114; 27 M, a twentieth visible 21 / 21 / 19; 5.6 M, a third visible 21 / 21 / 19;
+//   2.8 M in training 17 / 17 / 17, 333 333, all visible 13 / 14 / 19, 100 000 11 / 13 / 18.
 constexpr int kSortItemsFew = 4, kSortItems = 8, kSortItemsMany = 16;
-constexpr size_t kSortSome = (size_t)1 << 20, kSortMany = (size_t)1 << 23;  // pairs from which 8, and 16, are taken
+constexpr size_t kSortSome = (size_t)1 << 20, kSortMany = (size_t)1 << 25;  // pairs from which 8, and with nine-bit digits 16, are taken
 constexpr int kSortBlock = kSortThreads * kSortItemsFew;  // pairs of the smallest tile
-inline int sort_items(size_t pairs) { return pairs >= kSortMany ? kSortItemsMany : pairs >= kSortSome ? kSortItems : kSortItemsFew; }
+inline int sort_items(size_t pairs, int digit_bits)
+{
+	return digit_bits == 9 && pairs >= kSortMany ? kSortItemsMany : pairs >= kSortSome ? kSortItems : kSortItemsFew;
+}
 size_t scan_temp_words(size_t n);                 // u32 words of scratch for launch_inclusive_sum
 // `stage` (may be null) names the stage for the timing aid.
 void launch_inclusive_sum(const uint32_t* in, uint32_t* out, size_t n, uint32_t* temp, const char* stage,

@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from helpers import orc, scenes
+from test_gpu_rasterizer_parity import test_sorts_at_the_sizes_where_their_tiles_change as check_sorts
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -83,3 +84,8 @@ def test_groups_without_listed_gaussians(n, spread):
     assert (want[1] > 0).sum() > 2000 and torch.equal(want[1], got[1][at]) and int((got[1] > 0).sum()) == int((want[1] > 0).sum())
     for k in (0, 2, 3):
         assert torch.equal(want[k], got[k])
+
+
+def test_sorts_in_the_largest_tiles():
+    """2^26 Gaussians and some more, 2^25 instances and more under 17 tile bits: both sorts take tiles of 16 384 pairs."""
+    check_sorts((1 << 26) + 5, 4112, 4096)
