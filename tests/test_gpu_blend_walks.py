@@ -25,6 +25,16 @@ def test_more_strips_than_workgroups(width, height, n, grow):
     _check_backward(sub, cam, torch.tensor([0.2, 0.1, 0.05]), seed=3, with_depth_alpha=False)
 
 
+@pytest.mark.parametrize("width,height", [(1024, 1024), (1040, 1024), (1008, 1025)])   # 16 384, 16 640, 16 380 strips: ordered in one kernel or two
+def test_strips_ordered_at_once(width, height):
+    scene = scenes.cube_scene(1500, seed=12)
+    scene["scales"] = scene["scales"] * 8.0
+    cam = scenes.look_at_camera((0.0, 0.0, 0.0), (0.1, -0.05, 4.0), (0.05, -1, 0), width, height, 45.0)
+    sub = _scene_sub(scene)
+    _check_forward_stages(sub, cam, torch.tensor([0.2, 0.1, 0.05]), max_borderline=2e-3)
+    _check_backward(sub, cam, torch.tensor([0.2, 0.1, 0.05]), seed=5, with_depth_alpha=False)
+
+
 # (up to 4 096 strips, as in most tests of small images, a forward walk is shared by four wavefronts)
 @pytest.mark.parametrize("low,up", [((-0.31, -0.27, 3.6), (0.23, 0.19, 4.3)), ((-5.0, 0.05, -1.0), (5.0, 5.0, 9.0)),
                                     ((-5.0, -5.0, 4.95), (5.0, 5.0, 9.0))])
