@@ -1348,33 +1348,41 @@ __global__ __launch_bounds__(kFileBlock) void tile_ranges_kernel(Batch<TileRange
 	const size_t first = (size_t)blockIdx.x * kFileGroup;
 	if (first >= j.n)
 		return;  // the launch is sized for the job with the most keys
+	// A workgroup lives as long as its chain of reads: the keys (there is room for j.n, whatever they hold), the statuses and the count are
+	// asked for together, and a thread's previous key comes from its neighbour (71 M keys 100 -> 83 us, 42 M 61 -> 56).
+	const size_t idx0 = first + 4 * (size_t)threadIdx.x;
+	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+	uint32_t key[4] = {0u, 0u, 0u, 0u};
+	if (idx0 + 3 < j.n) {
+		const uint4 k4 = *reinterpret_cast<const uint4*>(keys + idx0);
+		key[0] = k4.x; key[1] = k4.y; key[2] = k4.z; key[3] = k4.w;
+	} else {
+#pragma unroll
+		for (int q = 0; q < 4; q++)
+			if (idx0 + q < j.n)
+				key[q] = keys[idx0 + q];
+	}
+	uint32_t prev = 0u;
+	if (lane == 0 && idx0 > 0 && idx0 < j.n)
+		prev = keys[idx0 - 1];
+	const uint32_t gave_up = (sort_status ? *sort_status : 0u) | (order_status ? *order_status : 0u);
+	if (n_device)
+		n = min(n, (size_t)*n_device);  // launched for an upper bound
 	// the sort has read its digit counts: zero again for the next to count into them
 	if (j.rezero) {
 		const size_t threads = (j.n + kFileGroup - 1) / kFileGroup * kFileBlock;
 		for (size_t w = (size_t)blockIdx.x * kFileBlock + threadIdx.x; w < (size_t)j.rezero_words; w += threads)
 			j.rezero[w] = 0u;
 	}
-	if ((sort_status && *sort_status != 0u) || (order_status && *order_status != 0u)) {
+	if (gave_up != 0u) {
 		if (blockIdx.x == 0 && threadIdx.x == 0 && fault)
 			__hip_atomic_store(fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 		return;
 	}
-	if (n_device)
-		n = min(n, (size_t)*n_device);  // launched for an upper bound
 	if (first >= n)
 		return;
-	const size_t idx0 = first + 4 * (size_t)threadIdx.x;
-	uint32_t key[4] = {0u, 0u, 0u, 0u};
-	if (idx0 + 3 < n) {
-		const uint4 k4 = *reinterpret_cast<const uint4*>(keys + idx0);
-		key[0] = k4.x; key[1] = k4.y; key[2] = k4.z; key[3] = k4.w;
-	} else {
-#pragma unroll
-		for (int q = 0; q < 4; q++)
-			if (idx0 + q < n)
-				key[q] = keys[idx0 + q];
-	}
-	uint32_t prev = (idx0 > 0 && idx0 < n) ? key_tile(keys[idx0 - 1]) : 0u;
+	const uint32_t lane_before = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key[3], 0x138, 0xF, 0xF, false);  // (wave_shr:1)
+	prev = key_tile(lane == 0 ? prev : lane_before);
 	const size_t last = min(n, first + kFileGroup) - 1;
 #pragma unroll
 	for (int q = 0; q < 4; q++) {
@@ -1406,7 +1414,6 @@ __global__ __launch_bounds__(kFileBlock) void tile_ranges_kernel(Batch<TileRange
 			own.x += (bits & 1u) | ((bits & 2u) << 15);
 			own.y += ((bits >> 2) & 1u) | ((bits & 8u) << 13);
 		}
-	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 	const uint2 inc = {wave_inclusive_scan_u32(own.x), wave_inclusive_scan_u32(own.y)};
 	if (lane == 63)
 		s_tail[wave] = inc;

@@ -240,23 +240,29 @@ __global__ __launch_bounds__(kFileBlock) void strip_file_place_kernel(BlendBatch
 	__shared__ FileStage st;
 	const BlendArgs& a = batch.job[blockIdx.y];
 	const uint32_t capacity = a.capacity;
-	const uint32_t R = a.count_device ? min(capacity, *a.count_device) : capacity;
 	const uint32_t first = blockIdx.x * (uint32_t)kFileGroup;
-	// after a sort that gave up the list is not sorted and the tile ranges are empty: nothing to place
-	if (first >= R || (a.sort_status && *a.sort_status != 0u) || (a.order_status && *a.order_status != 0u))
+	if (first >= capacity)
 		return;
+	// A workgroup lives as long as its chain of reads: the keys (there is room for `capacity`, whatever they hold), the statuses and the
+	// count are asked for together (71 M entries 262 -> 255 us, 42 M 132 -> 127).
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 	const uint32_t pos0 = first + 4u * (uint32_t)tid;
 	uint32_t key[4] = {0u, 0u, 0u, 0u};
-	if (pos0 + 3u < R) {
+	if (pos0 + 3u < capacity) {
 		const uint4 k4 = *reinterpret_cast<const uint4*>(a.tile_keys + pos0);
 		key[0] = k4.x; key[1] = k4.y; key[2] = k4.z; key[3] = k4.w;
 	} else {
 #pragma unroll
 		for (int q = 0; q < 4; q++)
-			if (pos0 + (uint32_t)q < R)
+			if (pos0 + (uint32_t)q < capacity)
 				key[q] = a.tile_keys[pos0 + q];
 	}
+	const uint32_t first_key = a.tile_keys[first];
+	const uint32_t gave_up = (a.sort_status ? *a.sort_status : 0u) | (a.order_status ? *a.order_status : 0u);
+	const uint32_t R = a.count_device ? min(capacity, *a.count_device) : capacity;
+	// after a sort that gave up the list is not sorted and the tile ranges are empty: nothing to place
+	if (first >= R || gave_up != 0u)
+		return;
 	uint2 range[4];
 	uint32_t filed[4];
 	uint2 own = {0u, 0u};
@@ -277,7 +283,7 @@ __global__ __launch_bounds__(kFileBlock) void strip_file_place_kernel(BlendBatch
 	st.bits[tid] = (uint16_t)all;
 	// what the tile of this workgroup's first entry filed in the workgroups before this one
 	{
-		const uint32_t begin0 = a.ranges[key_tile(a.tile_keys[first])].x;
+		const uint32_t begin0 = a.ranges[key_tile(first_key)].x;
 		uint4 sum = {0u, 0u, 0u, 0u};
 		if (begin0 < first)
 			for (uint32_t g = begin0 / (uint32_t)kFileGroup + (uint32_t)tid; g < blockIdx.x; g += kFileBlock) {
