@@ -1345,32 +1345,35 @@ __global__ __launch_bounds__(kFileBlock) void tile_ranges_kernel(Batch<TileRange
 	const uint32_t* __restrict__ order_status = j.order_status;
 	uint32_t* __restrict__ fault = j.fault;
 	uint4* __restrict__ file_tail = j.file_tail;
-	const size_t first = (size_t)blockIdx.x * kFileGroup;
+	size_t first = (size_t)blockIdx.x * kFileGroup;
 	if (first >= j.n)
 		return;  // the launch is sized for the job with the most keys
-	// A workgroup lives as long as its chain of reads: the keys (there is room for j.n, whatever they hold), the statuses and the count are
-	// asked for together, and a thread's previous key comes from its neighbour (71 M keys 100 -> 83 us, 42 M 61 -> 56).
-	const size_t idx0 = first + 4 * (size_t)threadIdx.x;
+	// A workgroup's time is its chain of reads: the keys (there is room for j.n, whatever they hold), the statuses and the count are
+	// asked for together, a group's keys while the one before it is worked on, and a thread's previous key comes from its neighbour
+	// (71 M keys 100 -> 68 us, 42 M 61 -> 52).
 	const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-	uint32_t key[4] = {0u, 0u, 0u, 0u};
-	if (idx0 + 3 < j.n) {
-		const uint4 k4 = *reinterpret_cast<const uint4*>(keys + idx0);
-		key[0] = k4.x; key[1] = k4.y; key[2] = k4.z; key[3] = k4.w;
-	} else {
+	uint32_t ahead[4] = {0u, 0u, 0u, 0u}, ahead_prev = 0u;
+	auto ask_for = [&](size_t group) {
+		const size_t at = group + 4 * (size_t)threadIdx.x;
+		if (at + 3 < j.n) {
+			const uint4 k4 = *reinterpret_cast<const uint4*>(keys + at);
+			ahead[0] = k4.x; ahead[1] = k4.y; ahead[2] = k4.z; ahead[3] = k4.w;
+		} else {
 #pragma unroll
-		for (int q = 0; q < 4; q++)
-			if (idx0 + q < j.n)
-				key[q] = keys[idx0 + q];
-	}
-	uint32_t prev = 0u;
-	if (lane == 0 && idx0 > 0 && idx0 < j.n)
-		prev = keys[idx0 - 1];
+			for (int q = 0; q < 4; q++)
+				if (at + q < j.n)
+					ahead[q] = keys[at + q];
+		}
+		if (lane == 0 && at > 0 && at < j.n)
+			ahead_prev = keys[at - 1];
+	};
+	ask_for(first);
 	const uint32_t gave_up = (sort_status ? *sort_status : 0u) | (order_status ? *order_status : 0u);
 	if (n_device)
 		n = min(n, (size_t)*n_device);  // launched for an upper bound
 	// the sort has read its digit counts: zero again for the next to count into them
 	if (j.rezero) {
-		const size_t threads = (j.n + kFileGroup - 1) / kFileGroup * kFileBlock;
+		const size_t threads = min((j.n + kFileGroup - 1) / kFileGroup, (size_t)gridDim.x) * kFileBlock;
 		for (size_t w = (size_t)blockIdx.x * kFileBlock + threadIdx.x; w < (size_t)j.rezero_words; w += threads)
 			j.rezero[w] = 0u;
 	}
@@ -1379,10 +1382,13 @@ __global__ __launch_bounds__(kFileBlock) void tile_ranges_kernel(Batch<TileRange
 			__hip_atomic_store(fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 		return;
 	}
-	if (first >= n)
-		return;
+	for (const size_t step = (size_t)gridDim.x * kFileGroup; first < n; first += step) {
+	const size_t idx0 = first + 4 * (size_t)threadIdx.x;
+	const uint32_t key[4] = {ahead[0], ahead[1], ahead[2], ahead[3]};
 	const uint32_t lane_before = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key[3], 0x138, 0xF, 0xF, false);  // (wave_shr:1)
-	prev = key_tile(lane == 0 ? prev : lane_before);
+	uint32_t prev = key_tile(lane == 0 ? ahead_prev : lane_before);
+	if (first + step < n)
+		ask_for(first + step);
 	const size_t last = min(n, first + kFileGroup) - 1;
 #pragma unroll
 	for (int q = 0; q < 4; q++) {
@@ -1403,7 +1409,7 @@ __global__ __launch_bounds__(kFileBlock) void tile_ranges_kernel(Batch<TileRange
 		prev = cur;
 	}
 	if (!file_tail)
-		return;
+		continue;
 	__syncthreads();
 	const uint32_t last_tile = s_last_tile;
 	uint2 own = {0u, 0u};
@@ -1421,7 +1427,8 @@ __global__ __launch_bounds__(kFileBlock) void tile_ranges_kernel(Batch<TileRange
 	if (threadIdx.x == 0) {
 		const uint32_t x = s_tail[0].x + s_tail[1].x + s_tail[2].x + s_tail[3].x;
 		const uint32_t y = s_tail[0].y + s_tail[1].y + s_tail[2].y + s_tail[3].y;
-		file_tail[blockIdx.x] = uint4{x & 0xFFFFu, x >> 16, y & 0xFFFFu, y >> 16};
+		file_tail[first / kFileGroup] = uint4{x & 0xFFFFu, x >> 16, y & 0xFFFFu, y >> 16};
+	}
 	}
 }
 
@@ -1456,8 +1463,10 @@ void launch_tile_ranges(const TileRangesJob* jobs, int count, hipStream_t s)
 			b.job[live++] = jobs[at + k];
 			max_n = jobs[at + k].n > max_n ? jobs[at + k].n : max_n;
 		}
+		// Up to 8 192 groups a workgroup each (as fast or faster), beyond that as many workgroups as are resident together, eight per CU.
+		const size_t groups = (max_n + kFileGroup - 1) / kFileGroup, most = groups * (size_t)live <= 8192 ? groups : max((size_t)2048 / (size_t)live, (size_t)1);
 		if (live)
-			hipLaunchKernelGGL(tile_ranges_kernel, dim3((unsigned)((max_n + kFileGroup - 1) / kFileGroup), (unsigned)live),
+			hipLaunchKernelGGL(tile_ranges_kernel, dim3((unsigned)min(groups, most), (unsigned)live),
 			                   dim3(kFileBlock), 0, s, b);
 	}
 }
