@@ -396,34 +396,37 @@ __global__ __launch_bounds__(256) void depth_pairs_kernel(Batch<DepthOrderJob> b
 	}
 }
 
-// The sum of every kScanGroup of the tile counts in depth order (the first level of the scan that follows),
-// four neighbouring ones per thread; the count of them is on the device.
+// The sum of every kScanGroup of the tile counts in depth order (the first level of the scan that follows), a wavefront per group, without
+// a barrier; the count of them is on the device.  The wavefronts that are resident together take all groups: with a workgroup per group
+// most had none (62.9 M Gaussians, a third listed: 28 -> 13 us).
 __global__ __launch_bounds__(256) void order_totals_kernel(Batch<DepthOrderJob> batch)
 {
-	__shared__ uint32_t lds[8];
+	static_assert(kScanGroup == 1024, "16 counts per lane");
 	const DepthOrderJob& j = batch.job[blockIdx.y];
 	// what the key duplication will count the digits of its tiles into
 	for (int w = (int)(blockIdx.x * 256 + threadIdx.x); w < (int)j.digit_copies * kDigitWords / 4; w += (int)gridDim.x * 256)
 		reinterpret_cast<uint4*>(j.digits)[w] = uint4{0u, 0u, 0u, 0u};
 	const size_t n = min((size_t)*j.visible_count, (size_t)j.P);
-	if ((size_t)blockIdx.x * kScanGroup >= n)
-		return;
 	const uint32_t* __restrict__ in = j.tiles_in_order;
-	const size_t k0 = (size_t)blockIdx.x * kScanGroup + 4 * (size_t)threadIdx.x;
-	uint32_t sum = 0;
-	if (k0 + 4 <= n) {
-		const uint4 v = *reinterpret_cast<const uint4*>(in + k0);
-		sum = v.x + v.y + v.z + v.w;
-	} else {
+	const int lane = threadIdx.x & 63;
+	for (size_t group = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6); group * kScanGroup < n; group += (size_t)gridDim.x * 4) {
+		const size_t k0 = group * kScanGroup + 4 * (size_t)lane;
+		uint4 v[4];
 #pragma unroll
 		for (int q = 0; q < 4; q++)
-			if (k0 + q < n)
-				sum += in[k0 + q];
+			v[q] = k0 + 256 * q + 4 <= n ? *reinterpret_cast<const uint4*>(in + k0 + 256 * q) : uint4{0u, 0u, 0u, 0u};
+		uint32_t sum = 0;
+#pragma unroll
+		for (int q = 0; q < 4; q++)
+			sum += v[q].x + v[q].y + v[q].z + v[q].w;
+		// the lane that holds the last counts, up to three of them
+		if (n - group * kScanGroup < kScanGroup && n > (n & ~(size_t)3) && (size_t)lane == (n >> 2 & 63))
+			for (size_t k = n & ~(size_t)3; k < n; k++)
+				sum += in[k];
+		sum = wave_inclusive_scan_u32(sum);
+		if (lane == 63)
+			j.scan_temp[group] = sum;
 	}
-	uint32_t total;
-	(void)block256_exclusive_scan_u32(sum, lds, total);
-	if (threadIdx.x == 0)
-		j.scan_temp[blockIdx.x] = total;
 }
 
 // Instances of the Gaussians in depth order, tiles row by row like the reference, at the offsets
@@ -1256,7 +1259,8 @@ void launch_depth_order(const DepthOrderJob* jobs, int count, hipStream_t s)
 		launch_sort_pass<uint32_t, 9, kPassPlain, true>(sorts, (size_t)max_p, pairs, nj, 1, 9, 511u, s);
 		launch_sort_pass<uint32_t, 9, kPassEndsUnless, true>(sorts, (size_t)max_p, pairs, nj, 2, 18, 511u, s);
 		launch_sort_pass<uint32_t, 9, kPassOnDemand, true>(sorts, (size_t)max_p, pairs, nj, 3, kDepthKeyBits, 31u, s);
-		hipLaunchKernelGGL(order_totals_kernel, grid, dim3(256), 0, s, b);
+		const unsigned resident = 2048u / (unsigned)nj;  // eight workgroups per CU
+		hipLaunchKernelGGL(order_totals_kernel, dim3(min(grid.x, resident), (unsigned)nj), dim3(256), 0, s, b);
 		if (!few_groups)
 			hipLaunchKernelGGL(single_block_exclusive_scan_kernel, dim3(1, (unsigned)nj), dim3(1024), 0, s, scan);
 		hipLaunchKernelGGL(block_inclusive_scan_kernel<4>, grid, dim3(256), 0, s, inc);

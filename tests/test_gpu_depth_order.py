@@ -89,3 +89,9 @@ def test_groups_without_listed_gaussians(n, spread):
 def test_sorts_in_the_largest_tiles():
     """2^26 Gaussians and some more, 2^25 instances and more under 17 tile bits: both sorts take tiles of 16 384 pairs."""
     check_sorts((1 << 26) + 5, 4112, 4096)
+
+
+@pytest.mark.parametrize("n", (8, 1023, 1024, 1025, 1026, 1027, 4096 + 6))
+def test_totals_of_ragged_groups(n):
+    """All in view: the sums of 1 024 tile counts where the last group is whole, short of a quad or a few counts beyond."""
+    check_sorts(n, 400, 300)
