@@ -385,7 +385,7 @@ void launch_depth_order(const DepthOrderJob* jobs, int count, hipStream_t s);
 // b * kDupPositions.  The scan that produces the offsets fills it; it has room for dup_first_words(P) workgroups,
 // those beyond (more than 16 instances per Gaussian on average) search the offsets instead.  One position per thread:
 // with 1 024 positions (four per thread) the kernel held 117 registers and 4 wavefronts per SIMD; with 256 it holds
-// 79 and 6, and is 22 % faster where the Gaussians are small.
+// 71 and 7, and is 22 % faster where the Gaussians are small.
 constexpr int kDupPositions = 256;
 constexpr size_t dup_first_words(size_t P) { return P / 16 + 2; }
 // The key duplication also counts the digits of the tiles it writes, which is what the sort of its keys starts
