@@ -144,7 +144,9 @@ __device__ __forceinline__ uint32_t strip_class(uint32_t filed) { return filed =
 // Words of strip_classes behind the counters and cursors of the two orders (1: the forward's, 0: the backward's).
 constexpr int kStripTail = 4 * kStripClasses;
 constexpr int strip_empty_word(int forward) { return kStripTail + 2 * forward; }  // how many strips are empty; behind it the placement cursor
-static_assert(strip_empty_word(1) + 1 < kRangeTailWords, "the words lie behind the ranges");
+constexpr int kStripLongWord = kStripTail + 4;   // how many strips at the front of the backward's order four wavefronts walk
+constexpr int kStripTotalWord = kStripTail + 5;  // the entries of all strips that the backward walks (where two kernels order them)
+static_assert(kStripTotalWord < kRangeTailWords, "the words lie behind the ranges");
 
 constexpr int kPerLane = 1;             // list entries per lane and step (2 was measured slower)
 constexpr int kChunk = 64 * kPerLane;   // list entries a wavefront takes per step
@@ -1145,12 +1147,15 @@ __device__ __forceinline__ Pair zero_pair()
 	return z;
 }
 
-struct BackwardStage {  // wave-private
-	// (each what one read of the walk takes; + padding up to a multiple of eight entries)
+struct BackwardChunk {  // each what one read of the walk takes; + padding up to a multiple of eight entries
 	float4 centre_conic[kChunk + kRows - 1];  // pixel x, pixel y, staged conic -xx / 2, -xy
 	float4 rest[kChunk + kRows - 1];          // staged conic -yy / 2, opacity, clip w, 0-based position in the tile list (as bits)
 	float4 cd[kChunk + kRows - 1];
 	uint32_t sum_row[kChunk + kRows - 1];  // where the Gaussian's row of `sums` begins, in 16 bytes
+};
+
+struct BackwardStage {  // wave-private
+	BackwardChunk chunk;
 	float2 u_at[kRows * kRowStride];  // [row][row_column(pixel)]: (u, alpha T)
 	float g_depth[72];                // upstream gradient of the depth image by pixel, eight of nine words
 	StripRays rays;
@@ -1202,7 +1207,7 @@ struct Blended {
 // kDepth: a gradient arrived for the depth image (without one, the usual case of a loss on the colour image alone, the
 // terms it multiplies are left out: the depth column of `sums` stays zero).
 template <bool kDepth>
-__device__ __forceinline__ void sum_rows(const BackwardStage& st, int slot0, const Blended& blended, const Sweep& sweep,
+__device__ __forceinline__ void sum_rows(const BackwardChunk& st, const float* g_depth, int slot0, const Blended& blended, const Sweep& sweep,
                                          const StripFrame& f, int lane)
 {
 #pragma clang fp contract(fast)
@@ -1216,7 +1221,7 @@ __device__ __forceinline__ void sum_rows(const BackwardStage& st, int slot0, con
 	Pair ua = sweep.row[0];
 	float s0 = ua.x, sx = ua.x * dx_first, sxx = sx * dx_first;
 	float cr = ua.y * sweep.r[0], cg = ua.y * sweep.g[0], cb = ua.y * sweep.b[0];
-	float cdp = kDepth ? ua.y * st.g_depth[9 * (lane & 7)] : 0.f;
+	float cdp = kDepth ? ua.y * g_depth[9 * (lane & 7)] : 0.f;
 #pragma unroll
 	for (int step = 1; step < 8; step++) {
 		ua = sweep.row[step];
@@ -1228,7 +1233,7 @@ __device__ __forceinline__ void sum_rows(const BackwardStage& st, int slot0, con
 		cg += ua.y * sweep.g[step];
 		cb += ua.y * sweep.b[step];
 		if (kDepth)
-			cdp += ua.y * st.g_depth[9 * (lane & 7) + step];
+			cdp += ua.y * g_depth[9 * (lane & 7) + step];
 	}
 	// the two halves of the strip row first (dy is theirs in common), then the four strip rows
 	float w[7] = {s0, sx, sxx, cr, cg, cb, cdp};
@@ -1276,17 +1281,21 @@ __device__ __forceinline__ void sum_rows(const BackwardStage& st, int slot0, con
 	__builtin_amdgcn_wave_barrier();
 }
 
-// Pixel-parallel part for the four entries staged from slot k on; `rows`: the pixel's place in the first of their rows.
-// Returns, as sum_rows asks for it (16 lanes per entry), which of them any pixel blended.
+// Pixel-parallel part for the four entries staged from slot k on: first what needs no other entry, then the recurrences.
 // kVisit: which comparisons the chunk's entries need (three of 29 vector instructions per entry; with an entry's words in
 // the order of their reads 2 775 -> 2 740 us at 5185x3359, 64.5 -> 63 for 100 000 Gaussians at 512x512).
 enum Visit { kVisitAll, kVisitPlain, kVisitPlainReached };  // plain: see plain_entry; reached: every pixel blended an entry behind the chunk
+struct VisitedEntries {
+	float alpha[4], G[4], inv[4], weighted[4];
+	uint64_t mask[4];  // the pixels that blended the entry
+};
 template <bool kDepth, BoxTest kBox, Visit kVisit>
-__device__ __forceinline__ uint64_t backward_rows(BackwardPixel& p, uint32_t last_contributor, const BackwardStage& st, int k,
-                                              LdsPair* rows, const float2 pixf, const BoxSpan& span, const BlendArgs& a)
+__device__ __forceinline__ void backward_visit(VisitedEntries& v, const BackwardPixel& p, uint32_t last_contributor, const BackwardChunk& st, int k,
+                                               const StripRays& rays, const float2 pixf, const BoxSpan& span, const BlendArgs& a)
 {
 	float power[4], clip_w[4], opacity[4];
-	uint64_t mask[4];
+	float (&alpha)[4] = v.alpha, (&G)[4] = v.G, (&inv)[4] = v.inv, (&weighted)[4] = v.weighted;
+	uint64_t (&mask)[4] = v.mask;
 #pragma unroll
 	for (int i = 0; i < 4; i++) {
 		const float4 centre_conic = st.centre_conic[k + i], rest = st.rest[k + i];
@@ -1307,16 +1316,15 @@ __device__ __forceinline__ uint64_t backward_rows(BackwardPixel& p, uint32_t las
 	for (int i = 0; i < 4; i++)
 		cd[i] = st.cd[k + i];
 	__builtin_amdgcn_sched_barrier(0);
-	float alpha[4], G[4], inv[4], weighted[4];
 #pragma unroll
 	for (int i = 0; i < 4; i++) {
 		G[i] = exp_of_exponent(power[i]);
 		alpha[i] = kVisit == kVisitAll ? fminf(0.99f, opacity[i] * G[i]) : opacity[i] * G[i];
 		mask[i] &= lanes_where(!(alpha[i] < 1.0f / 255.0f));
 		if (kBox == kBoxSpans)
-			mask[i] = lanes_inside_box(mask[i], clip_w[i], span, st.rays, a);
+			mask[i] = lanes_inside_box(mask[i], clip_w[i], span, rays, a);
 		if (kBox == kBoxExact)
-			mask[i] = lanes_inside_box(mask[i], clip_w[i], st.rays, a);
+			mask[i] = lanes_inside_box(mask[i], clip_w[i], rays, a);
 		// From here on nothing feeds a decision: gradients are compared by tolerance, so the divisions use the hardware
 		// reciprocal.
 		inv[i] = __builtin_amdgcn_rcpf(1.f - alpha[i]);
@@ -1324,6 +1332,12 @@ __device__ __forceinline__ uint64_t backward_rows(BackwardPixel& p, uint32_t las
 		if (kDepth)
 			weighted[i] = __builtin_fmaf(cd[i].w, p.g_depth, weighted[i]);
 	}
+}
+
+// `rows`: the pixel's place in the first of the four entries' rows.  Returns, as sum_rows asks for it (16 lanes per entry), which of them
+// any pixel blended.
+__device__ __forceinline__ uint64_t backward_rows(BackwardPixel& p, const VisitedEntries& v, LdsPair* rows)
+{
 	// The pixel's outputs are sums over its blended entries j of w_j (colour_j, depth_j, 1) with w_j = alpha_j T_j,
 	// T_j the product of (1 - alpha_k) over the entries in front, plus T_final times the background.  Their
 	// derivative with respect to alpha_i is T_i (colour_i, depth_i, 1) minus (the sum over the entries behind i +
@@ -1349,14 +1363,14 @@ __device__ __forceinline__ uint64_t backward_rows(BackwardPixel& p, uint32_t las
 		    "v_mul_f32 %[u], %[G], %[d]\n\t"
 		    "s_mov_b64 exec, %[active]"
 		    : [T] "+v"(p.T), [behind] "+v"(p.behind), [aT] "+v"(aT), [u] "+v"(u), [d] "=&v"(dL_dopa), [active] "=&s"(active)
-		    : [lanes] "s"(mask[i]), [inv] "v"(inv[i]), [alpha] "v"(alpha[i]), [weighted] "v"(weighted[i]), [G] "v"(G[i])
+		    : [lanes] "s"(v.mask[i]), [inv] "v"(v.inv[i]), [alpha] "v"(v.alpha[i]), [weighted] "v"(v.weighted[i]), [G] "v"(v.G[i])
 		    : "scc");
 		rows[i * kRowStride] = Pair{u, aT};
 	}
 	uint64_t blended = 0ull;
 #pragma unroll
 	for (int i = 0; i < 4; i++)
-		blended |= mask[i] != 0ull ? 0xFFFFull << (16 * i) : 0ull;
+		blended |= v.mask[i] != 0ull ? 0xFFFFull << (16 * i) : 0ull;
 	return blended;
 }
 
@@ -1367,10 +1381,33 @@ __device__ __forceinline__ void backward_chunk(BackwardPixel& p, uint32_t last_c
                                                const StripFrame& frame, int lane, const BlendArgs& a)
 {
 	for (int k = 0; k < count; k += kRows) {
-		const Blended blended = {backward_rows<kDepth, kBox, kVisit>(p, last_contributor, st, k, rows[0], pixf, span, a),
-		                         backward_rows<kDepth, kBox, kVisit>(p, last_contributor, st, k + 4, rows[1], pixf, span, a)};
+		VisitedEntries v;
+		Blended blended;
+		backward_visit<kDepth, kBox, kVisit>(v, p, last_contributor, st.chunk, k, st.rays, pixf, span, a);
+		blended.low = backward_rows(p, v, rows[0]);
+		backward_visit<kDepth, kBox, kVisit>(v, p, last_contributor, st.chunk, k + 4, st.rays, pixf, span, a);
+		blended.high = backward_rows(p, v, rows[1]);
 		if ((blended.low | blended.high) != 0ull)
-			sum_rows<kDepth>(st, k, blended, sweep, frame, lane);
+			sum_rows<kDepth>(st.chunk, st.g_depth, k, blended, sweep, frame, lane);
+	}
+}
+
+// Files a chunk's entry of this lane, and behind the last one entries up to a multiple of eight that lie behind every pixel's last one.
+__device__ __forceinline__ void stage_backward(BackwardChunk& st, const LoadedRecord& cur, uint32_t pos_cur, int count, int lane)
+{
+	if (lane < count) {
+		const float w = (pos_cur & 0x80000000u) ? __int_as_float(0x7FC00000) : cur.geom.w;  // (the strip lies inside the box: no per-pixel test)
+		const float4 conic = staged_conic(cur.conic);
+		st.centre_conic[lane] = float4{cur.geom.x, cur.geom.y, conic.x, conic.y};
+		st.rest[lane] = float4{conic.z, conic.w, w, __uint_as_float(pos_cur & kPosition)};
+		st.cd[lane] = cur.cd;
+		st.sum_row[lane] = kSumCols / 4 * cur.id;  // (32 bits hold it: a thousand million Gaussians' gradients fit no device)
+	}
+	if (lane < kRows - 1) {
+		st.centre_conic[count + lane] = float4{0.f, 0.f, 0.f, 0.f};
+		st.rest[count + lane] = float4{0.f, 0.f, 0.f, __uint_as_float(0xFFFFFFFFu)};
+		st.cd[count + lane] = float4{0.f, 0.f, 0.f, 0.f};
+		st.sum_row[count + lane] = 0u;
 	}
 }
 
@@ -1418,7 +1455,7 @@ __device__ __forceinline__ void backward_strip(const BlendArgs& a, uint32_t stri
 		sweep.row = lds_base(st.u_at + e * kRowStride + row_column(h * 16 + 8 * (lane & 1)));
 		sweep.column_low = a.sums + (upper ? 8 + j : j);
 		sweep.column_high = a.sums + (upper ? j : 8 + j);
-		float4* by_pixel = st.centre_conic;  // (not in use yet)
+		float4* by_pixel = st.chunk.centre_conic;  // (not in use yet)
 		by_pixel[lane] = float4{p.g_r, p.g_g, p.g_b, 0.f};
 		if (kDepth)
 			st.g_depth[lane + (lane >> 3)] = p.g_depth;
@@ -1451,20 +1488,7 @@ __device__ __forceinline__ void backward_strip(const BlendArgs& a, uint32_t stri
 	bool have_span = false;
 	for (uint32_t first = 0; first < filed; first += 64) {
 		const int count = (int)min(filed - first, 64u);
-		if (lane < count) {
-			const float w = (pos_cur & 0x80000000u) ? __int_as_float(0x7FC00000) : cur.geom.w;  // (the strip lies inside the box: no per-pixel test)
-			const float4 conic = staged_conic(cur.conic);
-			st.centre_conic[lane] = float4{cur.geom.x, cur.geom.y, conic.x, conic.y};
-			st.rest[lane] = float4{conic.z, conic.w, w, __uint_as_float(pos_cur & kPosition)};
-			st.cd[lane] = cur.cd;
-			st.sum_row[lane] = kSumCols / 4 * cur.id;  // (32 bits hold it: a thousand million Gaussians' gradients fit no device)
-		}
-		if (lane < kRows - 1) {  // pad to a multiple of eight with entries behind every pixel's last one
-			st.centre_conic[count + lane] = float4{0.f, 0.f, 0.f, 0.f};
-			st.rest[count + lane] = float4{0.f, 0.f, 0.f, __uint_as_float(0xFFFFFFFFu)};
-			st.cd[count + lane] = float4{0.f, 0.f, 0.f, 0.f};
-			st.sum_row[count + lane] = 0u;
-		}
+		stage_backward(st.chunk, cur, pos_cur, count, lane);
 		const bool straddles = lane < count && (pos_cur & 0x80000000u) == 0u;
 		const bool boxed = lanes_where(straddles) != 0ull, all_in_front = lanes_where(straddles && !(cur.geom.w > 0.f)) == 0ull;
 		// (lane 0 holds the chunk's entry that lies furthest back; the padding's opacity is 0)
@@ -1523,6 +1547,288 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 	}
 }
 
+// ---- a backward walk shared by four wavefronts -------------------------------------------------
+// A wavefront alone on its SIMD takes 0.2 us per entry, twice what issuing its instructions takes and far more than a
+// strip's share where the chip is full, so a launch of few strips lasts as long as its longest walks.  There (see long_strip_classes) four
+// wavefronts walk a strip, a pass of eight entries each in turn.  What needs no other entry (exponentials, alphas, reciprocals, colours
+// against the upstream gradient) and the sums over the pixels run side by side; transmittance and `behind` of the 64 pixels are
+// handed from pass to pass through LDS, and only three instructions per entry lie between taking and passing them on.  They and what
+// follows are the operations of one wavefront's walk on the same operands in the same order (factors of an entry that a pixel did not blend are made 1, 0
+// and 0, which leaves both as they are), and as many additions go to each Gaussian's row.  (Shared by pixels instead, as the forward's
+// walk, four times as many do, and additions to one address take 12 ns each.  Eight wavefronts: 67 to 75 us for 100 000 Gaussians at
+// 512x512, four 50, two 44; but two 112 for 61 000 Gaussians of two submodels at 397x251, four 72.)
+// Chunks are staged in turn as well, two ahead of their use, in kStagedChunks buffers.  The wavefronts of a workgroup run at the same
+// time and every word that one waits for is written by one that waits for earlier passes alone; the waits are bounded all the same.
+constexpr int kSharedWaves = 4;
+constexpr int kStagedChunks = 4;
+enum ChunkKind : uint32_t { kChunkSpans, kChunkExact, kChunkReached, kChunkPlain, kChunkAll };  // which copy of the loop a chunk runs
+constexpr int kSharedPolls = 1 << 20;
+
+struct SharedStage {
+	BackwardChunk chunk[kStagedChunks];
+	float2 u_at[kSharedWaves][kRows * kRowStride];
+	float2 carry[64];     // per pixel: transmittance and `behind`, as the pass before left them
+	float g_depth[72];
+	StripRays rays;
+	uint32_t turn;                    // the pass that may take `carry`
+	uint32_t staged[kStagedChunks];   // one more than the chunk that a buffer holds
+	uint32_t kind[kStagedChunks];
+	uint32_t walked[kSharedWaves];          // chunks that a wavefront is done with
+};
+
+// Waits until a word that another wavefront of the workgroup counts up has reached `value`.  (A wavefront's LDS accesses are served in
+// order, so what the writer stored ahead of the word is there when the word is; the empty assembly keeps the compiler to that order.)
+__device__ __forceinline__ void wait_for(const uint32_t* word, uint32_t value)
+{
+	for (int polls = 0; polls < kSharedPolls; polls++) {
+		const uint32_t v = (uint32_t)__builtin_amdgcn_readfirstlane((int)__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+		if ((int)(v - value) >= 0)
+			break;
+		__builtin_amdgcn_s_sleep(0);
+	}
+	asm volatile("" ::: "memory");
+}
+__device__ __forceinline__ void publish(uint32_t* word, uint32_t value, int lane)
+{
+	asm volatile("" ::: "memory");
+	if (lane == 0)
+		__hip_atomic_store(word, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+	asm volatile("" ::: "memory");
+}
+
+// The pixel's transmittance and `behind` once it is the turn of `pass`, read with the word that says so.
+__device__ __forceinline__ float2 wait_for_carry(const uint32_t& turn, const float2& carry, uint32_t pass)
+{
+	float2 c;
+	for (int polls = 0; polls < kSharedPolls; polls++) {
+		const uint32_t v = __hip_atomic_load(&turn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+		asm volatile("" ::: "memory");
+		c = carry;
+		asm volatile("" ::: "memory");
+		if ((uint32_t)__builtin_amdgcn_readfirstlane((int)v) == pass)
+			break;
+	}
+	return c;
+}
+
+template <bool kDepth, BoxTest kBox, Visit kVisit>
+__device__ __forceinline__ void backward_chunk_shared(BackwardPixel& p, uint32_t last_contributor, SharedStage& st, int buffer, uint32_t first_pass,
+                                                      int count, LdsPair* const (&rows)[2], const float2 pixf, const BoxSpan& span, const Sweep& sweep,
+                                                      const StripFrame& frame, int lane, int wave, const BlendArgs& a)
+{
+	const BackwardChunk& chunk = st.chunk[buffer];
+	for (int k = kRows * wave; k < count; k += kRows * kSharedWaves) {
+		VisitedEntries v[2];
+		backward_visit<kDepth, kBox, kVisit>(v[0], p, last_contributor, chunk, k, st.rays, pixf, span, a);
+		backward_visit<kDepth, kBox, kVisit>(v[1], p, last_contributor, chunk, k + 4, st.rays, pixf, span, a);
+		Blended blended = {0ull, 0ull};
+#pragma unroll
+		for (int i = 0; i < 8; i++) {
+			VisitedEntries& e = v[i >> 2];
+			const bool took = __builtin_amdgcn_inverse_ballot_w64(e.mask[i & 3]);
+			e.inv[i & 3] = took ? e.inv[i & 3] : 1.f;
+			e.alpha[i & 3] = took ? e.alpha[i & 3] : 0.f;
+			e.weighted[i & 3] = took ? e.weighted[i & 3] : 0.f;
+			uint64_t& b = i < 4 ? blended.low : blended.high;
+			b |= e.mask[i & 3] != 0ull ? 0xFFFFull << (16 * (i & 3)) : 0ull;
+		}
+		const uint32_t pass = first_pass + (uint32_t)k / kRows;
+		const float2 carry = wait_for_carry(st.turn, st.carry[lane], pass);
+		{
+			float T = carry.x, behind = carry.y;
+#pragma unroll
+			for (int i = 0; i < 8; i++) {
+				const VisitedEntries& e = v[i >> 2];
+				T *= e.inv[i & 3];
+				behind = __builtin_fmaf(e.alpha[i & 3] * T, e.weighted[i & 3], behind);
+			}
+			st.carry[lane] = float2{T, behind};
+		}
+		publish(&st.turn, pass + 1u, lane);
+		{
+			// (once more, with what it gives each entry: kept from above it would take 24 registers)
+			float T = carry.x, behind = carry.y;
+			asm volatile("" : "+v"(T), "+v"(behind));
+#pragma unroll
+			for (int i = 0; i < 8; i++) {
+				const VisitedEntries& e = v[i >> 2];
+				T *= e.inv[i & 3];
+				const float past = behind * e.inv[i & 3], aT = e.alpha[i & 3] * T, d = __builtin_fmaf(e.weighted[i & 3], T, -past);
+				behind = __builtin_fmaf(aT, e.weighted[i & 3], behind);
+				// (a transmittance that is not finite stays out of the rows of entries that the pixel did not blend)
+				const bool took = __builtin_amdgcn_inverse_ballot_w64(e.mask[i & 3]);
+				rows[i >> 2][(i & 3) * kRowStride] = Pair{took ? e.G[i & 3] * d : 0.f, took ? aT : 0.f};
+			}
+		}
+		if ((blended.low | blended.high) != 0ull)
+			sum_rows<kDepth>(chunk, st.g_depth, k, blended, sweep, frame, lane);
+	}
+}
+
+template <bool kDepth>
+__device__ __forceinline__ void backward_strip_shared(const BlendArgs& a, uint32_t strip_id, SharedStage& st, int lane, int wave)
+{
+	const int tile = (int)(strip_id >> 2), strip = (int)(strip_id & 3u);
+	uint2 range = a.ranges[tile];
+	range.y = min(range.y, a.capacity);
+	range.x = min(range.x, range.y);
+	const int tx = tile % a.grid_x, ty = tile / a.grid_x;
+	const uint32_t px = tx * kTile + (lane & 15), py = ty * kTile + strip * 4 + (lane >> 4);
+	const bool inside = px < (uint32_t)a.W && py < (uint32_t)a.H;
+	const uint32_t pix_id = (uint32_t)a.W * py + px;
+	const float2 pixf = {(float)px, (float)py};
+	const size_t plane = (size_t)a.H * a.W;
+	const StripFrame frame = {(float)(tx * kTile), (float)(ty * kTile + strip * 4), (float)(0.5 * a.W), (float)(0.5 * a.H)};
+	const uint32_t n = range.y - range.x;
+	const uint32_t filed = min(a.strip_filed[strip_id], n);
+	if (filed == 0u)  // (the same for every wavefront)
+		return;
+	const uint32_t last_contributor = inside ? a.n_contrib[pix_id] : 0u;
+
+	// the wavefront's own chunks, every kSharedWaves-th
+	const uint32_t* list = a.point_list + range.x;
+	const uint32_t* filed_list = a.strip_lists + 4 * (size_t)range.x + (size_t)strip * n;
+	auto position = [&](uint32_t chunk) {
+		const uint32_t e = 64u * chunk + (uint32_t)lane;
+		return e < filed ? filed_list[filed - 1u - e] : kNone;
+	};
+	auto index_of = [&](uint32_t pos) { return pos != kNone ? list[min(pos & kPosition, n - 1u)] : 0u; };
+	uint32_t next_chunk = (uint32_t)wave;
+	uint32_t pos_cur = position(next_chunk), pos_next = position(next_chunk + kSharedWaves), pos_after = position(next_chunk + 2 * kSharedWaves);
+	LoadedRecord cur = load_record(a, index_of(pos_cur), pos_cur != kNone);
+	uint32_t id_next = index_of(pos_next);
+
+	BackwardPixel p;
+	const float T_final = inside ? (1 - a.out_alpha[pix_id]) : 0.f;
+	p.T = T_final;
+	p.g_r = p.g_g = p.g_b = p.g_depth = p.g_alpha = 0.f;
+	if (inside) {
+		p.g_r = a.dL_dpix[pix_id];
+		p.g_g = a.dL_dpix[plane + pix_id];
+		p.g_b = a.dL_dpix[2 * plane + pix_id];
+		p.g_depth = a.dL_dpix_depth ? a.dL_dpix_depth[pix_id] : 0.f;
+		p.g_alpha = a.dL_dalpha ? a.dL_dalpha[pix_id] : 0.f;
+	}
+	p.behind = T_final * ((0.f + a.bg[0] * p.g_r + a.bg[1] * p.g_g) + a.bg[2] * p.g_b);
+
+	float4* by_pixel = reinterpret_cast<float4*>(st.u_at[0]);  // (not in use yet)
+	if (wave == 0) {
+		stage_rays(st.rays, pixf, a, lane);
+		by_pixel[lane] = float4{p.g_r, p.g_g, p.g_b, 0.f};
+		st.carry[lane] = float2{p.T, p.behind};
+		if (kDepth)
+			st.g_depth[lane + (lane >> 3)] = p.g_depth;
+		if (lane == 0)
+			st.turn = 0u;
+		if (lane < kStagedChunks)
+			st.staged[lane] = 0u;
+		if (lane < kSharedWaves)
+			st.walked[lane] = 0u;
+	}
+	__syncthreads();
+	Sweep sweep;
+	{
+		const int upper = (lane >> 3) & 1, e = (lane >> 4) + 4 * upper, h = (lane >> 1) & 3, j = lane & 7;
+		sweep.row = lds_base(st.u_at[wave] + e * kRowStride + row_column(h * 16 + 8 * (lane & 1)));
+		sweep.column_low = a.sums + (upper ? 8 + j : j);
+		sweep.column_high = a.sums + (upper ? j : 8 + j);
+#pragma unroll
+		for (int s = 0; s < 8; s++) {
+			const float4 g = by_pixel[8 * (lane & 7) + s];
+			sweep.r[s] = g.x;
+			sweep.g[s] = g.y;
+			sweep.b[s] = g.z;
+		}
+	}
+	__syncthreads();
+	LdsPair* const rows[2] = {lds_base(st.u_at[wave] + row_column(lane)), lds_base(st.u_at[wave] + 4 * kRowStride + row_column(lane))};
+
+	const uint32_t chunks = (filed + 63u) / 64u;
+	auto stage = [&]() {
+		const uint32_t buffer = next_chunk % kStagedChunks;
+		const int count = (int)min(filed - 64u * next_chunk, 64u);
+		stage_backward(st.chunk[buffer], cur, pos_cur, count, lane);
+		const bool straddles = lane < count && (pos_cur & 0x80000000u) == 0u;
+		const bool boxed = lanes_where(straddles) != 0ull, all_in_front = lanes_where(straddles && !(cur.geom.w > 0.f)) == 0ull;
+		const bool plain = lanes_where(lane < count && !plain_entry(cur)) == 0ull;
+		const bool reached = lanes_where((uint32_t)__builtin_amdgcn_readfirstlane((int)(pos_cur & kPosition)) >= last_contributor) == 0ull;
+		const uint32_t kind = boxed ? (all_in_front ? kChunkSpans : kChunkExact) : plain ? (reached ? kChunkReached : kChunkPlain) : kChunkAll;
+		if (lane == 0)
+			st.kind[buffer] = kind;
+		publish(&st.staged[buffer], next_chunk + 1u, lane);
+		next_chunk += kSharedWaves;
+		cur = load_record(a, id_next, pos_next != kNone);
+		pos_cur = pos_next;
+		pos_next = pos_after;
+		id_next = index_of(pos_next);
+		pos_after = position(next_chunk + 2 * kSharedWaves);
+	};
+	if (next_chunk < min(chunks, 2u))
+		stage();
+
+	BoxSpan span;
+	bool have_span = false;
+	for (uint32_t c = 0; c < chunks; c++) {
+		if (next_chunk == c + 2u && next_chunk < chunks) {
+			// its buffer held chunk c - 2
+#pragma unroll
+			for (int w = 0; w < kSharedWaves; w++)
+				if (c >= 2u)
+					wait_for(&st.walked[w], c - 1u);
+			stage();
+		}
+		const int buffer = (int)(c % kStagedChunks);
+		wait_for(&st.staged[buffer], c + 1u);
+		const uint32_t kind = (uint32_t)__builtin_amdgcn_readfirstlane((int)st.kind[buffer]);
+		const int count = (int)min(filed - 64u * c, 64u);
+		if (kind == kChunkSpans) {
+			if (kDepth || !have_span) {
+				span = w_inside_box(ray_of(st.rays), load_box_frame(a));
+				have_span = true;
+			}
+			backward_chunk_shared<kDepth, kBoxSpans, kVisitAll>(p, last_contributor, st, buffer, 8u * c, count, rows, pixf, span, sweep, frame, lane, wave, a);
+		} else if (kind == kChunkExact) {
+			backward_chunk_shared<kDepth, kBoxExact, kVisitAll>(p, last_contributor, st, buffer, 8u * c, count, rows, pixf, span, sweep, frame, lane, wave, a);
+		} else if (kind == kChunkReached) {
+			backward_chunk_shared<kDepth, kBoxNone, kVisitPlainReached>(p, last_contributor, st, buffer, 8u * c, count, rows, pixf, span, sweep, frame, lane, wave, a);
+		} else if (kind == kChunkPlain) {
+			backward_chunk_shared<kDepth, kBoxNone, kVisitPlain>(p, last_contributor, st, buffer, 8u * c, count, rows, pixf, span, sweep, frame, lane, wave, a);
+		} else {
+			backward_chunk_shared<kDepth, kBoxNone, kVisitAll>(p, last_contributor, st, buffer, 8u * c, count, rows, pixf, span, sweep, frame, lane, wave, a);
+		}
+		publish(&st.walked[wave], c + 1u, lane);
+	}
+}
+
+// Launches of few strips: the longest walks by a workgroup each, of the others one per wavefront (neighbours in the order, so they end at
+// about the same time).  Three wavefronts per SIMD: what the shared walk holds fits 168 registers, and the others run as fast as with four.
+template <bool kDepth>
+__global__ __launch_bounds__(64 * kSharedWaves) __attribute__((amdgpu_waves_per_eu(3, 3))) void blend_backward_shared_kernel(BlendBatch batch)
+{
+	__shared__ union Stages {
+		SharedStage shared;
+		BackwardStage alone[kSharedWaves];
+		__device__ Stages() {}
+	} st;
+	const BlendArgs& a = batch.job[blockIdx.x % (uint32_t)batch.count];
+	const uint32_t number = blockIdx.x / (uint32_t)batch.count;
+	const uint32_t filled = batch.strips - min(a.strip_classes[strip_empty_word(0)], batch.strips);
+	const uint32_t longer = min(a.strip_classes[kStripLongWord], filled), items = longer + (filled - longer + kSharedWaves - 1u) / kSharedWaves;
+	const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+	for (uint32_t at = number, turn = 0; at < items; at = turn_of_workgroup(number, ++turn, batch.workgroups)) {
+		int lane = (int)(threadIdx.x & 63u);
+		asm volatile("" : "+v"(lane));
+		if (at < longer) {
+			backward_strip_shared<kDepth>(a, min(a.strip_order[at], batch.strips - 1u), st.shared, lane, wave);
+			__syncthreads();  // the stage is the next strip's
+		} else {
+			const uint32_t mine = longer + kSharedWaves * (at - longer) + (uint32_t)wave;
+			if (mine < filled)
+				backward_strip<kDepth>(a, min(a.strip_order[mine], batch.strips - 1u), st.alone[wave], lane);
+		}
+	}
+}
+
 // Strips by decreasing number of entries to walk, in kStripClasses classes of 8 (longer ones share
 // the first class); the order inside a class is whatever the atomics give, which is all a
 // launch order needs; the strips without any come last.  Two small kernels: count the strips of every class, then place them; one
@@ -1533,6 +1839,19 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 4))) void
 // LDS counter as one
 // (5185x3359, both kernels and both orders: 92 us with a strip per thread, 31 now; 1600x1036: 19 and 20).
 constexpr uint32_t kOrderStrips = 1024;
+
+// How many classes, the longest ones, hold strips whose backward walk is shared by four wavefronts: those that one wavefront would be busy
+// with for 0.85 of the time that all the launch's entries take the chip (0.2 us per entry alone, 0.094 ns where every SIMD has four
+// walks), the entries of all jobs estimated from the job's own.  Backward blend in us, kernel of single wavefronts and this one by that
+// fraction (none shared, 2, 1, 0.82, 0.5, 0.35): 61 000 Gaussians of two submodels at 397x251 177, 179, 81, 71, 74, 74, 78; 100 000 at 512x512
+// 62, 64, 50, 53, 52, 48, 48; four submodels at 648x420 147, 148, 145, 143, 143, 162, 172; a call on each of four submodels at 1600x1036
+// 607, 592, 594, 568, 556, 589, 633; 333 000 at 1013x761 107, 106, 104, 102, 100, 110, 144.
+constexpr float kLongWalk = 0.85f * 0.094e-3f / 0.2f;
+__device__ __forceinline__ uint32_t long_strip_classes(uint32_t entries, float share)
+{
+	const float bound = fmaxf(share * (float)entries, 64.f);
+	return bound < 2048.f ? strip_class((uint32_t)bound) : 0u;
+}
 
 // The calling lane's place among its workgroup's strips of class c (all lanes come here).
 __device__ __forceinline__ uint32_t count_in_class(uint32_t* s_count, uint32_t c, bool valid)
@@ -1558,10 +1877,12 @@ struct StripOrderJob {
 	uint32_t* empty;         // how many strips are empty, and their placement cursor, zero beforehand
 	uint32_t* order;
 	uint32_t* clear;         // per strip, set to zero (may be null)
+	uint32_t* longer;        // receives how many strips are long ones (see long_strip_classes; may be null); behind it a word for the sum of lengths, zero beforehand
 };
 struct StripOrderBatch {
 	StripOrderJob job[kMaxBlendBatch];
 	uint32_t strips;
+	float long_share;  // of all entries: a walk of more is a long one
 };
 
 __global__ __launch_bounds__(256) void strip_count_kernel(StripOrderBatch batch)
@@ -1586,6 +1907,11 @@ __global__ __launch_bounds__(256) void strip_count_kernel(StripOrderBatch batch)
 		atomicAdd(&j.classes[threadIdx.x], s_count[threadIdx.x]);
 	if (threadIdx.x == 0 && s_count[kEmptyClass] != 0u)
 		atomicAdd(&j.empty[0], s_count[kEmptyClass]);
+	if (j.longer) {
+		const uint32_t sum = wave_inclusive_scan_u32(length[0] + length[1] + length[2] + length[3]);
+		if ((threadIdx.x & 63) == 63 && sum != 0u)
+			atomicAdd(&j.longer[1], sum);
+	}
 }
 
 __global__ __launch_bounds__(256) void strip_place_kernel(StripOrderBatch batch)
@@ -1610,6 +1936,8 @@ __global__ __launch_bounds__(256) void strip_place_kernel(StripOrderBatch batch)
 	__syncthreads();
 	uint32_t total;
 	const uint32_t start = block256_exclusive_scan_u32(in_class, s_scan, total);
+	if (j.longer && blockIdx.x == 0 && threadIdx.x == long_strip_classes(j.longer[1], batch.long_share))
+		j.longer[0] = start;
 	const uint32_t mine = s_count[threadIdx.x];
 	__syncthreads();
 	s_count[threadIdx.x] = start + (mine != 0u ? atomicAdd(&j.classes[kStripClasses + threadIdx.x], mine) : 0u);
@@ -1636,15 +1964,25 @@ __global__ __launch_bounds__(1024) void strip_order_kernel(StripOrderBatch batch
 	constexpr uint32_t kPerThread = kOrderAtOnce / 1024;
 	__shared__ uint32_t s_count[kStripClasses + 1];
 	__shared__ uint32_t s_scan[16];
+	__shared__ uint32_t s_total;
 	const StripOrderJob& j = batch.job[blockIdx.x];
 	const uint32_t tid = threadIdx.x, strips = batch.strips;
-	uint32_t c[kPerThread], rank[kPerThread];
+	uint32_t c[kPerThread], rank[kPerThread], sum = 0;
 #pragma unroll
-	for (uint32_t q = 0; q < kPerThread; q++)
+	for (uint32_t q = 0; q < kPerThread; q++) {
 		c[q] = 1024 * q + tid < strips ? j.length[1024 * q + tid] : 0u;
+		sum += c[q];
+	}
 	if (tid <= kStripClasses)
 		s_count[tid] = 0;
+	if (tid == 0)
+		s_total = 0;
 	__syncthreads();
+	if (j.longer) {
+		sum = wave_inclusive_scan_u32(sum);
+		if ((tid & 63) == 63)
+			atomicAdd(&s_total, sum);
+	}
 #pragma unroll
 	for (uint32_t q = 0; q < kPerThread; q++)
 		if (1024 * q < strips) {
@@ -1656,6 +1994,8 @@ __global__ __launch_bounds__(1024) void strip_order_kernel(StripOrderBatch batch
 	const uint32_t start = block_exclusive_scan_u32<16>(tid < kStripClasses ? s_count[tid] : 0u, s_scan, total);
 	if (tid == 0)
 		*j.empty = s_count[kEmptyClass];
+	if (j.longer && tid == long_strip_classes(s_total, batch.long_share))
+		j.longer[0] = start;
 	__syncthreads();
 	if (tid <= kStripClasses)
 		s_count[tid] = start;  // (of the empty class: all the others)
@@ -1676,11 +2016,13 @@ static void launch_strip_order(const BlendArgs* jobs, int count, int which, hipS
 {
 	StripOrderBatch b;
 	b.strips = (uint32_t)(4 * jobs[0].grid_x * jobs[0].grid_y);
+	b.long_share = kLongWalk * (float)count;
 	for (int k = 0; k < count; k++) {
 		b.job[k].length = which == 0 ? jobs[k].strip_total : jobs[k].strip_filed;
 		b.job[k].classes = jobs[k].strip_classes + (which == 0 ? 2 * kStripClasses : 0);
 		b.job[k].clear = which == 0 ? jobs[k].strip_filed : nullptr;  // (the wavefronts that share a strip take the largest of theirs)
 		b.job[k].empty = jobs[k].strip_classes + strip_empty_word(which == 0 ? 1 : 0);
+		b.job[k].longer = which == 0 ? nullptr : jobs[k].strip_classes + kStripLongWord;
 		b.job[k].order = which == 0 ? jobs[k].strip_order_forward : jobs[k].strip_order;
 	}
 	if (b.strips <= kOrderAtOnce) {
@@ -1770,11 +2112,22 @@ void launch_blend_backward(const BlendArgs* jobs, int count, hipStream_t s)
 		for (int k = 0; k < batch.count; k++)
 			batch.job[k] = jobs[at + k];
 		batch.strips = strips;
-		batch.workgroups = blend_workgroups(strips, batch.count);
-		const dim3 grid(batch.workgroups * (unsigned)batch.count);
 		bool depth = false;  // does any job of the batch bring a gradient of the depth image?
 		for (int k = 0; k < batch.count; k++)
 			depth = depth || batch.job[k].dL_dpix_depth != nullptr;
+		const unsigned jobs = (unsigned)batch.count;
+		if ((size_t)strips * jobs <= kStripWorkgroups) {
+			// (with more strips than that, few walks are long against the launch: 517 us for 1600x1036 and four submodels, 550 by this kernel)
+			batch.workgroups = (strips + kSharedWaves - 1) / kSharedWaves + 1024u / jobs;
+			const dim3 grid(batch.workgroups * jobs), threads(64 * kSharedWaves);
+			if (depth)
+				hipLaunchKernelGGL(blend_backward_shared_kernel<true>, grid, threads, 0, s, batch);
+			else
+				hipLaunchKernelGGL(blend_backward_shared_kernel<false>, grid, threads, 0, s, batch);
+			continue;
+		}
+		batch.workgroups = blend_workgroups(strips, batch.count);
+		const dim3 grid(batch.workgroups * jobs);
 		if (depth)
 			hipLaunchKernelGGL(blend_backward_kernel<true>, grid, dim3(64), 0, s, batch);
 		else

@@ -471,7 +471,7 @@ void launch_report_sort_status(const uint32_t* temp, uint32_t* fault, uint32_t* 
 // and sets *fault (host memory the device can write, may be null).  The caller has cleared `ranges`.  With a non-null
 // n_device the number of keys is min(n, *n_device) and the launch is sized for n.  file_tail (may be null)
 // receives, per kFileGroup keys, how many entries of the tile of the last of them have each strip bit set.
-constexpr int kRangeTailWords = 1028;   // words behind the ranges: the strip class counters of the blend
+constexpr int kRangeTailWords = 1032;   // words behind the ranges: the strip class counters of the blend
 struct TileRangesJob {
 	const uint32_t* keys;
 	size_t n;

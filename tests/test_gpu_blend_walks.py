@@ -99,3 +99,21 @@ def test_entries_that_need_every_comparison_of_a_visit(case):
     _check_forward_stages(sub, cam, torch.tensor([0.2, 0.1, 0.05]), max_borderline=5e-3)
     if case == "opaque":   # (a needle's gradients are differences of terms a million times as large, in the checker as here)
         _check_backward(sub, cam, torch.tensor([0.2, 0.1, 0.05]), seed=7, with_depth_alpha=True)
+
+
+@pytest.mark.parametrize("faces", (False, True))
+@pytest.mark.parametrize("n,with_depth_alpha", [(64, False), (65, True), (73, False), (200, True), (257, False), (521, True), (1203, False)])
+def test_backward_walks_shared_by_four_wavefronts(n, with_depth_alpha, faces):
+    """Strips that blend all of n entries: walks of one chunk by one wavefront, and by four with every number of chunks against the
+    buffers they are staged in, the last pass of a chunk full, partly filled or missing for some of the wavefronts."""
+    gen = torch.Generator().manual_seed(n)
+    scene = scenes.cube_scene(n, seed=71)
+    scene["xyz"] = torch.randn(n, 3, generator=gen) * torch.tensor([0.05, 0.05, 0.3]) + torch.tensor([0.0, 0.0, 4.0])
+    scene["scales"] = torch.full((n, 3), 0.3) * (0.5 + torch.rand(n, 3, generator=gen))
+    scene["opacity"] = 3.0 / n + 2.0 / n * torch.rand(n, 1, generator=gen) + 0.004
+    cam = scenes.look_at_camera((0.0, 0.0, 0.0), (0.03, -0.02, 4.0), (0.1, -1, 0), 43, 22, 12.0)
+    low, up = ((-0.2, -9.0, -9.0), (9.0, 0.15, 4.3)) if faces else ((-99.0,) * 3, (99.0,) * 3)
+    sub = _scene_sub(scene, low=torch.tensor(low), up=torch.tensor(up))
+    st = _check_forward_stages(sub, cam, torch.tensor([0.2, 0.1, 0.05]), max_borderline=5e-2)
+    assert faces or np.mean(st.n_contrib > 0.9 * n) > 0.5
+    _check_backward(sub, cam, torch.tensor([0.2, 0.1, 0.05]), seed=n, with_depth_alpha=with_depth_alpha)
