@@ -369,6 +369,19 @@ int rgs_composite_backward(int K, int height, int width,
                            const float* background, const float* g_image, const float* g_depth,
                            const float* g_alpha, float* const* d_images, float* const* d_depths,
                            float* const* d_alphas, void* stream);
+/* The same for layers as rgs_forward_raster or rgs_frame_forward_raster left them: strip_counts (HOST array of K device pointers, some
+ * may be NULL) names the layers' RGS_IMG_STRIP_TOTAL words in their image workspaces, unchanged since, and layer_background the three
+ * floats that all of them had as background.  If that is black, a layer's planes are not read where its strip
+ * lists nothing.  Without strip_counts or layer_background (NULL): as above. */
+int rgs_composite_layers_forward(int K, int height, int width,
+                                 const float* const* images, const float* const* depths, const float* const* alphas,
+                                 const float* background, const uint32_t* const* strip_counts, const float* layer_background,
+                                 float* out_image, float* out_depth, float* out_alpha, void* stream);
+int rgs_composite_layers_backward(int K, int height, int width,
+                                  const float* const* images, const float* const* depths, const float* const* alphas,
+                                  const float* background, const uint32_t* const* strip_counts, const float* layer_background,
+                                  const float* g_image, const float* g_depth, const float* g_alpha, float* const* d_images,
+                                  float* const* d_depths, float* const* d_alphas, void* stream);
 
 /* ---- boundary straddlers: what a submodel lends to its neighbours ---------------------------
  * The reference picks, per source submodel, the Gaussians whose 3-sigma cube reaches a face of

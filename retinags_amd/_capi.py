@@ -108,6 +108,8 @@ def _load():
     pp = C.POINTER(vp)
     lib.rgs_composite_forward.argtypes = [i, i, i, pp, pp, pp, vp, vp, vp, vp, vp]
     lib.rgs_composite_backward.argtypes = [i, i, i, pp, pp, pp, vp, vp, vp, vp, pp, pp, pp, vp]
+    lib.rgs_composite_layers_forward.argtypes = [i, i, i, pp, pp, pp, vp, pp, vp, vp, vp, vp, vp]
+    lib.rgs_composite_layers_backward.argtypes = [i, i, i, pp, pp, pp, vp, pp, vp, vp, vp, vp, pp, pp, pp, vp]
     lib.rgs_straddler_scratch_bytes.restype, lib.rgs_straddler_scratch_bytes.argtypes = sz, [i, i]
     fp = C.POINTER(C.c_float)
     lib.rgs_straddler_select.argtypes = [i, vp, vp, fp, fp, i, fp, fp, i, vp, vp, C.c_uint32, vp, vp]
@@ -124,7 +126,8 @@ def _load():
     lib.rgs_blend_work_counters.argtypes = [i, i, i, i, f, f, vp, vp, vp, vp, vp, vp, vp, vp, vp]
     for name in ("rgs_stage_timing", "rgs_stage_timing_read", "rgs_blend_work_counters", "rgs_geom_layout", "rgs_binning_layout", "rgs_image_layout", "rgs_mark_visible", "rgs_covariance3d",
                  "rgs_forward_geom", "rgs_forward_geom_enqueue", "rgs_forward_raster", "rgs_forward_raster_bounded", "rgs_backward", "rgs_inclusive_sum", "rgs_sort_pairs",
-                 "rgs_composite_forward", "rgs_composite_backward", "rgs_straddler_select", "rgs_merge_rows",
+                 "rgs_composite_forward", "rgs_composite_backward", "rgs_composite_layers_forward", "rgs_composite_layers_backward",
+                 "rgs_straddler_select", "rgs_merge_rows",
                  "rgs_merge_rows_backward", "rgs_l1_ssim_forward", "rgs_l1_ssim_backward", "rgs_adam_step",
                  "rgs_activate_forward", "rgs_activate_backward", "rgs_sort_pairs_static", "rgs_sort_fault",
                  "rgs_set_lookback_spin_limit", "rgs_frame_forward_geom", "rgs_frame_forward_raster",
@@ -139,6 +142,7 @@ EXPORTS = ("rgs_version", "rgs_last_error", "rgs_get_higher_msb", "rgs_geom_byte
            "rgs_image_bytes", "rgs_geom_layout", "rgs_binning_layout", "rgs_image_layout", "rgs_mark_visible", "rgs_covariance3d",
            "rgs_forward_geom", "rgs_forward_geom_enqueue", "rgs_forward_raster", "rgs_forward_raster_bounded", "rgs_backward", "rgs_scan_temp_bytes", "rgs_inclusive_sum",
            "rgs_sort_temp_bytes", "rgs_sort_pairs", "rgs_composite_forward", "rgs_composite_backward",
+           "rgs_composite_layers_forward", "rgs_composite_layers_backward",
            "rgs_stage_timing", "rgs_stage_timing_read", "rgs_blend_work_counters", "rgs_straddler_scratch_bytes",
            "rgs_straddler_select", "rgs_merge_rows", "rgs_merge_rows_backward", "rgs_loss_workspace_bytes",
            "rgs_l1_ssim_forward", "rgs_l1_ssim_backward", "rgs_adam_step", "rgs_activate_forward",

@@ -21,25 +21,35 @@ def composite_partial_images(images: Sequence[torch.Tensor], depths: Sequence[to
     images[k]: (3,H,W); depths[k], alphas[k]: (1,H,W).  Returns (image, depth, alpha).
     More than MAX_COMPOSITE inputs are folded in groups: compositing is associative in
     (image, depth, alpha) when the inner groups use a black background."""
+    return _composite(images, depths, alphas, background, None)
+
+
+def _composite(images, depths, alphas, background, strips):
+    """composite_partial_images; strips[k], if the list is given: what the rasterizer says of layer k beside its planes."""
     K = len(images)
     if K == 0 or len(depths) != K or len(alphas) != K:
         raise RuntimeError("composite_partial_images needs K >= 1 images, depths and alphas")
     images, depths, alphas = list(images), list(depths), list(alphas)
+    if K > _capi.MAX_COMPOSITE:
+        strips = None
     while len(images) > _capi.MAX_COMPOSITE:
         n = _capi.MAX_COMPOSITE
         img, dep, alp = _host.composite(None, images[:n] + depths[:n] + alphas[:n])
         images, depths, alphas = [img] + images[n:], [dep] + depths[n:], [alp] + alphas[n:]
-    return _host.composite(background, images + depths + alphas)
+    return _host.composite(background, images + depths + alphas, strips)
 
 
-def blender_render_result(render_results: Dict[int, dict], relation_vector, background: Optional[torch.Tensor]):
+def blender_render_result(render_results: Dict[int, dict], relation_vector, background: Optional[torch.Tensor],
+                          strips: Optional[Dict[int, tuple]] = None):
     """Same contract as the reference function of this name
     (parallel_utils/basic_parallel_trainer/result_aggregator.py:193-260) for one camera on
     one GPU: `render_results` maps submodel id -> {"render","depth","alpha"} (what
     render4renderinfo returns), `relation_vector[model_id]` is the compositing rank of that
     submodel or a negative value when it is not related to the camera.  Returns a dict with
     "render", "depth", "alpha".  A missing background draws a random colour, like the
-    reference (:256)."""
+    reference (:256).
+    strips: for results that come straight from rasterize_frame, what it handed out under that name by submodel id; planes
+    are then not read where their submodel shows nothing."""
     if isinstance(relation_vector, torch.Tensor):
         relation_vector = relation_vector.cpu().numpy()
     related = [(int(relation_vector[m]), m) for m in render_results if relation_vector[m] >= 0]
@@ -50,8 +60,8 @@ def blender_render_result(render_results: Dict[int, dict], relation_vector, back
     pk = [render_results[m] for _, m in related]
     device = pk[0]["render"].device
     bkg = background if background is not None else torch.rand((3,), device=device)
-    image, depth, alpha = composite_partial_images([p["render"] for p in pk], [p["depth"] for p in pk],
-                                                   [p["alpha"] for p in pk], bkg)
+    image, depth, alpha = _composite([p["render"] for p in pk], [p["depth"] for p in pk], [p["alpha"] for p in pk], bkg,
+                                     None if strips is None else [strips[m] for _, m in related])
     return {"render": image, "depth": depth, "alpha": alpha}
 
 

@@ -1254,7 +1254,8 @@ int rgs_sort_fault(void* stream)
 }
 
 static int fill_composite(rgs::CompositeArgs& a, int K, int height, int width, const float* const* images,
-                          const float* const* depths, const float* const* alphas, const float* background)
+                          const float* const* depths, const float* const* alphas, const float* background,
+                          const uint32_t* const* strip_counts, const float* layer_background)
 {
 	RGS_REQUIRE(K >= 1 && K <= RGS_MAX_COMPOSITE, "composite: K=%d outside 1..%d", K, RGS_MAX_COMPOSITE);
 	RGS_REQUIRE(height > 0 && width > 0, "composite: bad image size %dx%d", width, height);
@@ -1266,7 +1267,10 @@ static int fill_composite(rgs::CompositeArgs& a, int K, int height, int width, c
 		a.images[k] = images[k];
 		a.depths[k] = depths[k];
 		a.alphas[k] = alphas[k];
+		if (strip_counts)
+			a.strips[k] = strip_counts[k];
 	}
+	a.layer_bg = strip_counts ? layer_background : nullptr;
 	return 0;
 }
 
@@ -1275,11 +1279,20 @@ int rgs_composite_forward(int K, int height, int width,
                           const float* background, float* out_image, float* out_depth, float* out_alpha,
                           void* stream)
 {
+	return rgs_composite_layers_forward(K, height, width, images, depths, alphas, background, nullptr, nullptr, out_image, out_depth,
+	                                    out_alpha, stream);
+}
+
+int rgs_composite_layers_forward(int K, int height, int width,
+                                 const float* const* images, const float* const* depths, const float* const* alphas,
+                                 const float* background, const uint32_t* const* strip_counts, const float* layer_background,
+                                 float* out_image, float* out_depth, float* out_alpha, void* stream)
+{
 	hipStream_t s = static_cast<hipStream_t>(stream);
 	EntryScope scope_(s);
 	const int debug = 0;
 	rgs::CompositeArgs a;
-	if (int rc = fill_composite(a, K, height, width, images, depths, alphas, background))
+	if (int rc = fill_composite(a, K, height, width, images, depths, alphas, background, strip_counts, layer_background))
 		return rc;
 	RGS_REQUIRE(out_image && out_depth && out_alpha, "rgs_composite_forward: null output");
 	a.out_image = out_image; a.out_depth = out_depth; a.out_alpha = out_alpha;
@@ -1294,11 +1307,21 @@ int rgs_composite_backward(int K, int height, int width,
                            const float* g_alpha, float* const* d_images, float* const* d_depths,
                            float* const* d_alphas, void* stream)
 {
+	return rgs_composite_layers_backward(K, height, width, images, depths, alphas, background, nullptr, nullptr, g_image, g_depth,
+	                                     g_alpha, d_images, d_depths, d_alphas, stream);
+}
+
+int rgs_composite_layers_backward(int K, int height, int width,
+                                  const float* const* images, const float* const* depths, const float* const* alphas,
+                                  const float* background, const uint32_t* const* strip_counts, const float* layer_background,
+                                  const float* g_image, const float* g_depth, const float* g_alpha, float* const* d_images,
+                                  float* const* d_depths, float* const* d_alphas, void* stream)
+{
 	hipStream_t s = static_cast<hipStream_t>(stream);
 	EntryScope scope_(s);
 	const int debug = 0;
 	rgs::CompositeArgs a;
-	if (int rc = fill_composite(a, K, height, width, images, depths, alphas, background))
+	if (int rc = fill_composite(a, K, height, width, images, depths, alphas, background, strip_counts, layer_background))
 		return rc;
 	RGS_REQUIRE(g_image && d_images && d_alphas && (d_depths || !g_depth), "rgs_composite_backward: null pointer");
 	a.g_image = g_image; a.g_depth = g_depth; a.g_alpha = g_alpha;

@@ -46,9 +46,29 @@ struct PlaneTables {
 	}
 };
 
+// What the layers of a frame bring beside their planes, if they come straight from the rasterizer: their image workspaces, in which it says what
+// each strip lists, and the background they all had.
+struct LayerStrips {
+	variable_list images;  // per layer, undefined ones for layers without
+	Tensor background;
+};
+
 // Outputs image, depth, alpha.  `planes`: the layers' colours, then their depths, then their alphas.
 struct Composite : torch::autograd::Function<Composite> {
-	static variable_list forward(AutogradContext* ctx, at::TensorList planes, const std::optional<Tensor>* background)
+	using StripTable = std::array<const uint32_t*, RGS_MAX_COMPOSITE>;
+	static StripTable strip_table(const Tensor* images, int K, int64_t H, int64_t W)
+	{
+		std::array<size_t, RGS_IMG_FIELDS> offset;
+		check(rgs_image_layout(W, H, offset.data()));
+		StripTable t{};
+		for (int k = 0; k < K; k++)
+			if (const char* image = ptr<const char>(images[k]))
+				t[k] = reinterpret_cast<const uint32_t*>(image + offset[RGS_IMG_STRIP_TOTAL]);
+		return t;
+	}
+
+	static variable_list forward(AutogradContext* ctx, at::TensorList planes, const std::optional<Tensor>* background,
+	                             const LayerStrips* strips)
 	{
 		const int K = static_cast<int>(planes.size() / 3);
 		const at::Device device = planes[0].device();
@@ -56,7 +76,7 @@ struct Composite : torch::autograd::Function<Composite> {
 			throw std::runtime_error("the compositor needs its inputs on a GPU (device memory)");
 		const int64_t H = planes[0].size(-2), W = planes[0].size(-1);
 		variable_list saved;
-		saved.reserve(3 * K + 1);
+		saved.reserve(4 * K + 2);
 		for (int k = 0; k < 3 * K; k++)
 			saved.push_back(plane(planes[k], device, k < K ? 3 : 1, H, W));
 		const Tensor bg = background_of(*background, device);
@@ -65,12 +85,22 @@ struct Composite : torch::autograd::Function<Composite> {
 			in.set(k, saved[k], saved[K + k], saved[2 * K + k]);
 		const Tensor image = new_f32({3, H, W}, device), depth = new_f32({1, H, W}, device), alpha = new_f32({1, H, W}, device);
 		c10::DeviceGuard guard(device);
-		check(rgs_composite_forward(K, H, W, in.images.data(), in.depths.data(), in.alphas.data(), ptr(bg), ptr(image), ptr(depth),
-		                            ptr(alpha), current_stream(device)));
+		const bool with_strips = strips->background.defined();
+		StripTable counts{};
+		if (with_strips)
+			counts = strip_table(strips->images.data(), K, H, W);
+		check(rgs_composite_layers_forward(K, H, W, in.images.data(), in.depths.data(), in.alphas.data(), ptr(bg),
+		                                   with_strips ? counts.data() : nullptr, ptr(strips->background), ptr(image), ptr(depth),
+		                                   ptr(alpha), current_stream(device)));
 		// an absent depth or alpha gradient comes back undefined and goes down as a null pointer
 		ctx->set_materialize_grads(false);
 		saved.push_back(bg);
+		if (with_strips) {
+			saved.push_back(strips->background);
+			saved.insert(saved.end(), strips->images.begin(), strips->images.end());
+		}
 		ctx->save_for_backward(std::move(saved));
+		ctx->saved_data["strips"] = with_strips;
 		return {image, depth, alpha};
 	}
 
@@ -78,7 +108,8 @@ struct Composite : torch::autograd::Function<Composite> {
 	{
 		return in_backward([&]() -> variable_list {
 			const variable_list saved = ctx->get_saved_variables();
-			const int K = static_cast<int>(saved.size() / 3);
+			const bool with_strips = ctx->saved_data["strips"].toBool();
+			const int K = static_cast<int>(with_strips ? (saved.size() - 2) / 4 : saved.size() / 3);
 			const at::Device device = saved[0].device();
 			const int64_t H = saved[0].size(1), W = saved[0].size(2);
 			auto given = [&](const Tensor& g, int64_t channels) { return g.defined() ? plane(g, device, channels, H, W) : Tensor(); };
@@ -92,7 +123,7 @@ struct Composite : torch::autograd::Function<Composite> {
 			// depths have none either; told so, the rasterizer's backward leaves out the terms it would multiply.
 			const bool with_depth = g_depth.defined();
 			const int64_t planes = with_depth ? 5 : 4;
-			variable_list out(3 * K + 1);
+			variable_list out(3 * K + 2);
 			for (int k = 0; k < K; k++) {
 				in.set(k, saved[k], saved[K + k], saved[2 * K + k]);
 				// a layer's three gradients in one (5,H,W) block, the layout of RenderResult.zip_grad
@@ -107,22 +138,49 @@ struct Composite : torch::autograd::Function<Composite> {
 				out[2 * K + k] = block.narrow(0, planes - 1, 1);
 			}
 			c10::DeviceGuard guard(device);
-			check(rgs_composite_backward(K, H, W, in.images.data(), in.depths.data(), in.alphas.data(), ptr(saved[3 * K]), ptr(g_image),
-			                             ptr(g_depth), ptr(g_alpha), d_images.data(), with_depth ? d_depths.data() : nullptr,
-			                             d_alphas.data(), current_stream(device)));
+			StripTable counts{};
+			if (with_strips)
+				counts = strip_table(&saved[3 * K + 2], K, H, W);
+			check(rgs_composite_layers_backward(K, H, W, in.images.data(), in.depths.data(), in.alphas.data(), ptr(saved[3 * K]),
+			                                    with_strips ? counts.data() : nullptr, with_strips ? ptr(saved[3 * K + 1]) : nullptr,
+			                                    ptr(g_image), ptr(g_depth), ptr(g_alpha), d_images.data(),
+			                                    with_depth ? d_depths.data() : nullptr, d_alphas.data(), current_stream(device)));
 			return out;
 		});
 	}
 };
 
-py::tuple composite(const std::optional<Tensor>& background, const std::vector<Tensor>& planes)
+// `strips`: None, or what rasterize_frame handed out under that name for these layers, in their order here.
+py::tuple composite(const std::optional<Tensor>& background, const std::vector<Tensor>& planes, py::handle strips)
 {
 	if (planes.empty() || planes.size() % 3 != 0 || planes.size() > 3 * RGS_MAX_COMPOSITE)
 		throw std::runtime_error("the compositor takes between one layer and " + std::to_string(RGS_MAX_COMPOSITE) + " layers");
+	LayerStrips known;
+	if (!strips.is_none()) {
+		const size_t K = planes.size() / 3;
+		const int64_t bytes = static_cast<int64_t>(rgs_image_bytes(planes[0].size(-1), planes[0].size(-2)));
+		bool one_background = true;
+		for (py::handle h : py::reinterpret_borrow<py::sequence>(strips)) {
+			const py::tuple layer = py::reinterpret_borrow<py::tuple>(h);
+			const Tensor image = from_python(layer[0], "an image workspace"), bg = tensor_from_python(layer[1], "a background");
+			if (present(image) && (image.numel() != bytes || image.scalar_type() != at::kByte || !image.is_contiguous() ||
+			                       image.device() != planes[0].device()))
+				throw std::runtime_error("the image workspace is not that of such an image");
+			if (!known.background.defined())
+				known.background = bg;
+			one_background = one_background && bg.data_ptr() == known.background.data_ptr();
+			known.images.push_back(image);
+		}
+		if (known.images.size() != K)
+			throw std::runtime_error("the strips of every layer are needed");
+		if (!one_background || known.background.numel() != 3 || known.background.scalar_type() != at::kFloat ||
+		    known.background.device() != planes[0].device() || !known.background.is_contiguous())
+			known = LayerStrips();
+	}
 	variable_list out;
 	{
 		py::gil_scoped_release no_gil;
-		out = Composite::apply(at::TensorList(planes), &background);
+		out = Composite::apply(at::TensorList(planes), &background, &known);
 	}
 	return py::make_tuple(out[0], out[1], out[2]);
 }
@@ -661,11 +719,13 @@ struct FrameLayer {
 	int M = 0;
 	Rendered rendered;
 	Tensor radii, geom;
+	Tensor image, background;  // see Frame::keep_strips
 };
 
 struct Frame : torch::CustomClassHolder {
 	std::vector<FrameLayer> layers;
 	bool keep_workspaces = false;
+	bool keep_strips = false;  // the image workspaces, and the backgrounds as the library saw them, for the compositor
 };
 
 // The submodels that a camera sees ("layers"), rasterized together: what the reference does with one call per submodel
@@ -729,6 +789,7 @@ struct RasterizeFrame : torch::autograd::Function<RasterizeFrame> {
 				rgs_frame_layer& L = arr.back();
 				const Tensor bg = device_f32(l.s.bg, device), low = device_f32(l.s.low, device), up = device_f32(l.s.up, device);
 				keep.insert(keep.end(), {bg, low, up, t[kOpacities]});
+				l.background = bg;
 				const size_t geom_bytes = rgs_geom_bytes(l.P);
 				l.geom = new_bytes(geom_bytes, device);
 				r.image = new_bytes(image_bytes, device);
@@ -781,6 +842,9 @@ struct RasterizeFrame : torch::autograd::Function<RasterizeFrame> {
 			}
 			check(rgs_frame_forward_raster(n, arr.data(), &view, main, s0.debug));
 		}
+		if (frame.keep_strips)
+			for (int k : live)
+				frame.layers[k].image = frame.layers[k].rendered.image;
 		ctx->set_materialize_grads(false);  // an output that took no part in the loss comes back undefined
 		ctx->save_for_backward(std::move(saved));
 		ctx->mark_non_differentiable(radii);
@@ -889,7 +953,10 @@ struct RasterizeFrame : torch::autograd::Function<RasterizeFrame> {
 
 // `inputs`: per layer the kInputs tensors, empty ones for those that are absent.  `streams`: None, or a stream handle per layer.
 // `workspaces`: None, or a list that receives (instances, geometry, binning and image workspace) per layer.
-py::list rasterize_frame(const py::sequence& settings, const py::sequence& inputs, py::handle streams, py::handle workspaces)
+// `strips`: None, or a list that receives per layer its image workspace (None for a layer without Gaussians) and its background, which is
+// what _host.composite takes under that name.
+py::list rasterize_frame(const py::sequence& settings, const py::sequence& inputs, py::handle streams, py::handle workspaces,
+                         py::handle strips)
 {
 	const size_t K = settings.size();
 	if (K == 0 || inputs.size() != kInputs * K)
@@ -899,6 +966,7 @@ py::list rasterize_frame(const py::sequence& settings, const py::sequence& input
 	auto frame = c10::make_intrusive<Frame>();
 	frame->layers.resize(K);
 	frame->keep_workspaces = !workspaces.is_none();
+	frame->keep_strips = !strips.is_none();
 	variable_list flat;
 	flat.reserve(K * kInputs);
 	for (size_t k = 0; k < K; k++) {
@@ -922,6 +990,11 @@ py::list rasterize_frame(const py::sequence& settings, const py::sequence& input
 			workspaces.attr("append")(py::make_tuple(l.rendered.instances, l.geom, l.rendered.binning, l.rendered.image));
 			l.geom = l.rendered.binning = l.rendered.image = Tensor();
 		}
+	for (FrameLayer& l : frame->layers) {
+		if (frame->keep_strips)
+			strips.attr("append")(py::make_tuple(to_python(l.image), l.background.defined() ? l.background : l.s.bg));
+		l.image = l.background = Tensor();
+	}
 	py::list result;
 	for (size_t k = 0; k < K; k++)
 		result.append(py::make_tuple(out[4 * k], out[4 * k + 1], out[4 * k + 2], out[4 * k + 3]));
@@ -970,14 +1043,15 @@ PYBIND11_MODULE(_host, m)
 		}
 	});
 
-	m.def("composite", &composite);
+	m.def("composite", &composite, py::arg("background"), py::arg("planes"), py::arg("strips") = py::none());
 	m.def("gradient_outputs", &gradient_outputs);
 	m.def("set_original_gradient_outputs", &set_original_gradient_outputs);
 	m.def("rasterize", &rasterize);
 	m.def("rasterize_forward", &rasterize_forward);
 	m.def("rasterize_forward_from_stage", &rasterize_forward_from_stage);
 	m.def("rasterize_backward", &rasterize_backward);
-	m.def("rasterize_frame", &rasterize_frame);
+	m.def("rasterize_frame", &rasterize_frame, py::arg("settings"), py::arg("inputs"), py::arg("streams"), py::arg("workspaces"),
+	      py::arg("strips") = py::none());
 	m.def("enqueue_geometry", &enqueue_geometry);
 	define_training(m);
 

@@ -135,6 +135,10 @@ struct CompositeArgs {
 	float* d_images[kMaxComposite];
 	float* d_depths[kMaxComposite];
 	float* d_alphas[kMaxComposite];
+	// Layers as the rasterizer left them: entries filed per 16x4 strip (four per tile, tiles row by row; null for a layer that came
+	// otherwise) and their common background.  No layer has any if layer_bg is null.
+	const uint32_t* strips[kMaxComposite];
+	const float* layer_bg;
 };
 
 // Boundary straddlers (sharing.hip).  Boxes are passed by value: at most kMaxShareBoxes per launch.

@@ -355,6 +355,7 @@ def render_frame(cam: Camera, subs: List[Submodel], relation: np.ndarray, backgr
         submodel_bg = torch.zeros(3, device=device)
     related = [m for m in range(len(subs)) if relation[m] >= 0]
     stages = {}
+    strips = None
     if together:
         if instance_bounds is not None or host_threads:
             raise ValueError("together=True takes neither instance_bounds nor host_threads")
@@ -369,9 +370,13 @@ def render_frame(cam: Camera, subs: List[Submodel], relation: np.ndarray, backgr
             inputs.append(dict(means3D=sub.means3D, means2D=means2D, shs=sub.shs, opacities=sub.opacity, scales=sub.scales,
                                rotations=sub.rotations))
         taps = [] if keep_workspaces else None
+        # from two million pixels of all layers on the compositor passes over what they do not show (four submodels, both
+        # directions: 63 -> 49 us at 1600x1036, 808 -> 530 at 5185x3359; 13.0 -> 13.5 at 648x420)
+        listed = [] if cam.image_height * cam.image_width * len(related) >= 1 << 21 else None
         outs = _rasterize_layers(settings, inputs,
                                  streams=[lanes[k % len(lanes)].cuda_stream for k in range(len(related))] if streams else None,
-                                 workspaces=taps)
+                                 workspaces=taps, strips=listed)
+        strips = None if listed is None else dict(zip(related, listed))
         partial = {}
         for k, m in enumerate(related):
             color, radii, depth, alpha = outs[k]
@@ -447,7 +452,7 @@ def render_frame(cam: Camera, subs: List[Submodel], relation: np.ndarray, backgr
             for t in res.values():
                 if torch.is_tensor(t) and t.is_cuda:
                     t.record_stream(main)
-    out = blender_render_result(partial, relation, background)
+    out = blender_render_result(partial, relation, background, strips)
     out["partial"] = partial
     out["stages"] = stages
     if together and keep_workspaces:

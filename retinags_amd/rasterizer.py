@@ -227,14 +227,15 @@ def rasterize_frame(rasterizers, inputs, streams=None, workspaces=None):
     return _rasterize_layers([rz.raster_settings for rz in rasterizers], inputs, streams, workspaces)
 
 
-def _rasterize_layers(settings, inputs, streams=None, workspaces=None):
-    """rasterize_frame from the layers' settings."""
+def _rasterize_layers(settings, inputs, streams=None, workspaces=None, strips=None):
+    """rasterize_frame from the layers' settings.  `strips`: a list that receives what the compositor can use of each layer
+    (see _host.composite)."""
     flat = []
     for kw in inputs:
         shs, colors_precomp, scales, rotations, cov3D = _checked_inputs(kw.get("shs"), kw.get("colors_precomp"), kw.get("scales"),
                                                                         kw.get("rotations"), kw.get("cov3D_precomp"))
         flat += (kw["means3D"], kw["means2D"], shs, colors_precomp, kw["opacities"], scales, rotations, cov3D)
-    return _host.rasterize_frame(settings, flat, streams, workspaces)
+    return _host.rasterize_frame(settings, flat, streams, workspaces, strips)
 
 
 def _checked_inputs(shs, colors_precomp, scales, rotations, cov3D_precomp):
