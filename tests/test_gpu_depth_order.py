@@ -95,3 +95,26 @@ def test_sorts_in_the_largest_tiles():
 def test_totals_of_ragged_groups(n):
     """All in view: the sums of 1 024 tile counts where the last group is whole, short of a quad or a few counts beyond."""
     check_sorts(n, 400, 300)
+
+
+@pytest.mark.parametrize("n", (9, 65, 4095, 4096, 4097, 8191, 8192, 8193, 8192 + 1027))
+def test_order_of_few_gaussians_by_one_workgroup(n):
+    """Up to 8 192 Gaussians are ordered out of LDS, four or eight per thread; one more by the general path."""
+    check_sorts(n, 400, 300)
+
+
+@pytest.mark.parametrize("n", (900, 4096, 8000, 9000))
+def test_depths_that_need_the_fourth_pass(n):
+    """Gaussians at depths below and beyond 8 192, equal depths among them and a third behind the camera, on both sides of the bound up to which one
+    workgroup orders them: depth order and offsets against a stable argsort, the images against the checker."""
+    from test_gpu_rasterizer_parity import _check_forward_stages, _scene_sub
+    scene = scenes.cube_scene(n, seed=n)
+    scene["xyz"][1::2] = scene["xyz"][::2][:scene["xyz"][1::2].shape[0]]
+    far, behind = torch.arange(n) % 4 >= 2, torch.arange(n) % 3 == 0
+    scene["xyz"][far] *= 4000.0
+    scene["scales"][far] *= 4000.0
+    scene["xyz"][behind, 2] *= -1.0
+    cam = scenes.look_at_camera((0, 0, 0), (0, 0, 1), (0, -1, 0), 160, 100, 60.0)
+    st = _check_forward_stages(_scene_sub(scene), cam, torch.tensor([0.1, 0.2, 0.3]), max_borderline=2e-3)
+    listed = st.depths[st.radii > 0]
+    assert listed.max() > 8192 and listed.min() < 8 and 0.3 * n < len(listed) < 0.8 * n
