@@ -271,6 +271,14 @@ typedef struct rgs_frame_layer {
 	void* stream;              /* NULL, or a second HIP stream for rgs_frame_backward (the forward calls ignore it): work that is
 	                              bound by memory bandwidth (the per-Gaussian backward of the layers whose blend is done) then
 	                              runs on it beside the blend, which is bound by instruction issue; the frame's stream waits for it */
+	/* SH rows in parts, of every layer of a call or of none (sh_rest NULL): M is 16; of Gaussians 0..sh_own-1 shs holds the first
+	 * coefficients (sh_own, 3) and sh_rest the others (sh_own, 45), of the rest sh_lent holds whole rows (P - sh_own, 48).  Their
+	 * gradients go to dL_dsh, dL_dsh_rest and dL_dsh_lent; those three and sh_lent start at multiples of 16 bytes. */
+	const float* sh_rest;
+	const float* sh_lent;
+	int sh_own;
+	float* dL_dsh_rest;
+	float* dL_dsh_lent;
 } rgs_frame_layer;
 /* rgs_forward_geom for every layer (P > 0 each): every geometry stage of every layer is queued on `stream` (one
  * launch per stage for all layers; rgs_frame_layer.stream is not looked at by the forward) before the host waits for
@@ -476,6 +484,91 @@ int rgs_activate_backward(int n, int rest, const float* rotation, const float* s
                           const float* g_shs, const float* g_scales, const float* g_rotations, const float* g_opacities,
                           float* d_features_dc, float* d_features_rest, float* d_scaling, float* d_rotation,
                           float* d_opacity, void* stream);
+
+/* ---- the stored models of a frame together ------------------------------------------------------
+ * Activation, selection and lending for up to RGS_MAX_STORED_MODELS models that the frame's rasterizer reads with SH rows in parts (see
+ * rgs_frame_layer.sh_rest), one launch per step for all of them.  All tables are HOST arrays of device pointers; arrays start at multiples
+ * of 16 bytes but for features_dc / features_rest and the gradients of those. */
+#define RGS_MAX_STORED_MODELS 16
+/* rgs_activate_forward but for the SH rows: scaling (n,3), rotation (n,4), opacity (n,1) -> scales, rotations, opacities; and zero_rows rows
+ * of means2D (.,3), the screen-space placeholder (render_half_gs.py:7-14), set to zero. */
+typedef struct rgs_stored_model {
+	int n, zero_rows;
+	const float* scaling;
+	const float* rotation;
+	const float* opacity;
+	float* scales;
+	float* rotations;
+	float* opacities;
+	float* means2D;
+} rgs_stored_model;
+int rgs_activate_models(int n_models, const rgs_stored_model* models, void* stream);
+/* Its backward, all gradients present; d_meta (n,1) receives the length of the (x, y) gradient of each row of means2D
+ * (render_half_gs.py:16-18). */
+typedef struct rgs_stored_model_grads {
+	int n;
+	const float* rotation;
+	const float* scales;
+	const float* opacities;
+	const float* g_scales;
+	const float* g_rotations;
+	const float* g_opacities;
+	const float* g_means2D;
+	float* d_scaling;
+	float* d_rotation;
+	float* d_opacity;
+	float* d_meta;
+} rgs_stored_model_grads;
+int rgs_activate_models_backward(int n_models, const rgs_stored_model_grads* models, void* stream);
+/* rgs_straddler_select for every source, source k in box k of the n_sources boxes and lending to the others. */
+typedef struct rgs_straddler_source {
+	int n;
+	const float* means3D;
+	const float* scales;
+	uint32_t* counts;
+	uint32_t* rows;
+	uint32_t capacity;
+	void* scratch;
+} rgs_straddler_source;
+int rgs_straddler_select_many(int n_sources, const rgs_straddler_source* sources, const float* boxes_low, const float* boxes_up,
+                              void* stream);
+/* One list of rows that `source` lends to `destination`: row rows[j] of the source goes to row at + j of the destination's merged arrays and
+ * to row sh_at + j of its sh_lent.  rows NULL, for a source that is its own destination: positions 0..count-1 from means3D_from to
+ * means3D, for merged positions in an array of their own. */
+typedef struct rgs_lend_segment {
+	int source, destination;
+	const uint32_t* rows;
+	uint32_t count, at, sh_at;
+} rgs_lend_segment;
+typedef struct rgs_lend_model {
+	const float* means3D_from;
+	float* means3D;
+	float* opacity;             /* activated: own rows, with room for the lent ones behind */
+	float* scales;
+	float* rotations;
+	const float* sh_first;      /* features_dc, features_rest with 15 coefficients */
+	const float* sh_rest;
+	float* sh_lent;             /* (lent, 48) */
+} rgs_lend_model;
+int rgs_lend_rows(int n_models, const rgs_lend_model* models, int n_segments, const rgs_lend_segment* segments, void* stream);
+/* The adjoint: the gradients of lent rows are added to the rows they were read from, per lender in the order of `segments`.  Gradient arrays
+ * of merged rows with the own ones in front, sh_first / sh_rest of the own rows and sh_lent of the lent ones; a borrower's array may be
+ * NULL (nothing is added from it), a lender's may not. */
+typedef struct rgs_lend_gradients {
+	float* means3D;
+	float* means2D;
+	float* opacity;
+	float* scales;
+	float* rotations;
+	float* sh_first;
+	float* sh_rest;
+	const float* sh_lent;
+} rgs_lend_gradients;
+int rgs_lend_rows_backward(int n_models, const rgs_lend_gradients* models, int n_segments, const rgs_lend_segment* segments, void* stream);
+/* n floats of host memory, at most RGS_MAX_WRITTEN_FLOATS, to device memory: they travel with the launch, so nothing waits and the host
+ * memory is free again when this returns. */
+#define RGS_MAX_WRITTEN_FLOATS 768
+int rgs_write_floats(int n, const float* values, float* device, void* stream);
 
 /* ---- optimiser step ---------------------------------------------------------------------------
  * torch.optim.Adam without weight decay or amsgrad, as the reference sets it up per submodel

@@ -61,7 +61,9 @@ class FrameLayer(C.Structure):
                 ("grad_accum", C.c_void_p), ("dL_dmean2D", C.c_void_p), ("dL_dopacity", C.c_void_p),
                 ("dL_dcolor", C.c_void_p), ("dL_dmean3D", C.c_void_p), ("dL_dcov3D", C.c_void_p), ("dL_dsh", C.c_void_p),
                 ("dL_dscale", C.c_void_p), ("dL_drot", C.c_void_p), ("accum_zeroed", C.c_int),
-                ("stream", C.c_void_p)]
+                ("stream", C.c_void_p),
+                ("sh_rest", C.c_void_p), ("sh_lent", C.c_void_p), ("sh_own", C.c_int), ("dL_dsh_rest", C.c_void_p),
+                ("dL_dsh_lent", C.c_void_p)]
 
 
 class RgsError(RuntimeError):
@@ -120,6 +122,12 @@ def _load():
     lib.rgs_l1_ssim_backward.argtypes = [i, i, i, vp, vp, f, vp, vp, vp, vp]
     lib.rgs_activate_forward.argtypes = [i, i] + [vp] * 10
     lib.rgs_activate_backward.argtypes = [i, i] + [vp] * 13
+    for name in ("rgs_activate_models", "rgs_activate_models_backward"):
+        getattr(lib, name).argtypes = [i, vp, vp]
+    lib.rgs_straddler_select_many.argtypes = [i, vp, fp, fp, vp]
+    for name in ("rgs_lend_rows", "rgs_lend_rows_backward"):
+        getattr(lib, name).argtypes = [i, vp, i, vp, vp]
+    lib.rgs_write_floats.argtypes = [i, fp, vp, vp]
     lib.rgs_adam_step.argtypes = [i, C.POINTER(AdamTensor), C.c_double, C.c_double, C.c_double, vp]
     lib.rgs_stage_timing.argtypes = [i]
     lib.rgs_stage_timing_read.argtypes = [i, C.POINTER(C.c_char_p), C.POINTER(C.c_float), C.POINTER(C.c_int)]
@@ -131,7 +139,8 @@ def _load():
                  "rgs_merge_rows_backward", "rgs_l1_ssim_forward", "rgs_l1_ssim_backward", "rgs_adam_step",
                  "rgs_activate_forward", "rgs_activate_backward", "rgs_sort_pairs_static", "rgs_sort_fault",
                  "rgs_set_lookback_spin_limit", "rgs_frame_forward_geom", "rgs_frame_forward_raster",
-                 "rgs_frame_backward"):
+                 "rgs_frame_backward", "rgs_activate_models", "rgs_activate_models_backward", "rgs_straddler_select_many",
+                 "rgs_lend_rows", "rgs_lend_rows_backward", "rgs_write_floats"):
         getattr(lib, name).restype = i
     return lib
 
@@ -147,7 +156,9 @@ EXPORTS = ("rgs_version", "rgs_last_error", "rgs_get_higher_msb", "rgs_geom_byte
            "rgs_straddler_select", "rgs_merge_rows", "rgs_merge_rows_backward", "rgs_loss_workspace_bytes",
            "rgs_l1_ssim_forward", "rgs_l1_ssim_backward", "rgs_adam_step", "rgs_activate_forward",
            "rgs_activate_backward", "rgs_sort_pairs_static", "rgs_sort_fault", "rgs_set_lookback_spin_limit",
-           "rgs_frame_forward_geom", "rgs_frame_forward_raster", "rgs_frame_backward")
+           "rgs_frame_forward_geom", "rgs_frame_forward_raster", "rgs_frame_backward", "rgs_activate_models",
+           "rgs_activate_models_backward", "rgs_straddler_select_many", "rgs_lend_rows", "rgs_lend_rows_backward",
+           "rgs_write_floats")
 MAX_FRAME_LAYERS = 64
 STATIC_SORT_MAX_PAIRS = 1 << 22
 WORK_COUNTERS = 8

@@ -4,6 +4,8 @@
 #include "../../include/rgs.h"
 #include "rgs_kernels.h"
 
+#include <algorithm>
+
 #include <atomic>
 #include <cmath>
 #include <cstdarg>
@@ -480,6 +482,17 @@ static bool sh_rows_by_16_bytes(const float* shs, int M, int D)
 	return shs && (reinterpret_cast<uintptr_t>(shs) & 15) == 0 && (n & 3) == 0 && n <= 48 && needed <= n;
 }
 
+// SH rows in parts, if they are.
+static int check_split_sh(const char* who, int P, int M, const float* shs, const rgs::SplitSh& sh)
+{
+	if (!sh.rest)
+		return 0;
+	RGS_REQUIRE(shs && M == 16 && sh.own >= 0 && sh.own <= P, "%s: SH rows in parts need 16 coefficients and 0 <= sh_own <= P", who);
+	RGS_REQUIRE(sh.own == P || (sh.lent && (reinterpret_cast<uintptr_t>(sh.lent) & 15) == 0),
+	            "%s: whole SH rows missing or not at a multiple of 16 bytes", who);
+	return 0;
+}
+
 // One event per host thread and device, for waiting on the copy of the instance count alone.
 static hipEvent_t count_event_of_this_thread()
 {
@@ -507,6 +520,7 @@ struct GeomCall {
 	int* radii;
 	void* geom_ws;
 	size_t geom_bytes;
+	rgs::SplitSh sh;
 };
 
 // The geometry stage of `K` layers that share a camera, every kernel launched once for all of them: preprocess,
@@ -563,6 +577,10 @@ static int forward_geom(bool wait_for_count, void* count_ready_event, const char
 		a.blend_record = at<float4>(ws, off[RGS_GEOM_BLEND_RECORD]);
 		a.block_visible = at<uint32_t>(ws, off[RGS_GEOM_BLOCK_VISIBLE]);
 		a.sh_rows_by_16_bytes = sh_rows_by_16_bytes(c.shs, c.M, c.D);
+		a.sh = c.sh;
+		RGS_REQUIRE((c.sh.rest != nullptr) == (calls[0].sh.rest != nullptr), "%s: SH rows in parts in some layers alone", who);
+		if (int rc = check_split_sh(who, c.P, c.M, c.shs, c.sh))
+			return rc;
 		const OrderScratch o = order_scratch((size_t)c.P);
 		char* scratch = at<char>(ws, off[RGS_GEOM_ORDER_SCRATCH]);
 		a.clear = at<uint32_t>(scratch, o.digits);
@@ -622,7 +640,7 @@ int rgs_forward_geom(int P, int D, int M, int width, int height,
 	RGS_REQUIRE(P > 0, "rgs_forward_geom: P must be positive (the caller short-circuits P == 0)");
 	RGS_REQUIRE(num_rendered_host, "rgs_forward_geom: null pointer");
 	const GeomCall c = {P, D, M, means3D, shs, colors_precomp, opacities, scales, scale_modifier, rotations, cov3D_precomp, radii,
-	                    geom_ws, geom_bytes};
+	                    geom_ws, geom_bytes, {}};
 	return forward_geom(true, nullptr, "rgs_forward_geom", 1, &c, width, height, viewmatrix, projmatrix, cam_pos, tan_fovx,
 	                    tan_fovy, num_rendered_host, stream, debug);
 }
@@ -639,7 +657,7 @@ int rgs_forward_geom_enqueue(int P, int D, int M, int width, int height,
 	RGS_REQUIRE(P > 0, "rgs_forward_geom_enqueue: P must be positive (the caller short-circuits P == 0)");
 	RGS_REQUIRE(num_rendered_pinned, "rgs_forward_geom_enqueue: null pointer");
 	const GeomCall c = {P, D, M, means3D, shs, colors_precomp, opacities, scales, scale_modifier, rotations, cov3D_precomp, radii,
-	                    geom_ws, geom_bytes};
+	                    geom_ws, geom_bytes, {}};
 	return forward_geom(false, count_ready_event, "rgs_forward_geom_enqueue", 1, &c, width, height, viewmatrix, projmatrix, cam_pos,
 	                    tan_fovx, tan_fovy, num_rendered_pinned, stream, debug);
 }
@@ -1003,7 +1021,8 @@ int rgs_frame_forward_geom(int K, const rgs_frame_layer* layers, const rgs_frame
 	for (int k = 0; k < K; k++) {
 		const rgs_frame_layer& l = layers[k];
 		calls[(size_t)k] = GeomCall{l.P, l.D, l.M, l.means3D, l.shs, l.colors_precomp, l.opacities, l.scales, l.scale_modifier,
-		                            l.rotations, l.cov3D_precomp, const_cast<int*>(l.radii), l.geom_ws, l.geom_bytes};
+		                            l.rotations, l.cov3D_precomp, const_cast<int*>(l.radii), l.geom_ws, l.geom_bytes,
+		                            rgs::SplitSh{l.sh_rest, l.sh_lent, l.sh_own}};
 	}
 	return forward_geom(true, nullptr, "rgs_frame_forward_geom", K, calls.data(), view->width, view->height, view->viewmatrix,
 	                    view->projmatrix, view->cam_pos, view->tan_fovx, view->tan_fovy, counts_pinned, stream, debug);
@@ -1076,6 +1095,17 @@ int rgs_frame_backward(int K, const rgs_frame_layer* layers, const rgs_frame_vie
 		                       l.scale_modifier, l.rotations, l.cov3D_precomp, view->viewmatrix, view->projmatrix, view->cam_pos,
 		                       view->tan_fovx, view->tan_fovy, l.radii, l.geom_ws, l.grad_accum, l.dL_dmean2D, l.dL_dopacity,
 		                       l.dL_dcolor, l.dL_dmean3D, l.dL_dcov3D, l.dL_dsh, l.dL_dscale, l.dL_drot);
+		rgs::PreprocessBackwardArgs& p = geometry[(size_t)k];
+		p.sh = rgs::SplitSh{l.sh_rest, l.sh_lent, l.sh_own};
+		p.dL_dsh_rest = l.dL_dsh_rest;
+		p.dL_dsh_lent = l.dL_dsh_lent;
+		RGS_REQUIRE((l.sh_rest != nullptr) == (layers[0].sh_rest != nullptr), "rgs_frame_backward: SH rows in parts in some layers alone");
+		if (int rc = check_split_sh("rgs_frame_backward", l.P, l.M, l.shs, p.sh))
+			return rc;
+		if (l.sh_rest)
+			RGS_REQUIRE((l.sh_own == 0 || (l.dL_dsh && l.dL_dsh_rest && ((reinterpret_cast<uintptr_t>(l.dL_dsh) | reinterpret_cast<uintptr_t>(l.dL_dsh_rest)) & 15) == 0)) &&
+			                (l.sh_own == l.P || (l.dL_dsh_lent && (reinterpret_cast<uintptr_t>(l.dL_dsh_lent) & 15) == 0)),
+			            "rgs_frame_backward: gradients of SH rows in parts missing or not at multiples of 16 bytes");
 	}
 	if (!sums_to_clear.empty()) {
 		rgs::stage_mark("clear_gradients", s);
@@ -1343,6 +1373,18 @@ size_t rgs_straddler_scratch_bytes(int n, int n_boxes)
 	return sizeof(uint32_t) * (size_t)n_boxes * (rgs::straddler_select_blocks(n) + 1);
 }
 
+static rgs::ShareBoxes share_boxes(int n, const float* low, const float* up)
+{
+	rgs::ShareBoxes boxes;
+	boxes.count = n;
+	for (int b = 0; b < n; b++)
+		for (int c = 0; c < 3; c++) {
+			boxes.low[b][c] = low[3 * b + c];
+			boxes.up[b][c] = up[3 * b + c];
+		}
+	return boxes;
+}
+
 int rgs_straddler_select(int n, const float* means3D, const float* scales, const float* src_low, const float* src_up,
                          int n_boxes, const float* boxes_low, const float* boxes_up, int skip, uint32_t* counts,
                          uint32_t* rows, uint32_t capacity, void* scratch, void* stream)
@@ -1358,7 +1400,7 @@ int rgs_straddler_select(int n, const float* means3D, const float* scales, const
 	RGS_REQUIRE(counts && scratch, "rgs_straddler_select: null counts or scratch");
 	RGS_REQUIRE(n == 0 || (means3D && scales), "rgs_straddler_select: null input");
 	RGS_REQUIRE(capacity == 0 || rows, "rgs_straddler_select: null rows");
-	rgs::StraddlerSelectArgs a;
+	rgs::StraddlerJob a;
 	a.n = n;
 	a.means3D = means3D;
 	a.scales = scales;
@@ -1366,18 +1408,12 @@ int rgs_straddler_select(int n, const float* means3D, const float* scales, const
 		a.src_low[c] = src_low[c];
 		a.src_up[c] = src_up[c];
 	}
-	a.boxes.count = n_boxes;
-	for (int b = 0; b < n_boxes; b++)
-		for (int c = 0; c < 3; c++) {
-			a.boxes.low[b][c] = boxes_low[3 * b + c];
-			a.boxes.up[b][c] = boxes_up[3 * b + c];
-		}
 	a.skip = skip;
 	a.block_counts = static_cast<uint32_t*>(scratch);
 	a.counts = counts;
 	a.rows = rows;
 	a.capacity = capacity;
-	rgs::launch_straddler_select(a, s);
+	rgs::launch_straddler_select(&a, 1, share_boxes(n_boxes, boxes_low, boxes_up), s);
 	RGS_STAGE("straddler_select");
 	return 0;
 }
@@ -1610,6 +1646,189 @@ int rgs_activate_backward(int n, int rest, const float* rotation, const float* s
 	a.features_by_16_bytes = aligned16(d_features_dc) && aligned16(d_features_rest);
 	rgs::launch_activate_backward(a, s);
 	RGS_STAGE("activate_backward");
+	return 0;
+}
+
+int rgs_activate_models(int n_models, const rgs_stored_model* models, void* stream)
+{
+	hipStream_t s = static_cast<hipStream_t>(stream);
+	EntryScope scope_(s);
+	const int debug = 0;
+	RGS_REQUIRE(n_models >= 0 && n_models <= RGS_MAX_STORED_MODELS && (n_models == 0 || models), "rgs_activate_models: bad table of %d models", n_models);
+	rgs::ActivateJob jobs[RGS_MAX_STORED_MODELS];
+	for (int k = 0; k < n_models; k++) {
+		const rgs_stored_model& m = models[k];
+		RGS_REQUIRE(m.n >= 0 && m.zero_rows >= 0, "rgs_activate_models: bad sizes of model %d", k);
+		RGS_REQUIRE(m.n == 0 || (m.scaling && m.rotation && m.opacity && m.scales && m.rotations && m.opacities), "rgs_activate_models: null pointer in model %d", k);
+		RGS_REQUIRE(m.zero_rows == 0 || m.means2D, "rgs_activate_models: null pointer in model %d", k);
+		RGS_REQUIRE(aligned16(m.scaling) && aligned16(m.rotation) && aligned16(m.opacity) && aligned16(m.scales) && aligned16(m.rotations) &&
+		                aligned16(m.opacities) && aligned16(m.means2D),
+		            "rgs_activate_models: arrays must start at multiples of 16 bytes");
+		jobs[k] = rgs::ActivateJob{m.n, m.zero_rows, m.scaling, m.rotation, m.opacity, m.scales, m.rotations, m.opacities, m.means2D};
+	}
+	rgs::launch_activate_many(jobs, n_models, s);
+	RGS_STAGE("activate_models");
+	return 0;
+}
+
+int rgs_activate_models_backward(int n_models, const rgs_stored_model_grads* models, void* stream)
+{
+	hipStream_t s = static_cast<hipStream_t>(stream);
+	EntryScope scope_(s);
+	const int debug = 0;
+	RGS_REQUIRE(n_models >= 0 && n_models <= RGS_MAX_STORED_MODELS && (n_models == 0 || models),
+	            "rgs_activate_models_backward: bad table of %d models", n_models);
+	rgs::ActivateBackwardJob jobs[RGS_MAX_STORED_MODELS];
+	for (int k = 0; k < n_models; k++) {
+		const rgs_stored_model_grads& m = models[k];
+		RGS_REQUIRE(m.n >= 0, "rgs_activate_models_backward: bad size of model %d", k);
+		for (const float* t : {m.rotation, m.scales, m.opacities, m.g_scales, m.g_rotations, m.g_opacities, m.g_means2D,
+		                       (const float*)m.d_scaling, (const float*)m.d_rotation, (const float*)m.d_opacity, (const float*)m.d_meta})
+			RGS_REQUIRE(m.n == 0 || (t && aligned16(t)), "rgs_activate_models_backward: an array of model %d is missing or not at a multiple of 16 bytes", k);
+		jobs[k] = rgs::ActivateBackwardJob{m.n, m.rotation, m.scales, m.opacities, m.g_scales, m.g_rotations, m.g_opacities, m.g_means2D,
+		                                   m.d_scaling, m.d_rotation, m.d_opacity, m.d_meta};
+	}
+	rgs::launch_activate_many_backward(jobs, n_models, s);
+	RGS_STAGE("activate_models_backward");
+	return 0;
+}
+
+int rgs_straddler_select_many(int n_sources, const rgs_straddler_source* sources, const float* boxes_low, const float* boxes_up, void* stream)
+{
+	hipStream_t s = static_cast<hipStream_t>(stream);
+	EntryScope scope_(s);
+	const int debug = 0;
+	RGS_REQUIRE(n_sources >= 1 && n_sources <= rgs::kMaxShareBoxes && sources && boxes_low && boxes_up,
+	            "rgs_straddler_select_many: %d sources, must be 1..%d, or null", n_sources, rgs::kMaxShareBoxes);
+	rgs::StraddlerJob jobs[rgs::kMaxShareBoxes];
+	for (int k = 0; k < n_sources; k++) {
+		const rgs_straddler_source& f = sources[k];
+		RGS_REQUIRE(f.n >= 0 && f.counts && f.scratch && (f.n == 0 || (f.means3D && f.scales)) && (f.capacity == 0 || f.rows),
+		            "rgs_straddler_select_many: bad source %d", k);
+		rgs::StraddlerJob& a = jobs[k];
+		a.n = f.n;
+		a.means3D = f.means3D;
+		a.scales = f.scales;
+		for (int c = 0; c < 3; c++) {
+			a.src_low[c] = boxes_low[3 * k + c];
+			a.src_up[c] = boxes_up[3 * k + c];
+		}
+		a.skip = k;
+		a.block_counts = static_cast<uint32_t*>(f.scratch);
+		a.counts = f.counts;
+		a.rows = f.rows;
+		a.capacity = f.capacity;
+	}
+	rgs::launch_straddler_select(jobs, n_sources, share_boxes(n_sources, boxes_low, boxes_up), s);
+	RGS_STAGE("straddler_select");
+	return 0;
+}
+
+extern "C++" {
+// The segments of one launch, of those not done yet as many as it takes; `take` says whether a segment may join.
+template <typename Args, typename Take>
+static uint32_t fill_lend_segments(Args& a, const rgs_lend_segment* segments, int n, std::vector<char>& done, Take take)
+{
+	uint32_t blocks = 0;
+	a.segments = 0;
+	for (int i = 0; i < n && a.segments < rgs::kMaxLendSegments; i++) {
+		const rgs_lend_segment& g = segments[i];
+		if (done[(size_t)i] || !take(g))
+			continue;
+		done[(size_t)i] = 1;
+		if (g.count == 0)
+			continue;
+		a.seg[a.segments++] = rgs::LendSegment{g.rows, g.count, g.at, g.sh_at, blocks, (uint16_t)g.source, (uint16_t)g.destination};
+		blocks += rgs::merge_blocks_for(g.count);
+	}
+	return blocks;
+}
+}
+
+int rgs_lend_rows(int n_models, const rgs_lend_model* models, int n_segments, const rgs_lend_segment* segments, void* stream)
+{
+	hipStream_t s = static_cast<hipStream_t>(stream);
+	EntryScope scope_(s);
+	const int debug = 0;
+	RGS_REQUIRE(n_models >= 0 && n_models <= RGS_MAX_STORED_MODELS && (n_models == 0 || models) && n_segments >= 0 && (n_segments == 0 || segments),
+	            "rgs_lend_rows: bad tables of %d models, %d segments", n_models, n_segments);
+	rgs::LendArgs a;
+	for (int k = 0; k < n_models; k++) {
+		const rgs_lend_model& m = models[k];
+		RGS_REQUIRE(aligned16(m.rotations) && aligned16(m.sh_lent), "rgs_lend_rows: arrays must start at multiples of 16 bytes");
+		a.model[k] = rgs::LendModel{m.means3D_from, m.means3D, m.opacity, m.scales, m.rotations, m.sh_first, m.sh_rest, m.sh_lent};
+	}
+	for (int i = 0; i < n_segments; i++) {
+		const rgs_lend_segment& g = segments[i];
+		RGS_REQUIRE(g.source >= 0 && g.source < n_models && g.destination >= 0 && g.destination < n_models && (g.rows || g.source == g.destination),
+		            "rgs_lend_rows: bad segment %d", i);
+		const rgs_lend_model &f = models[g.source], &t = models[g.destination];
+		RGS_REQUIRE(g.count == 0 || (f.means3D_from && t.means3D), "rgs_lend_rows: null pointer in segment %d", i);
+		RGS_REQUIRE(g.count == 0 || !g.rows || (f.opacity && f.scales && f.rotations && f.sh_first && f.sh_rest && t.opacity && t.scales && t.rotations && t.sh_lent),
+		            "rgs_lend_rows: null pointer in segment %d", i);
+	}
+	std::vector<char> done((size_t)n_segments, 0);
+	for (int left = n_segments; left > 0;) {
+		const uint32_t blocks = fill_lend_segments(a, segments, n_segments, done, [](const rgs_lend_segment&) { return true; });
+		rgs::launch_lend_rows(a, blocks, s);
+		RGS_STAGE("lend_rows");
+		left = (int)std::count(done.begin(), done.end(), 0);
+	}
+	return 0;
+}
+
+int rgs_lend_rows_backward(int n_models, const rgs_lend_gradients* models, int n_segments, const rgs_lend_segment* segments, void* stream)
+{
+	hipStream_t s = static_cast<hipStream_t>(stream);
+	EntryScope scope_(s);
+	const int debug = 0;
+	RGS_REQUIRE(n_models >= 0 && n_models <= RGS_MAX_STORED_MODELS && (n_models == 0 || models) && n_segments >= 0 && (n_segments == 0 || segments),
+	            "rgs_lend_rows_backward: bad tables of %d models, %d segments", n_models, n_segments);
+	rgs::LendBackwardArgs a;
+	for (int k = 0; k < n_models; k++) {
+		const rgs_lend_gradients& m = models[k];
+		RGS_REQUIRE(aligned16(m.sh_lent), "rgs_lend_rows_backward: sh_lent must start at a multiple of 16 bytes");
+		a.model[k] = rgs::LendGradients{m.means3D, m.means2D, m.opacity, m.scales, m.rotations, m.sh_first, m.sh_rest, m.sh_lent};
+	}
+	for (int i = 0; i < n_segments; i++) {
+		const rgs_lend_segment& g = segments[i];
+		RGS_REQUIRE(g.source >= 0 && g.source < n_models && g.destination >= 0 && g.destination < n_models && g.rows,
+		            "rgs_lend_rows_backward: bad segment %d", i);
+		const rgs_lend_gradients& f = models[g.source];
+		RGS_REQUIRE(g.count == 0 || (f.means3D && f.means2D && f.opacity && f.scales && f.rotations && f.sh_first && f.sh_rest),
+		            "rgs_lend_rows_backward: null pointer in segment %d", i);
+	}
+	// every lender once per launch
+	std::vector<char> done((size_t)n_segments, 0);
+	for (int left = n_segments; left > 0;) {
+		uint32_t taken = 0;
+		const uint32_t blocks = fill_lend_segments(a, segments, n_segments, done, [&](const rgs_lend_segment& g) {
+			const bool first = (taken >> g.source & 1u) == 0u;
+			taken |= 1u << g.source;
+			return first;
+		});
+		rgs::launch_lend_rows_backward(a, blocks, s);
+		RGS_STAGE("lend_rows_backward");
+		left = (int)std::count(done.begin(), done.end(), 0);
+	}
+	return 0;
+}
+
+int rgs_write_floats(int n, const float* values, float* device, void* stream)
+{
+	hipStream_t s = static_cast<hipStream_t>(stream);
+	EntryScope scope_(s);
+	const int debug = 0;
+	RGS_REQUIRE(n >= 0 && n <= RGS_MAX_WRITTEN_FLOATS && (n == 0 || (values && device)), "rgs_write_floats: %d floats, at most %d, or null", n,
+	            RGS_MAX_WRITTEN_FLOATS);
+	if (n == 0)
+		return 0;
+	rgs::WriteFloatsArgs a;
+	memcpy(a.v, values, sizeof(float) * (size_t)n);
+	a.to = device;
+	a.n = n;
+	rgs::launch_write_floats(a, s);
+	RGS_STAGE("write_floats");
 	return 0;
 }
 

@@ -1457,7 +1457,19 @@ __global__ __launch_bounds__(256) void fill_u32_kernel(uint32_t* __restrict__ p,
 		p[done + tid] = v;
 }
 
-// The same for several arrays in one launch (the array in blockIdx.y).
+// A few floats that travel with the launch.
+__global__ __launch_bounds__(256) void write_floats_kernel(WriteFloatsArgs a)
+{
+	for (int k = threadIdx.x; k < a.n; k += 256)
+		a.to[k] = a.v[k];
+}
+
+void launch_write_floats(const WriteFloatsArgs& a, hipStream_t s)
+{
+	hipLaunchKernelGGL(write_floats_kernel, dim3(1), dim3(256), 0, s, a);
+}
+
+// fill_u32_kernel for several arrays in one launch (the array in blockIdx.y).
 __global__ __launch_bounds__(256) void fill_many_kernel(Batch<FillJob> batch, uint32_t v)
 {
 	uint32_t* __restrict__ p = batch.job[blockIdx.y].p;

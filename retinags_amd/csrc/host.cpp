@@ -726,12 +726,17 @@ struct Frame : torch::CustomClassHolder {
 	std::vector<FrameLayer> layers;
 	bool keep_workspaces = false;
 	bool keep_strips = false;  // the image workspaces, and the backgrounds as the library saw them, for the compositor
+	bool split_sh = false;     // SH rows in parts: see rgs_frame_layer::sh_rest
 };
+
+// The parts of a layer's SH rows beside the first coefficients.
+enum SplitInput { kSplitRest, kSplitLent, kSplitInputs };
 
 // The submodels that a camera sees ("layers"), rasterized together: what the reference does with one call per submodel
 // (gather_RenderResult_pool, parallel_utils/basic_parallel_trainer/result_aggregator.py:22-38), as three library calls per
 // frame (every layer's geometry stage, then binning and one blend launch for all, and for the backward one blend launch for
-// all and every layer's per-Gaussian backward).  `flat`: kInputs tensors per layer.  Outputs per layer colour, radii, depth, alpha.
+// all and every layer's per-Gaussian backward).  `flat`: kInputs tensors per layer, then, with SH rows in parts, kSplitInputs per layer
+// (kSH then holds the first coefficients).  Outputs per layer colour, radii, depth, alpha.
 struct RasterizeFrame : torch::autograd::Function<RasterizeFrame> {
 	static rgs_frame_view view_of(const Settings& s, const std::array<Tensor, 4>& t)
 	{
@@ -761,8 +766,8 @@ struct RasterizeFrame : torch::autograd::Function<RasterizeFrame> {
 		std::vector<rgs_frame_layer> arr;
 		std::vector<int> live;
 		arr.reserve(K);
-		variable_list saved, out, radii, keep;
-		saved.reserve(K * kSavedPerLayer);
+		variable_list saved, out, radii, keep, split;
+		saved.reserve(K * (kSavedPerLayer + kSplitInputs));
 		out.reserve(4 * K);
 		for (int k = 0; k < K; k++) {
 			FrameLayer& l = frame.layers[k];
@@ -774,6 +779,17 @@ struct RasterizeFrame : torch::autograd::Function<RasterizeFrame> {
 			check_means(flat[kInputs * k + kMeans3D]);
 			l.P = t[kMeans3D].size(0);
 			l.M = sh_rows(t[kSH]);
+			std::array<Tensor, kSplitInputs> parts;
+			if (frame.split_sh) {
+				for (int i = 0; i < kSplitInputs; i++)
+					parts[i] = device_f32(flat[kInputs * K + kSplitInputs * k + i], device);
+				const int64_t own = t[kSH].dim() == 3 ? t[kSH].size(0) : 0;
+				if (own < 1 || t[kSH].sizes() != at::IntArrayRef({own, 1, 3}) || parts[kSplitRest].sizes() != at::IntArrayRef({own, 15, 3}) ||
+				    parts[kSplitLent].sizes() != at::IntArrayRef({l.P - own, 16, 3}))
+					throw std::runtime_error("rasterize_frame: SH rows in parts are (N,1,3), (N,15,3) and (P-N,16,3) with N >= 1");
+				l.M = 16;
+				split.insert(split.end(), parts.begin(), parts.end());
+			}
 			Rendered& r = l.rendered;
 			make_package(r, H, W, device);
 			l.radii = at::empty({l.P}, at::TensorOptions().dtype(at::kInt).device(device));
@@ -798,6 +814,11 @@ struct RasterizeFrame : torch::autograd::Function<RasterizeFrame> {
 				L.M = l.M;
 				L.means3D = ptr(t[kMeans3D]);
 				L.shs = ptr(t[kSH]);
+				if (frame.split_sh) {
+					L.sh_rest = ptr(parts[kSplitRest]);
+					L.sh_lent = ptr(parts[kSplitLent]);
+					L.sh_own = static_cast<int>(t[kSH].size(0));
+				}
 				L.colors_precomp = ptr(t[kColors]);
 				L.opacities = ptr(t[kOpacities]);
 				L.scales = ptr(t[kScales]);
@@ -846,6 +867,7 @@ struct RasterizeFrame : torch::autograd::Function<RasterizeFrame> {
 			for (int k : live)
 				frame.layers[k].image = frame.layers[k].rendered.image;
 		ctx->set_materialize_grads(false);  // an output that took no part in the loss comes back undefined
+		saved.insert(saved.end(), split.begin(), split.end());
 		ctx->save_for_backward(std::move(saved));
 		ctx->mark_non_differentiable(radii);
 		ctx->saved_data["frame"] = c10::IValue::make_capsule(*held);
@@ -879,6 +901,7 @@ struct RasterizeFrame : torch::autograd::Function<RasterizeFrame> {
 			const hipStream_t main = current_stream(device);
 			auto sv = [&](int k, int i) -> const Tensor& { return saved[k * kSavedPerLayer + i]; };
 			std::vector<GradientArrays> made(K);
+			variable_list split_grads(frame.split_sh ? K * kSplitInputs : 0);
 			for (int k = 0; k < K; k++) {
 				if (frame.layers[k].P == 0)
 					continue;
@@ -887,13 +910,20 @@ struct RasterizeFrame : torch::autograd::Function<RasterizeFrame> {
 				std::array<bool, kGradients> left_out{};
 				left_out[kGradColors] = !present(sv(k, kSavedColors));
 				left_out[kGradCov3D] = !present(sv(k, kSavedCov3D));
+				left_out[kGradSH] = frame.split_sh;
 				made[k] = make_gradients(frame.layers[k].P, frame.layers[k].M, device, left_out);
+				if (frame.split_sh) {
+					made[k].g[kGradSH] = new_f32(sv(k, kSavedSH).sizes(), device);
+					for (int i = 0; i < kSplitInputs; i++)
+						split_grads[kSplitInputs * k + i] = new_f32(saved[kSavedPerLayer * K + kSplitInputs * k + i].sizes(), device);
+				}
 			}
 			const std::array<Tensor, 4> vt = view_tensors(s0, device);
 			const rgs_frame_view view = view_of(s0, vt);
 			std::vector<rgs_frame_layer> arr;
 			arr.reserve(K);
-			variable_list keep, out(K * kInputs + 1);
+			variable_list keep, out(K * kInputs + split_grads.size() + 1);
+			std::copy(split_grads.begin(), split_grads.end(), out.begin() + K * kInputs);
 			for (int k = 0; k < K; k++) {
 				const FrameLayer& l = frame.layers[k];
 				if (l.P == 0) {
@@ -912,6 +942,14 @@ struct RasterizeFrame : torch::autograd::Function<RasterizeFrame> {
 					L.R = l.rendered.instances;
 					L.means3D = ptr(sv(k, kSavedMeans3D));
 					L.shs = ptr(sv(k, kSavedSH));
+					if (frame.split_sh) {
+						const Tensor* parts = &saved[kSavedPerLayer * K + kSplitInputs * k];
+						L.sh_rest = ptr(parts[kSplitRest]);
+						L.sh_lent = ptr(parts[kSplitLent]);
+						L.sh_own = static_cast<int>(sv(k, kSavedSH).size(0));
+						L.dL_dsh_rest = ptr(split_grads[kSplitInputs * k + kSplitRest]);
+						L.dL_dsh_lent = ptr(split_grads[kSplitInputs * k + kSplitLent]);
+					}
 					L.colors_precomp = ptr(sv(k, kSavedColors));
 					L.scales = ptr(sv(k, kSavedScales));
 					L.rotations = ptr(sv(k, kSavedRotations));
@@ -954,9 +992,10 @@ struct RasterizeFrame : torch::autograd::Function<RasterizeFrame> {
 // `inputs`: per layer the kInputs tensors, empty ones for those that are absent.  `streams`: None, or a stream handle per layer.
 // `workspaces`: None, or a list that receives (instances, geometry, binning and image workspace) per layer.
 // `strips`: None, or a list that receives per layer its image workspace (None for a layer without Gaussians) and its background, which is
-// what _host.composite takes under that name.
+// what _host.composite takes under that name.  `split`: None, or per layer the further parts of SH rows whose first coefficients are given
+// as the layer's sh: (N,15,3) and, of the Gaussians behind those N, whole rows (P-N,16,3).
 py::list rasterize_frame(const py::sequence& settings, const py::sequence& inputs, py::handle streams, py::handle workspaces,
-                         py::handle strips)
+                         py::handle strips, py::handle split)
 {
 	const size_t K = settings.size();
 	if (K == 0 || inputs.size() != kInputs * K)
@@ -979,6 +1018,16 @@ py::list rasterize_frame(const py::sequence& settings, const py::sequence& input
 			given[i] = held[i] = inputs[k * kInputs + i];
 		const std::array<Tensor, kInputs> in = inputs_from_python(given.data());
 		flat.insert(flat.end(), in.begin(), in.end());
+	}
+	if (!split.is_none()) {
+		frame->split_sh = true;
+		for (py::handle h : py::reinterpret_borrow<py::sequence>(split)) {
+			const py::tuple parts = py::reinterpret_borrow<py::tuple>(h);
+			for (int i = 0; i < kSplitInputs; i++)
+				flat.push_back(tensor_from_python(parts[i], "a part of the SH rows"));
+		}
+		if (flat.size() != (kInputs + kSplitInputs) * K)
+			throw std::runtime_error("rasterize_frame: the parts of the SH rows of every layer are needed");
 	}
 	variable_list out;
 	{
@@ -1051,7 +1100,7 @@ PYBIND11_MODULE(_host, m)
 	m.def("rasterize_forward_from_stage", &rasterize_forward_from_stage);
 	m.def("rasterize_backward", &rasterize_backward);
 	m.def("rasterize_frame", &rasterize_frame, py::arg("settings"), py::arg("inputs"), py::arg("streams"), py::arg("workspaces"),
-	      py::arg("strips") = py::none());
+	      py::arg("strips") = py::none(), py::arg("split") = py::none());
 	m.def("enqueue_geometry", &enqueue_geometry);
 	define_training(m);
 

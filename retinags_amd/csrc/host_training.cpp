@@ -336,6 +336,247 @@ std::vector<Tensor> merge_shared(const std::vector<int64_t>& own, const py::sequ
 	return MergeShared::apply(at::TensorList(flat), &merge);
 }
 
+// ---- the stored models of an iteration ----------------------------------------------------------------------------
+
+// A stored model's tensors in the order of StoredModel.parameters but for the placeholder, which comes last.
+enum StoredField { kStoredXyz, kStoredFirst, kStoredRest, kStoredScaling, kStoredRotation, kStoredOpacity, kStoredMeta, kStoredFields };
+// What a model becomes for the frame: merged rows (own, then lent ones), its SH rows in parts.
+enum ShownField { kShownMeans3D, kShownMeans2D, kShownOpacity, kShownScales, kShownRotations, kShownFirst, kShownRest, kShownLent, kShownFields };
+
+struct Stored : torch::CustomClassHolder {
+	int K = 0;
+	std::vector<float> boxes;               // lower corners, then upper corners
+	std::vector<int64_t> spare;             // rows of room that the models' positions have behind them; used if append
+	bool append = false;
+	std::vector<int64_t> own, total, counts;  // counts[source * K + destination]
+	std::vector<rgs_lend_segment> segments;
+	variable_list lists;                    // the row lists that the segments point into
+};
+
+// Activation, selection, lending for all models of an iteration at once: what activate, select_straddlers and merge_shared do one
+// after another, with one launch per step whatever the number of models (an iteration of two models is 36 kernels instead of 49), and
+// without a joined copy of the SH rows, which the rasterizer reads, and whose gradients it writes, as they are stored.
+struct ShowStored : torch::autograd::Function<ShowStored> {
+	static Tensor with_rows(const Tensor& room, int64_t rows)
+	{
+		return carved(room, 0, rows_of(rows, room.sizes()));
+	}
+
+	static variable_list forward(AutogradContext* ctx, at::TensorList in, const c10::intrusive_ptr<Stored>* held)
+	{
+		Stored& m = **held;
+		const int K = m.K;
+		const at::Device device = in[0].device();
+		c10::DeviceGuard guard(device);
+		const hipStream_t stream = current_stream(device);
+		auto given = [&](int k, int f) -> const Tensor& { return in[kStoredFields * k + f]; };
+		// activated tensors with room behind them for the lent rows: as much as the positions have, or a guess
+		std::vector<std::array<Tensor, 4>> act(K);  // scales, rotations, opacity, means2D
+		std::vector<rgs_stored_model> models(K);
+		std::vector<int64_t> room(K);
+		for (int k = 0; k < K; k++) {
+			const int64_t n = given(k, kStoredXyz).size(0);
+			m.own.push_back(n);
+			room[k] = m.append ? m.spare[k] : n / 8 + 4096;
+			act[k] = {new_f32({n + room[k], 3}, device), new_f32({n + room[k], 4}, device), new_f32({n + room[k], 1}, device),
+			          new_f32({n + room[k], 3}, device)};
+			models[k] = {static_cast<int>(n), static_cast<int>(n + room[k]), ptr(given(k, kStoredScaling)), ptr(given(k, kStoredRotation)),
+			             ptr(given(k, kStoredOpacity)), ptr(act[k][0]), ptr(act[k][1]), ptr(act[k][2]), ptr(act[k][3])};
+		}
+		check(rgs_activate_models(K, models.data(), stream));
+		select(m, in, act, device, stream);
+		// where lent rows go: destination by destination, lenders in ascending order
+		variable_list out;
+		out.reserve(K * kShownFields);
+		std::vector<rgs_lend_model> lend(K);
+		std::vector<rgs_lend_segment> copies;
+		for (int d = 0; d < K; d++) {
+			int64_t lent = 0;
+			for (int s = 0; s < K; s++) {
+				const int64_t count = m.counts[s * K + d];
+				if (s != d && count > 0) {
+					m.segments.push_back({s, d, static_cast<const uint32_t*>(m.lists[s].data_ptr()) + d * m.lists[s].size(1), static_cast<uint32_t>(count),
+					                      static_cast<uint32_t>(m.own[d] + lent), static_cast<uint32_t>(lent)});
+					lent += count;
+				}
+			}
+			const int64_t n = m.own[d], P = n + lent;
+			m.total.push_back(P);
+			const Tensor& xyz = given(d, kStoredXyz);
+			Tensor means3D;
+			if (m.append) {
+				const size_t end = (xyz.storage_offset() + 3 * P) * sizeof(float);
+				if (lent > room[d] || end > xyz.storage().nbytes())
+					throw std::runtime_error("submodel " + std::to_string(d) + ": no room for " + std::to_string(lent) +
+					                         " lent rows behind its means3D; allocate the field with spare rows or merge with append=False");
+				means3D = carved(xyz, 0, {P, 3});
+			} else {
+				means3D = new_f32({P, 3}, device);
+				copies.push_back({d, d, nullptr, static_cast<uint32_t>(n), 0u, 0u});
+				if (lent > room[d])  // more than guessed: once more, with room for them all
+					for (Tensor& t : act[d]) {
+						const Tensor larger = new_f32(rows_of(P, t.sizes()), device).zero_();
+						larger.narrow(0, 0, n).copy_(t.narrow(0, 0, n));
+						t = larger;
+					}
+			}
+			const Tensor sh_lent = new_f32({lent, 16, 3}, device);
+			const Tensor &first = given(d, kStoredFirst), &rest = given(d, kStoredRest);
+			lend[d] = {ptr(xyz), ptr(means3D), ptr(act[d][2]), ptr(act[d][0]), ptr(act[d][1]), ptr(first), ptr(rest), ptr(sh_lent)};
+			out.insert(out.end(), {means3D, with_rows(act[d][3], P), with_rows(act[d][2], P), with_rows(act[d][0], P), with_rows(act[d][1], P),
+			                       carved(first, 0, first.sizes()), carved(rest, 0, rest.sizes()), sh_lent});
+		}
+		copies.insert(copies.end(), m.segments.begin(), m.segments.end());
+		check(rgs_lend_rows(K, lend.data(), static_cast<int>(copies.size()), copies.data(), stream));
+		variable_list saved;
+		for (int k = 0; k < K; k++)
+			saved.insert(saved.end(), {given(k, kStoredRotation), with_rows(act[k][0], m.own[k]), with_rows(act[k][2], m.own[k])});
+		ctx->save_for_backward(std::move(saved));
+		ctx->set_materialize_grads(false);
+		ctx->saved_data["stored"] = c10::IValue::make_capsule(*held);
+		return out;
+	}
+
+	// Counts and row lists of all pairs; a list that did not fit is written again with room for it.
+	static void select(Stored& m, at::TensorList in, const std::vector<std::array<Tensor, 4>>& act, const at::Device& device, hipStream_t stream)
+	{
+		const int K = m.K;
+		const at::TensorOptions ints = at::TensorOptions().dtype(at::kInt).device(device);
+		const Tensor counts_dev = at::empty({K, K}, ints);
+		std::vector<rgs_straddler_source> sources(K);
+		variable_list scratch;
+		m.lists.resize(K);
+		auto source = [&](int k, int64_t capacity) {
+			m.lists[k] = at::empty({K, capacity}, ints);
+			scratch.push_back(new_bytes(std::max<size_t>(1, rgs_straddler_scratch_bytes(m.own[k], K)), device));
+			return rgs_straddler_source{static_cast<int>(m.own[k]), ptr(in[kStoredFields * k + kStoredXyz]), ptr(act[k][0]),
+			                            ptr<uint32_t>(counts_dev) + k * K, ptr<uint32_t>(m.lists[k]), static_cast<uint32_t>(capacity),
+			                            scratch.back().data_ptr()};
+		};
+		for (int k = 0; k < K; k++)
+			sources[k] = source(k, std::min(m.own[k], m.own[k] / 8 + 4096));
+		const float *low = m.boxes.data(), *up = low + 3 * K;
+		check(rgs_straddler_select_many(K, sources.data(), low, up, stream));
+		const CountSlot slot = slot_pool().take(device.index());
+		const bool arrived = hipMemcpyAsync(slot.words, counts_dev.data_ptr(), K * K * sizeof(uint32_t), hipMemcpyDeviceToHost, stream) ==
+		                         hipSuccess &&
+		                     hipEventRecord(slot.event, stream) == hipSuccess && hipEventSynchronize(slot.event) == hipSuccess;
+		m.counts.assign(slot.words, slot.words + K * K);
+		slot_pool().give_back(device.index(), slot);
+		if (!arrived)
+			throw std::runtime_error("reading the straddlers' counts failed");
+		for (int k = 0; k < K; k++) {
+			const int64_t longest = *std::max_element(m.counts.begin() + k * K, m.counts.begin() + (k + 1) * K);
+			if (longest > m.lists[k].size(1)) {
+				const rgs_straddler_source f = source(k, longest);
+				check(rgs_straddler_select(f.n, f.means3D, f.scales, low + 3 * k, up + 3 * k, K, low, up, k, f.counts, f.rows, f.capacity,
+				                           f.scratch, stream));
+			}
+		}
+	}
+
+	static variable_list backward(AutogradContext* ctx, variable_list grads)
+	{
+		return in_backward([&]() -> variable_list {
+			const auto holder = ctx->saved_data["stored"].toCapsule();
+			const Stored& m = static_cast<const Stored&>(*holder);
+			const int K = m.K;
+			const variable_list saved = ctx->get_saved_variables();
+			const at::Device device = saved[0].device();
+			c10::DeviceGuard guard(device);
+			const hipStream_t stream = current_stream(device);
+			// gradients that did not come are zeros, unless only borrowers would read them
+			std::vector<rgs_lend_gradients> all(K);
+			for (int k = 0; k < K; k++) {
+				const int64_t n = m.own[k], P = m.total[k];
+				const std::array<std::vector<int64_t>, kShownFields> shapes = {{{P, 3}, {P, 3}, {P, 1}, {P, 3}, {P, 4}, {n, 1, 3}, {n, 15, 3}, {P - n, 16, 3}}};
+				for (int f = 0; f < kShownFields; f++) {
+					Tensor& g = grads[kShownFields * k + f];
+					if (g.defined())
+						g = g.contiguous();
+					else if (f != kShownLent)
+						g = new_f32(shapes[f], device).zero_();
+				}
+				auto at = [&](int f) { return ptr(grads[kShownFields * k + f]); };
+				all[k] = {at(kShownMeans3D), at(kShownMeans2D), at(kShownOpacity), at(kShownScales), at(kShownRotations), at(kShownFirst), at(kShownRest),
+				          at(kShownLent)};
+			}
+			check(rgs_lend_rows_backward(K, all.data(), static_cast<int>(m.segments.size()), m.segments.data(), stream));
+			variable_list out(K * kStoredFields + 1);
+			std::vector<rgs_stored_model_grads> models(K);
+			for (int k = 0; k < K; k++) {
+				const int64_t n = m.own[k];
+				const Tensor* g = &grads[kShownFields * k];
+				Tensor* d = &out[kStoredFields * k];
+				d[kStoredXyz] = carved(g[kShownMeans3D], 0, {n, 3});
+				d[kStoredFirst] = g[kShownFirst];
+				d[kStoredRest] = g[kShownRest];
+				d[kStoredScaling] = new_f32({n, 3}, device);
+				d[kStoredRotation] = new_f32({n, 4}, device);
+				d[kStoredOpacity] = new_f32({n, 1}, device);
+				d[kStoredMeta] = new_f32({n, 1}, device);
+				models[k] = {static_cast<int>(n), ptr(saved[3 * k]), ptr(saved[3 * k + 1]), ptr(saved[3 * k + 2]), all[k].scales, all[k].rotations,
+				             all[k].opacity, all[k].means2D, ptr(d[kStoredScaling]), ptr(d[kStoredRotation]), ptr(d[kStoredOpacity]),
+				             ptr(d[kStoredMeta])};
+			}
+			check(rgs_activate_models_backward(K, models.data(), stream));
+			return out;
+		});
+	}
+};
+
+// Whether show_stored takes these models (kStoredFields tensors each): what one launch can hold, as its kernels read it.
+bool stored_together(const variable_list& in)
+{
+	const size_t K = in.size() / kStoredFields;
+	if (K < 1 || K > RGS_MAX_STORED_MODELS)
+		return false;
+	for (size_t k = 0; k < K; k++) {
+		const Tensor* t = &in[kStoredFields * k];
+		const int64_t n = t[kStoredXyz].dim() == 2 ? t[kStoredXyz].size(0) : 0;
+		if (n < 1 || n >= int64_t(1) << 30)
+			return false;
+		const std::array<std::vector<int64_t>, kStoredFields> shapes = {{{n, 3}, {n, 1, 3}, {n, 15, 3}, {n, 3}, {n, 4}, {n, 1}, {n, 1}}};
+		for (int f = 0; f < kStoredFields; f++)
+			if (!t[f].is_cuda() || t[f].device() != in[0].device() || t[f].scalar_type() != at::kFloat || !t[f].is_contiguous() ||
+			    t[f].sizes() != at::IntArrayRef(shapes[f]) ||
+			    ((f == kStoredScaling || f == kStoredRotation || f == kStoredOpacity) && (reinterpret_cast<uintptr_t>(t[f].data_ptr()) & 15) != 0))
+				return false;
+	}
+	return true;
+}
+
+// None where the models cannot be taken together; otherwise (counts[K*K], kShownFields tensors per model).  `boxes` as in select_straddlers.
+py::object show_stored(const variable_list& in, const std::vector<float>& boxes, const std::vector<int64_t>& spare, bool append)
+{
+	if (!stored_together(in))
+		return py::none();
+	auto stored = c10::make_intrusive<Stored>();
+	stored->K = static_cast<int>(in.size() / kStoredFields);
+	if (static_cast<int>(boxes.size()) != 6 * stored->K || static_cast<int>(spare.size()) != stored->K)
+		throw std::runtime_error("show_stored: a box and a number of spare rows per model");
+	stored->boxes = boxes;
+	stored->spare = spare;
+	stored->append = append;
+	variable_list out;
+	{
+		py::gil_scoped_release no_gil;
+		out = ShowStored::apply(at::TensorList(in), &stored);
+	}
+	return py::make_tuple(stored->counts, out);
+}
+
+// Values on the device that the host need not keep: they travel with a launch.
+Tensor floats_on_device(const std::vector<float>& values, const Tensor& like)
+{
+	py::gil_scoped_release no_gil;
+	const at::Device device = like.device();
+	const Tensor t = new_f32({static_cast<int64_t>(values.size())}, device);
+	c10::DeviceGuard guard(device);
+	check(rgs_write_floats(static_cast<int>(values.size()), values.data(), ptr(t), current_stream(device)));
+	return t;
+}
+
 // ---- image loss --------------------------------------------------------------------------------------------------
 
 // (1 - lambda) L1 + lambda (1 - SSIM).  Outputs the loss and (loss, L1, SSIM), of which only the first is differentiable.
@@ -467,6 +708,8 @@ void define_training(py::module_& m)
 	m.def("screen_placeholder", &screen_placeholder);
 	m.def("select_straddlers", &select_straddlers);
 	m.def("merge_shared", &merge_shared);
+	m.def("show_stored", &show_stored);
+	m.def("floats_on_device", &floats_on_device);
 	m.def("l1_ssim", &l1_ssim);
 	m.def("adam_step", &adam_step);
 }

@@ -155,8 +155,24 @@ __device__ __forceinline__ void wave_lds_fence()
 
 constexpr int kShRowStride = 13;  // float4 per parked row: 52 words, so 8 lanes' 16-byte reads meet no bank twice
 
-// kStream: records and per-Gaussian arrays are stored as streaming data (see launch_preprocess_forward).
-template <bool kStream>
+// SH rows in parts: a training iteration's parameters hold the first coefficient and the others in two tensors.  Joining them into whole rows
+// ahead of the rasterizer, and splitting their gradients behind it, moved 2.2 GB per iteration at 2.8 M Gaussians (447 us with the
+// rest of the activation, 89 without the rows); read and written where they are, rows of 180 bytes and of 12 in place of one of 192, the forward
+// geometry takes 114 us instead of 93 and the per-Gaussian backward 258 instead of 220.
+// Floats 4 piece to 4 piece + 3 of a row in parts (the accesses start at any float):
+typedef float UnalignedFloat4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float4 split_row_piece(const float* __restrict__ first, const SplitSh& sh, size_t row, int piece)
+{
+	if (row >= (size_t)sh.own)
+		return reinterpret_cast<const float4*>(sh.lent)[12 * (row - (size_t)sh.own) + piece];
+	if (piece == 0)
+		return float4{first[3 * row], first[3 * row + 1], first[3 * row + 2], sh.rest[45 * row]};
+	const UnalignedFloat4 v = *reinterpret_cast<const UnalignedFloat4*>(sh.rest + 45 * row + 4 * piece - 3);
+	return float4{v.x, v.y, v.z, v.w};
+}
+
+// kStream: records and per-Gaussian arrays are stored as streaming data (see launch_preprocess_forward).  kSplit: SH rows in parts.
+template <bool kStream, bool kSplit>
 __global__ __launch_bounds__(256) void preprocess_forward_kernel(Batch<PreprocessArgs> batch)
 {
 	__shared__ uint32_t s_scan[8];
@@ -246,9 +262,9 @@ __global__ __launch_bounds__(256) void preprocess_forward_kernel(Batch<Preproces
 		const float len = sqrtf(dir.x * dir.x + dir.y * dir.y + dir.z * dir.z);
 		const float dx = dir.x / len, dy = dir.y / len, dz = dir.z / len;
 		float raw[3] = {0.f, 0.f, 0.f};
-		if (a.sh_rows_by_16_bytes) {
+		if (kSplit || a.sh_rows_by_16_bytes) {
 			const int piece = lane & 15, sub = lane >> 4;
-			const int row_pieces = a.M * 3 / 4;
+			const int row_pieces = kSplit ? 12 : a.M * 3 / 4;
 			const int needed = 3 * (a.D + 1) * (a.D + 1);
 			const float4* __restrict__ rows =
 			    reinterpret_cast<const float4*>(a.shs) + (size_t)(idx - lane) * row_pieces;
@@ -259,7 +275,8 @@ __global__ __launch_bounds__(256) void preprocess_forward_kernel(Batch<Preproces
 					const int slot = base + 4 * r + sub;
 					v[r] = float4{0.f, 0.f, 0.f, 0.f};
 					if (4 * piece < needed && slot < n_seen)
-						v[r] = rows[(size_t)listed[slot] * row_pieces + piece];
+						v[r] = kSplit ? split_row_piece(a.shs, a.sh, (size_t)(idx - lane) + listed[slot], piece)
+						              : rows[(size_t)listed[slot] * row_pieces + piece];
 				}
 #pragma unroll
 				for (int r = 0; r < 8; r++)
@@ -443,6 +460,8 @@ __device__ __forceinline__ void store_rows(const PreprocessBackwardArgs& a, floa
 
 // Built for 4 wavefronts per SIMD (left alone the compiler keeps both turns of the SH part in registers: 168
 // of them, 3 wavefronts; 3, 4 and 5 measure the same: the kernel is bound by its stores).
+// kSplit: SH rows and their gradients in parts.
+template <bool kSplit>
 __attribute__((amdgpu_waves_per_eu(4, 4)))
 __global__ __launch_bounds__(128) void preprocess_backward_kernel(Batch<PreprocessBackwardArgs> batch)
 {
@@ -498,12 +517,12 @@ __global__ __launch_bounds__(128) void preprocess_backward_kernel(Batch<Preproce
 #pragma unroll
 		for (int ch = 0; ch < 3; ch++)
 			g[ch] = sum_color[ch] * (((cl >> ch) & 1u) ? 0.f : 1.f);
-		if (a.sh_rows_by_16_bytes) {
+		if (kSplit || a.sh_rows_by_16_bytes) {
 			// The usual case.  The wavefront reads the SH rows of its rendered Gaussians together,
 			// 16 lanes to a row and 16 bytes a lane, parks them in LDS (32 rows at a time) where
 			// each lane picks up its own; the rows of dL_dsh, zeros for the others, leave the same way.
 			const int piece = lane & 15, sub = lane >> 4;
-			const int row_pieces = n_sh / 4;
+			const int row_pieces = kSplit ? 12 : n_sh / 4;
 			const int needed = 3 * (a.D + 1) * (a.D + 1);
 			const int needed_pieces = (needed + 3) / 4;
 			float4* parked = s_rows[wave];
@@ -513,7 +532,11 @@ __global__ __launch_bounds__(128) void preprocess_backward_kernel(Batch<Preproce
 			const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(seen >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)seen, 0u));
 			const size_t wave_first = i - (size_t)lane;
 			const float4* __restrict__ rows = reinterpret_cast<const float4*>(a.shs) + wave_first * row_pieces;
-			float4* __restrict__ grads = reinterpret_cast<float4*>(a.dL_dsh) + wave_first * row_pieces;
+			// rows in parts: a wavefront's rows are all stored in two parts, all whole or, at the border of the two, row by row
+			const size_t own = kSplit ? (size_t)a.sh.own : 0;
+			const bool in_parts = kSplit && wave_first + 64 <= own, at_border = kSplit && !in_parts && wave_first < own;
+			float4* __restrict__ grads = kSplit ? reinterpret_cast<float4*>(a.dL_dsh_lent) + 12 * (wave_first - own)
+			                                    : reinterpret_cast<float4*>(a.dL_dsh) + wave_first * row_pieces;
 			if (rendered)
 				listed[rank] = (uint8_t)lane;
 			wave_lds_fence();
@@ -529,7 +552,8 @@ __global__ __launch_bounds__(128) void preprocess_backward_kernel(Batch<Preproce
 						const int slot = base + 4 * r + sub;
 						v[r] = float4{0.f, 0.f, 0.f, 0.f};
 						if (piece < needed_pieces && slot < n_seen)
-							v[r] = rows[(size_t)listed[slot] * row_pieces + piece];
+							v[r] = kSplit ? split_row_piece(a.shs, a.sh, wave_first + listed[slot], piece)
+							              : rows[(size_t)listed[slot] * row_pieces + piece];
 					}
 #pragma unroll
 					for (int r = 0; r < 8; r++)
@@ -579,13 +603,41 @@ __global__ __launch_bounds__(128) void preprocess_backward_kernel(Batch<Preproce
 						for (int ch = 0; ch < 3; ch++)
 							sh_backward_channel(a.D, xo, yo, zo, none + ch, go[ch], out + ch, t0, t1, t2);
 					}
+					if (in_parts) {
+						// 32 rows of 45 floats, then 32 of 3, as they lie in memory
+						float* words = reinterpret_cast<float*>(parked);
 #pragma unroll
-					for (int k = 0; k < kShRegs; k += 4)
-						if (k < n_sh)
-							mine[k / 4] = float4{out[k], out[k + 1], out[k + 2], out[k + 3]};
+						for (int k = 0; k < kShRegs; k++)
+							words[k < 3 ? 32 * 45 + 3 * (lane & 31) + k : 45 * (lane & 31) + k - 3] = out[k];
+					} else if (at_border) {
+						if (i < own) {
+#pragma unroll
+							for (int k = 0; k < kShRegs; k++)
+								(k < 3 ? a.dL_dsh + 3 * i : a.dL_dsh_rest + 45 * i - 3)[k] = out[k];
+						} else if (present) {
+#pragma unroll
+							for (int k = 0; k < kShRegs; k++)
+								a.dL_dsh_lent[48 * (i - own) + k] = out[k];
+						}
+					} else {
+#pragma unroll
+						for (int k = 0; k < kShRegs; k += 4)
+							if (kSplit || k < n_sh)
+								mine[k / 4] = float4{out[k], out[k + 1], out[k + 2], out[k + 3]};
+					}
 				}
 				wave_lds_fence();
 				__builtin_amdgcn_sched_barrier(0);
+				if (in_parts) {
+					float4* __restrict__ rest_to = reinterpret_cast<float4*>(a.dL_dsh_rest + 45 * (wave_first + 32 * h));
+					float4* __restrict__ first_to = reinterpret_cast<float4*>(a.dL_dsh + 3 * (wave_first + 32 * h));
+#pragma unroll
+					for (int u = 0; u < 32 * 45 / 4; u += 64)
+						if (u + lane < 32 * 45 / 4)
+							store_streaming(rest_to + u + lane, parked[u + lane]);
+					if (lane < 32 * 3 / 4)
+						store_streaming(first_to + lane, parked[32 * 45 / 4 + lane]);
+				} else if (!at_border)
 #pragma unroll
 				for (int r = 0; r < 8; r++) {
 					const int row = 32 * h + 4 * r + sub;
@@ -816,10 +868,15 @@ void launch_preprocess_forward(const PreprocessArgs* jobs, int count, hipStream_
 			all += (size_t)b.job[k].P;
 		}
 		const dim3 grid((unsigned)((max_p + 255) / 256), (unsigned)nj);
-		if (all >= kStreamedGaussians)
-			hipLaunchKernelGGL(preprocess_forward_kernel<true>, grid, dim3(256), 0, s, b);
+		const bool split = jobs[at].sh.rest != nullptr;  // (of all jobs or of none)
+		if (all >= kStreamedGaussians && split)
+			hipLaunchKernelGGL((preprocess_forward_kernel<true, true>), grid, dim3(256), 0, s, b);
+		else if (all >= kStreamedGaussians)
+			hipLaunchKernelGGL((preprocess_forward_kernel<true, false>), grid, dim3(256), 0, s, b);
+		else if (split)
+			hipLaunchKernelGGL((preprocess_forward_kernel<false, true>), grid, dim3(256), 0, s, b);
 		else
-			hipLaunchKernelGGL(preprocess_forward_kernel<false>, grid, dim3(256), 0, s, b);
+			hipLaunchKernelGGL((preprocess_forward_kernel<false, false>), grid, dim3(256), 0, s, b);
 	}
 }
 
@@ -834,7 +891,11 @@ void launch_preprocess_backward(const PreprocessBackwardArgs* jobs, int count, h
 			b.job[k] = jobs[at + k];
 			max_p = b.job[k].P > max_p ? b.job[k].P : max_p;
 		}
-		hipLaunchKernelGGL(preprocess_backward_kernel, dim3((unsigned)((max_p + 127) / 128), (unsigned)nj), dim3(128), 0, s, b);
+		const dim3 grid((unsigned)((max_p + 127) / 128), (unsigned)nj);
+		if (jobs[at].sh.rest)
+			hipLaunchKernelGGL(preprocess_backward_kernel<true>, grid, dim3(128), 0, s, b);
+		else
+			hipLaunchKernelGGL(preprocess_backward_kernel<false>, grid, dim3(128), 0, s, b);
 	}
 }
 

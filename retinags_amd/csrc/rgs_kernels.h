@@ -16,6 +16,14 @@ struct Batch {
 	T job[kMaxBatch];
 };
 
+// SH rows of 16 coefficients that are stored in parts: of the first `own` Gaussians the first coefficient (3 floats) where PreprocessArgs::shs
+// says and the other fifteen (45 floats) here, of the others whole rows of 48 floats here.  rest null: one tensor of whole rows.
+struct SplitSh {
+	const float* rest;
+	const float* lent;
+	int own;
+};
+
 struct PreprocessArgs {
 	int P, D, M;
 	const float* means;
@@ -43,6 +51,7 @@ struct PreprocessArgs {
 	uint32_t* clear;          // clear_words words that the kernel sets to zero for a later stage
 	size_t clear_words;
 	float4* blend_record;  // 4 float4 per Gaussian, see blend.hip
+	SplitSh sh;
 };
 
 struct PreprocessBackwardArgs {
@@ -71,6 +80,9 @@ struct PreprocessBackwardArgs {
 	float* dL_dsh;      // (P,M,3)
 	float* dL_dscale;   // (P,3)
 	float* dL_drot;     // (P,4)
+	SplitSh sh;
+	float* dL_dsh_rest;  // gradients of the rows in parts, where there are any (dL_dsh: of the first coefficients)
+	float* dL_dsh_lent;
 };
 
 struct BlendArgs {
@@ -148,17 +160,21 @@ struct ShareBoxes {
 	float up[kMaxShareBoxes][3];
 	int count;
 };
-struct StraddlerSelectArgs {
+struct StraddlerJob {       // one source
 	int n;
 	const float* means3D;   // (n,3)
 	const float* scales;    // (n,3) activated
 	float src_low[3], src_up[3];
-	ShareBoxes boxes;       // destinations
 	int skip;               // index of a destination that is never lent to (the source itself), or -1
 	uint32_t* block_counts; // boxes.count x straddler_select_blocks(n) words of scratch
 	uint32_t* counts;       // boxes.count
 	uint32_t* rows;         // boxes.count x capacity; rows beyond capacity are counted, not stored
 	uint32_t capacity;
+	uint32_t blocks;        // set by the launcher
+};
+struct StraddlerBatch {
+	StraddlerJob job[kMaxBatch];
+	ShareBoxes boxes;       // destinations
 };
 constexpr int kMaxMergeSegments = 32;
 struct MergeSegment {
@@ -202,6 +218,44 @@ struct MergeBackwardArgs {
 	const float* shs;
 };
 
+// Rows lent between the stored models of a frame, every model's arrays in one table (sharing.hip).
+constexpr int kMaxLendSegments = 48;
+struct LendModel {
+	const float* means3D_from;  // own rows; and where merged rows go, own ones in front (the same array: own rows are there already)
+	float* means3D;
+	float* opacity;             // activated, with room behind the own rows
+	float* scales;
+	float* rotations;
+	const float* sh_first;      // (own, 3) and (own, 45)
+	const float* sh_rest;
+	float* sh_lent;             // (lent, 48)
+};
+struct LendSegment {
+	const uint32_t* rows;       // of the source; null: its own positions, rows 0..count-1, to the front of its merged array
+	uint32_t count, at, sh_at, block0;
+	uint16_t source, destination;
+};
+struct LendArgs {
+	LendModel model[kMaxBatch];
+	LendSegment seg[kMaxLendSegments];
+	int segments;
+};
+struct LendGradients {          // of the merged arrays, own rows in front; any may be null but those that segments name
+	float* means3D;
+	float* means2D;
+	float* opacity;
+	float* scales;
+	float* rotations;
+	float* sh_first;            // of the own rows
+	float* sh_rest;
+	const float* sh_lent;       // of the lent ones
+};
+struct LendBackwardArgs {
+	LendGradients model[kMaxBatch];
+	LendSegment seg[kMaxLendSegments];  // every source once
+	int segments;
+};
+
 // Image loss and optimiser step (training.hip).
 struct LossArgs {
 	int C, H, W;
@@ -243,6 +297,31 @@ struct ActivateBackwardArgs {
 	float* d_rotation;
 	float* d_opacity;
 	bool features_by_16_bytes;   // as above, for their gradients
+};
+// The activation of a frame's stored models but for their SH rows, which the rasterizer reads where they are stored.
+struct ActivateJob {
+	int n, zero_rows;            // Gaussians; rows of means2D to set to zero
+	const float* scaling;
+	const float* rotation;
+	const float* opacity;
+	float* scales;
+	float* rotations;
+	float* opacities;
+	float* means2D;
+};
+struct ActivateBackwardJob {
+	int n;
+	const float* rotation;       // stored quaternions
+	const float* scales;         // activated values
+	const float* opacities;
+	const float* g_scales;
+	const float* g_rotations;
+	const float* g_opacities;
+	const float* g_means2D;      // (n,3)
+	float* d_scaling;
+	float* d_rotation;
+	float* d_opacity;
+	float* d_meta;               // (n,1): length of the (x, y) of g_means2D's row
 };
 constexpr int kMaxAdamTensors = 16;
 struct AdamTensor {
@@ -507,6 +586,13 @@ void launch_blend_count(const BlendArgs& a, hipStream_t s);    // the work-accou
 void launch_composite_forward(const CompositeArgs& a, hipStream_t s);
 void launch_composite_backward(const CompositeArgs& a, hipStream_t s);
 void launch_fill_u32(uint32_t* p, uint32_t v, size_t n, hipStream_t s);
+constexpr int kMaxWrittenFloats = 768;
+struct WriteFloatsArgs {
+	float v[kMaxWrittenFloats];
+	float* to;
+	int n;
+};
+void launch_write_floats(const WriteFloatsArgs& a, hipStream_t s);
 struct FillJob {
 	uint32_t* p;
 	size_t n;  // words
@@ -515,7 +601,9 @@ void launch_fill_many(const FillJob* jobs, int count, uint32_t v, hipStream_t s)
 
 // sharing.hip
 uint32_t straddler_select_blocks(int n);
-void launch_straddler_select(const StraddlerSelectArgs& a, hipStream_t s);
+void launch_straddler_select(const StraddlerJob* jobs, int count, const ShareBoxes& boxes, hipStream_t s);
+void launch_lend_rows(const LendArgs& a, uint32_t blocks, hipStream_t s);
+void launch_lend_rows_backward(const LendBackwardArgs& a, uint32_t blocks, hipStream_t s);
 uint32_t merge_blocks_for(uint32_t rows);   // workgroups one segment of that many rows takes
 void launch_merge_rows(const MergeArgs& a, uint32_t blocks, bool by_16_bytes, hipStream_t s);
 void launch_merge_rows_backward(const MergeBackwardArgs& a, uint32_t blocks, bool by_16_bytes, hipStream_t s);
@@ -526,6 +614,8 @@ void launch_l1_ssim_forward(const LossArgs& a, hipStream_t s);
 void launch_l1_ssim_backward(const LossArgs& a, hipStream_t s);
 void launch_activate_forward(const ActivateArgs& a, hipStream_t s);
 void launch_activate_backward(const ActivateBackwardArgs& a, hipStream_t s);
+void launch_activate_many(const ActivateJob* jobs, int count, hipStream_t s);
+void launch_activate_many_backward(const ActivateBackwardJob* jobs, int count, hipStream_t s);
 uint32_t adam_blocks_for(size_t n);
 void launch_adam_step(const AdamArgs& a, uint32_t blocks, hipStream_t s);
 

@@ -28,7 +28,7 @@ constexpr int kSelectBlock = kSelectThreads * kSelectItems;   // Gaussians per w
 constexpr int kSelectWaves = kSelectThreads / kWave;
 constexpr int kSelectCells = kSelectItems * kSelectWaves;     // (item, wave) cells of a workgroup, in row order
 
-__device__ __forceinline__ uint64_t lend_mask(const StraddlerSelectArgs& a, uint32_t i)
+__device__ __forceinline__ uint64_t lend_mask(const StraddlerJob& a, const ShareBoxes& boxes, uint32_t i)
 {
 	const float* m = a.means3D + 3 * (size_t)i;
 	const float* s = a.scales + 3 * (size_t)i;
@@ -42,19 +42,24 @@ __device__ __forceinline__ uint64_t lend_mask(const StraddlerSelectArgs& a, uint
 	if (!candidate)
 		return 0;
 	uint64_t mask = 0;
-	for (int d = 0; d < a.boxes.count; d++) {
+	for (int d = 0; d < boxes.count; d++) {
 		if (d == a.skip)
 			continue;
-		const bool meets = hx >= a.boxes.low[d][0] && hy >= a.boxes.low[d][1] && hz >= a.boxes.low[d][2] &&
-		                   lx <= a.boxes.up[d][0] && ly <= a.boxes.up[d][1] && lz <= a.boxes.up[d][2];
+		const bool meets = hx >= boxes.low[d][0] && hy >= boxes.low[d][1] && hz >= boxes.low[d][2] &&
+		                   lx <= boxes.up[d][0] && ly <= boxes.up[d][1] && lz <= boxes.up[d][2];
 		mask |= (uint64_t)meets << d;
 	}
 	return mask;
 }
 
-__global__ __launch_bounds__(kSelectThreads) void straddler_count_kernel(StraddlerSelectArgs a, uint32_t blocks)
+__global__ __launch_bounds__(kSelectThreads) void straddler_count_kernel(StraddlerBatch batch)
 {
 	__shared__ uint32_t total[kMaxShareBoxes];
+	const StraddlerJob& a = batch.job[blockIdx.y];
+	const ShareBoxes& boxes = batch.boxes;
+	const uint32_t blocks = a.blocks;
+	if (blockIdx.x >= blocks)
+		return;
 	const int tid = threadIdx.x;
 	if (tid < kMaxShareBoxes)
 		total[tid] = 0;
@@ -63,25 +68,27 @@ __global__ __launch_bounds__(kSelectThreads) void straddler_count_kernel(Straddl
 #pragma unroll
 	for (int j = 0; j < kSelectItems; j++) {
 		const uint32_t i = base + j * kSelectThreads + tid;
-		const uint64_t m = i < (uint32_t)a.n ? lend_mask(a, i) : 0;
+		const uint64_t m = i < (uint32_t)a.n ? lend_mask(a, boxes, i) : 0;
 		if (__ballot(m != 0) == 0)
 			continue;
-		for (int d = 0; d < a.boxes.count; d++) {
+		for (int d = 0; d < boxes.count; d++) {
 			const uint64_t lent = __ballot((m >> d) & 1);
 			if (lent && (tid & (kWave - 1)) == 0)
 				atomicAdd(&total[d], (uint32_t)__popcll(lent));
 		}
 	}
 	__syncthreads();
-	if (tid < a.boxes.count)
+	if (tid < boxes.count)
 		a.block_counts[(size_t)tid * blocks + blockIdx.x] = total[tid];
 }
 
-// One workgroup per destination: exclusive scan of that destination's per-block counts, in place.
-__global__ __launch_bounds__(256) void straddler_scan_kernel(uint32_t* block_counts, uint32_t blocks, uint32_t* counts)
+// One workgroup per source and destination: exclusive scan of that destination's per-block counts, in place.
+__global__ __launch_bounds__(256) void straddler_scan_kernel(StraddlerBatch batch)
 {
 	__shared__ uint32_t lds[8];
-	uint32_t* row = block_counts + (size_t)blockIdx.x * blocks;
+	const StraddlerJob& a = batch.job[blockIdx.y];
+	const uint32_t blocks = a.blocks;
+	uint32_t* row = a.block_counts + (size_t)blockIdx.x * blocks;
 	uint32_t carry = 0;
 	for (uint32_t at = 0; at < blocks; at += 256) {
 		const uint32_t i = at + threadIdx.x;
@@ -94,12 +101,17 @@ __global__ __launch_bounds__(256) void straddler_scan_kernel(uint32_t* block_cou
 		__syncthreads();
 	}
 	if (threadIdx.x == 0)
-		counts[blockIdx.x] = carry;
+		a.counts[blockIdx.x] = carry;
 }
 
-__global__ __launch_bounds__(kSelectThreads) void straddler_emit_kernel(StraddlerSelectArgs a, uint32_t blocks)
+__global__ __launch_bounds__(kSelectThreads) void straddler_emit_kernel(StraddlerBatch batch)
 {
 	__shared__ uint32_t cell[kSelectCells][kMaxShareBoxes];
+	const StraddlerJob& a = batch.job[blockIdx.y];
+	const ShareBoxes& boxes = batch.boxes;
+	const uint32_t blocks = a.blocks;
+	if (blockIdx.x >= blocks)
+		return;
 	const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
 	for (int c = tid; c < kSelectCells * kMaxShareBoxes; c += kSelectThreads)
 		(&cell[0][0])[c] = 0;
@@ -109,10 +121,10 @@ __global__ __launch_bounds__(kSelectThreads) void straddler_emit_kernel(Straddle
 #pragma unroll
 	for (int j = 0; j < kSelectItems; j++) {
 		const uint32_t i = base + j * kSelectThreads + tid;
-		masks[j] = i < (uint32_t)a.n ? lend_mask(a, i) : 0;
+		masks[j] = i < (uint32_t)a.n ? lend_mask(a, boxes, i) : 0;
 		if (__ballot(masks[j] != 0) == 0)
 			continue;
-		for (int d = 0; d < a.boxes.count; d++) {
+		for (int d = 0; d < boxes.count; d++) {
 			const uint64_t lent = __ballot((masks[j] >> d) & 1);
 			if (lent && lane == 0)
 				cell[j * kSelectWaves + wave][d] = (uint32_t)__popcll(lent);
@@ -125,7 +137,7 @@ __global__ __launch_bounds__(kSelectThreads) void straddler_emit_kernel(Straddle
 			continue;
 		const uint32_t i = base + j * kSelectThreads + tid;
 		const int mine = j * kSelectWaves + wave;
-		for (int d = 0; d < a.boxes.count; d++) {
+		for (int d = 0; d < boxes.count; d++) {
 			const bool bit = (masks[j] >> d) & 1;
 			const uint64_t lent = __ballot(bit);
 			if (!lent)
@@ -241,23 +253,158 @@ __global__ __launch_bounds__(256) void merge_rows_backward_kernel(MergeBackwardA
 	}
 }
 
+// ---- rows lent between stored models --------------------------------------------------------------
+// As the merge above, for models whose SH rows stay where they are stored, in two parts: only lent rows are joined, into an array of their
+// own, and all pairs of lender and borrower go in one launch.
+typedef float UnalignedFloat4 __attribute__((ext_vector_type(4), aligned(4)));
+
+template <int kFloats>
+__device__ __forceinline__ void copy_narrow(const float* __restrict__ from, float* __restrict__ to)
+{
+	float v[kFloats];
+#pragma unroll
+	for (int c = 0; c < kFloats; c++)
+		v[c] = from[c];
+#pragma unroll
+	for (int c = 0; c < kFloats; c++)
+		to[c] = v[c];
+}
+
+__global__ __launch_bounds__(256) void lend_rows_kernel(LendArgs a)
+{
+	int k = 0;
+	while (k + 1 < a.segments && blockIdx.x >= a.seg[k + 1].block0)
+		k++;
+	const LendSegment& seg = a.seg[k];
+	const LendModel &source = a.model[seg.source], &dest = a.model[seg.destination];
+	const uint32_t j = (blockIdx.x - seg.block0) * kRowsPerBlock + threadIdx.x / kRowLanes;
+	if (j >= seg.count)
+		return;
+	const int part = threadIdx.x % kRowLanes;
+	const size_t from = seg.rows ? seg.rows[j] : j, to = (size_t)seg.at + j;
+	if (part == 13)
+		copy_narrow<3>(source.means3D_from + 3 * from, dest.means3D + 3 * to);
+	if (!seg.rows)
+		return;
+	if (part < 12) {
+		float4 v;
+		if (part == 0) {
+			const float* first = source.sh_first + 3 * from;
+			v = float4{first[0], first[1], first[2], source.sh_rest[45 * from]};
+		} else {
+			const UnalignedFloat4 r = *reinterpret_cast<const UnalignedFloat4*>(source.sh_rest + 45 * from + 4 * part - 3);
+			v = float4{r.x, r.y, r.z, r.w};
+		}
+		reinterpret_cast<float4*>(dest.sh_lent)[12 * ((size_t)seg.sh_at + j) + part] = v;
+	} else if (part == 12) {
+		reinterpret_cast<float4*>(dest.rotations)[to] = reinterpret_cast<const float4*>(source.rotations)[from];
+	} else if (part == 14) {
+		copy_narrow<3>(source.scales + 3 * from, dest.scales + 3 * to);
+	} else if (part == 15) {
+		dest.opacity[to] = source.opacity[from];
+	}
+}
+
+template <int kFloats>
+__device__ __forceinline__ void add_narrow(const float* __restrict__ g, float* __restrict__ into)
+{
+	float v[kFloats];
+#pragma unroll
+	for (int c = 0; c < kFloats; c++)
+		v[c] = into[c] + g[c];
+#pragma unroll
+	for (int c = 0; c < kFloats; c++)
+		into[c] = v[c];
+}
+
+// The gradients of lent rows are added to those of the rows they were read from.  Every segment of a launch has another source and a
+// segment's rows are distinct, so the additions need no atomics.
+__global__ __launch_bounds__(256) void lend_rows_backward_kernel(LendBackwardArgs a)
+{
+	int k = 0;
+	while (k + 1 < a.segments && blockIdx.x >= a.seg[k + 1].block0)
+		k++;
+	const LendSegment& seg = a.seg[k];
+	const LendGradients &into = a.model[seg.source], &g = a.model[seg.destination];
+	const uint32_t j = (blockIdx.x - seg.block0) * kRowsPerBlock + threadIdx.x / kRowLanes;
+	if (j >= seg.count)
+		return;
+	const int part = threadIdx.x % kRowLanes;
+	const size_t to = seg.rows[j], at = (size_t)seg.at + j;
+	if (part < 12) {
+		if (!g.sh_lent)
+			return;
+		const float4 v = reinterpret_cast<const float4*>(g.sh_lent)[12 * ((size_t)seg.sh_at + j) + part];
+		if (part == 0) {
+			float* first = into.sh_first + 3 * to;
+			first[0] += v.x;
+			first[1] += v.y;
+			first[2] += v.z;
+			into.sh_rest[45 * to] += v.w;
+		} else {
+			UnalignedFloat4* p = reinterpret_cast<UnalignedFloat4*>(into.sh_rest + 45 * to + 4 * part - 3);
+			UnalignedFloat4 t = *p;
+			t.x += v.x; t.y += v.y; t.z += v.z; t.w += v.w;
+			*p = t;
+		}
+	} else if (part == 12) {
+		if (g.rotations)
+			add_narrow<4>(g.rotations + 4 * at, into.rotations + 4 * to);
+	} else if (part == 13) {
+		if (g.means3D)
+			add_narrow<3>(g.means3D + 3 * at, into.means3D + 3 * to);
+	} else if (part == 14) {
+		if (g.scales)
+			add_narrow<3>(g.scales + 3 * at, into.scales + 3 * to);
+		if (g.opacity)
+			add_narrow<1>(g.opacity + at, into.opacity + to);
+	} else {
+		if (g.means2D)
+			add_narrow<3>(g.means2D + 3 * at, into.means2D + 3 * to);
+	}
+}
+
 }  // namespace
+
+void launch_lend_rows(const LendArgs& a, uint32_t blocks, hipStream_t s)
+{
+	stage_mark("lend_rows", s);
+	if (blocks)
+		hipLaunchKernelGGL(lend_rows_kernel, dim3(blocks), dim3(256), 0, s, a);
+}
+
+void launch_lend_rows_backward(const LendBackwardArgs& a, uint32_t blocks, hipStream_t s)
+{
+	stage_mark("lend_rows_backward", s);
+	if (blocks)
+		hipLaunchKernelGGL(lend_rows_backward_kernel, dim3(blocks), dim3(256), 0, s, a);
+}
 
 uint32_t straddler_select_blocks(int n)
 {
 	return (uint32_t)((n + kSelectBlock - 1) / kSelectBlock);
 }
 
-void launch_straddler_select(const StraddlerSelectArgs& a, hipStream_t s)
+// The sources of a frame in one launch per step (kMaxBatch of them at a time).
+void launch_straddler_select(const StraddlerJob* jobs, int count, const ShareBoxes& boxes, hipStream_t s)
 {
-	const uint32_t blocks = straddler_select_blocks(a.n);
 	stage_mark("straddler_select", s);
-	if (blocks) {
-		hipLaunchKernelGGL(straddler_count_kernel, dim3(blocks), dim3(kSelectThreads), 0, s, a, blocks);
-		hipLaunchKernelGGL(straddler_scan_kernel, dim3(a.boxes.count), dim3(256), 0, s, a.block_counts, blocks, a.counts);
-		hipLaunchKernelGGL(straddler_emit_kernel, dim3(blocks), dim3(kSelectThreads), 0, s, a, blocks);
-	} else {
-		launch_fill_u32(a.counts, 0, a.boxes.count, s);
+	for (int at = 0; at < count; at += kMaxBatch) {
+		const int nj = count - at < kMaxBatch ? count - at : kMaxBatch;
+		StraddlerBatch b;
+		b.boxes = boxes;
+		uint32_t most = 0;
+		for (int k = 0; k < nj; k++) {
+			b.job[k] = jobs[at + k];
+			b.job[k].blocks = straddler_select_blocks(jobs[at + k].n);
+			most = b.job[k].blocks > most ? b.job[k].blocks : most;
+		}
+		const dim3 grid(most, (unsigned)nj);
+		if (most)
+			hipLaunchKernelGGL(straddler_count_kernel, grid, dim3(kSelectThreads), 0, s, b);
+		hipLaunchKernelGGL(straddler_scan_kernel, dim3((unsigned)boxes.count, (unsigned)nj), dim3(256), 0, s, b);
+		if (most)
+			hipLaunchKernelGGL(straddler_emit_kernel, grid, dim3(kSelectThreads), 0, s, b);
 	}
 }
 

@@ -333,6 +333,8 @@ constexpr int kActRows = 128;     // SH rows per workgroup: six workgroups' rows
 constexpr int kActMaxRest = 15;
 static_assert(kActRows % 4 == 0, "a workgroup's rows begin at a multiple of 16 bytes in each of the tensors");
 
+__host__ __device__ inline uint32_t blocks_of(size_t units, size_t per_block) { return (uint32_t)((units + per_block - 1) / per_block); }
+
 struct ActParts {
 	uint32_t sh_blocks, rot_blocks, scale_blocks, opacity_blocks;
 	uint32_t rest_reciprocal;  // 0: the SH rows go by 4-byte accesses, kActUnits per workgroup; otherwise kActRows rows per workgroup
@@ -345,14 +347,13 @@ static_assert((size_t)kActRows * 3 * kActMaxRest * 3 * kActMaxRest < (1u << 20),
 inline ActParts act_parts(int n, int rest, bool sh_by_16_bytes)
 {
 	const size_t sh_floats = 3 * (size_t)(1 + rest);
-	auto blocks = [](size_t units, size_t per_block) { return (uint32_t)((units + per_block - 1) / per_block); };
 	ActParts p;
 	const bool by_rows = sh_by_16_bytes && rest >= 1 && rest <= kActMaxRest;
 	p.rest_reciprocal = by_rows ? ((1u << 20) + 3 * (uint32_t)rest - 1) / (3 * (uint32_t)rest) : 0u;
-	p.sh_blocks = by_rows ? blocks((size_t)n, kActRows) : blocks(((size_t)n * sh_floats + 3) / 4, kActUnits);
-	p.rot_blocks = blocks((size_t)n, kActUnits);
-	p.scale_blocks = blocks(((size_t)n * 3 + 3) / 4, kActUnits);
-	p.opacity_blocks = blocks(((size_t)n + 3) / 4, kActUnits);
+	p.sh_blocks = by_rows ? blocks_of((size_t)n, kActRows) : blocks_of(((size_t)n * sh_floats + 3) / 4, kActUnits);
+	p.rot_blocks = blocks_of((size_t)n, kActUnits);
+	p.scale_blocks = blocks_of(((size_t)n * 3 + 3) / 4, kActUnits);
+	p.opacity_blocks = blocks_of(((size_t)n + 3) / 4, kActUnits);
 	return p;
 }
 
@@ -497,6 +498,124 @@ __device__ __forceinline__ void flat_units(uint32_t block, size_t total, const f
 	}
 }
 
+// kActUnits quaternions per workgroup: made unit ones, and the gradient through that.
+__device__ __forceinline__ void unit_quaternions(uint32_t block, size_t n, const float* __restrict__ from, float* __restrict__ to)
+{
+	constexpr int kTurns = kActUnits / 256;
+	const size_t i0 = (size_t)block * kActUnits + threadIdx.x;
+	float4 v[kTurns];
+#pragma unroll
+	for (int t = 0; t < kTurns; t++)
+		if (i0 + 256 * t < n)
+			v[t] = load_streaming(reinterpret_cast<const float4*>(from) + i0 + 256 * t);
+#pragma unroll
+	for (int t = 0; t < kTurns; t++)
+		if (i0 + 256 * t < n) {
+			const float4 q = v[t];
+			const float len = fmaxf(sqrtf(q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w), 1e-12f);  // torch.nn.functional.normalize
+			store_streaming(reinterpret_cast<float4*>(to) + i0 + 256 * t, float4{q.x / len, q.y / len, q.z / len, q.w / len});
+		}
+}
+__device__ __forceinline__ void unit_quaternions_backward(uint32_t block, size_t n, const float* __restrict__ from, const float* __restrict__ grad,
+                                                          float* __restrict__ to)
+{
+	constexpr int kTurns = kActUnits / 256;
+	const size_t i0 = (size_t)block * kActUnits + threadIdx.x;
+	float4 v[kTurns], w[kTurns];
+#pragma unroll
+	for (int t = 0; t < kTurns; t++)
+		if (i0 + 256 * t < n) {
+			v[t] = load_streaming(reinterpret_cast<const float4*>(from) + i0 + 256 * t);
+			w[t] = load_streaming(reinterpret_cast<const float4*>(grad) + i0 + 256 * t);
+		}
+#pragma unroll
+	for (int t = 0; t < kTurns; t++)
+		if (i0 + 256 * t < n) {
+			// d/dq of q / |q|: (g - u (u . g)) / |q| with u = q / |q|
+			const float4 q = v[t], g = w[t];
+			const float len = fmaxf(sqrtf(q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w), 1e-12f);
+			const float u0 = q.x / len, u1 = q.y / len, u2 = q.z / len, u3 = q.w / len;
+			const float along = u0 * g.x + u1 * g.y + u2 * g.z + u3 * g.w;
+			store_streaming(reinterpret_cast<float4*>(to) + i0 + 256 * t,
+			                float4{(g.x - u0 * along) / len, (g.y - u1 * along) / len, (g.z - u2 * along) / len,
+			                       (g.w - u3 * along) / len});
+		}
+}
+
+__device__ __forceinline__ float activated_scale(float v) { return expf(v); }
+__device__ __forceinline__ float activated_opacity(float v) { return 1.0f / (1.0f + expf(-v)); }
+
+// Scales, rotations, opacities and the zeros of the screen-space placeholder of every stored model of a frame (blockIdx.y), in units as above.
+__global__ __launch_bounds__(256) void activate_many_kernel(Batch<ActivateJob> batch)
+{
+	const ActivateJob& j = batch.job[blockIdx.y];
+	const size_t n = (size_t)j.n;
+	uint32_t block = blockIdx.x;
+	const uint32_t rot_blocks = blocks_of(n, kActUnits), scale_blocks = blocks_of((3 * n + 3) / 4, kActUnits),
+	               opacity_blocks = blocks_of((n + 3) / 4, kActUnits);
+	if (block < rot_blocks) {
+		unit_quaternions(block, n, j.rotation, j.rotations);
+		return;
+	}
+	block -= rot_blocks;
+	if (block < scale_blocks) {
+		flat_units(block, 3 * n, j.scaling, nullptr, j.scales, [](float v, float) { return activated_scale(v); });
+		return;
+	}
+	block -= scale_blocks;
+	if (block < opacity_blocks) {
+		flat_units(block, n, j.opacity, nullptr, j.opacities, [](float v, float) { return activated_opacity(v); });
+		return;
+	}
+	block -= opacity_blocks;
+	const size_t floats = 3 * (size_t)j.zero_rows;
+#pragma unroll
+	for (int t = 0; t < kActUnits / 256; t++) {
+		const size_t at = 4 * ((size_t)block * kActUnits + 256 * t + threadIdx.x);
+		if (at + 4 <= floats)
+			*reinterpret_cast<float4*>(j.means2D + at) = float4{0.f, 0.f, 0.f, 0.f};
+		else
+			for (size_t k = at; k < floats; k++)
+				j.means2D[k] = 0.f;
+	}
+}
+
+__global__ __launch_bounds__(256) void activate_many_backward_kernel(Batch<ActivateBackwardJob> batch)
+{
+	const ActivateBackwardJob& j = batch.job[blockIdx.y];
+	const size_t n = (size_t)j.n;
+	uint32_t block = blockIdx.x;
+	const uint32_t rot_blocks = blocks_of(n, kActUnits), scale_blocks = blocks_of((3 * n + 3) / 4, kActUnits),
+	               opacity_blocks = blocks_of((n + 3) / 4, kActUnits);
+	if (block < rot_blocks) {
+		unit_quaternions_backward(block, n, j.rotation, j.g_rotations, j.d_rotation);
+		return;
+	}
+	block -= rot_blocks;
+	if (block < scale_blocks) {
+		flat_units(block, 3 * n, j.g_scales, j.scales, j.d_scaling, [](float g, float s) { return g * s; });
+		return;
+	}
+	block -= scale_blocks;
+	if (block < opacity_blocks) {
+		flat_units(block, n, j.g_opacities, j.opacities, j.d_opacity, [](float g, float o) { return g * (o * (1.0f - o)); });
+		return;
+	}
+	block -= opacity_blocks;
+	float x[kActUnits / 256], y[kActUnits / 256];
+	const size_t i0 = (size_t)block * kActUnits + threadIdx.x;
+#pragma unroll
+	for (int t = 0; t < kActUnits / 256; t++)
+		if (i0 + 256 * t < n) {
+			x[t] = j.g_means2D[3 * (i0 + 256 * t)];
+			y[t] = j.g_means2D[3 * (i0 + 256 * t) + 1];
+		}
+#pragma unroll
+	for (int t = 0; t < kActUnits / 256; t++)
+		if (i0 + 256 * t < n)
+			j.d_meta[i0 + 256 * t] = sqrtf(x[t] * x[t] + y[t] * y[t]);
+}
+
 __global__ __launch_bounds__(256) void activate_forward_kernel(ActivateArgs a, ActParts parts)
 {
 	__shared__ __attribute__((aligned(16))) float joined[kActRows * 3 * (1 + kActMaxRest)];
@@ -534,29 +653,16 @@ __global__ __launch_bounds__(256) void activate_forward_kernel(ActivateArgs a, A
 	}
 	block -= parts.sh_blocks;
 	if (block < parts.rot_blocks) {
-		constexpr int kTurns = kActUnits / 256;
-		const size_t i0 = (size_t)block * kActUnits + threadIdx.x;
-		float4 v[kTurns];
-#pragma unroll
-		for (int t = 0; t < kTurns; t++)
-			if (i0 + 256 * t < n)
-				v[t] = load_streaming(reinterpret_cast<const float4*>(a.rotation) + i0 + 256 * t);
-#pragma unroll
-		for (int t = 0; t < kTurns; t++)
-			if (i0 + 256 * t < n) {
-				const float4 q = v[t];
-				const float len = fmaxf(sqrtf(q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w), 1e-12f);  // torch.nn.functional.normalize
-				store_streaming(reinterpret_cast<float4*>(a.rotations) + i0 + 256 * t, float4{q.x / len, q.y / len, q.z / len, q.w / len});
-			}
+		unit_quaternions(block, n, a.rotation, a.rotations);
 		return;
 	}
 	block -= parts.rot_blocks;
 	if (block < parts.scale_blocks) {
-		flat_units(block, 3 * n, a.scaling, nullptr, a.scales, [](float v, float) { return expf(v); });
+		flat_units(block, 3 * n, a.scaling, nullptr, a.scales, [](float v, float) { return activated_scale(v); });
 		return;
 	}
 	block -= parts.scale_blocks;
-	flat_units(block, n, a.opacity, nullptr, a.opacities, [](float v, float) { return 1.0f / (1.0f + expf(-v)); });
+	flat_units(block, n, a.opacity, nullptr, a.opacities, [](float v, float) { return activated_opacity(v); });
 }
 
 __global__ __launch_bounds__(256) void activate_backward_kernel(ActivateBackwardArgs a, ActParts parts)
@@ -603,27 +709,7 @@ __global__ __launch_bounds__(256) void activate_backward_kernel(ActivateBackward
 	if (block < parts.rot_blocks) {
 		if (!a.g_rotations)
 			return;
-		constexpr int kTurns = kActUnits / 256;
-		const size_t i0 = (size_t)block * kActUnits + threadIdx.x;
-		float4 v[kTurns], w[kTurns];
-#pragma unroll
-		for (int t = 0; t < kTurns; t++)
-			if (i0 + 256 * t < n) {
-				v[t] = load_streaming(reinterpret_cast<const float4*>(a.rotation) + i0 + 256 * t);
-				w[t] = load_streaming(reinterpret_cast<const float4*>(a.g_rotations) + i0 + 256 * t);
-			}
-#pragma unroll
-		for (int t = 0; t < kTurns; t++)
-			if (i0 + 256 * t < n) {
-				// d/dq of q / |q|: (g - u (u . g)) / |q| with u = q / |q|
-				const float4 q = v[t], g = w[t];
-				const float len = fmaxf(sqrtf(q.x * q.x + q.y * q.y + q.z * q.z + q.w * q.w), 1e-12f);
-				const float u0 = q.x / len, u1 = q.y / len, u2 = q.z / len, u3 = q.w / len;
-				const float along = u0 * g.x + u1 * g.y + u2 * g.z + u3 * g.w;
-				store_streaming(reinterpret_cast<float4*>(a.d_rotation) + i0 + 256 * t,
-				                float4{(g.x - u0 * along) / len, (g.y - u1 * along) / len, (g.z - u2 * along) / len,
-				                       (g.w - u3 * along) / len});
-			}
+		unit_quaternions_backward(block, n, a.rotation, a.g_rotations, a.d_rotation);
 		return;
 	}
 	block -= parts.rot_blocks;
@@ -657,6 +743,42 @@ void launch_activate_backward(const ActivateBackwardArgs& a, hipStream_t s)
 	const ActParts p = act_parts(a.n, a.rest, a.features_by_16_bytes);
 	hipLaunchKernelGGL(activate_backward_kernel, dim3(p.sh_blocks + p.rot_blocks + p.scale_blocks + p.opacity_blocks), dim3(256),
 	                   0, s, a, p);
+}
+
+void launch_activate_many(const ActivateJob* jobs, int count, hipStream_t s)
+{
+	stage_mark("activate_forward", s);
+	for (int at = 0; at < count; at += kMaxBatch) {
+		const int nj = count - at < kMaxBatch ? count - at : kMaxBatch;
+		Batch<ActivateJob> b;
+		uint32_t most = 0;
+		for (int k = 0; k < nj; k++) {
+			const ActivateJob& j = b.job[k] = jobs[at + k];
+			const size_t n = (size_t)j.n;
+			const uint32_t blocks = blocks_of(n, kActUnits) + blocks_of((3 * n + 3) / 4, kActUnits) + blocks_of((n + 3) / 4, kActUnits) +
+			                        blocks_of((3 * (size_t)j.zero_rows + 3) / 4, kActUnits);
+			most = blocks > most ? blocks : most;
+		}
+		if (most)
+			hipLaunchKernelGGL(activate_many_kernel, dim3(most, (unsigned)nj), dim3(256), 0, s, b);
+	}
+}
+
+void launch_activate_many_backward(const ActivateBackwardJob* jobs, int count, hipStream_t s)
+{
+	stage_mark("activate_backward", s);
+	for (int at = 0; at < count; at += kMaxBatch) {
+		const int nj = count - at < kMaxBatch ? count - at : kMaxBatch;
+		Batch<ActivateBackwardJob> b;
+		uint32_t most = 0;
+		for (int k = 0; k < nj; k++) {
+			const size_t n = (size_t)(b.job[k] = jobs[at + k]).n;
+			const uint32_t blocks = 2 * blocks_of(n, kActUnits) + blocks_of((3 * n + 3) / 4, kActUnits) + blocks_of((n + 3) / 4, kActUnits);
+			most = blocks > most ? blocks : most;
+		}
+		if (most)
+			hipLaunchKernelGGL(activate_many_backward_kernel, dim3(most, (unsigned)nj), dim3(256), 0, s, b);
+	}
 }
 
 uint32_t loss_blocks(int C, int H, int W)

@@ -33,6 +33,9 @@ class Submodel:
     range_up: torch.Tensor
     active_sh_degree: int = 3
     means2D: Optional[torch.Tensor] = None   # screen-space placeholder whose gradient densification reads
+    # SH rows in parts: shs holds the first coefficients of the first N Gaussians, these their others and the others' whole rows
+    # (read by render_frame(together=True) alone)
+    sh_parts: Optional[tuple] = None
 
     def parameters(self) -> List[torch.Tensor]:
         return [self.means3D, self.opacity, self.scales, self.rotations, self.shs]
@@ -369,6 +372,8 @@ def render_frame(cam: Camera, subs: List[Submodel], relation: np.ndarray, backgr
             settings.append(raster_settings(cam, sub, submodel_bg))
             inputs.append(dict(means3D=sub.means3D, means2D=means2D, shs=sub.shs, opacities=sub.opacity, scales=sub.scales,
                                rotations=sub.rotations))
+            if sub.sh_parts is not None:
+                inputs[-1]["sh_parts"] = sub.sh_parts
         taps = [] if keep_workspaces else None
         # from two million pixels of all layers on the compositor passes over what they do not show (four submodels, both
         # directions: 63 -> 49 us at 1600x1036, 808 -> 530 at 5185x3359; 13.0 -> 13.5 at 648x420)
@@ -555,6 +560,27 @@ def make_stored_optimisers(models: List[StoredModel], scale: float = 1.0):
     return out
 
 
+def _shown_together(models: List[StoredModel], part: Partition, append: bool):
+    """Activation, selection and lending of all models at once, as far as the library's kernels for that take them (16 models of
+    contiguous float32 tensors on one GPU, 16 SH coefficients): (lent rows, submodels whose SH rows are read where they are
+    stored), or None.  The rows and values are those of activated(), select_straddlers and merge_shared."""
+    if any(type(m).activated is not StoredModel.activated for m in models):
+        return None
+    flat = [t for m in models for t in (m.xyz, m.features_dc, m.features_rest, m.scaling, m.rotation, m.opacity, m.means2D_meta)]
+    boxes = np.stack([part.box_low, part.box_up]).astype(np.float32).ravel().tolist()
+    made = _host.show_stored(flat, boxes, [int(m.spare_rows) for m in models], append)
+    if made is None:
+        return None
+    counts, rows = made
+    K = len(models)
+    corners = _host.floats_on_device(boxes, models[0].xyz).view(2, K, 3)
+    shown = []
+    for k, low, up in zip(range(K), corners[0].unbind(), corners[1].unbind()):
+        means3D, means2D, opacity, scales, rotations, first, rest, lent = rows[8 * k:8 * k + 8]
+        shown.append(Submodel(means3D, opacity, scales, rotations, first, low, up, means2D=means2D, sh_parts=(rest, lent)))
+    return sum(counts), shown
+
+
 def stored_training_iteration(models: List[StoredModel], optimisers, part: Partition, cam: Camera, relation: np.ndarray,
                               gt_image: torch.Tensor, background: torch.Tensor, lambda_dssim: float = 0.2,
                               streams: Optional[List["torch.cuda.Stream"]] = None) -> dict:
@@ -563,14 +589,20 @@ def stored_training_iteration(models: List[StoredModel], optimisers, part: Parti
     SH coefficients).  Lent rows are appended when the models were made with spare rows."""
     from ..loss import l1_ssim_loss
     from ..sharing import merge_shared, select_straddlers
-    device = models[0].xyz.device
-    shown = [m.activated() for m in models]
-    table = select_straddlers(shown, part.box_low, part.box_up)
-    merged = merge_shared(shown, table, reuse_gradients=True, append=all(m.spare_rows > 0 for m in models))
-    frame = render_frame(cam, submodels_from_shared(merged, part, device), relation, background, streams=streams, together=True)
+    append = all(m.spare_rows > 0 for m in models)
+    together = _shown_together(models, part, append)
+    if together is not None:
+        lent_rows, shown = together
+    else:
+        device = models[0].xyz.device
+        activated = [m.activated() for m in models]
+        table = select_straddlers(activated, part.box_low, part.box_up)
+        merged = merge_shared(activated, table, reuse_gradients=True, append=append)
+        lent_rows, shown = int(table.counts.sum()), submodels_from_shared(merged, part, device)
+    frame = render_frame(cam, shown, relation, background, streams=streams, together=True)
     loss, l1 = l1_ssim_loss(frame["render"], gt_image, lambda_dssim)
     loss.backward()
     for opt in optimisers:
         opt.step()
         opt.zero_grad(set_to_none=True)
-    return {"loss": loss.detach(), "l1": l1, "frame": frame, "lent_rows": int(table.counts.sum())}
+    return {"loss": loss.detach(), "l1": l1, "frame": frame, "lent_rows": lent_rows}

@@ -229,13 +229,15 @@ def rasterize_frame(rasterizers, inputs, streams=None, workspaces=None):
 
 def _rasterize_layers(settings, inputs, streams=None, workspaces=None, strips=None):
     """rasterize_frame from the layers' settings.  `strips`: a list that receives what the compositor can use of each layer
-    (see _host.composite)."""
+    (see _host.composite).  A layer's "sh_parts", of all layers or of none: the further parts of SH rows of which "shs" holds
+    the first coefficients (see _host.rasterize_frame)."""
     flat = []
+    split = None if not any("sh_parts" in kw for kw in inputs) else [kw["sh_parts"] for kw in inputs]
     for kw in inputs:
         shs, colors_precomp, scales, rotations, cov3D = _checked_inputs(kw.get("shs"), kw.get("colors_precomp"), kw.get("scales"),
                                                                         kw.get("rotations"), kw.get("cov3D_precomp"))
         flat += (kw["means3D"], kw["means2D"], shs, colors_precomp, kw["opacities"], scales, rotations, cov3D)
-    return _host.rasterize_frame(settings, flat, streams, workspaces, strips)
+    return _host.rasterize_frame(settings, flat, streams, workspaces, strips, split)
 
 
 def _checked_inputs(shs, colors_precomp, scales, rotations, cov3D_precomp):

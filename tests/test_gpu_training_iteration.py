@@ -150,3 +150,55 @@ def test_the_loss_goes_down_from_stored_parameters(spare):
         seen_meta_grad = seen_meta_grad or float(g.max()) > 0.0
         assert all(p.grad is not None and torch.isfinite(p.grad).all() for p in m.parameters())
     assert seen_meta_grad
+
+
+class _Still:
+    def step(self):
+        pass
+
+    def zero_grad(self, set_to_none=True):
+        pass
+
+
+@pytest.mark.parametrize("depth,spare,grow,unrelated", [(1, 0.0, 2.0, False), (1, 0.3, 2.0, False), (2, 0.0, 2.0, True), (2, 3.0, 100.0, False),
+                                                        (1, 0.0, 100.0, False), (3, 4.0, 12.0, True)])
+def test_models_shown_together_are_models_shown_one_by_one(depth, spare, grow, unrelated):
+    """An iteration's gradients with activation, selection and lending of all models in one launch each and SH rows read as they are
+    stored, against activated(), select_straddlers and merge_shared: from a few lent rows to lists longer than the room there is at
+    first, with room behind the positions and without, models that the camera does not see, two to eight of them."""
+    from retinags_amd.harness import partition, pipeline
+
+    class OneByOne(pipeline.StoredModel):
+        def activated(self):
+            return super().activated()
+
+    scene, cam, _ = scenes.make_config("C1", shrink=100 if grow > 20 else 150, resolution_scale=0.25)
+    scene["scales"] = scene["scales"] * grow
+    part = partition.partition_scene(scene["xyz"], scene["scales"], depth)
+    rel = partition.relation_vector(part, cam)
+    if unrelated:
+        rel = np.where(rel == rel.max(), -1.0, rel)
+    cam_d, bg = cam.to(DEV), torch.rand(3, device=DEV)
+    gt = torch.rand(3, cam.image_height, cam.image_width, device=DEV)
+    grads, lent, renders = [], [], []
+    for kind in (pipeline.StoredModel, OneByOne):
+        models = [kind(**vars(m)) for m in pipeline.stored_models_from_partition(scene, part, DEV, spare)]
+        for m in models:
+            for t in m.parameters():
+                t.requires_grad_(True)
+        step = pipeline.stored_training_iteration(models, [_Still() for _ in models], part, cam_d, rel, gt, bg)
+        grads.append([[t.grad for t in m.parameters()] for m in models])
+        lent.append(step["lent_rows"])
+        renders.append(step["frame"]["render"].detach())
+    own = [int(m.xyz.shape[0]) for m in models]
+    if grow > 20:   # some list is longer than the room for it at first, some model borrows more than there is room for at first
+        from retinags_amd.sharing import select_straddlers
+        counts = select_straddlers([m.activated() for m in models], part.box_low, part.box_up).counts
+        assert any(counts[k].max() > n // 8 + 4096 for k, n in enumerate(own)) and any(counts[:, k].sum() > n // 8 + 4096 for k, n in enumerate(own))
+    assert lent[0] == lent[1] > 20 and torch.equal(renders[0], renders[1])
+    for a, b in zip(*grads):
+        for k, (got, want) in enumerate(zip(a, b)):
+            assert got.shape == want.shape
+            # (sums of float atomics: equal up to their order)
+            assert torch.linalg.norm(got - want) <= 1e-4 * torch.linalg.norm(want), k
+    assert any(float(torch.linalg.norm(g[1])) > 0 for g in grads[0])
