@@ -267,7 +267,7 @@ size_t geom_layout(size_t P, size_t* off)
 int tile_key_bits(int width, int height)
 {
 	const uint32_t tiles = (uint32_t)((width + rgs::kTile - 1) / rgs::kTile) * (uint32_t)((height + rgs::kTile - 1) / rgs::kTile);
-	return (int)rgs_get_higher_msb(tiles);
+	return (int)rgs_get_higher_msb(tiles > 1 ? tiles - 1 : 1);
 }
 
 // Passes of the instance sort on the tile bits.

@@ -462,7 +462,7 @@ __global__ __launch_bounds__(256) void duplicate_with_keys_kernel(Batch<Duplicat
 {
 	__shared__ DuplicateStage st;
 	__shared__ uint32_t s_first;
-	constexpr int kTileDigitWords = 3 * 512;  // tiles have at most 24 bits: three passes at most
+	constexpr int kTileDigitWords = 4 * 512;  // one digit of up to 11 bits, or up to three of 9 (tiles have at most 24 bits)
 	__shared__ uint32_t s_digits[kTileDigitWords];  // digit counts of the tiles this workgroup writes
 	extern __shared__ __align__(16) float s_ndc[];  // NDC of the middle of every tile column, then of every tile row
 	const DuplicateJob& job = batch.job[blockIdx.y];
@@ -676,7 +676,7 @@ __global__ __launch_bounds__(256) void duplicate_with_keys_kernel(Batch<Duplicat
 	}
 	}
 	__syncthreads();
-	for (int w = tid; w < 512 * passes; w += 256) {
+	for (int w = tid; w < (passes == 1 ? 1 << job.end_bit : 512 * passes); w += 256) {
 		const uint32_t c = s_digits[w];
 		if (c)
 			atomicAdd(&job.tile_digits[(blockIdx.x & (job.digit_copies - 1u)) * kDigitWords + w], c);
@@ -717,9 +717,8 @@ void launch_duplicate_with_keys(const DuplicateJob* jobs, int count, int grid_x,
 // kSortThreads * kItems pairs in arrival order, rank them in LDS, obtain their global digit offsets from
 // the blocks before them through a chained look-back over per-tile status words, and scatter.
 // Element order inside a tile is (wave, round, lane); ranking preserves it, and tiles are
-// ordered by their id, so every pass is stable.  A digit has up to kBits bits (template parameter): 9 for 32-bit
-// keys, which sorts 17 or 18 tile bits in two passes and 27 depth bits in three, 8 for 64-bit keys, whose tiles of
-// pairs fill the LDS.
+// ordered by their id, so every pass is stable.  A digit has up to kBits bits (template parameter): 7 to 11 for 32-bit
+// keys (sort_max_digit_bits_u32), 8 for 64-bit keys, whose tiles of pairs fill the LDS.
 //
 // Scratch layout (u32 words), B = 2^kBits:
 //   [0, 2048)      digit histograms, B words per pass, where the job names no digit_counts (every block of a pass scans its counts itself)
@@ -822,8 +821,8 @@ enum SortPassKind { kPassPlain = 0, kPassEndsUnless = 1, kPassOnDemand = 2 };
 // Per-wave digit counts fit 16 bits (a wavefront ranks kSortItems * 64 keys), and so does a digit's place inside a tile.
 template <int kBits>
 struct SortCounts {
-	uint16_t digit_base[1 << kBits];    // exclusive prefix over digits within the tile
-	uint32_t global_base[1 << kBits];   // where this tile's run of each digit starts globally
+	uint16_t digit_base[1 << kBits];                  // exclusive prefix over digits within the tile
+	__align__(8) uint32_t global_base[1 << kBits];    // where this tile's run of each digit starts globally
 };
 
 // How many wavefronts stand by to fill the gaps of the others' phases (loads, ranking, look-back, stores) and how long the runs are
@@ -833,12 +832,17 @@ struct SortCounts {
 // to memory, ahead of the ranking, and sixteen took 119 registers instead of 89 (per pass, us: instances of two submodels of 2.8 M
 // 64 -> 58, of two at 5185x3359 378 -> 328, of one of 2.8 M in training 45 -> 42, its depths 20 -> 17).
 template <typename KeyT, int kBits, int kKind, int kItems>
-__global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(sizeof(KeyT) == 4 && kItems <= 8 ? 8 : 4))) void sort_onesweep_kernel(
+__global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(sizeof(KeyT) == 4 && kItems <= 8 && kBits <= 10 ? 8 : 4))) void sort_onesweep_kernel(
 	Batch<SortJob<KeyT>> batch, int pass, int shift, uint32_t mask, int spin_limit)
 {
 	constexpr int kBins = 1 << kBits;
 	constexpr int kWaves = kSortThreads / 64, kBlock = kSortThreads * kItems;
-	static_assert(kBins <= kSortThreads, "a thread owns at most one digit value");
+	// A thread owns one digit value, or two neighbouring ones whose counts and look-back words it handles as halves of one number.
+	constexpr int kOwn = kBins > kSortThreads ? 2 : 1;
+	static_assert(kBins <= 2 * kSortThreads, "a thread owns at most two digit values");
+	typedef std::conditional_t<kOwn == 2, uint64_t, uint32_t> Word;
+	constexpr Word kBoth = kOwn == 2 ? (Word)0x100000001ull : (Word)1u;
+	constexpr Word kAggregates = kFlagAggregate * kBoth, kInclusives = kFlagInclusive * kBoth, kValues = kValueMask * kBoth;
 	const SortJob<KeyT>& j = batch.job[blockIdx.y];
 	// the passes ping-pong between the two buffer pairs, starting in -> out
 	const KeyT* __restrict__ keys_in = (pass & 1) ? j.keys_out : j.keys_in;
@@ -868,7 +872,8 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 	uint32_t* __restrict__ lookback = j.temp + kSortHeader + (size_t)pass * kBins * job_tiles;
 	uint32_t* __restrict__ tile_counter = j.temp + kSortCounters + pass;
 	uint32_t* __restrict__ status = j.temp + kSortStatus;
-	__shared__ KeyT s_keys[kBlock];
+	constexpr int kCountKeys = kWaves * kBins * (int)sizeof(uint16_t) / (int)sizeof(KeyT);  // the room that the counts take
+	__shared__ __align__(16) KeyT s_keys[kBlock > kCountKeys ? kBlock : kCountKeys];
 	__shared__ uint32_t s_vals[kBlock];
 	__shared__ SortCounts<kBits> sc;
 	__shared__ uint32_t s_scan[kWaves];
@@ -879,6 +884,7 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 	const bool owns = tid < kBins;
+	const int own = tid * kOwn;  // the first digit value that the thread owns
 	// Tiles are handed out in arrival order, so every tile a block waits for below belongs to
 	// a block that is already running.
 	if (tid == 0)
@@ -922,12 +928,12 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 		uint32_t same_lo = ~0u, same_hi = ~0u;
 #pragma unroll
 		for (int b = 0; b < kBits; b++) {
-			int own = (int)(d << (31 - b)) >> 31;
-			asm("" : "+v"(own));  // (or the compiler forms the bit a second time for the vote)
-			const uint64_t vote = lanes_where(own != 0);
-			// same & ~(vote ^ own), one instruction
-			same_lo = (uint32_t)__builtin_amdgcn_bitop3_b32((int)same_lo, (int)(uint32_t)vote, own, 0x90);
-			same_hi = (uint32_t)__builtin_amdgcn_bitop3_b32((int)same_hi, (int)(uint32_t)(vote >> 32), own, 0x90);
+			int bit = (int)(d << (31 - b)) >> 31;
+			asm("" : "+v"(bit));  // (or the compiler forms the bit a second time for the vote)
+			const uint64_t vote = lanes_where(bit != 0);
+			// same & ~(vote ^ bit), one instruction
+			same_lo = (uint32_t)__builtin_amdgcn_bitop3_b32((int)same_lo, (int)(uint32_t)vote, bit, 0x90);
+			same_hi = (uint32_t)__builtin_amdgcn_bitop3_b32((int)same_hi, (int)(uint32_t)(vote >> 32), bit, 0x90);
 		}
 		const uint32_t below = __builtin_amdgcn_mbcnt_hi(same_hi, __builtin_amdgcn_mbcnt_lo(same_lo, 0u));
 		// every lane reads its digit's count (lanes of one digit the same word), then the first of each digit's lanes adds theirs:
@@ -940,47 +946,62 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 		__builtin_amdgcn_wave_barrier();
 	}
 	// the counts of the thread's digit value in all tiles, needed once this tile's are published
-	uint32_t totals[kDigitCopies] = {};
+	Word totals[kDigitCopies] = {};
 	if (owns) {
-		totals[0] = digit_count[tid];
+		totals[0] = *reinterpret_cast<const Word*>(digit_count + own);
 		if (j.digit_copies > 1u)
 #pragma unroll
 			for (int c = 1; c < kDigitCopies; c++)
-				totals[c] = digit_count[c * kDigitWords + tid];
+				totals[c] = *reinterpret_cast<const Word*>(digit_count + c * kDigitWords + own);
 	}
 	__syncthreads();
 
-	// A thread owns a digit value: prefix over the waves, publish the tile's count.
+	// For the digit values that a thread owns: prefix over the waves, publish the tile's counts.
 	const uint32_t valid = min(n - block_base, (uint32_t)kBlock);
 	// (by its distance in bytes, below 2^32: an address of 64 bits takes its registers through the whole kernel)
-	auto word_of = [&](uint32_t t) { return reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(lookback) + (t * (uint32_t)kBins + (uint32_t)tid) * 4u); };
-	uint32_t count = 0, digit_start;
+	auto word_of = [&](uint32_t t) { return reinterpret_cast<Word*>(reinterpret_cast<char*>(lookback) + (t * (uint32_t)kBins + (uint32_t)own) * 4u); };
+	Word count = 0, digit_start;
 	{
+		typedef std::conditional_t<kOwn == 2, uint32_t, uint16_t> Counts;  // (two counts of 16 bits are added as one number)
+		uint32_t prefix = 0;
 		if (owns) {
 			uint32_t c[kWaves];
 #pragma unroll
 			for (int w = 0; w < kWaves; w++)
-				c[w] = wave_hist[w][tid];
+				c[w] = *reinterpret_cast<const Counts*>(&wave_hist[w][own]);
 #pragma unroll
 			for (int w = 0; w < kWaves; w++) {
-				wave_hist[w][tid] = (uint16_t)count;
-				count += c[w];
+				*reinterpret_cast<Counts*>(&wave_hist[w][own]) = (Counts)prefix;
+				prefix += c[w];
 			}
 		}
+		count = kOwn == 2 ? (Word)(prefix & 0xFFFFu) | (Word)(prefix >> 16) << (32 * (kOwn - 1)) : (Word)prefix;
 		uint32_t total;
-		const uint32_t ex = block_exclusive_scan_u32<kWaves>(count, s_scan, total);
+		const uint32_t ex = block_exclusive_scan_u32<kWaves>(kOwn == 2 ? (prefix & 0xFFFFu) + (prefix >> 16) : prefix, s_scan, total);
+		if (owns) {
+			sc.digit_base[own] = (uint16_t)ex;
+			if (kOwn == 2)
+				sc.digit_base[own + kOwn - 1] = (uint16_t)(ex + (prefix & 0xFFFFu));
+		}
+		// what fills the tile up is not published
+		if ((uint32_t)(own + kOwn - 1) == mask)
+			count -= (Word)((uint32_t)kBlock - valid) << (32 * (kOwn - 1));
+		else if ((uint32_t)own == mask)
+			count -= (Word)((uint32_t)kBlock - valid);
 		if (owns)
-			sc.digit_base[tid] = (uint16_t)ex;
-		if ((uint32_t)tid == mask)
-			count -= (uint32_t)kBlock - valid;  // what fills the tile up is not published
-		if (owns)
-			__hip_atomic_store(word_of(tile), count | (tile == 0 ? kFlagInclusive : kFlagAggregate), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+			__hip_atomic_store(word_of(tile), count | (tile == 0 ? kInclusives : kAggregates), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 		// where the digit's run starts in the whole array: the exclusive scan of the digit counts
-		uint32_t all, digit_total = 0;
+		uint32_t all;
+		Word digit_total = 0;
 #pragma unroll
 		for (int c = 0; c < kDigitCopies; c++)
 			digit_total += totals[c];
-		digit_start = block_exclusive_scan_u32<kWaves>(digit_total, s_scan, all);
+		if (kOwn == 2) {
+			const uint32_t start = block_exclusive_scan_u32<kWaves>((uint32_t)digit_total + (uint32_t)(digit_total >> (32 * (kOwn - 1))), s_scan, all);
+			digit_start = (Word)start | (Word)(start + (uint32_t)digit_total) << (32 * (kOwn - 1));
+		} else {
+			digit_start = block_exclusive_scan_u32<kWaves>((uint32_t)digit_total, s_scan, all);
+		}
 	}
 
 	// The tile's pairs in digit order, through LDS.  None of this needs the tiles before this one: by the time
@@ -1008,29 +1029,29 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 		out_val[i] = s_vals[q];
 	}
 
-	// Look back: the pairs of this thread's digit value in all earlier tiles.
+	// Look back: the pairs of this thread's digit values in all earlier tiles.
 	if (owns) {
-		uint32_t exclusive = 0;
+		Word exclusive = 0;
 		if (tile != 0) {
 			// Words of the tiles below t are still to be added.  Up to kLookBatch of them are requested
 			// together: walked one load at a time, the chain of tiles and not memory sets the pace of a pass.
 			uint32_t t = tile;
 			bool gave_up = spin_limit < 0, done = false;
 			while (!gave_up && !done) {
-				uint32_t v[kLookBatch];
+				Word v[kLookBatch];
 #pragma unroll
 				for (int q = 0; q < kLookBatch; q++)
 					v[q] = (uint32_t)q < t ? __hip_atomic_load(word_of(t - 1u - (uint32_t)q), __ATOMIC_RELAXED,
 					                                           __HIP_MEMORY_SCOPE_AGENT)
-					                       : kFlagInclusive;  // below the first tile there is nothing
+					                       : kInclusives;  // below the first tile there is nothing
 				uint32_t used = 0;
 #pragma unroll
 				for (int q = 0; q < kLookBatch; q++) {
 					// a word counts once every nearer one has been published and none of them closed the sum
-					if (!done && used == (uint32_t)q && (v[q] >> 30) != 0u) {
-						exclusive += v[q] & kValueMask;
+					if (!done && used == (uint32_t)q && (v[q] & (kAggregates | kInclusives)) != 0u) {
+						exclusive += v[q] & kValues;
 						used = (uint32_t)q + 1u;
-						done = (v[q] & kFlagInclusive) != 0u;
+						done = (v[q] & kInclusives) != 0u;
 					}
 				}
 				t -= used < t ? used : t;
@@ -1038,9 +1059,9 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 					done = true;
 				if (!done && used < (uint32_t)kLookBatch) {
 					// tile t - 1 has not published yet: wait for its word, then look again from there
-					const uint32_t* word = word_of(t - 1u);
-					uint32_t w = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-					for (int spins = 0; (w >> 30) == 0u; spins++) {
+					const Word* word = word_of(t - 1u);
+					Word w = __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+					for (int spins = 0; (w & (kAggregates | kInclusives)) == 0u; spins++) {
 						// give up after a bounded wait, or as soon as any other look-back has
 						if (spins >= spin_limit ||
 						    ((spins & 255) == 255 &&
@@ -1057,9 +1078,9 @@ __global__ __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(si
 				atomicOr(status, 1u);
 			// On the (never expected) give-up path `exclusive` is too small, which keeps every
 			// scatter address inside the array; the status word tells the consumer to discard it.
-			__hip_atomic_store(word_of(tile), ((exclusive + count) & kValueMask) | kFlagInclusive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+			__hip_atomic_store(word_of(tile), ((exclusive + count) & kValues) | kInclusives, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 		}
-		sc.global_base[tid] = digit_start + exclusive;
+		*reinterpret_cast<Word*>(&sc.global_base[own]) = digit_start + exclusive;
 	}
 	__syncthreads();
 
@@ -1142,7 +1163,7 @@ static void launch_sort_pass(const Batch<SortJob<KeyT>>& b, size_t most_pairs, s
 	const dim3 grid((unsigned)sort_tiles(most_pairs, items), (unsigned)jobs);
 	const int spin = g_lookback_spin_limit.load();
 	if constexpr (sizeof(KeyT) == 4) {
-		if constexpr (kBits == 9) {
+		if constexpr (kBits >= 9) {
 			if (items == kSortItemsMany) {
 				hipLaunchKernelGGL((sort_onesweep_kernel<KeyT, kBits, kKind, kSortItemsMany>), grid, dim3(kSortThreads), 0, s, b, pass, shift, mask, spin);
 				return;
@@ -1212,10 +1233,13 @@ void launch_sort_pairs(uint64_t* keys_in, uint64_t* keys_out, uint32_t* vals_in,
 void launch_sort_pairs_u32(const SortJob<uint32_t>* jobs, int count, int end_bit, bool temp_cleared, bool histograms_done,
                            const char* stage, hipStream_t s)
 {
-	if (sort_max_digit_bits_u32(end_bit) == 9)
-		sort_pairs<uint32_t, 9>(jobs, count, end_bit, temp_cleared, histograms_done, stage != nullptr, s);
-	else
-		sort_pairs<uint32_t, 8>(jobs, count, end_bit, temp_cleared, histograms_done, stage != nullptr, s);
+	switch (sort_max_digit_bits_u32(end_bit)) {
+	case 11: sort_pairs<uint32_t, 11>(jobs, count, end_bit, temp_cleared, histograms_done, stage != nullptr, s); break;
+	case 10: sort_pairs<uint32_t, 10>(jobs, count, end_bit, temp_cleared, histograms_done, stage != nullptr, s); break;
+	case 9: sort_pairs<uint32_t, 9>(jobs, count, end_bit, temp_cleared, histograms_done, stage != nullptr, s); break;
+	case 8: sort_pairs<uint32_t, 8>(jobs, count, end_bit, temp_cleared, histograms_done, stage != nullptr, s); break;
+	default: sort_pairs<uint32_t, 7>(jobs, count, end_bit, temp_cleared, histograms_done, stage != nullptr, s);
+	}
 }
 
 // ---- depth order of few Gaussians: one workgroup per job, out of LDS -------------------------------

@@ -370,16 +370,22 @@ void launch_preprocess_backward(const PreprocessBackwardArgs* jobs, int count, h
 
 // binning.hip
 // A sort on the lowest end_bit bits of its keys takes ceil(end_bit / max_bits) passes, max_bits being the widest digit
-// its kernel handles (kDigitBitsU32 for 32-bit keys, kDigitBitsU64 for 64-bit ones); the bits are shared out evenly
+// its kernel handles (sort_max_digit_bits_u32 for 32-bit keys, kDigitBitsU64 for 64-bit ones); the bits are shared out evenly
 // between the passes, the wider digits first (13 bits: 7 then 6, not 9 then 4: the fewer values a digit has, the longer
 // the runs of neighbouring keys a pass writes).
-constexpr int kDigitBitsU32 = 9;   // 512 digit values: the 17 tile bits of a 5185x3359 image in two passes, 27 depth bits in three
 constexpr int kDigitBitsU64 = 8;
-// The widest digit the sort of 32-bit keys on end_bit bits uses: 9 bits where that saves a pass, 8 otherwise (a pass
-// over 512 digit values writes shorter runs and was measured 14 % slower than one over 256).
+// The widest digit the sort of 32-bit keys on end_bit bits uses.  Up to 11 bits (2 048 tiles) are sorted in one pass, whose 2 048 digit values
+// are two per thread: a pass over the instances of a small image is a chain of a few dependent waits for memory, whatever it ranks (per
+// call, us, one pass and two: 100 000 Gaussians at 512x512 153 and 159, at 720x640 162 and 169; 2 M 440 and 461, 455 and 473; 20 000 at 700x700
+// 145 and 152.  12 bits would need 128 KB of LDS for the counts of sixteen wavefronts).  Beyond, as few passes as nine bits allow
+// (18 tile bits in two, 27 depth bits in three), and no wider than those need: a pass votes once per bit and pair, and one
+// over 512 digit values writes shorter runs (13 bits, two submodels of 2.8 M: 117 us as eight bits, 111 as seven; 62.9 M 356 and 344).
 __host__ __device__ inline int sort_max_digit_bits_u32(int end_bit)
 {
-	return (end_bit + 8) / 9 < (end_bit + 7) / 8 ? 9 : 8;
+	if (end_bit <= 11)
+		return end_bit < 7 ? 7 : end_bit;
+	const int passes = (end_bit + 8) / 9, bits = (end_bit + passes - 1) / passes;
+	return bits < 7 ? 7 : bits;
 }
 __host__ __device__ inline int sort_passes(int end_bit, int max_bits)
 {
@@ -400,16 +406,16 @@ constexpr int kSortThreads = 1024;
 // fewer cache lines two workgroups (on two XCDs) share; but fewer, larger tiles leave part of the chip idle when the pairs
 // are few.  By what a launch has room for: the instances of all its jobs, which the host knows, and for the depth sort all their
 // Gaussians, of which the host does not know how many are visible (16 from twice as many on).  Per pass, us, with 4 / 8 / 16:
-//   instances: 5185x3359 with 5.6 M Gaussians (nine-bit digits; those that follow have eight bits) 501 / 350 / 328, 62.9 M at 1600x1036 259 / 174 / 186, 5.6 M there
+//   instances: 5185x3359 with 5.6 M Gaussians (nine-bit digits; those that follow were measured with eight bits) 501 / 350 / 328, 62.9 M at 1600x1036 259 / 174 / 186, 5.6 M there
 //   78 / 58 / 60, 2.8 M in training 51 / 42 / 42, a call of 333 333 Gaussians 22 / 18 / 21, of 100 000 12 / 13 / 17;
 //   depths: 62.9 M, a third visible 153 / 100 / 114; 27 M, a twentieth visible 21 / 21 / 19; 5.6 M, a third visible 21 / 21 / 19;
 //   2.8 M in training 17 / 17 / 17, 333 333, all visible 13 / 14 / 19, 100 000 11 / 13 / 18.
 constexpr int kSortItemsFew = 4, kSortItems = 8, kSortItemsMany = 16;
-constexpr size_t kSortSome = (size_t)1 << 20, kSortMany = (size_t)1 << 25;  // pairs from which 8, and with nine-bit digits 16, are taken
+constexpr size_t kSortSome = (size_t)1 << 20, kSortMany = (size_t)1 << 25;  // pairs from which 8, and with digits of nine bits and more 16, are taken
 constexpr int kSortBlock = kSortThreads * kSortItemsFew;  // pairs of the smallest tile
 inline int sort_items(size_t pairs, int digit_bits)
 {
-	return digit_bits == 9 && pairs >= kSortMany ? kSortItemsMany : pairs >= kSortSome ? kSortItems : kSortItemsFew;
+	return digit_bits >= 9 && pairs >= kSortMany ? kSortItemsMany : pairs >= kSortSome ? kSortItems : kSortItemsFew;
 }
 size_t scan_temp_words(size_t n);                 // u32 words of scratch for launch_inclusive_sum
 // `stage` (may be null) names the stage for the timing aid.
@@ -438,7 +444,7 @@ void launch_totals_from_block_sums(const TotalsJob* jobs, int count, hipStream_t
 // copy of its number, and the sort adds the copies up (0.2 us per launch).  With 1, 4, 8 and 16 copies the key duplication takes 27.0, 14.2,
 // 12.8 and 12.4 us at 100 000 Gaussians and 77, 45, 45 and 45 for three submodels of a city; with 1 and 8 the listing of pairs 39 and 15 us
 // there, 36 and 20 for two submodels of 2.8 M each.  Up to 128 workgroups (4 000 Gaussians: 4) one copy is the faster.
-constexpr int kDigitWords = 4 * 512;  // keys have at most four digits
+constexpr int kDigitWords = 4 * 512;  // keys have at most four digits of nine bits, or one of eleven
 constexpr int kDigitCopies = 8;
 constexpr uint32_t digit_copies(size_t workgroups) { return workgroups > 128 ? kDigitCopies : 1; }
 struct DepthOrderJob {
@@ -499,7 +505,7 @@ void launch_duplicate_with_keys(const DuplicateJob* jobs, int count, int grid_x,
 size_t sort_clear_words(size_t n, int end_bit, int max_bits);
 size_t depth_sort_clear_words(size_t n);          // the same for the depth sort of launch_depth_order
 // The scratch has room for 2048 digit counts and as many look-back words per tile of kSortBlock pairs, the smallest: 8 passes of 256
-// digit values (64-bit keys) or 4 passes of 512 (32-bit keys).
+// digit values (64-bit keys), 4 passes of 512 or one of 2048 (32-bit keys).
 constexpr uint32_t kSortScratchPerTile = 2048;
 constexpr uint32_t kSortHeader = 2112;            // words ahead of the look-back words: histograms, counters, status
 constexpr size_t sort_temp_words_for(size_t n)

@@ -91,6 +91,20 @@ def test_sorts_in_the_largest_tiles():
     check_sorts((1 << 26) + 5, 4112, 4096)
 
 
+@pytest.mark.parametrize("width,height", ((16, 16), (256, 128), (192, 176), (256, 256), (272, 256), (512, 256), (384, 352), (512, 512), (656, 400),
+                                          (1024, 512), (832, 640)))
+def test_tile_digits_of_every_width(width, height):
+    """1, 128, 132, 256, 272, 512, 528, 1 024, 1 025, 2 048 and 2 080 tiles: on both sides of every width of the instance sort's digit, up to one
+    pass of 11 bits (two digit values per thread) and the first two passes beyond."""
+    check_sorts(70_001, width, height)
+
+
+@pytest.mark.parametrize("n", ((1 << 20) + 4097, 34_000_003))   # sort tiles of 8 192 and of 16 384 pairs
+@pytest.mark.parametrize("width,height", ((512, 512), (1024, 512)))
+def test_wide_tile_digits_in_larger_tiles(n, width, height):
+    check_sorts(n, width, height)
+
+
 @pytest.mark.parametrize("n", (8, 1023, 1024, 1025, 1026, 1027, 4096 + 6))
 def test_totals_of_ragged_groups(n):
     """All in view: the sums of 1 024 tile counts where the last group is whole, short of a quad or a few counts beyond."""
