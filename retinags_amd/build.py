@@ -39,7 +39,7 @@ SOURCES = {
 }
 
 HOST_SOURCES = ["host.cpp", "host_training.cpp"]
-HEADERS = ["rgs_device.h", "rgs_kernels.h", "strip_filing.h", "tile_order.h", os.path.join("..", "..", "include", "rgs.h")]
+HEADERS = ["counts.h", "rgs_device.h", "rgs_kernels.h", "strip_filing.h", "tile_order.h", os.path.join("..", "..", "include", "rgs.h")]
 
 
 def _hipcc() -> str:
@@ -91,7 +91,7 @@ def build(force: bool = False, verbose: bool = True) -> str:
     link = force or bool(jobs) or _stale(LIB, objs)
     host_parts, host_link = _host_commands()
     for source, command, o in host_parts:
-        if force or _stale(o, [source, os.path.join(CSRC, "host.h"), hdrs[-1]]):
+        if force or _stale(o, [source, os.path.join(CSRC, "host.h"), os.path.join(CSRC, "counts.h"), hdrs[-1]]):
             jobs.insert(0, command)
 
     def run(cmd):

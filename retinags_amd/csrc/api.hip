@@ -2,6 +2,7 @@
 // sequencing and error reporting.  The declarations and the reference interfaces they
 // replace are in include/rgs.h.
 #include "../../include/rgs.h"
+#include "counts.h"
 #include "rgs_kernels.h"
 
 #include <algorithm>
@@ -506,6 +507,17 @@ static hipEvent_t count_event_of_this_thread()
 	return events[dev];
 }
 
+// The address under which the current device writes to host memory that the runtime has allocated (pinned); null for any other memory.
+static uint32_t* device_address_of_host_memory(uint32_t* host)
+{
+	hipPointerAttribute_t a;
+	if (hipPointerGetAttributes(&a, host) != hipSuccess) {
+		(void)hipGetLastError();
+		return nullptr;
+	}
+	return a.type == hipMemoryTypeHost && a.hostPointer == host ? static_cast<uint32_t*>(a.devicePointer) : nullptr;
+}
+
 // One layer's arguments of the geometry stage.
 struct GeomCall {
 	int P, D, M;
@@ -524,7 +536,8 @@ struct GeomCall {
 };
 
 // The geometry stage of `K` layers that share a camera, every kernel launched once for all of them: preprocess,
-// the instance counts (one copy to counts_host[0..K)), and, behind that copy, the depth order.
+// the instance counts, which the kernel that adds them up writes to counts_host[0..K) where that is pinned memory (a copy brings them
+// otherwise), and, behind them, the depth order.
 static int forward_geom(bool wait_for_count, void* count_ready_event, const char* who, int K, const GeomCall* calls,
                         int width, int height, const float* viewmatrix, const float* projmatrix, const float* cam_pos,
                         float tan_fovx, float tan_fovy, uint32_t* counts_host, void* stream, int debug)
@@ -537,7 +550,8 @@ static int forward_geom(bool wait_for_count, void* count_ready_event, const char
 	std::vector<rgs::PreprocessArgs> pre((size_t)K);
 	std::vector<rgs::TotalsJob> totals((size_t)K);
 	std::vector<rgs::DepthOrderJob> orders((size_t)K);
-	uint32_t* frame_counts = nullptr;  // K words in the first layer's workspace, so that one copy brings all counts
+	uint32_t* const counts_seen = device_address_of_host_memory(counts_host);
+	uint32_t* frame_counts = counts_seen;  // or K words in the first layer's workspace, so that one copy brings all counts
 	for (int k = 0; k < K; k++) {
 		const GeomCall& c = calls[k];
 		RGS_REQUIRE(c.P > 0, "%s: P must be positive (the caller short-circuits P == 0)", who);
@@ -555,7 +569,7 @@ static int forward_geom(bool wait_for_count, void* count_ready_event, const char
 		size_t off[RGS_GEOM_FIELDS];
 		geom_layout((size_t)c.P, off);
 		void* ws = c.geom_ws;
-		if (k == 0)
+		if (k == 0 && !counts_seen)
 			frame_counts = at<uint32_t>(ws, off[RGS_GEOM_TOTAL]) + 1;
 		rgs::PreprocessArgs& a = pre[(size_t)k];
 		a.P = c.P; a.D = c.D; a.M = c.M;
@@ -601,13 +615,17 @@ static int forward_geom(bool wait_for_count, void* count_ready_event, const char
 		d.dup_first = at<uint32_t>(scratch, o.dup_first);
 		d.digits = at<uint32_t>(scratch, o.digits);
 	}
+	if (counts_seen && wait_for_count)
+		rgs::expect_counts(counts_host, K);
 	rgs::launch_preprocess_forward(pre.data(), K, s);
 	RGS_STAGE("preprocess");
 	rgs::launch_totals_from_block_sums(totals.data(), K, s);
 	RGS_STAGE("instance count");
-	hipError_t e = hipMemcpyAsync(counts_host, frame_counts, sizeof(uint32_t) * (size_t)K, hipMemcpyDeviceToHost, s);
-	// the host only needs the counts: it waits for this event, not for the kernels queued below
-	hipEvent_t ready = wait_for_count ? count_event_of_this_thread() : static_cast<hipEvent_t>(count_ready_event);
+	hipError_t e = hipSuccess;
+	if (!counts_seen)
+		e = hipMemcpyAsync(counts_host, frame_counts, sizeof(uint32_t) * (size_t)K, hipMemcpyDeviceToHost, s);
+	// the host only needs the counts: it waits for them or for this event, not for the kernels queued below
+	hipEvent_t ready = !wait_for_count ? static_cast<hipEvent_t>(count_ready_event) : counts_seen ? nullptr : count_event_of_this_thread();
 	if (e == hipSuccess && ready)
 		e = hipEventRecord(ready, s);
 	// depth order of the Gaussians and the offsets of their instances in that order: needs
@@ -615,7 +633,7 @@ static int forward_geom(bool wait_for_count, void* count_ready_event, const char
 	rgs::launch_depth_order(orders.data(), K, s);
 	RGS_STAGE("depth order");
 	if (e == hipSuccess && wait_for_count)
-		e = ready ? hipEventSynchronize(ready) : hipStreamSynchronize(s);
+		e = counts_seen ? rgs::wait_for_counts(counts_host, K, s) : ready ? hipEventSynchronize(ready) : hipStreamSynchronize(s);
 	if (e != hipSuccess)
 		return fail("%s: reading the instance count failed: %s", who, hipGetErrorString(e));
 	if (wait_for_count)

@@ -109,6 +109,8 @@ __global__ __launch_bounds__(1024) void single_block_exclusive_scan_kernel(Batch
 			base += s;
 		total += s;
 	}
+	if (tid == 0 && total_copy)
+		__hip_atomic_store(total_copy, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);  // (host memory: the host waits for this word)
 	uint32_t run = base + inc - sum;
 	for (size_t i = lo; i < hi; i++) {
 		const uint32_t v = from[i];
@@ -122,8 +124,6 @@ __global__ __launch_bounds__(1024) void single_block_exclusive_scan_kernel(Batch
 	}
 	if (tid == 0 && total_out)
 		*total_out = total;
-	if (tid == 0 && total_copy)
-		*total_copy = total;
 }
 
 struct BlockInclusiveJob {

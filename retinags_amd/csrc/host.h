@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "../../include/rgs.h"
+#include "counts.h"
 
 namespace rgs_host {
 
@@ -134,6 +135,7 @@ inline hipStream_t current_stream(const at::Device& device) { return c10::hip::g
 // A few pinned words and an event that says they have arrived.
 struct CountSlot {
 	uint32_t* words = nullptr;
+	uint32_t* on_device = nullptr;  // the same words as kernels write them
 	hipEvent_t event = nullptr;
 };
 
@@ -184,10 +186,13 @@ public:
 		}
 		CountSlot s;
 		void* memory = nullptr;
+		void* address = nullptr;
 		if (hipHostMalloc(&memory, kSlotWords * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess ||
+		    hipHostGetDevicePointer(&address, memory, 0) != hipSuccess ||
 		    hipEventCreateWithFlags(&s.event, hipEventDisableTiming) != hipSuccess)
 			throw std::runtime_error("no pinned memory for an instance count");
 		s.words = static_cast<uint32_t*>(memory);
+		s.on_device = static_cast<uint32_t*>(address);
 		return s;
 	}
 	void give_back(int device, CountSlot s)
@@ -226,6 +231,37 @@ inline SlotPool& slot_pool()
 	static SlotPool* pool = new SlotPool;  // stays until the process ends: the runtime may be gone before static objects are
 	return *pool;
 }
+
+// A slot whose words kernels of `stream` write, for as long as the caller is about to launch them and waits for what they write.
+class AwaitedCounts {
+public:
+	AwaitedCounts(int device, hipStream_t stream, int n) : device_(device), stream_(stream), n_(n), slot_(slot_pool().take(device))
+	{
+		rgs::expect_counts(slot_.words, n);
+	}
+	~AwaitedCounts()
+	{
+		if (!arrived_)
+			(void)hipStreamSynchronize(stream_);  // a kernel may yet write them
+		slot_pool().give_back(device_, slot_);
+	}
+	AwaitedCounts(const AwaitedCounts&) = delete;
+	AwaitedCounts& operator=(const AwaitedCounts&) = delete;
+	uint32_t* on_device() const { return slot_.on_device; }
+	// The words, or null if they did not come.
+	const uint32_t* wait()
+	{
+		arrived_ = rgs::wait_for_counts(slot_.words, n_, stream_) == hipSuccess;
+		return arrived_ ? slot_.words : nullptr;
+	}
+
+private:
+	const int device_;
+	const hipStream_t stream_;
+	const int n_;
+	const CountSlot slot_;
+	bool arrived_ = false;
+};
 
 
 void define_training(py::module_& m);  // host_training.cpp

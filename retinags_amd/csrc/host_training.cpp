@@ -144,35 +144,32 @@ py::tuple select_straddlers(const std::vector<Tensor>& means3D, const std::vecto
 		const hipStream_t stream = current_stream(device);
 		const float *low = boxes.data(), *up = low + 3 * K;
 		const at::TensorOptions ints = at::TensorOptions().dtype(at::kInt).device(device);
-		const Tensor counts_dev = at::empty({K, K}, ints);
+		AwaitedCounts awaited(device.index(), stream, K * K);
 		variable_list scratch;
 		std::vector<int64_t> caps(K);
-		auto run = [&](int src) {
+		auto run = [&](int src, uint32_t* counts_at) {
 			const int64_t n = means3D[src].size(0);
 			lists[src] = at::empty({K, caps[src]}, ints);
 			scratch.push_back(new_bytes(std::max<size_t>(1, rgs_straddler_scratch_bytes(n, K)), device));
 			check(rgs_straddler_select(n, ptr(means3D[src]), ptr(scales[src]), low + 3 * src, up + 3 * src, K, low, up, src,
-			                           ptr<uint32_t>(counts_dev) + src * K, ptr<uint32_t>(lists[src]), caps[src],
+			                           counts_at, ptr<uint32_t>(lists[src]), caps[src],
 			                           scratch.back().data_ptr(), stream));
 		};
 		for (int src = 0; src < K; src++) {
 			const int64_t n = means3D[src].size(0);
 			caps[src] = std::min(n, capacity < 0 ? n / 8 + 4096 : capacity);
-			run(src);
+			run(src, awaited.on_device() + src * K);
 		}
-		const CountSlot slot = slot_pool().take(device.index());
-		const bool arrived = hipMemcpyAsync(slot.words, counts_dev.data_ptr(), K * K * sizeof(uint32_t), hipMemcpyDeviceToHost,
-		                                    stream) == hipSuccess &&
-		                     hipEventRecord(slot.event, stream) == hipSuccess && hipEventSynchronize(slot.event) == hipSuccess;
-		std::copy(slot.words, slot.words + K * K, counts.begin());
-		slot_pool().give_back(device.index(), slot);
+		const uint32_t* arrived = awaited.wait();
 		if (!arrived)
 			throw std::runtime_error("reading the straddlers' counts failed");
+		std::copy(arrived, arrived + K * K, counts.begin());
 		for (int src = 0; src < K; src++) {
 			const int64_t longest = *std::max_element(counts.begin() + src * K, counts.begin() + (src + 1) * K);
 			if (longest > caps[src]) {  // a list was cut short: once more with room for the longest
 				caps[src] = longest;
-				run(src);
+				scratch.push_back(at::empty({K}, ints));  // (the awaited words go to another call when this one returns)
+				run(src, ptr<uint32_t>(scratch.back()));
 			}
 		}
 	}
@@ -442,7 +439,7 @@ struct ShowStored : torch::autograd::Function<ShowStored> {
 	{
 		const int K = m.K;
 		const at::TensorOptions ints = at::TensorOptions().dtype(at::kInt).device(device);
-		const Tensor counts_dev = at::empty({K, K}, ints);
+		AwaitedCounts awaited(device.index(), stream, K * K);
 		std::vector<rgs_straddler_source> sources(K);
 		variable_list scratch;
 		m.lists.resize(K);
@@ -450,25 +447,23 @@ struct ShowStored : torch::autograd::Function<ShowStored> {
 			m.lists[k] = at::empty({K, capacity}, ints);
 			scratch.push_back(new_bytes(std::max<size_t>(1, rgs_straddler_scratch_bytes(m.own[k], K)), device));
 			return rgs_straddler_source{static_cast<int>(m.own[k]), ptr(in[kStoredFields * k + kStoredXyz]), ptr(act[k][0]),
-			                            ptr<uint32_t>(counts_dev) + k * K, ptr<uint32_t>(m.lists[k]), static_cast<uint32_t>(capacity),
+			                            awaited.on_device() + k * K, ptr<uint32_t>(m.lists[k]), static_cast<uint32_t>(capacity),
 			                            scratch.back().data_ptr()};
 		};
 		for (int k = 0; k < K; k++)
 			sources[k] = source(k, std::min(m.own[k], m.own[k] / 8 + 4096));
 		const float *low = m.boxes.data(), *up = low + 3 * K;
 		check(rgs_straddler_select_many(K, sources.data(), low, up, stream));
-		const CountSlot slot = slot_pool().take(device.index());
-		const bool arrived = hipMemcpyAsync(slot.words, counts_dev.data_ptr(), K * K * sizeof(uint32_t), hipMemcpyDeviceToHost, stream) ==
-		                         hipSuccess &&
-		                     hipEventRecord(slot.event, stream) == hipSuccess && hipEventSynchronize(slot.event) == hipSuccess;
-		m.counts.assign(slot.words, slot.words + K * K);
-		slot_pool().give_back(device.index(), slot);
+		const uint32_t* arrived = awaited.wait();
 		if (!arrived)
 			throw std::runtime_error("reading the straddlers' counts failed");
+		m.counts.assign(arrived, arrived + K * K);
 		for (int k = 0; k < K; k++) {
 			const int64_t longest = *std::max_element(m.counts.begin() + k * K, m.counts.begin() + (k + 1) * K);
 			if (longest > m.lists[k].size(1)) {
-				const rgs_straddler_source f = source(k, longest);
+				rgs_straddler_source f = source(k, longest);
+				scratch.push_back(at::empty({K}, ints));  // (the awaited words go to another call when this one returns)
+				f.counts = ptr<uint32_t>(scratch.back());
 				check(rgs_straddler_select(f.n, f.means3D, f.scales, low + 3 * k, up + 3 * k, K, low, up, k, f.counts, f.rows, f.capacity,
 				                           f.scratch, stream));
 			}

@@ -101,7 +101,7 @@ __global__ __launch_bounds__(256) void straddler_scan_kernel(StraddlerBatch batc
 		__syncthreads();
 	}
 	if (threadIdx.x == 0)
-		a.counts[blockIdx.x] = carry;
+		__hip_atomic_store(&a.counts[blockIdx.x], carry, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);  // (may be host memory that the host polls)
 }
 
 __global__ __launch_bounds__(kSelectThreads) void straddler_emit_kernel(StraddlerBatch batch)
