@@ -118,6 +118,25 @@ __device__ __forceinline__ uint64_t lanes_inside_box(uint64_t lanes, float w, co
 		lanes &= ~lanes_where(clipped_by_box(ray_of(rays), w, load_box_frame(a)));
 	return lanes;
 }
+// The same for the entries of a group: their comparisons stand together and one branch is for all of them.  (A branch per entry waits for
+// its comparisons each time, and the walks that last longest are those along a face of the box: forward of four submodels of 5.6 M, a call
+// each, 435 -> 410 us; in one launch 254 -> 247; 62.9 M 730 -> 716.  The backward, which has more to do between them, gained nothing.)
+template <int kEntries, typename Rays>
+__device__ __forceinline__ void keep_lanes_inside_box(uint64_t (&mask)[kEntries], const float (&w)[kEntries], const BoxSpan& s, const Rays& rays, const BlendArgs& a)
+{
+	uint64_t unsure[kEntries], any = 0ull;
+#pragma unroll
+	for (int i = 0; i < kEntries; i++) {
+		mask[i] &= ~(lanes_where(w[i] < s.from) | lanes_where(w[i] > s.to));
+		unsure[i] = mask[i] & (lanes_where(w[i] <= s.from_sure) | lanes_where(w[i] >= s.to_sure));
+		any |= unsure[i];
+	}
+	if (any != 0ull)
+#pragma unroll
+		for (int i = 0; i < kEntries; i++)
+			if (unsure[i] != 0ull)
+				mask[i] &= ~lanes_where(clipped_by_box(ray_of(rays), w[i], load_box_frame(a)));
+}
 // The same by the exact test alone, where some entry of the chunk lies at a clip w that is not positive.
 template <typename Rays>
 __device__ __forceinline__ uint64_t lanes_inside_box(uint64_t lanes, float w, const Rays& rays, const BlendArgs& a)
@@ -455,10 +474,12 @@ __device__ __forceinline__ void forward_alphas(FourEntries& e, uint64_t live, co
 		if (!kPlain)
 			e.mask[i] &= lanes_where(!(e.power[i] > 0.0f));
 	}
-	if (kBox == kBoxSpans)
+	if (kBox == kBoxSpans) {
 #pragma unroll
 		for (int i = 0; i < 4; i++)
-			e.mask[i] = lanes_inside_box(e.mask[i] & live, e.clip_w[i], span, rays, a);
+			e.mask[i] &= live;
+		keep_lanes_inside_box(e.mask, e.clip_w, span, rays, a);
+	}
 	if (kBox == kBoxExact)
 #pragma unroll
 		for (int i = 0; i < 4; i++)
