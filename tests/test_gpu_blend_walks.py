@@ -117,3 +117,54 @@ def test_backward_walks_shared_by_four_wavefronts(n, with_depth_alpha, faces):
     st = _check_forward_stages(sub, cam, torch.tensor([0.2, 0.1, 0.05]), max_borderline=5e-2)
     assert faces or np.mean(st.n_contrib > 0.9 * n) > 0.5
     _check_backward(sub, cam, torch.tensor([0.2, 0.1, 0.05]), seed=n, with_depth_alpha=with_depth_alpha)
+
+
+def _slab_along_a_face(n):
+    """Opaque Gaussians about a face of the box that the camera sees at 45 degrees: neighbouring pixels enter the box at depths with many
+    chunks of entries between them, and what lies behind the box's other faces is blended by no pixel."""
+    gen = torch.Generator().manual_seed(n)
+    scene = scenes.cube_scene(n, seed=n)
+    z = 2.0 + 0.3 * torch.rand(n, generator=gen) - 0.15
+    z[::5] = 2.0 + 3.0 * torch.rand(z[::5].shape, generator=gen)
+    side = z * (0.8 + 0.4 * torch.rand(n, generator=gen))
+    scene["xyz"] = torch.stack([side, (torch.rand(n, generator=gen) - 0.5) * 0.4 * (side + z), z], 1)
+    scene["scales"] = torch.full((n, 3), 0.012)
+    scene["opacity"] = torch.full((n, 1), 0.97)
+    return scene, (-9.0, -9.0, 2.0), (9.0, 0.4, 2.6)
+
+
+def test_chunks_that_no_pixel_can_blend_are_passed_over():
+    """Whole walks, which pass over chunks that the box clips for every unfinished pixel, against walks shared by four wavefronts, which
+    stage every chunk (the same view as two jobs of a launch and as one): equal images and last blended entries."""
+    from retinags_amd import GaussianRasterizationSettings, GaussianRasterizer, _capi, rasterizer
+    dev, n = "cuda:0", 250_000
+    scene, low, up = _slab_along_a_face(n)
+    cam = scenes.look_at_camera((0.0, 0.0, 0.0), (1.0, 0.0, 1.0), (0.0, -1, 0), 509, 501, 40.0).to(dev)
+    r = GaussianRasterizer(GaussianRasterizationSettings(
+        image_height=501, image_width=509, tanfovx=cam.tanfovx, tanfovy=cam.tanfovy, bg=torch.zeros(3, device=dev), scale_modifier=1.0,
+        viewmatrix=cam.world_view_transform, projmatrix=cam.full_proj_transform, projmatrix_inv=cam.projection_matrix_inv,
+        range_low=torch.tensor(low, device=dev), range_up=torch.tensor(up, device=dev), sh_degree=0, campos=cam.camera_center,
+        prefiltered=False, debug=False))
+    given = dict(means3D=scene["xyz"].to(dev), means2D=torch.zeros(n, 3, device=dev), opacities=scene["opacity"].to(dev),
+                 colors_precomp=torch.rand(n, 3, generator=torch.Generator().manual_seed(1)).to(dev), scales=scene["scales"].to(dev),
+                 rotations=scene["rotations"].to(dev))
+    im = _capi.image_layout(509, 501)
+    read = lambda img, key, count: img[im[key]:im[key] + 4 * count].view(torch.int32)
+    alone, both = [], []
+    with torch.no_grad():
+        one = rasterizer.rasterize_frame([r], [given], workspaces=alone)[0]
+        two = rasterizer.rasterize_frame([r, r], [given, given], workspaces=both)
+    totals, walked = (read(alone[0][3], key, 4096).long() for key in ("strip_total", "strip_filed"))
+    # some lists go on for more chunks than are looked at together behind the last entry that is blended
+    assert int((totals - walked).max()) > 64 * 16 and int(walked.max()) > 64 * 5
+    for k in range(2):
+        for name, a, b in zip(("colour", "radii", "depth", "alpha"), one, two[k]):
+            assert torch.equal(a, b), name
+        for key, count in (("strip_filed", 4096), ("n_contrib", 509 * 501)):
+            assert torch.equal(read(alone[0][3], key, count), read(both[k][3], key, count)), key
+
+
+def test_chunks_passed_over_against_the_checker():
+    scene, low, up = _slab_along_a_face(60_000)
+    cam = scenes.look_at_camera((0.0, 0.0, 0.0), (1.0, 0.0, 1.0), (0.0, -1, 0), 515, 497, 40.0)
+    _check_forward_stages(_scene_sub(scene, low=torch.tensor(low), up=torch.tensor(up)), cam, torch.tensor([0.2, 0.1, 0.05]), max_borderline=2e-3)
