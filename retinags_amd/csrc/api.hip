@@ -619,8 +619,20 @@ static int forward_geom(bool wait_for_count, void* count_ready_event, const char
 		rgs::expect_counts(counts_host, K);
 	rgs::launch_preprocess_forward(pre.data(), K, s);
 	RGS_STAGE("preprocess");
-	rgs::launch_totals_from_block_sums(totals.data(), K, s);
-	RGS_STAGE("instance count");
+	// The one workgroup that orders a few Gaussians has their tile counts at hand: it adds them up, a launch less in a chain of a dozen (calls of
+	// 4 000 Gaussians 86.7 -> 82.8 us, four submodels of 2 000 165 -> 161).
+	bool totals_with_order = true;
+	for (int k = 0; k < K; k++)
+		totals_with_order = totals_with_order && calls[k].P <= rgs::kSmallOrder;
+	if (totals_with_order) {
+		for (int k = 0; k < K; k++)
+			orders[(size_t)k].totals = totals[(size_t)k];
+		rgs::launch_depth_order(orders.data(), K, s);
+		RGS_STAGE("depth order");
+	} else {
+		rgs::launch_totals_from_block_sums(totals.data(), K, s);
+		RGS_STAGE("instance count");
+	}
 	hipError_t e = hipSuccess;
 	if (!counts_seen)
 		e = hipMemcpyAsync(counts_host, frame_counts, sizeof(uint32_t) * (size_t)K, hipMemcpyDeviceToHost, s);
@@ -630,8 +642,10 @@ static int forward_geom(bool wait_for_count, void* count_ready_event, const char
 		e = hipEventRecord(ready, s);
 	// depth order of the Gaussians and the offsets of their instances in that order: needs
 	// nothing from the host, so it is queued behind the counts' copy
-	rgs::launch_depth_order(orders.data(), K, s);
-	RGS_STAGE("depth order");
+	if (!totals_with_order) {
+		rgs::launch_depth_order(orders.data(), K, s);
+		RGS_STAGE("depth order");
+	}
 	if (e == hipSuccess && wait_for_count)
 		e = counts_seen ? rgs::wait_for_counts(counts_host, K, s) : ready ? hipEventSynchronize(ready) : hipStreamSynchronize(s);
 	if (e != hipSuccess)

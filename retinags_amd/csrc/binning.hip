@@ -1256,6 +1256,7 @@ __global__ __launch_bounds__(1024) void small_depth_order_kernel(Batch<DepthOrde
 	__shared__ uint16_t s_digit_base[kBins];
 	__shared__ uint32_t s_scan[kWaves];
 	__shared__ uint32_t s_above;  // bits above those of the three passes
+	__shared__ uint32_t s_tiles[kWaves];
 	const DepthOrderJob& j = batch.job[blockIdx.x];
 	const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
 	const uint32_t P = (uint32_t)j.P, index_bits = depth_index_bits(P), cap = 0xFFFFFFFFu >> index_bits, index_mask = (1u << index_bits) - 1u;
@@ -1290,7 +1291,24 @@ __global__ __launch_bounds__(1024) void small_depth_order_kernel(Batch<DepthOrde
 #pragma unroll
 		for (int q = 0; q < kItems; q++)
 			mine += __float_as_uint(depth[q]) != 0u ? 1u : 0u;
+		uint32_t tiles = 0;
+#pragma unroll
+		for (int q = 0; q < kItems; q++)
+			tiles += count[q];
+		tiles = wave_inclusive_scan_u32(tiles);
+		if (lane == 63)
+			s_tiles[wave] = tiles;
 		uint32_t at = block_exclusive_scan_u32<kWaves>(mine, s_scan, n);
+		if (tid == 0 && j.totals.total_out) {
+			uint32_t total = 0;
+#pragma unroll
+			for (int w = 0; w < kWaves; w++)
+				total += s_tiles[w];
+			if (j.totals.total_copy)
+				__hip_atomic_store(j.totals.total_copy, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);  // (the host waits for this word)
+			*j.totals.total_out = total;
+			*j.totals.visible_count = n;
+		}
 #pragma unroll
 		for (int q = 0; q < kItems; q++)
 			if (__float_as_uint(depth[q]) != 0u) {
@@ -1400,7 +1418,6 @@ __global__ __launch_bounds__(1024) void small_depth_order_kernel(Batch<DepthOrde
 
 // A call's images from the Gaussians, general path and this, us: 4 000 Gaussians at 160x120 111 and 87, 8 000 114 and 99, 8 000 at 800x600
 // 147 and 132; with sixteen per thread 12 000 at 320x240 121 and 122, 16 000 122 and 129.
-constexpr int kSmallOrder = 8192;
 
 static void launch_small_depth_order(const Batch<DepthOrderJob>& b, int jobs, int most, hipStream_t s)
 {

@@ -465,8 +465,10 @@ struct DepthOrderJob {
 	uint32_t* dup_first;       // dup_first_words(P) words: see launch_duplicate_with_keys
 	uint32_t* digits;          // kDigitCopies x kDigitWords words, zero beforehand and left zero: see also DuplicateJob
 	uint32_t digit_copies;     // how many of the copies the launch uses: it sets this itself
+	TotalsJob totals;          // of jobs of up to kSmallOrder Gaussians: with a total_out, the launch makes the totals too (no launch_totals_from_block_sums)
 };
 void launch_depth_order(const DepthOrderJob* jobs, int count, hipStream_t s);
+constexpr int kSmallOrder = 8192;  // Gaussians that one workgroup puts in order
 // Also sets clear[0..clear_words) to zero (the scratch of the sort that follows).  Instances whose
 // position is `capacity` or more are not written.
 // Output positions a workgroup of the key duplication writes, and the table that tells each such workgroup at
