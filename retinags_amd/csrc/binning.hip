@@ -629,7 +629,7 @@ __global__ __launch_bounds__(256) void duplicate_with_keys_kernel(Batch<Duplicat
 			// t / w through the reciprocal in single precision (both are below 2^24, so exact as floats; the quotient
 			// is off by one at most, which the remainder shows): a third of the instructions of the integer division
 			uint32_t row = (uint32_t)((float)t * __builtin_amdgcn_rcpf((float)w));
-			int col = (int)(t - row * w);
+			int col = (int)(t - __umul24(row, w));
 			if (col < 0) {
 				row--;
 				col += (int)w;

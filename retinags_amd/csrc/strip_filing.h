@@ -179,14 +179,15 @@ __device__ __forceinline__ uint32_t strips_filed_for(const StripTests& t, float 
 		dy_high = ((!(-bY < first) & !(-bY > last)) ? Y : top) + margin;
 		dy_low = ((!(bY < first) & !(bY > last)) ? -Y : bottom) - margin;
 	}
-	// Which strips the entry reaches, without a branch: all four are answered by comparisons and lane masks.  Of a tile inside the box
-	// that is all.
+	// Which strips the entry reaches, without a branch: all four are answered by two comparisons each and lane masks (four against each of
+	// the ends, with their differences, took 19 instructions more: 621 -> 606 us at 5185x3359, 185 -> 181 for four calls at 1600x1036).  Of a
+	// tile inside the box that is all.
 	uint32_t bits = 0;
+	const float cy = t.gy - y0;
+	const float top = fminf(cy + t.hy, cy - dy_low), bottom = fmaxf(cy - t.hy, cy - dy_high);  // the last and first row it reaches, from y0
 #pragma unroll
 	for (int s = 0; s < 4; s++) {
-		const float ya = y0 + (float)(4 * s);
-		const float dyl = t.gy - (ya + 3.f), dyh = t.gy - ya;
-		const bool beside = (t.gy + t.hy < ya) | (t.gy - t.hy > ya + 3.f) | (dyh < dy_low) | (dyl > dy_high);
+		const bool beside = (top < (float)(4 * s)) | (bottom > (float)(4 * s + 3));
 		bits |= beside ? 0u : 0x11u << s;
 	}
 	if (!tile_inside) {
