@@ -323,8 +323,8 @@ def measure(args, config, forward_only, asides, cpu, apart_too=False, morton_too
     K = len(related)
     T = ((W + 15) // 16) * ((H + 15) // 16)
     N = W * H
-    tile_bits = int(_capi.lib.rgs_get_higher_msb(T))
-    passes = min((tile_bits + 8) // 9, (tile_bits + 7) // 8)   # of the instance sort, on the tile key: digits of up to 9 bits
+    tile_bits = int(_capi.lib.rgs_get_higher_msb(max(T - 1, 1)))
+    passes = 1 if tile_bits <= 11 else (tile_bits + 8) // 9   # of the instance sort, on the tile key: one digit of up to 11 bits, or several of up to 9
     # The backward revisits, per pixel, the entries up to the last blended one: nAl of the nA visits.  These are the visits of
     # the reference's loop, which looks at every entry of a tile's list in every pixel; the kernels here leave out most of those
     # that blend nothing.  So achieved_TFLOPs of the blends is the rate at which that loop's work gets done, and not that of the
@@ -364,7 +364,7 @@ def measure(args, config, forward_only, asides, cpu, apart_too=False, morton_too
     # preprocess writes the rendered rows only, into arrays its caller has cleared (4 P + 559 P_vis, or with that clearing
     # 304 P more); here every row of the dense outputs is written once, zeros included.  The reference sorts 12-byte pairs
     # on (tile << 32 | depth) in ceil((32 + bits) / 8) passes after one read of the keys (R (8 + 24 p)); here the instances
-    # are emitted in depth order and sorted on the tile alone, 8-byte pairs, ceil(bits / 8) passes.
+    # are emitted in depth order and sorted on the tile alone, 8-byte pairs, `passes` passes.
     ref_passes = (32 + int(_capi.lib.rgs_get_higher_msb(T)) + 7) // 8
     reference_design_bytes = {
         "preprocess_backward": {"rendered_rows_only": 4.0 * P_tot + 559.0 * P_vis,
@@ -617,9 +617,10 @@ def whole_iteration(scene, part, cam_d, rel, bg, streams, dev, repeats):
            "activation_tensor_expression_wall_ms": round(_timed_ms(activations_by_tensor_expressions, repeats), 3),
            "steps": f"activate, select + merge straddlers (appended), render + composite, L1+SSIM loss, backward, "
                     f"Adam ({7 * len(models)} tensors)"}
-    # algorithmic bytes: 224 in + 224 out per Gaussian forward (56 floats: SH, scale, rotation, opacity);
-    # backward reads their gradients, the stored rotation and the activated scale / opacity, writes 224
-    for name, per_gaussian in (("activate_forward", 448.0), ("activate_backward", 224.0 + 32.0 + 224.0)):
+    # algorithmic bytes (the SH rows stay where they are stored): forward 8 floats in (scale, rotation, opacity), 8 and the 3 zeros
+    # of the screen-space placeholder out; backward the gradients of those 11 in (8 bytes of the placeholder's 12), the stored
+    # rotation, the activated scale and opacity in, 9 floats out
+    for name, per_gaussian in (("activate_forward", 4.0 * 19), ("activate_backward", 4.0 * (10 + 8 + 9))):
         if name in stage and stage[name][0] > 0:
             t = stage[name][0]
             out[name] = {"ms_per_iteration": round(t, 4), "launches": stage[name][1],
