@@ -17,20 +17,26 @@ inline void expect_counts(uint32_t* words, int n)
 // Until a kernel on `s` has written all of words[0..n), which expect_counts set before it was launched.  A copy to the host and an
 // event behind it put two launches between that kernel and the next one of the stream and as many into the host's path: polled, a call takes
 // 4 us less (4 000 Gaussians at 160x120 88 -> 84 us, 100 000 at 512x512 150 -> 146).  The stream is asked now and then, so that a kernel that
-// never wrote them (a failed launch, a stream under capture) ends the wait, with the stream's error if it has one.
+// never wrote them (a failed launch, a stream under capture) ends the wait with an error, the stream's if it has one.
 inline hipError_t wait_for_counts(const uint32_t* words, int n, hipStream_t s)
 {
+	bool done = false;  // the stream has nothing left that could write them
 	for (uint32_t polls = 1;; polls++) {
 		int k = 0;
 		while (k < n && __atomic_load_n(&words[k], __ATOMIC_ACQUIRE) != kNoCount)
 			k++;
 		if (k == n)
 			return hipSuccess;
+		if (done)
+			return hipErrorLaunchFailure;
 		if (polls % 65536u == 0u) {
 			const hipError_t e = hipStreamQuery(s);
-			if (e != hipErrorNotReady)
+			if (e == hipErrorNotReady)
+				(void)hipGetLastError();  // not there yet: no error of the caller's
+			else if (e != hipSuccess)
 				return e;
-			(void)hipGetLastError();  // not there yet: no error of the caller's
+			else
+				done = true;
 		}
 		__builtin_ia32_pause();
 	}
