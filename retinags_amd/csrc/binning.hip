@@ -311,62 +311,63 @@ __global__ __launch_bounds__(256) void depth_pairs_kernel(Batch<DepthOrderJob> b
 	__syncthreads();
 	uint32_t written = 0;
 	// How many of a group's Gaussians are listed is known ahead of it.  Where neighbours in memory are neighbours in the scene most
-	// groups have none (a city stored along a space-filling curve, 5 % in view: 39.5 -> 29 us; 62.9 M Gaussians in random order 124 -> 101; both before the digit counts had copies), so a workgroup with many groups
-	// looks for those that have some, 64 at a time; one with few would only wait for the answer.
+	// groups have none (a city stored along a space-filling curve, 5 % in view: 39.5 -> 29 us; 62.9 M Gaussians in random order
+	// 124 -> 101; both before the digit counts had copies), so a workgroup with many groups looks for those that have some, 64 at a
+	// time; one with few would only wait for the answer.
 	const size_t blocks = (P + 255) / 256, groups = (P + kScanGroup - 1) / kScanGroup;
 	const bool many = groups > 4 * (size_t)gridDim.x;
 	auto listed_up_to = [&](size_t group) { return 4 * group < blocks ? visible_base[4 * group] : *j.visible_count; };
 	for (size_t ahead = blockIdx.x; ahead < groups; ahead += 64 * (size_t)gridDim.x) {
-	const size_t looked_at = ahead + (size_t)(threadIdx.x & 63) * gridDim.x;
-	uint32_t base = 0u;
-	bool some = looked_at < groups;
-	if (some) {
-		base = listed_up_to(looked_at);
-		if (many)
-			some = base != listed_up_to(looked_at + 1);
-	}
-	for (uint64_t todo = lanes_where(some); todo != 0ull; todo &= todo - 1ull) {  // (the same in every wavefront of the workgroup)
-		const int which = __builtin_ctzll(todo);
-		const size_t group = ahead + (size_t)which * gridDim.x;
-		const size_t idx0 = group * kScanGroup + 4 * (size_t)threadIdx.x;
-		// the depth of a Gaussian that touches no tile is stored as 0, that of one that does exceeds 0.2: the
-		// depths alone say which ones are listed
-		float depth[4] = {0.f, 0.f, 0.f, 0.f};
-		uint32_t count[4] = {0u, 0u, 0u, 0u};
-		if (idx0 + 4 <= P) {
-			const float4 d4 = *reinterpret_cast<const float4*>(depths + idx0);
-			const uint4 c4 = *reinterpret_cast<const uint4*>(tiles_touched + idx0);
-			depth[0] = d4.x; depth[1] = d4.y; depth[2] = d4.z; depth[3] = d4.w;
-			count[0] = c4.x; count[1] = c4.y; count[2] = c4.z; count[3] = c4.w;
-		} else {
+		const size_t looked_at = ahead + (size_t)(threadIdx.x & 63) * gridDim.x;
+		uint32_t base = 0u;
+		bool some = looked_at < groups;
+		if (some) {
+			base = listed_up_to(looked_at);
+			if (many)
+				some = base != listed_up_to(looked_at + 1);
+		}
+		for (uint64_t todo = lanes_where(some); todo != 0ull; todo &= todo - 1ull) {  // (the same in every wavefront of the workgroup)
+			const int which = __builtin_ctzll(todo);
+			const size_t group = ahead + (size_t)which * gridDim.x;
+			const size_t idx0 = group * kScanGroup + 4 * (size_t)threadIdx.x;
+			// the depth of a Gaussian that touches no tile is stored as 0, that of one that does exceeds 0.2: the
+			// depths alone say which ones are listed
+			float depth[4] = {0.f, 0.f, 0.f, 0.f};
+			uint32_t count[4] = {0u, 0u, 0u, 0u};
+			if (idx0 + 4 <= P) {
+				const float4 d4 = *reinterpret_cast<const float4*>(depths + idx0);
+				const uint4 c4 = *reinterpret_cast<const uint4*>(tiles_touched + idx0);
+				depth[0] = d4.x; depth[1] = d4.y; depth[2] = d4.z; depth[3] = d4.w;
+				count[0] = c4.x; count[1] = c4.y; count[2] = c4.z; count[3] = c4.w;
+			} else {
+#pragma unroll
+				for (int q = 0; q < 4; q++)
+					if (idx0 + q < P) {
+						depth[q] = depths[idx0 + q];
+						count[q] = tiles_touched[idx0 + q];
+					}
+			}
+			uint32_t mine = 0;
 #pragma unroll
 			for (int q = 0; q < 4; q++)
-				if (idx0 + q < P) {
-					depth[q] = depths[idx0 + q];
-					count[q] = tiles_touched[idx0 + q];
+				mine += __float_as_uint(depth[q]) != 0u ? 1u : 0u;
+			uint32_t total;
+			uint32_t at = (uint32_t)__builtin_amdgcn_readlane((int)base, which) + block256_exclusive_scan_u32(mine, lds, total);
+			written += mine;
+#pragma unroll
+			for (int q = 0; q < 4; q++)
+				if (__float_as_uint(depth[q]) != 0u) {
+					const uint32_t key = __float_as_uint(depth[q]) - kDepthKeyBase;
+					keys[at] = key;
+					values[at] = (uint32_t)(idx0 + q) | (min(count[q], cap) << index_bits);
+					at++;
+#pragma unroll
+					for (int p = 0; p < kDepthPasses; p++)
+						atomicAdd(&s_hist[p][(key >> (9 * p)) & 511u], 1u);
+					if (key >> kDepthKeyBits)
+						atomicAdd(&s_top[key >> kDepthKeyBits], 1u);
 				}
 		}
-		uint32_t mine = 0;
-#pragma unroll
-		for (int q = 0; q < 4; q++)
-			mine += __float_as_uint(depth[q]) != 0u ? 1u : 0u;
-		uint32_t total;
-		uint32_t at = (uint32_t)__builtin_amdgcn_readlane((int)base, which) + block256_exclusive_scan_u32(mine, lds, total);
-		written += mine;
-#pragma unroll
-		for (int q = 0; q < 4; q++)
-			if (__float_as_uint(depth[q]) != 0u) {
-				const uint32_t key = __float_as_uint(depth[q]) - kDepthKeyBase;
-				keys[at] = key;
-				values[at] = (uint32_t)(idx0 + q) | (min(count[q], cap) << index_bits);
-				at++;
-#pragma unroll
-				for (int p = 0; p < kDepthPasses; p++)
-					atomicAdd(&s_hist[p][(key >> (9 * p)) & 511u], 1u);
-				if (key >> kDepthKeyBits)
-					atomicAdd(&s_top[key >> kDepthKeyBits], 1u);
-			}
-	}
 	}
 	__syncthreads();
 	uint32_t* digits = j.digits + (blockIdx.x & (j.digit_copies - 1u)) * kDigitWords;
@@ -525,155 +526,155 @@ __global__ __launch_bounds__(256) void duplicate_with_keys_kernel(Batch<Duplicat
 	if (blockIdx.x < table_runs)
 		ask_for(blockIdx.x);
 	for (uint32_t run = blockIdx.x; (uint64_t)run * kDupPositions < (uint64_t)limit; run += gridDim.x) {
-	const uint32_t start = run * (uint32_t)kDupPositions;
-	const uint32_t stop = min(start + (uint32_t)kDupPositions, limit);
-	__syncthreads();  // the previous run is done with s_first and the staged Gaussians; the tables are written
-	uint32_t staged_begin, own_end;
-	if (ahead) {
-		own_end = ahead_end;
-		st.index[tid] = ahead_index;
-		staged_begin = ahead_begin;
-	} else {
-		// beyond the table (more than 16 instances per Gaussian on average): the first Gaussian whose inclusive offset
-		// exceeds `start` by a 64-ary search of the first wavefront
-		if (tid < 64) {
-			uint32_t lo = 0, hi = n;  // the answer lies in [lo, hi]
-			while (lo < hi) {
-				const uint32_t step = (hi - lo + 63u) / 64u;
-				const uint32_t probe = lo + (uint32_t)lane * step;
-				const bool below = probe < hi && offsets[probe] <= start;
-				const uint32_t c = (uint32_t)__popcll(lanes_where(below));  // the predicate is monotone: the first c probes hold
-				if (c == 0u) {
-					hi = lo;
-				} else {
-					const uint32_t last_true = lo + (c - 1u) * step;
-					lo = last_true + 1u;
-					hi = min(last_true + step, hi);
-				}
-			}
-			if (lane == 0)
-				s_first = min(lo, n - 1u);
-		}
-		__syncthreads();
-		const uint32_t g0 = s_first, g = g0 + (uint32_t)tid;
-		own_end = g < n ? offsets[g] : total;
-		st.index[tid] = g < n ? min(order[g], P - 1u) : 0u;
-		staged_begin = g0 == 0u ? 0u : offsets[g0 - 1];
-	}
-	st.end[tid] = own_end;
-	const uint32_t next_begins = own_end - start;
-	if (next_begins - 1u < 255u)
-		atomicOr(&st.begins[which][next_begins >> 5], 1u << (next_begins & 31u));
-	__syncthreads();
-	ahead = false;
-	if (tid < 8)
-		st.begins[which ^ 1][tid] = 0u;
-	if ((uint64_t)(run + gridDim.x) * kDupPositions < (uint64_t)limit && run + gridDim.x < table_runs)
-		ask_for(run + gridDim.x);
-
-	{
-		const uint32_t staged_end = st.end[255];
-		const uint32_t from = max(start, staged_begin), to = min(stop, staged_end);
-		// Up to kDupPositions / 256 positions per thread.  First all of them find their Gaussian and ask for its
-		// record (pixel centre, conic, extents, radius: everything else follows from those), then each is finished:
-		// the records of a thread arrive together, not one wait after another.
-		constexpr int kPerThread = kDupPositions / 256;
-		static_assert(kPerThread == 1, "a bit per thread");
-		// The staged Gaussian of a position: as many as have begun up to it since the run's first (every listed one has an instance).
-		// One read of the bits and a count where a binary search took eight reads in LDS, each after the one before: 611 -> 587 us for
-		// 62.9 M Gaussians, where most have an instance or two; nothing where they have many.
-		const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-		uint32_t begun = 0, own_lo = 0, own_hi = 0;
-		{
-			const uint4 m0 = *reinterpret_cast<const uint4*>(&st.begins[which][0]), m1 = *reinterpret_cast<const uint4*>(&st.begins[which][4]);
-			const uint32_t m[8] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
-			which ^= 1;
-#pragma unroll
-			for (int w = 0; w < 4; w++) {
-				const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)m[2 * w]), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)m[2 * w + 1]);
-				begun += w < wave ? (uint32_t)(__popc(lo) + __popc(hi)) : 0u;
-				own_lo = w == wave ? lo : own_lo;
-				own_hi = w == wave ? hi : own_hi;
-			}
-			// (a lane counts the bits below its own: its own bit is shifted down to be one of them)
-			begun += own_lo & 1u;
-			own_lo = own_lo >> 1 | own_hi << 31;
-			own_hi >>= 1;
-		}
-		uint32_t first[kPerThread], index[kPerThread];
-		float4 r0[kPerThread], r1[kPerThread], r3[kPerThread];
-#pragma unroll
-		for (int q = 0; q < kPerThread; q++) {
-			const uint32_t pos = from + (uint32_t)tid + 256u * (uint32_t)q;
-			first[q] = 0u;
-			index[q] = 0u;
-			if (pos < to) {
-				const int lo = (int)(begun + __builtin_amdgcn_mbcnt_hi(own_hi, __builtin_amdgcn_mbcnt_lo(own_lo, 0u)));
-				first[q] = lo == 0 ? staged_begin : min(st.end[lo - 1], pos);
-				index[q] = st.index[lo];
-				const float4* rec = filing.record + 4 * (size_t)index[q];
-				r0[q] = rec[0];
-				r1[q] = rec[1];
-				r3[q] = rec[3];
-			}
-		}
-		uint32_t tile_of[kPerThread];
-#pragma unroll
-		for (int q = 0; q < kPerThread; q++) {
-			const uint32_t pos = from + (uint32_t)tid + 256u * (uint32_t)q;
-			tile_of[q] = 0xFFFFFFFFu;
-			if (pos >= to)
-				continue;
-			const TileRect rc = tile_rect(r0[q].x, r0[q].y, __float_as_int(r3[q].z), gx, gy);
-			const uint32_t t = pos - first[q], w = max(rc.x1 - rc.x0, 1u);
-			// t / w through the reciprocal in single precision (both are below 2^24, so exact as floats; the quotient
-			// is off by one at most, which the remainder shows): a third of the instructions of the integer division
-			uint32_t row = (uint32_t)((float)t * __builtin_amdgcn_rcpf((float)w));
-			int col = (int)(t - __umul24(row, w));
-			if (col < 0) {
-				row--;
-				col += (int)w;
-			} else if (col >= (int)w) {
-				row++;
-				col -= (int)w;
-			}
-			const int tx = (int)rc.x0 + col, ty = (int)(rc.y0 + row);
-			const uint32_t tile = (uint32_t)ty * (uint32_t)gx + (uint32_t)tx;
-			float nx, ny;
-			if (ndc_in_lds) {
-				nx = s_ndc[tx];
-				ny = s_ndc[gx + ty];
-			} else {
-				nx = tile_middle_ndc(tx, filing.W);
-				ny = tile_middle_ndc(ty, filing.H);
-			}
-			const StripTests tests = prepare_strip_tests(FiledGeometry{r0[q], r1[q], float2{r3[q].x, r3[q].y}}, box);
-			const uint32_t strips = strips_filed_for(tests, (float)(tx * kTile), (float)(ty * kTile), nx, ny, steps, box);
-			keys[pos] = tile | (strips << kKeyTileBits);
-			values[pos] = index[q];
-			tile_of[q] = tile;
-		}
-		// the digits of the tiles just written, for the sort (every lane comes here: the narrow digits are counted by ballot)
-#pragma unroll
-		for (int q = 0; q < kPerThread; q++) {
-			const bool have = tile_of[q] != 0xFFFFFFFFu;
-			for (int p = 0; p < passes; p++) {
-				const int shift = sort_digit_shift(job.end_bit, p, digit_bits);
-				const int bits = sort_digit_bits(job.end_bit, p, digit_bits);
-				const uint32_t d = (tile_of[q] >> shift) & ((1u << bits) - 1u);
-				if (bits <= 2) {
-					// a digit of one or two bits: every lane would add to one of a few words, one after the other
-					for (uint32_t v = 0; v < (1u << bits); v++) {
-						const uint32_t c = (uint32_t)__popcll(lanes_where(have && d == v));
-						if (lane == 0 && c != 0u)
-							atomicAdd(&s_digits[512 * p + v], c);
+		const uint32_t start = run * (uint32_t)kDupPositions;
+		const uint32_t stop = min(start + (uint32_t)kDupPositions, limit);
+		__syncthreads();  // the previous run is done with s_first and the staged Gaussians; the tables are written
+		uint32_t staged_begin, own_end;
+		if (ahead) {
+			own_end = ahead_end;
+			st.index[tid] = ahead_index;
+			staged_begin = ahead_begin;
+		} else {
+			// beyond the table (more than 16 instances per Gaussian on average): the first Gaussian whose inclusive offset
+			// exceeds `start` by a 64-ary search of the first wavefront
+			if (tid < 64) {
+				uint32_t lo = 0, hi = n;  // the answer lies in [lo, hi]
+				while (lo < hi) {
+					const uint32_t step = (hi - lo + 63u) / 64u;
+					const uint32_t probe = lo + (uint32_t)lane * step;
+					const bool below = probe < hi && offsets[probe] <= start;
+					const uint32_t c = (uint32_t)__popcll(lanes_where(below));  // the predicate is monotone: the first c probes hold
+					if (c == 0u) {
+						hi = lo;
+					} else {
+						const uint32_t last_true = lo + (c - 1u) * step;
+						lo = last_true + 1u;
+						hi = min(last_true + step, hi);
 					}
-				} else if (have) {
-					atomicAdd(&s_digits[512 * p + d], 1u);
+				}
+				if (lane == 0)
+					s_first = min(lo, n - 1u);
+			}
+			__syncthreads();
+			const uint32_t g0 = s_first, g = g0 + (uint32_t)tid;
+			own_end = g < n ? offsets[g] : total;
+			st.index[tid] = g < n ? min(order[g], P - 1u) : 0u;
+			staged_begin = g0 == 0u ? 0u : offsets[g0 - 1];
+		}
+		st.end[tid] = own_end;
+		const uint32_t next_begins = own_end - start;
+		if (next_begins - 1u < 255u)
+			atomicOr(&st.begins[which][next_begins >> 5], 1u << (next_begins & 31u));
+		__syncthreads();
+		ahead = false;
+		if (tid < 8)
+			st.begins[which ^ 1][tid] = 0u;
+		if ((uint64_t)(run + gridDim.x) * kDupPositions < (uint64_t)limit && run + gridDim.x < table_runs)
+			ask_for(run + gridDim.x);
+
+		{
+			const uint32_t staged_end = st.end[255];
+			const uint32_t from = max(start, staged_begin), to = min(stop, staged_end);
+			// Up to kDupPositions / 256 positions per thread.  First all of them find their Gaussian and ask for its
+			// record (pixel centre, conic, extents, radius: everything else follows from those), then each is finished:
+			// the records of a thread arrive together, not one wait after another.
+			constexpr int kPerThread = kDupPositions / 256;
+			static_assert(kPerThread == 1, "a bit per thread");
+			// The staged Gaussian of a position: as many as have begun up to it since the run's first (every listed one has an instance).
+			// One read of the bits and a count where a binary search took eight reads in LDS, each after the one before: 611 -> 587 us for
+			// 62.9 M Gaussians, where most have an instance or two; nothing where they have many.
+			const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+			uint32_t begun = 0, own_lo = 0, own_hi = 0;
+			{
+				const uint4 m0 = *reinterpret_cast<const uint4*>(&st.begins[which][0]), m1 = *reinterpret_cast<const uint4*>(&st.begins[which][4]);
+				const uint32_t m[8] = {m0.x, m0.y, m0.z, m0.w, m1.x, m1.y, m1.z, m1.w};
+				which ^= 1;
+#pragma unroll
+				for (int w = 0; w < 4; w++) {
+					const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)m[2 * w]), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)m[2 * w + 1]);
+					begun += w < wave ? (uint32_t)(__popc(lo) + __popc(hi)) : 0u;
+					own_lo = w == wave ? lo : own_lo;
+					own_hi = w == wave ? hi : own_hi;
+				}
+				// (a lane counts the bits below its own: its own bit is shifted down to be one of them)
+				begun += own_lo & 1u;
+				own_lo = own_lo >> 1 | own_hi << 31;
+				own_hi >>= 1;
+			}
+			uint32_t first[kPerThread], index[kPerThread];
+			float4 r0[kPerThread], r1[kPerThread], r3[kPerThread];
+#pragma unroll
+			for (int q = 0; q < kPerThread; q++) {
+				const uint32_t pos = from + (uint32_t)tid + 256u * (uint32_t)q;
+				first[q] = 0u;
+				index[q] = 0u;
+				if (pos < to) {
+					const int lo = (int)(begun + __builtin_amdgcn_mbcnt_hi(own_hi, __builtin_amdgcn_mbcnt_lo(own_lo, 0u)));
+					first[q] = lo == 0 ? staged_begin : min(st.end[lo - 1], pos);
+					index[q] = st.index[lo];
+					const float4* rec = filing.record + 4 * (size_t)index[q];
+					r0[q] = rec[0];
+					r1[q] = rec[1];
+					r3[q] = rec[3];
+				}
+			}
+			uint32_t tile_of[kPerThread];
+#pragma unroll
+			for (int q = 0; q < kPerThread; q++) {
+				const uint32_t pos = from + (uint32_t)tid + 256u * (uint32_t)q;
+				tile_of[q] = 0xFFFFFFFFu;
+				if (pos >= to)
+					continue;
+				const TileRect rc = tile_rect(r0[q].x, r0[q].y, __float_as_int(r3[q].z), gx, gy);
+				const uint32_t t = pos - first[q], w = max(rc.x1 - rc.x0, 1u);
+				// t / w through the reciprocal in single precision (both are below 2^24, so exact as floats; the quotient
+				// is off by one at most, which the remainder shows): a third of the instructions of the integer division
+				uint32_t row = (uint32_t)((float)t * __builtin_amdgcn_rcpf((float)w));
+				int col = (int)(t - __umul24(row, w));
+				if (col < 0) {
+					row--;
+					col += (int)w;
+				} else if (col >= (int)w) {
+					row++;
+					col -= (int)w;
+				}
+				const int tx = (int)rc.x0 + col, ty = (int)(rc.y0 + row);
+				const uint32_t tile = (uint32_t)ty * (uint32_t)gx + (uint32_t)tx;
+				float nx, ny;
+				if (ndc_in_lds) {
+					nx = s_ndc[tx];
+					ny = s_ndc[gx + ty];
+				} else {
+					nx = tile_middle_ndc(tx, filing.W);
+					ny = tile_middle_ndc(ty, filing.H);
+				}
+				const StripTests tests = prepare_strip_tests(FiledGeometry{r0[q], r1[q], float2{r3[q].x, r3[q].y}}, box);
+				const uint32_t strips = strips_filed_for(tests, (float)(tx * kTile), (float)(ty * kTile), nx, ny, steps, box);
+				keys[pos] = tile | (strips << kKeyTileBits);
+				values[pos] = index[q];
+				tile_of[q] = tile;
+			}
+			// the digits of the tiles just written, for the sort (every lane comes here: the narrow digits are counted by ballot)
+#pragma unroll
+			for (int q = 0; q < kPerThread; q++) {
+				const bool have = tile_of[q] != 0xFFFFFFFFu;
+				for (int p = 0; p < passes; p++) {
+					const int shift = sort_digit_shift(job.end_bit, p, digit_bits);
+					const int bits = sort_digit_bits(job.end_bit, p, digit_bits);
+					const uint32_t d = (tile_of[q] >> shift) & ((1u << bits) - 1u);
+					if (bits <= 2) {
+						// a digit of one or two bits: every lane would add to one of a few words, one after the other
+						for (uint32_t v = 0; v < (1u << bits); v++) {
+							const uint32_t c = (uint32_t)__popcll(lanes_where(have && d == v));
+							if (lane == 0 && c != 0u)
+								atomicAdd(&s_digits[512 * p + v], c);
+						}
+					} else if (have) {
+						atomicAdd(&s_digits[512 * p + d], 1u);
+					}
 				}
 			}
 		}
-	}
 	}
 	__syncthreads();
 	for (int w = tid; w < (passes == 1 ? 1 << job.end_bit : 512 * passes); w += 256) {
@@ -1612,52 +1613,52 @@ __global__ __launch_bounds__(kFileBlock) void tile_ranges_kernel(Batch<TileRange
 		return;
 	}
 	for (const size_t step = (size_t)gridDim.x * kFileGroup; first < n; first += step) {
-	const size_t idx0 = first + 4 * (size_t)threadIdx.x;
-	const uint32_t key[4] = {ahead[0], ahead[1], ahead[2], ahead[3]};
-	const uint32_t lane_before = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key[3], 0x138, 0xF, 0xF, false);  // (wave_shr:1)
-	uint32_t prev = key_tile(lane == 0 ? ahead_prev : lane_before);
-	if (first + step < n)
-		ask_for(first + step);
-	const size_t last = min(n, first + kFileGroup) - 1;
+		const size_t idx0 = first + 4 * (size_t)threadIdx.x;
+		const uint32_t key[4] = {ahead[0], ahead[1], ahead[2], ahead[3]};
+		const uint32_t lane_before = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key[3], 0x138, 0xF, 0xF, false);  // (wave_shr:1)
+		uint32_t prev = key_tile(lane == 0 ? ahead_prev : lane_before);
+		if (first + step < n)
+			ask_for(first + step);
+		const size_t last = min(n, first + kFileGroup) - 1;
 #pragma unroll
-	for (int q = 0; q < 4; q++) {
-		const size_t idx = idx0 + q;
-		const uint32_t cur = key_tile(key[q]);
-		if (idx < n) {
-			if (idx == 0) {
-				ranges[cur].x = 0;
-			} else if (cur != prev) {
-				ranges[prev].y = (uint32_t)idx;
-				ranges[cur].x = (uint32_t)idx;
+		for (int q = 0; q < 4; q++) {
+			const size_t idx = idx0 + q;
+			const uint32_t cur = key_tile(key[q]);
+			if (idx < n) {
+				if (idx == 0) {
+					ranges[cur].x = 0;
+				} else if (cur != prev) {
+					ranges[prev].y = (uint32_t)idx;
+					ranges[cur].x = (uint32_t)idx;
+				}
+				if (idx == n - 1)
+					ranges[cur].y = (uint32_t)n;
+				if (idx == last)
+					s_last_tile = cur;
 			}
-			if (idx == n - 1)
-				ranges[cur].y = (uint32_t)n;
-			if (idx == last)
-				s_last_tile = cur;
+			prev = cur;
 		}
-		prev = cur;
-	}
-	if (!file_tail)
-		continue;
-	__syncthreads();
-	const uint32_t last_tile = s_last_tile;
-	uint2 own = {0u, 0u};
+		if (!file_tail)
+			continue;
+		__syncthreads();
+		const uint32_t last_tile = s_last_tile;
+		uint2 own = {0u, 0u};
 #pragma unroll
-	for (int q = 0; q < 4; q++)
-		if (idx0 + q < n && key_tile(key[q]) == last_tile) {  // sorted: these are the workgroup's last keys
-			const uint32_t bits = key_strips(key[q]);
-			own.x += (bits & 1u) | ((bits & 2u) << 15);
-			own.y += ((bits >> 2) & 1u) | ((bits & 8u) << 13);
+		for (int q = 0; q < 4; q++)
+			if (idx0 + q < n && key_tile(key[q]) == last_tile) {  // sorted: these are the workgroup's last keys
+				const uint32_t bits = key_strips(key[q]);
+				own.x += (bits & 1u) | ((bits & 2u) << 15);
+				own.y += ((bits >> 2) & 1u) | ((bits & 8u) << 13);
+			}
+		const uint2 inc = {wave_inclusive_scan_u32(own.x), wave_inclusive_scan_u32(own.y)};
+		if (lane == 63)
+			s_tail[wave] = inc;
+		__syncthreads();
+		if (threadIdx.x == 0) {
+			const uint32_t x = s_tail[0].x + s_tail[1].x + s_tail[2].x + s_tail[3].x;
+			const uint32_t y = s_tail[0].y + s_tail[1].y + s_tail[2].y + s_tail[3].y;
+			file_tail[first / kFileGroup] = uint4{x & 0xFFFFu, x >> 16, y & 0xFFFFu, y >> 16};
 		}
-	const uint2 inc = {wave_inclusive_scan_u32(own.x), wave_inclusive_scan_u32(own.y)};
-	if (lane == 63)
-		s_tail[wave] = inc;
-	__syncthreads();
-	if (threadIdx.x == 0) {
-		const uint32_t x = s_tail[0].x + s_tail[1].x + s_tail[2].x + s_tail[3].x;
-		const uint32_t y = s_tail[0].y + s_tail[1].y + s_tail[2].y + s_tail[3].y;
-		file_tail[first / kFileGroup] = uint4{x & 0xFFFFu, x >> 16, y & 0xFFFFu, y >> 16};
-	}
 	}
 }
 
